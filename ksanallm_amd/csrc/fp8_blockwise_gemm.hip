@@ -329,9 +329,10 @@ int launch_fp8_tile(const Fp8Params& q, const TilePlan& plan, float* partial, hi
 template <typename TO, int WM>
 int launch_fp8_tile_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s) {
   constexpr int kLdsMax = 160 * 1024;
-  // (the 256-slot kernel runs half-empty blocks on the 128-token tile's three stages)
-  const size_t lds = WM == 8 ? std::max(fp8_tile_lds_bytes(8, q.K / 128), fp8_tile_lds_bytes(4, q.K / 128))
-                             : fp8_tile_lds_bytes(WM, q.K / 128);
+  // (the 256-slot kernel runs blocks of at most 160 tokens on three stages, as long as K <= 28672 leaves room for them)
+  const size_t deep_lds = fp8_tile_lds_bytes(5, q.K / 128);
+  const bool deep = WM == 8 && deep_lds <= kLdsMax;
+  const size_t lds = deep ? std::max(fp8_tile_lds_bytes(WM, q.K / 128), deep_lds) : fp8_tile_lds_bytes(WM, q.K / 128);
   if (lds > kLdsMax) return fail(KSQ_ERR_UNSUPPORTED, "k range of %u blocks per workgroup does not fit the LDS", q.K / 128);
   // more dynamic LDS than a kernel may use without asking: once per device
   static std::atomic<uint64_t> configured{0};
@@ -359,6 +360,7 @@ int launch_fp8_tile_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s) 
   p.numel = q.numel;
   p.top_k = q.top_k;
   p.scale_rows = q.scale_rows;
+  p.deep_rows = deep ? 160 : 0;
   fp8_tile_kernel<TO, true, WM><<<p.tiles_m * p.tiles_n, 512, lds, s>>>(p);
   return KSQ_OK;
 }

@@ -40,6 +40,7 @@ struct Fp8TileParams {
   const int32_t* num_post_pad;
   const float* topk_w;
   uint32_t numel, top_k, scale_rows;  // scale_rows = ceil(N/128): rows of one expert's b_s
+  uint32_t deep_rows;                 // 256-slot blocks of at most this many slots run on the three-stage tile
 };
 
 __device__ __forceinline__ f32x4 mfma_fp8_k128(i32x8 a, i32x8 b, f32x4 c) {
@@ -51,27 +52,30 @@ __device__ __forceinline__ f32x4 mfma_fp8_k128(i32x8 a, i32x8 b, f32x4 c) {
 // expert_ids[tile_m], results go to out[s, :] (times topk_w[s] when given).  Blocks past num_post_pad leave at once;
 // there is no cut along K in this form.
 // WM = 8: 256-token tiles.  WM = 4: 128-token tiles (each wavefront 64 tokens x 64 weight rows) for row counts that
-// would leave half of a 256-token tile to padding; a stage then holds 8 activation fragments.
+// would leave half of a 256-token tile to padding; a stage then holds 8 activation fragments.  WM = 5: 160-token tiles,
+// the most that three stages leave room for.
 constexpr int fp8_tile_stage_bytes(int wm) { return (2 * wm + 16) * 2048; }
-// LDS stages: the 48 KiB stages of the 128-token tile fit three times, and need it - a stage of that tile is over in
-// less time than a load takes to come back
-constexpr int fp8_tile_stages(int wm) { return wm == 4 ? 3 : 2; }
+// LDS stages: the 48 KiB stages of the 128-token tile (52 KiB: 160 tokens) fit three times, and need it - a stage of
+// that tile is over in less time than a load takes to come back
+constexpr int fp8_tile_stages(int wm) { return wm <= 5 ? 3 : 2; }
+constexpr int fp8_tile_scale_bytes(int wm) { return wm == 5 ? 768 : 1024; }  // activation scales of a stage, 64 at a time
 constexpr size_t fp8_tile_lds_bytes(int wm, size_t kb_max) {
-  return static_cast<size_t>(fp8_tile_stages(wm)) * (fp8_tile_stage_bytes(wm) + 1024) + 2 * kb_max * 4;
+  return static_cast<size_t>(fp8_tile_stages(wm)) * (fp8_tile_stage_bytes(wm) + fp8_tile_scale_bytes(wm)) + 2 * kb_max * 4;
 }
 
 // BLOCK: slots between consecutive row blocks (tile_m * BLOCK is the block's first slot): the tile's own 32 * WM rows, or
-// - grouped form - 256 for a 128-token tile that serves a 256-slot block of which at most the lower half holds tokens.
+// - grouped form - 256 for a 160-token tile that serves a 256-slot block with at most 160 tokens.
 template <typename TO, bool GROUPED, int WM, int BLOCK>
 __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds) {
-  static_assert(WM == 8 || WM == 4, "256- or 128-token tiles");
-  static_assert(BLOCK == 2 * WM * 16 || (GROUPED && WM == 4 && BLOCK == 256), "block stride");
+  static_assert(WM == 8 || WM == 5 || WM == 4, "256-, 160- or 128-token tiles");
+  static_assert(BLOCK == 2 * WM * 16 || (GROUPED && WM == 5 && BLOCK == 256), "block stride");
   constexpr int WAVES_N = 4;
   constexpr int WN = 4;  // 16x16 tiles per wavefront: 16*WM tokens x 64 weight rows
   constexpr int BM = 2 * WM * 16, BN = 256;
   constexpr int FRAG = 2048;                  // bytes of one 16 x 128 operand fragment
   constexpr int AF = BM / 16;                 // activation fragments of a stage
-  constexpr int AFW = AF / 4;                 // ... fetched by each of the wavefronts 0..3
+  constexpr int BM_WAVES = (BM + 63) / 64;    // wavefronts that copy activation scales, 64 each
+  constexpr int AFW = AF / 4;                 // ... fetched by each of the wavefronts 0..3 (WM = 5: by halves, see below)
   constexpr int STAGE_BYTES = fp8_tile_stage_bytes(WM);  // AF activation + 16 weight fragments
   constexpr int W_FRAG0 = AF;                 // first weight fragment of a stage
   constexpr int NS = fp8_tile_stages(WM);     // LDS stages
@@ -119,16 +123,18 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
     }
     live_tiles = __builtin_amdgcn_readfirstlane((rows + 15) / 16);
   }
-  // The two wavefront rows split the block's row tiles: WM each - or, when at most WM of the 2 * WM hold tokens (a
-  // grouped block at most half full: an expert with half a block's slots), WM / 2 each of the lower WM, so that no SIMD
-  // is left with one working wavefront and one that only takes part in loads and barriers.
-  const bool lower_half = GROUPED && live_tiles <= WM;
-  const uint32_t per_wave = lower_half ? WM / 2 : WM;  // row tiles a wavefront covers
-  const uint32_t rt0 = wm * per_wave;                   // its first row tile
+  // The two wavefront rows share the row tiles that hold tokens evenly: no SIMD is left with one working wavefront and
+  // one that only takes part in loads and barriers (200 tokens: 7 and 6 row tiles, not 8 and 5).
+  const uint32_t per_wave = (live_tiles + 1) / 2;  // row tiles a wavefront covers
+  const uint32_t rt0 = wm * per_wave;              // its first row tile
   const uint32_t mine = live_tiles > rt0 ? (live_tiles - rt0 < per_wave ? live_tiles - rt0 : per_wave) : 0;
   const bool idle = mine == 0;  // none of this wavefront's row tiles holds a token
   const bool stage_act = wave < 4;
   const uint32_t frag0 = (wave & 3) * (stage_act ? AFW : 4);
+  // WM = 5: the halves of the activation fragments that hold tokens are dealt out, per_wave to each of wavefronts 0..3
+  // (4 * per_wave halves cover 2 * per_wave >= live_tiles fragments); the rest is not fetched
+  constexpr bool BY_HALVES = WM == 5;
+  const uint32_t half0 = (wave & 3) * per_wave;
   // Weights come as packed 2 KiB fragments (ksq_fp8_repack_weight), fragment (strip, k-block) at (strip*KB + kb)*2048:
   // a half of a fragment is one contiguous KiB, fetched by one load with lane j taking bytes 16j, and lands in LDS as
   // it lies in memory - MFMA lane l then reads 16 bytes at 16l of each half, consecutive lanes consecutive addresses,
@@ -140,9 +146,21 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   g_tile += static_cast<size_t>(kb_begin) * k_step;
   const uint32_t row_limit = p.M - m0;  // token rows of this tile inside the matrix
   uint32_t d_voff[4], d_voff_hi[4];     // per fragment: first load, and second load minus its instruction offset of 64
+  uint32_t h_voff[5];                   // WM = 5, activations: per half
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    h_voff[i] = 0;
+    if (BY_HALVES && stage_act) {
+      const uint32_t hh = half0 + i;  // half hh & 1 of fragment hh / 2
+      const uint32_t in_block = (hh / 2) * 16 + (lane >> 2);
+      uint32_t sid = static_cast<uint32_t>(p.sorted_ids[m0 + (in_block < static_cast<uint32_t>(BM) ? in_block : BM - 1)]);
+      sid = sid < p.numel ? sid : p.numel - 1;
+      h_voff[i] = (sid / p.top_k) * p.K + 64 * (hh & 1) + 16 * ((lane & 3) ^ (lane >> 4));
+    }
+  }
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
-    if (stage_act && f >= AFW) {
+    if (stage_act && (f >= AFW || BY_HALVES)) {
       d_voff[f] = d_voff_hi[f] = 0;  // not fetched
     } else if (stage_act) {
       uint32_t row = (frag0 + f) * 16 + (lane >> 2);
@@ -169,8 +187,9 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   // copy 64 of them each into LDS with one 4-byte-per-lane LDS-targeted load per stage.  The weight scales of the
   // workgroup's two 128-row scale blocks, for its whole k range, are copied into LDS once.  A lane needs one activation
   // scale per row tile (token = column l%16 of the MFMA result) and one weight scale per k-block.
+  constexpr int SCALE_SLOT = fp8_tile_scale_bytes(WM);
   constexpr int SCALE_BASE = NS * STAGE_BYTES;    // [NS slots][256] activation scales, then [2][kb_count] weight scales
-  constexpr int BS_BASE = SCALE_BASE + NS * 1024;
+  constexpr int BS_BASE = SCALE_BASE + NS * SCALE_SLOT;
   // M % 4 == 0: wavefront 0 copies all 256 with one 16-byte-per-lane load (lanes whose four tokens lie past M repeat
   // the last four).  Otherwise wavefronts 0..3 copy 64 each, 4 bytes per lane, every lane clamped on its own.
   // (the one-load form needs the 256 scales of a k-block contiguous: dense form with token-contiguous scales)
@@ -207,21 +226,23 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   auto load_scales = [&](uint32_t kb) {
     const uint32_t k = kb < kb_count ? kb : kb_count - 1;
     const char* ap = as_base + static_cast<size_t>(k) * p.as_kb_bytes;
-    const uint32_t d = __builtin_amdgcn_readfirstlane(s_lds + (kb % NS) * 1024);
+    const uint32_t d = __builtin_amdgcn_readfirstlane(s_lds + (kb % NS) * SCALE_SLOT);
     if (s_vec) {
       if (wave == 0)
         asm volatile("s_nop 4\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" ::"v"(s_voff), "s"(d), "s"(ap)
                      : "memory", "m0");
-    } else if (wave < BM / 64) {
+    } else if (wave < BM_WAVES) {
       asm volatile("s_nop 4\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2" ::"v"(s_voff), "s"(d), "s"(ap)
                    : "memory", "m0");
     }
   };
   // operands of k-block `kb` -> LDS slot kb % 2.  The instruction offset of an LDS-targeted load is added to the LDS
   // address as well as to the global one: the second half's 64-byte global offset is taken out of its LDS base.
-  // (a block at most half full: the activation fragments of its upper half are never read and, where every wait is
-  // for all of a wavefront's loads - two stages -, not fetched either)
-  const bool skip_act = NS == 2 && lower_half && stage_act && frag0 >= static_cast<uint32_t>(WM);
+  // (two stages: every wait is for all of a wavefront's loads, and activation fragments past the last one that holds
+  // tokens are not fetched - pairwise, the loads being written for four or two fragments)
+  const uint32_t frags_mine = live_tiles > frag0 ? live_tiles - frag0 : 0;
+  const bool skip_act = GROUPED && NS == 2 && stage_act && frags_mine == 0;
+  const bool pair_act = stage_act && (AFW == 2 || (GROUPED && NS == 2 && frags_mine <= 2));
   auto load_operands = [&](uint32_t kb) {
     if (skip_act) return;
     const uint32_t k = kb < kb_count ? kb : kb_count - 1;
@@ -229,7 +250,19 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
     const uint32_t f0 = __builtin_amdgcn_readfirstlane(d_lds + (kb % NS) * STAGE_BYTES);
     const uint32_t f0h = f0 + 1024 - 64;
     const uint32_t f1 = f0 + FRAG, f1h = f0h + FRAG;
-    if (AFW == 2 && stage_act) {  // two activation fragments per wavefront (128-token tiles)
+    if (BY_HALVES && stage_act) {
+      const uint32_t h0 = lds_base + (kb % NS) * STAGE_BYTES + half0 * (FRAG / 2);
+#pragma unroll
+      for (int i = 0; i < 5; ++i) {
+        if (static_cast<uint32_t>(i) < per_wave) {
+          const uint32_t d = __builtin_amdgcn_readfirstlane(h0 + i * (FRAG / 2));
+          asm volatile("s_nop 4\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" ::"v"(h_voff[i]), "s"(d), "s"(src)
+                       : "memory", "m0");
+        }
+      }
+      return;
+    }
+    if (pair_act) {  // two activation fragments
       asm volatile(
           "s_nop 4\n\t"
           "s_mov_b32 m0, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %8\n\t"
@@ -263,7 +296,7 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   // Everything this wavefront issued has landed, except the loads of the youngest stage when three stages are in use
   // (vmcnt retires in issue order; a wavefront issues the same loads every stage: 8 weight loads, or 2*AFW activation
   // loads with or without the one scale load in front of them).
-  const bool has_scale_load = s_vec ? wave == 0 : wave < BM / 64;
+  const bool has_scale_load = s_vec ? wave == 0 : wave < BM_WAVES;
   // This wavefront's fragment reads of the stage have returned: behind the barrier other wavefronts refill the slot they
   // came from, and a bare s_barrier waits for nothing by itself.
   auto reads_done = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
@@ -272,6 +305,15 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     } else if (!stage_act) {
       asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    } else if (BY_HALVES) {  // per_wave (1..5) activation loads, with or without the one scale load
+      switch (per_wave + (has_scale_load ? 1 : 0)) {
+        case 1: asm volatile("s_waitcnt vmcnt(1)" ::: "memory"); break;
+        case 2: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
+        case 3: asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); break;
+        case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
+        case 5: asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); break;
+        default: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
+      }
     } else if (has_scale_load) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * AFW + 1) : "memory");
     } else {
@@ -308,7 +350,7 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
     {
       const float bs = bs_lds[kb];
 #pragma unroll
-      for (int i = 0; i < WMV; ++i) sc[i] = as_lds[slot * 256 + i * 16] * bs;
+      for (int i = 0; i < WMV; ++i) sc[i] = as_lds[slot * (SCALE_SLOT / 4) + i * 16] * bs;
     }
     const char* act = lds + slot * STAGE_BYTES + rt0 * FRAG;
     const char* wgt = lds + slot * STAGE_BYTES + (W_FRAG0 + wn * WN) * FRAG;
@@ -423,9 +465,11 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   }
 }
 
-// A 256-slot block of the grouped form of which at most 128 slots hold tokens (an expert with half a block's tokens or
-// fewer) runs the 128-token tile's code: three stages of 48 KiB instead of two of 64 - a half-empty stage is over in
-// less time than its successor's loads take to arrive - and every wavefront at work.
+// A 256-slot block of the grouped form with at most 160 tokens (deep_rows) runs the 160-token tile's code: three stages
+// of 52 KiB instead of two of 64, because what bounds such a block is the stream of its weights, and only the activation
+// fragments that hold tokens are fetched.  160 is what the LDS has room for; that it lies above 128 matters: with 125
+// tokens per expert on average four experts in ten hold more than 128, and in 128-slot blocks each of those reads its
+// weights a second time (256 experts, hidden 7168, inter 2048, 4000 tokens, whole block: 3.18 -> 2.87 ms).
 template <typename TO, bool GROUPED = false, int WM = 8>
 __global__ void __launch_bounds__(512, 1) fp8_tile_kernel(Fp8TileParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];  // fp8_tile_lds_bytes (the larger of both forms)
@@ -439,8 +483,8 @@ __global__ void __launch_bounds__(512, 1) fp8_tile_kernel(Fp8TileParams p) {
       const bool is_row = static_cast<uint32_t>(p.sorted_ids[m0 + h * 64 + (threadIdx.x & 63)]) < p.numel;
       rows += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(is_row)));
     }
-    if (__builtin_amdgcn_readfirstlane(rows) <= 128) {
-      fp8_tile_body<TO, true, 4, 256>(p, lds);
+    if (__builtin_amdgcn_readfirstlane(rows) <= p.deep_rows) {
+      fp8_tile_body<TO, true, 5, 256>(p, lds);
       return;
     }
   }

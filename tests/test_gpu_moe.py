@@ -528,6 +528,26 @@ def test_grouped_fp8_tile_kernel_every_count_of_live_row_tiles(ops, oracle, bm):
     H.check_gemm(out, ref, H.BF16, "grouped fp8 tile kernel, %d-slot blocks" % bm)
 
 
+@pytest.mark.parametrize("n,k", [(256, 128), (272, 384), (528, 1024)])
+def test_grouped_fp8_tile_kernel_at_the_edges_of_the_three_stage_tile(ops, oracle, n, k):
+    """A 256-slot block of at most 160 slots runs on three LDS stages, a larger one on two, a 128-slot block on its own
+    tile: every output is the same sum in the same order of k, so the bits are the same."""
+    rows = [1, 16, 17, 32, 33, 127, 128, 129, 144, 145, 159, 160, 161, 176, 255, 256, 257, 417]
+    E, T = len(rows), sum(rows)
+    g = H.gen(7800 + n + k)
+    bq, bs = _fp8_experts(oracle, 7810 + n, E, n, k)
+    x = torch.randn((T, k), generator=g).to(torch.bfloat16)
+    ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
+    ids = ids[torch.randperm(T, generator=g)].reshape(T, 1).contiguous().cuda()
+    q, s = ops.per_token_group_quant_fp8(x.cuda(), k, 128, False)
+    wp, wsc = ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda()
+    outs = []
+    for bm in (128, 256):
+        sorted_ids, expert_ids, npp = ops.moe_align_block_size(ids, E, bm)
+        outs.append(ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, None, sorted_ids, expert_ids, npp, T, 1, bm, torch.bfloat16))
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
 @pytest.mark.parametrize("T,E,topk,hidden,inter", [(1, 8, 2, 256, 128), (48, 16, 4, 512, 256), (200, 8, 2, 384, 640),
                                                    (1200, 8, 2, 512, 256)])   # the last: 300 slots per expert, 256-slot blocks
