@@ -128,6 +128,26 @@ def build_layers():
     return LAYERS_LIB, LAYER_TEST
 
 
+OPS_HOST = os.path.join(HERE, "_ops_host.so")
+
+
+def build_ops_host():
+    """The host side of ops.py (host code only, against the installed torch) -> _ops_host.so, an extension module."""
+    import sysconfig
+    import torch
+    t = os.path.dirname(torch.__file__)
+    cmd = [HIPCC, "-std=c++17", "-O2", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(), "-I" + os.path.join(ROOT, "include"),
+           "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(t, "include"), "-Wno-unused-command-line-argument",
+           "-o", OPS_HOST, os.path.join(HERE, "host", "ops_host.cpp"),
+           "-L" + os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("host extension build failed:\n" + r.stderr)
+    return OPS_HOST
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
     print(build_layers())
+    print(build_ops_host())

@@ -108,6 +108,12 @@ def load():
     return _lib
 
 
+def addresses():
+    """Entry points of the loaded library as addresses, for the C++ side of ops.py (host/ops_host.cpp)."""
+    lib = load()
+    return {name: ctypes.cast(getattr(lib, name), c_p).value for name in SIGNATURES}
+
+
 def check(rc):
     if rc != 0:
         raise KsqError(rc, load().ksq_last_error_string().decode())

@@ -10,6 +10,13 @@ from . import lib as _l
 
 _lib = _l.load()
 
+# The hot calls run in C++ (host/ops_host.cpp), on the library's own entry points; there is no other path for them.
+try:
+    from . import _ops_host as _h
+except ImportError as e:
+    raise ImportError("_ops_host.so is not built: run `python -m ksanallm_amd.build` (%s)" % e) from e
+_h.bind(_l.addresses(), _l.check)
+
 F16, BF16 = _l.F16, _l.BF16
 
 
@@ -28,7 +35,7 @@ def _torch_dt(tag):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    return _h.current_stream()
 
 
 def _ptr(t):
@@ -106,37 +113,14 @@ def w4a16_workspace_size(max_m, n, k, group, dtype):
     return _lib.ksq_w4a16_workspace_size(max_m, n, k, group, dtype)
 
 
-_WORKSPACES = {}
-
-
-def _w4a16_workspace(device, m, n, k, group, dt):
-    """A per-device scratch tensor large enough for this call (grown on demand, like the engine's shared workspace)."""
-    need = _lib.ksq_w4a16_workspace_size(m, n, k, group, dt)
-    if need == 0:
-        return None
-    cur = _WORKSPACES.get(device)
-    if cur is None or cur.numel() < need:
-        cur = torch.empty(need, dtype=torch.uint8, device=device)
-        _WORKSPACES[device] = cur
-    return cur
+def _scratch(nbytes, device):
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
 
 
 def w4a16_gemm(x, w_packed, scales_packed, zeros_packed, n, k, group, out=None, workspace=None):
-    """InvokeFpAIntBGroupCudaGemm / InvokeFpAIntBGroupCutlassGemm / InvokeMarlinGemm / InvokeMacheteGemm."""
-    m = x.shape[0]
-    _need_bytes(x, m * k * 2, "w4a16_gemm: x")
-    _need_bytes(w_packed, k * n // 2, "w4a16_gemm: packed weight")
-    _need_bytes(scales_packed, (k // group) * n * 2, "w4a16_gemm: scales")
-    if zeros_packed is not None:
-        _need_bytes(zeros_packed, (k // group) * n, "w4a16_gemm: zero points")
-    if out is None:
-        out = torch.empty((m, n), dtype=x.dtype, device=x.device)
-    if workspace is None:
-        workspace = _w4a16_workspace(x.device, m, n, k, group, _dt(x))
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    _l.check(_lib.ksq_w4a16_gemm(_ptr(out), _ptr(x), _ptr(w_packed), _ptr(scales_packed), _ptr(zeros_packed),
-                                 _ptr(workspace), ws_bytes, m, n, k, group, _dt(x), _stream()))
-    return out
+    """InvokeFpAIntBGroupCudaGemm / InvokeFpAIntBGroupCutlassGemm / InvokeMarlinGemm / InvokeMacheteGemm.  Scratch that is
+    not given comes from torch's allocator, for this call."""
+    return _h.w4a16_gemm(x, w_packed, scales_packed, zeros_packed, n, k, group, out, workspace)
 
 
 def w4a16_gemm_f32(x, w_packed, scales_packed, zeros_packed, n, k, group, workspace=None):
@@ -147,7 +131,7 @@ def w4a16_gemm_f32(x, w_packed, scales_packed, zeros_packed, n, k, group, worksp
     _need_bytes(scales_packed, (k // group) * n * 2, "w4a16_gemm_f32: scales")
     out = torch.empty((m, n), dtype=torch.float32, device=x.device)
     if workspace is None:
-        workspace = _w4a16_workspace(x.device, m, n, k, group, _dt(x))
+        workspace = _scratch(_lib.ksq_w4a16_workspace_size(m, n, k, group, _dt(x)), x.device)
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     _l.check(_lib.ksq_w4a16_gemm_f32(_ptr(out), _ptr(x), _ptr(w_packed), _ptr(scales_packed), _ptr(zeros_packed),
                                      _ptr(workspace), ws_bytes, m, n, k, group, _dt(x), _stream()))
@@ -157,36 +141,13 @@ def w4a16_gemm_f32(x, w_packed, scales_packed, zeros_packed, n, k, group, worksp
 # ----------------------------------------------------------------------------------------------- FP8
 def per_token_group_quant_fp8(x, k, group=128, column_major=True, fuse_silu_mul=False, q=None, s=None):
     """InvokePerTokenGroupQuantFp8E4m3: returns (codes uint8 [m,k], scales fp32 [k/group,m] or [m,k/group])."""
-    m = x.shape[0]
-    if q is None:
-        q = torch.empty((m, k), dtype=torch.uint8, device=x.device)
-    if s is None:
-        s = torch.empty((k // group, m) if column_major else (m, k // group), dtype=torch.float32, device=x.device)
-    _l.check(_lib.ksq_fp8_group_quant(_ptr(x), _ptr(q), _ptr(s), m, k, group, int(column_major), int(fuse_silu_mul),
-                                      _dt(x, allow_f32=True), _stream()))
-    return q, s
+    return _h.per_token_group_quant_fp8(x, k, group, column_major, fuse_silu_mul, q, s)
 
 
 def fp8_blockwise_gemm(a_q, a_s, b, b_s, out_dtype=torch.bfloat16, out=None, workspace=None):
     """InvokeBlockGemm / DeepGEMMWrapper::Gemm: a_q [m,k] e4m3 bytes, a_s [k/128,m], b [n,k] packed by
     fp8_repack_weight, b_s [n/128,k/128]."""
-    m, k = a_q.shape
-    n = b.shape[0]
-    _need_bytes(a_s, (k // 128) * m * 4, "fp8_blockwise_gemm: activation scales")
-    _need_bytes(b, n * k, "fp8_blockwise_gemm: weight")
-    _need_bytes(b_s, ((n + 127) // 128) * (k // 128) * 4, "fp8_blockwise_gemm: weight scales")
-    if out is None:
-        out = torch.empty((m, n), dtype=out_dtype, device=a_q.device)
-    if workspace is None:
-        need = _lib.ksq_fp8_blockwise_workspace_size(m, n, k)
-        if need:
-            workspace = _WORKSPACES.get(a_q.device)
-            if workspace is None or workspace.numel() < need:
-                workspace = _WORKSPACES[a_q.device] = torch.empty(need, dtype=torch.uint8, device=a_q.device)
-    ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    _l.check(_lib.ksq_fp8_blockwise_gemm(_ptr(a_q), _ptr(a_s), _ptr(b), _ptr(b_s), _ptr(out), m, n, k,
-                                         _dt(out, allow_f32=True), _ptr(workspace), ws_bytes, _stream()))
-    return out
+    return _h.fp8_blockwise_gemm(a_q, a_s, b, b_s, out_dtype, out, workspace)
 
 
 def fp8_blockwise_gemm_f32(a_q, a_s, b, b_s, workspace=None):
@@ -198,11 +159,7 @@ def fp8_blockwise_gemm_f32(a_q, a_s, b, b_s, workspace=None):
     _need_bytes(b_s, ((n + 127) // 128) * (k // 128) * 4, "fp8_blockwise_gemm_f32: weight scales")
     out = torch.empty((m, n), dtype=torch.float32, device=a_q.device)
     if workspace is None:
-        need = _lib.ksq_fp8_blockwise_workspace_size(m, n, k)
-        if need:
-            workspace = _WORKSPACES.get(a_q.device)
-            if workspace is None or workspace.numel() < need:
-                workspace = _WORKSPACES[a_q.device] = torch.empty(need, dtype=torch.uint8, device=a_q.device)
+        workspace = _scratch(_lib.ksq_fp8_blockwise_workspace_size(m, n, k), a_q.device)
     ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
     _l.check(_lib.ksq_fp8_blockwise_gemm_f32(_ptr(a_q), _ptr(a_s), _ptr(b), _ptr(b_s), _ptr(out), m, n, k,
                                              _ptr(workspace), ws_bytes, _stream()))
@@ -256,31 +213,16 @@ def moe_w4a16_gate_up_silu(x, w_packed, scales_packed, sorted_ids, expert_ids, n
 
 def moe_topk_softmax(gating, top_k, norm_topk_prob=False, routed_scaling_factor=1.0):
     """InvokeBasicSoftmaxTopk: (topk_weights fp32 [T, top_k], topk_ids int32 [T, top_k])."""
-    tokens, E = gating.shape
-    dt = _l.F32 if gating.dtype == torch.float32 else _dt(gating)
-    w = torch.empty((tokens, top_k), dtype=torch.float32, device=gating.device)
-    ids = torch.empty((tokens, top_k), dtype=torch.int32, device=gating.device)
-    _l.check(_lib.ksq_moe_topk_softmax(_ptr(gating), _ptr(w), _ptr(ids), tokens, E, top_k, int(norm_topk_prob),
-                                       float(routed_scaling_factor), dt, _stream()))
-    return w, ids
+    return _h.moe_topk_softmax(gating, top_k, norm_topk_prob, routed_scaling_factor)
 
 
 def moe_grouped_topk(gating, top_k, num_expert_group=1, topk_group=1, scoring_func="softmax", e_bias=None,
                      renormalize=False, routed_scaling_factor=1.0):
     """InvokeGroupedTopk: (topk_weights fp32 [T, top_k], topk_ids int32 [T, top_k]); e_bias fp32 [E] or None."""
-    tokens, E = gating.shape
     if scoring_func not in ("softmax", "sigmoid"):
         raise ValueError("Unsupported scoring function: %s" % scoring_func)
-    dt = _l.F32 if gating.dtype == torch.float32 else _dt(gating)
-    w = torch.empty((tokens, top_k), dtype=torch.float32, device=gating.device)
-    ids = torch.empty((tokens, top_k), dtype=torch.int32, device=gating.device)
-    if e_bias is not None and e_bias.dtype != torch.float32:
-        raise ValueError("e_bias must be fp32")
-    _l.check(_lib.ksq_moe_grouped_topk(_ptr(gating), _ptr(e_bias) if e_bias is not None else None, _ptr(w), _ptr(ids),
-                                       tokens, E, top_k, num_expert_group, topk_group,
-                                       1 if scoring_func == "sigmoid" else 0, int(renormalize),
-                                       float(routed_scaling_factor), dt, _stream()))
-    return w, ids
+    return _h.moe_grouped_topk(gating, top_k, num_expert_group, topk_group, scoring_func == "sigmoid", e_bias, renormalize,
+                               routed_scaling_factor)
 
 
 def silu_and_mul(x, out=None):
@@ -310,35 +252,8 @@ def fused_moe_w4a16(x, w13_packed, s13_packed, w2_packed, s2_packed, topk_ids, t
                     block_m=None):
     """InvokeFusedMoe<T,false> for int4 weights (S/kernels/nvidia/moe_kernel_wrapper.cpp:463-654):
     align -> GEMM1 -> silu*mul -> GEMM2 (* routed weight) -> sum over top-k."""
-    T, topk = topk_ids.shape
-    numel = T * topk
-    tw = topk_w.reshape(-1).to(torch.float32).contiguous()
-    if block_m is None and T <= FEW_TOKENS and numel <= 64 and topk <= 32 and (2 * inter) % 32 == 0:
-        # a few decode tokens: two launches - the first GEMM with every slot a block of its own (no aligned
-        # permutation) and the activation in its epilogue, the second with the sum over top-k in it
-        ids = topk_ids.reshape(-1).to(torch.int32).contiguous()
-        c2 = torch.empty((numel, inter), dtype=x.dtype, device=x.device)
-        _l.check(_lib.ksq_moe_w4a16_gate_up_silu(_ptr(c2), _ptr(x), _ptr(w13_packed), _ptr(s13_packed), None, None, _ptr(ids),
-                                                 None, numel, topk, E, 2 * inter, hidden, group, 16, _dt(x), _stream()))
-        out = torch.empty((T, hidden), dtype=x.dtype, device=x.device)
-        _l.check(_lib.ksq_moe_w4a16_down_sum(_ptr(out), _ptr(c2), _ptr(w2_packed), _ptr(s2_packed), _ptr(tw), _ptr(ids), T,
-                                             topk, E, hidden, inter, group, _dt(x), _stream()))
-        return out
-    if block_m is None:
-        block_m = _lib.ksq_moe_block_m(numel, E)
-    sorted_ids, expert_ids, npp = moe_align_block_size(topk_ids, E, block_m)
-    # the activation runs in the first GEMM's epilogue, except with 128-row blocks (a size ksq_moe_block_m no longer
-    # picks but a caller may ask for), where the two launches measured faster (64 rows per expert: 1.75 against 1.87 ms)
-    if block_m != 128 and (2 * inter) % 32 == 0:
-        c2 = moe_w4a16_gate_up_silu(x, w13_packed, s13_packed, sorted_ids, expert_ids, npp, numel, topk, E, 2 * inter,
-                                    hidden, group, block_m)
-    else:
-        c1 = moe_w4a16_gemm(x, w13_packed, s13_packed, None, sorted_ids, expert_ids, npp, numel, topk, E, 2 * inter,
-                            hidden, group, block_m)
-        c2 = silu_and_mul(c1)
-    c3 = moe_w4a16_gemm(c2, w2_packed, s2_packed, tw, sorted_ids, expert_ids, npp, numel, 1, E, hidden, inter, group,
-                        block_m)
-    return moe_sum(c3.view(T, topk, hidden))
+    return _h.fused_moe_w4a16(x, w13_packed, s13_packed, w2_packed, s2_packed, topk_ids, topk_w, E, hidden, inter, group,
+                              block_m, FEW_TOKENS)
 
 
 def moe_fp8_blockwise_gemm(a_q, a_s, a_s_column_major, b, b_s, topk_w, sorted_ids, expert_ids, num_post_pad, numel,
@@ -361,31 +276,7 @@ def fused_moe_fp8_blockwise(x, w13, w13_scale, w2, w2_scale, topk_ids, topk_w, b
     compute_dtype TYPE_BLOCK_FP8_E4M3): quantize x per token and 128 channels -> align -> GEMM1 -> silu*mul fused into
     the second quantization -> GEMM2 (* routed weight) -> sum over top-k.  w13 [E, 2*inter, hidden], w2 [E, hidden, inter]
     e4m3 bytes packed by fp8_repack_weight, scales fp32 per 128 x 128 block."""
-    T, topk = topk_ids.shape
-    E, two_inter, hidden = w13.shape
-    inter = two_inter // 2
-    numel = T * topk
-    tw = topk_w.reshape(-1).to(torch.float32).contiguous()
-    if block_m is None and T <= FEW_TOKENS and numel <= 64 and topk <= 32:
-        # a few decode tokens: no aligned permutation, the sum over top-k inside the second GEMM (as fused_moe_w4a16)
-        ids = topk_ids.reshape(-1).to(torch.int32).contiguous()
-        a1_q, a1_s = per_token_group_quant_fp8(x, hidden, 128, False)
-        c1 = moe_fp8_blockwise_gemm(a1_q, a1_s, False, w13, w13_scale, None, None, ids, None, numel, topk, 16, x.dtype)
-        a2_q, a2_s = per_token_group_quant_fp8(c1, inter, 128, False, fuse_silu_mul=True)
-        out = torch.empty((T, hidden), dtype=x.dtype, device=x.device)
-        _l.check(_lib.ksq_moe_fp8_down_sum(_ptr(out), _ptr(a2_q), _ptr(a2_s), _ptr(w2), _ptr(w2_scale), _ptr(tw), _ptr(ids), T,
-                                           topk, E, hidden, inter, _dt(out), _stream()))
-        return out
-    if block_m is None:
-        block_m = _lib.ksq_moe_fp8_block_m(numel, E)
-    sorted_ids, expert_ids, npp = moe_align_block_size(topk_ids, E, block_m)
-    a1_q, a1_s = per_token_group_quant_fp8(x, hidden, 128, False)
-    c1 = moe_fp8_blockwise_gemm(a1_q, a1_s, False, w13, w13_scale, None, sorted_ids, expert_ids, npp, numel, topk,
-                                block_m, x.dtype)
-    a2_q, a2_s = per_token_group_quant_fp8(c1, inter, 128, False, fuse_silu_mul=True)
-    c3 = moe_fp8_blockwise_gemm(a2_q, a2_s, False, w2, w2_scale, tw, sorted_ids, expert_ids, npp, numel, 1, block_m,
-                                x.dtype)
-    return moe_sum(c3.view(T, topk, hidden))
+    return _h.fused_moe_fp8_blockwise(x, w13, w13_scale, w2, w2_scale, topk_ids, topk_w, block_m, FEW_TOKENS)
 
 
 def fp8_e4m3_quantize(x, scale=None):
@@ -481,14 +372,7 @@ def w4a8_unpack_weight(packed, K, N):
 def w4a8_static_quant(x, scale, per_channel=False, per_token=False, group=128):
     """StaticQuantizeE4M3PerTensor / PerChannel / PerToken: x [m,k] T, scale fp32 [1], [k] or [m] -> (codes uint8
     [m,k], group sums fp32 [k/group, m]); group 128 or 64."""
-    m, k = x.shape
-    q = torch.empty((m, k), dtype=torch.uint8, device=x.device)
-    xsum = torch.empty((k // group, m), dtype=torch.float32, device=x.device)
-    mode = _l.W4A8_PER_CHANNEL if per_channel else (_l.W4A8_PER_TOKEN if per_token else _l.W4A8_PER_TENSOR)
-    if group == 64:
-        mode |= _l.W4A8_SUMS_PER_64
-    _l.check(_lib.ksq_w4a8_static_quant(_ptr(x), _ptr(scale), _ptr(q), _ptr(xsum), m, k, mode, _dt(x), _stream()))
-    return q, xsum
+    return _h.w4a8_static_quant(x, scale, per_channel, per_token, group)
 
 
 def w4a8_group_sums(a_q, group=128):
@@ -502,16 +386,4 @@ def w4a8_group_sums(a_q, group=128):
 
 def w4a8_gemm(a_q, xsum, w_packed, scales, alpha, n, out_dtype=torch.bfloat16, out=None, workspace=None, group=128):
     """FinegrainedMixedDtypeGemmWrapper::Forward: a_q [m,k] e4m3 bytes, xsum [k/group, m], scales fp16 [k/group, n]."""
-    m, k = a_q.shape
-    _need_bytes(xsum, (k // group) * m * 4, "w4a8_gemm: group sums")
-    _need_bytes(w_packed, n * k // 2, "w4a8_gemm: packed weight")
-    _need_bytes(scales, (k // group) * n * 2, "w4a8_gemm: scales")
-    if out is None:
-        out = torch.empty((m, n), dtype=out_dtype, device=a_q.device)
-    if workspace is None:
-        need = _lib.ksq_w4a8_workspace_size(m, n, k)
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=a_q.device)
-    assert scales.dtype == torch.float16
-    _l.check(_lib.ksq_w4a8_gemm(_ptr(a_q), _ptr(xsum), _ptr(w_packed), _ptr(scales), float(alpha), _ptr(out), m, n, k,
-                                group, _dt(out), _ptr(workspace), workspace.numel(), _stream()))
-    return out
+    return _h.w4a8_gemm(a_q, xsum, w_packed, scales, alpha, n, out_dtype, out, workspace, group)
