@@ -315,9 +315,9 @@ __global__ void __launch_bounds__(512, 1) w4a16_tile_kernel(TileParams p) {
   // blocks and lose the interleaving of LDS reads, conversions and MFMAs (measured: 20 % slower, not faster).
   auto run = [&](auto wmv_c) {
     constexpr int WMV = decltype(wmv_c)::value;
-    // Fragments this wavefront stages per x stage.  A 256-slot expert block of which at most the lower eight row tiles
-    // hold slots stages those only (two fragments per wavefront instead of four); the reads below never reach further.
-    constexpr int APV = (GROUPED && WM == 16 && WMV <= 8) ? 2 : AP;
+    // Fragments this wavefront stages per x stage.  A 256-row block of which at most the lower eight row tiles hold
+    // rows stages those only (two fragments per wavefront instead of four); the reads below never reach further.
+    constexpr int APV = (WM == 16 && WMV <= 8) ? 2 : AP;
     uint32_t a_voff[APV / 2];
 #pragma unroll
     for (int j = 0; j < APV / 2; ++j) {
@@ -479,11 +479,14 @@ __global__ void __launch_bounds__(512, 1) w4a16_tile_kernel(TileParams p) {
       stage(std::integral_constant<int, 5>{}, base);
     }
   };
-  if (GROUPED) {
-    // expert blocks: an instance of the main loop for every number of row tiles that hold slots, from four (the depth
-    // of the fragment prefetch) to all of them.  What a padded row tile costs is not so much time in the loop as power
-    // - its MFMAs multiply real rows -, and the clock: at 128 slots per expert on average, instances over 9 and 10
-    // row tiles next to those over 8 and 12 took a tenth off the whole call.
+  // An instance of the main loop for every number of row tiles that hold rows, from four (the depth of the fragment
+  // prefetch) to all of them.  Expert blocks: what a padded row tile costs is not so much time in the loop as power - its
+  // MFMAs multiply real rows -, and the clock: at 128 slots per expert on average, instances over 9 and 10 row tiles next
+  // to those over 8 and 12 took a tenth off the whole call.  Dense form: a prompt or a batch of 129..255 rows is one
+  // 256-row tile, all of which was multiplied as soon as more than half of it held rows (n = 14336, k = 4096, 150 rows,
+  // bf16 with zero points: 40.9 -> 34.6 us with ten of sixteen row tiles multiplied).
+  // (groups of 64 and 32 rows, dense: half of the tile or all of it)
+  if constexpr (GROUPED || GROUP == 128) {
     for_tile_count<4, WM>(live_tiles, run);
   } else if (live_tiles <= WM / 2) {
     run(std::integral_constant<int, WM / 2>{});

@@ -112,6 +112,23 @@ def test_prefill_256_row_tiles(ops, dtype, awq, M, N, K, tile_kernels):
                  weights_rounded=True)
 
 
+# the main loop of the tile kernel exists once per number of row tiles that hold rows: every count, 128- and 256-row tiles
+@pytest.mark.parametrize("awq", [False, True])
+@pytest.mark.parametrize("M,N,K", [(m, 8448, 128) for m in (129, 145, 161, 177, 193, 209, 225, 241)] +
+                         [(m, 272, 384) for m in (33, 65, 81, 97, 113)])
+def test_prefill_every_row_tile_count(ops, awq, M, N, K, tile_kernels):
+    from ksanallm_amd import lib as L
+    full = 256 if M > 128 else 128
+    assert L.select_tile(L.KIND_W4A16, M, N, K, H.BF16)["block_m"] == full
+    d = H.make_w4a16(3500 + M, full, N, K, 128, H.BF16, awq=awq, x_std=0.5, s_lo=0.002, s_hi=0.01, z_lo=0, z_hi=15)
+    y = run_case(ops, d)
+    short = run_case(ops, dict(d, M=M, x=d["x"][:M].contiguous()))
+    assert (short == y[:M]).all(), "a row's sum depends on how many rows the tile holds"
+    n = 64   # the oracle on the first columns: what a wrong row tile would show in every column
+    sub = H.w4a16_oracle(d)[:M, :n]
+    H.check_gemm(short[:, :n], sub, H.BF16, "row tiles M=%d" % M, weights_rounded=True)
+
+
 # few output tiles: K is split over workgroups, fp32 partials go through the workspace and a second kernel sums them
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
 @pytest.mark.parametrize("M,N,K", [(128, 4096, 14336), (512, 4096, 14336), (64, 512, 2048), (200, 256, 1664)])
