@@ -62,6 +62,13 @@ SplitKChoice select_splitk(size_t m, size_t n, size_t k) {
   //   47.8 -> 46.3 us; n = 25600, k = 5120 at 16 rows 15.9 -> 15.0 us), not below (n = 14336, k = 4096 at 8 rows:
   //   7.9 us in registers, 8.4 us through LDS), and with up to 8 rows four column tiles per wavefront beat eight
   //   (n = 57344, k = 8192, 1 row: 40.7 against 43.1 us).
+  // - K cut over workgroups, 17 rows and more: x outweighs the weights there by construction (n = 4096, k = 14336: 20 rows
+  //   13.2 -> 12.9 us, 32 rows 15.8 -> 14.3, 64 rows 21.6 -> 19.0, 128 rows 36.7 -> 31.5; n = k = 5120 at 32 rows
+  //   12.7 -> 11.6; n = 5120, k = 25600 at 32 rows 34.4 -> 29.0; n = 2048, k = 8192 at 32 rows 11.5 -> 11.0).
+  if (c.parts > 1 && mt == 2) {
+    c.waves = 8;
+    c.xc = 8;
+  }
   if (c.parts == 1 && strips % 4 == 0) {
     if (mt == 2 && c.nt == 8) {
       c.waves = 4;

@@ -292,6 +292,19 @@ def test_prefill_full_size_properties(ops, N, K):
     assert torch.equal(yp, y[perm])
 
 
+# the same with the activations through LDS (17 rows and more): parts of K that are no whole number of chunks or of 4-k-tile
+# loads, a short last part, several row blocks
+@pytest.mark.parametrize("dtype,awq", [(H.F16, False), (H.BF16, True)])
+@pytest.mark.parametrize("M,N,K", [(17, 1024, 4096), (25, 2048, 8064), (32, 4096, 14336), (33, 2048, 5248), (95, 1024, 4224)])
+def test_decode_k_parts_x_through_lds(ops, dtype, awq, M, N, K):
+    from ksanallm_amd import lib as L
+    desc = L.select_tile(L.KIND_W4A16, M, N, K, dtype)
+    assert desc["kernel"] == 0 and desc["x_chunk"] == 8 and desc["waves"] == 8 and desc["split_k"] > 8
+    d = H.make_w4a16(4100 + M + N, M, N, K, 128, dtype, awq=awq, z_lo=0, z_hi=15)
+    y = run_case(ops, d)
+    H.check_gemm(y, H.w4a16_oracle(d), dtype, "decode K parts, x through LDS M=%d N=%d K=%d" % (M, N, K))
+
+
 # decode regime with the activations staged through LDS (17..32 rows; up to 16 rows from 48 MB of weights): K that is
 # not a whole number of 4-k-tile loads, one chunk and several, ragged row counts, both dtypes, with and without zero points
 @pytest.mark.parametrize("dtype,awq", [(H.F16, False), (H.BF16, True), (H.F16, True), (H.BF16, False)])
