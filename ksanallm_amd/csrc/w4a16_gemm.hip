@@ -290,13 +290,13 @@ KSQ_EXPORT int ksq_w4a16_gemm_f32(float* y, const void* x, const void* w_packed,
 }
 
 namespace {
-template <typename T, int NT>
+template <typename T, int NT, int WAVES>
 int launch_token_sum(const SplitKParams& p, uint32_t tokens, hipStream_t s) {
-  // one row of x per workgroup: the narrow decode instances' ring depths
-  constexpr int LOOK = NT == 1 ? 4 : 3, OCC = NT == 1 ? 4 : 3;
-  typedef SplitKLds<1, NT, 4, 0> Lds;
+  // one row of x per workgroup: the narrow decode instances' ring depths; eight wavefronts keep more in flight with two
+  constexpr int LOOK = WAVES == 8 ? 2 : (NT == 1 ? 4 : 3), OCC = WAVES == 8 ? 2 : (NT == 1 ? 4 : 3);
+  typedef SplitKLds<1, NT, WAVES, 0> Lds;
   dim3 grid(p.N / 16 / NT, tokens, 1);
-  w4a16_splitk_kernel<T, 1, NT, 4, LOOK, OCC, 128, false, true, 0, 16, true><<<grid, 4 * 64, Lds::kBytes, s>>>(p);
+  w4a16_splitk_kernel<T, 1, NT, WAVES, LOOK, OCC, 128, false, true, 0, 16, true><<<grid, WAVES * 64, Lds::kBytes, s>>>(p);
   return KSQ_OK;
 }
 }  // namespace
@@ -332,12 +332,19 @@ KSQ_EXPORT int ksq_moe_w4a16_down_sum(void* out, const void* x, const void* w_pa
   const bool two = (n / 16) % 2 == 0 && (n / 32) * tokens >= 192;
   p.magic2 = dtype == KSQ_F16 ? F16::kMagic2 : BF16::kMagic2;
   int rc;
-  if (dtype == KSQ_F16)
-    rc = two ? launch_token_sum<F16, 2>(p, static_cast<uint32_t>(tokens), as_stream(stream))
-             : launch_token_sum<F16, 1>(p, static_cast<uint32_t>(tokens), as_stream(stream));
-  else
-    rc = two ? launch_token_sum<BF16, 2>(p, static_cast<uint32_t>(tokens), as_stream(stream))
-             : launch_token_sum<BF16, 1>(p, static_cast<uint32_t>(tokens), as_stream(stream));
+  // ... and eight wavefronts instead of four where their rings of two k-tiles fill: what bounds the kernel is the bytes a
+  // CU keeps in flight, and 224 workgroups of four wavefronts keep 24 KiB (whole one-token block, 8 of 256 experts, hidden
+  // 7168, inter 2048: 44.1 -> 42.4 us; 4 experts 26.2 -> 25.0; 2 experts of inter 1024, 16 k-tiles: 17.9 -> 17.4; four
+  // tokens 127.9 -> 127.0; eight wavefronts with a ring of three or four 0.4-0.9 us behind two)
+  const bool eight = two && top_k * k >= 16 * 128;
+  auto go = [&](auto t) {
+    typedef decltype(t) T;
+    const uint32_t rows = static_cast<uint32_t>(tokens);
+    return eight ? launch_token_sum<T, 2, 8>(p, rows, as_stream(stream))
+           : two ? launch_token_sum<T, 2, 4>(p, rows, as_stream(stream))
+                 : launch_token_sum<T, 1, 4>(p, rows, as_stream(stream));
+  };
+  rc = dtype == KSQ_F16 ? go(F16{}) : go(BF16{});
   if (rc) return rc;
   return check_launch(fn);
 }

@@ -364,6 +364,35 @@ def test_silu_over_every_input_of_the_type(ops, dtype):
     print("silu %s: %d of %d inputs one unit off the correctly rounded value (%.3f %%)" % (td, int((d > 0).sum()), n, 100 * share))
 
 
+@pytest.mark.parametrize("topk,k", [(5, 384), (4, 512), (17, 128), (2, 1024), (3, 1408)])
+def test_down_sum_with_eight_wavefronts(topk, k):
+    """15 k-tiles run on four wavefronts, 16 and more on eight, one token (few workgroups) on the one-column form of four:
+    the same fp32 sum in another order, so an fp16 output differs by one unit (2^-10 of its value) at most."""
+    from ksanallm_amd import lib as L
+    from ksanallm_amd import ops
+    E, n, T = 24, 2048, 3
+    g = H.gen(6100 + topk)
+    codes = torch.randint(0, 256, (E, n, k // 2), generator=g, dtype=torch.uint8)
+    w = ops.repack_weight(codes.cuda(), L.SRC_MOE_NK, E, k, n)
+    s = ops.repack_scales((torch.rand((E, n, k // 128), generator=g) * 0.01).half().cuda(), L.SCALE_NG, E, k, n, 128)
+    x = torch.randn((T * topk, k), generator=g).half().cuda()
+    ids = torch.stack([torch.randperm(E, generator=g)[:topk] for _ in range(T)]).to(torch.int32).cuda()
+    tw = torch.rand((T, topk), generator=g).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def down(t0, t1):
+        out = torch.full((t1 - t0, n), float("nan"), dtype=torch.float16, device="cuda")
+        L.check(L.load().ksq_moe_w4a16_down_sum(out.data_ptr(), x[t0 * topk:].data_ptr(), w.data_ptr(), s.data_ptr(),
+                                                tw[t0:].contiguous().data_ptr(), ids[t0:].contiguous().data_ptr(), t1 - t0, topk,
+                                                E, n, k, 128, H.F16, stream))
+        torch.cuda.synchronize()
+        return out.float()
+    whole = down(0, T)
+    one = torch.cat([down(t, t + 1) for t in range(T)])
+    assert torch.isfinite(one).all()
+    assert float((whole - one).norm() / one.norm()) < 2.0 ** -10
+
+
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
 @pytest.mark.parametrize("T,E,topk,hidden,inter", [(1, 16, 4, 256, 128), (2, 16, 8, 512, 256), (3, 8, 2, 384, 128), (8, 16, 4, 256, 384),
                                                    (1, 256, 8, 7168, 2048)])
