@@ -245,9 +245,12 @@ TilePlan plan_fp8_tile(size_t m, size_t n, size_t k) {
 // W4A8: the blockwise-FP8 tile shapes; a k-step moves three quarters of the bytes and its prologue is shorter, so a
 // cut along K pays earlier (measured at n = 25600, k = 5120: with the FP8 costs 64 / 128 / 256 tokens ran whole tiles
 // on 100 of the 256 CUs in 38 / 51 / 83 us, with these they are cut in two or three: 28 / 38 / 60 us)
+// Up to 64 tokens, 64-token tiles: the two wavefront rows share the row tiles (of a 128-token tile the lower one would
+// stand idle) and a barrier comes every two k-blocks (n = 25600, k = 5120 at 64 tokens, quantizer included:
+// 29.65 -> 28.3 us).
 TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k) {
   TilePlan t{};
-  t.block_m = (m <= 128 || (m < 1024 && (m - 1) % 256 < 128)) ? 128 : 256;
+  t.block_m = m <= 64 ? 64 : (m <= 128 || (m < 1024 && (m - 1) % 256 < 128)) ? 128 : 256;
   // as in plan_mfma_tile: at most 32 tiles of 256 tokens are better served by 128-token tiles and half the cut along K
   // (n = k = 5120 at 256 tokens: 31 -> 25 us; n = k = 4096 at 512 tokens: 33 -> 27 us)
   if (t.block_m == 256 && div_up(m, 256) * div_up(n, 256) <= 32 && k <= 16384) t.block_m = 128;

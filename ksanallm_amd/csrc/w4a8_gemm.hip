@@ -450,10 +450,10 @@ KSQ_EXPORT int ksq_w4a8_static_quant(const void* x, const void* scale, void* q, 
 
 KSQ_EXPORT size_t ksq_w4a8_workspace_size(size_t max_m, size_t n, size_t k) {
   if (n == 0 || k == 0 || k % 128 != 0) return 0;
-  // only the split-K form of the tile kernel needs scratch (fp32 partial tiles); the plan is the same for all m of a
-  // band of 128 rows
+  // only the split-K form of the tile kernel needs scratch (fp32 partial tiles); the plan is the same for
+  // 33..64 rows, 65..128 rows and all m of every further band of 128 rows
   size_t need = 0;
-  for (size_t band_end = 128; max_m > 32; band_end += 128) {
+  for (size_t band_end = 64; max_m > 32; band_end += band_end == 64 ? 64 : 128) {
     const size_t m = band_end < max_m ? band_end : max_m;
     const TilePlan t = plan_w4a8_tile(m, n, k);
     need = t.workspace_bytes > need ? t.workspace_bytes : need;
@@ -511,7 +511,9 @@ KSQ_EXPORT int ksq_w4a8_gemm(const void* a_q, const void* xsum, const void* w_pa
                   n, k, plan.workspace_bytes, workspace ? workspace_bytes : size_t(0));
     if (256 * k > 0xffffffffull || 16 * (k / 128) * 1024 > 0xffffffffull) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: k too large", fn);
     float* partial = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
-    if (plan.block_m == 128)
+    if (plan.block_m == 64)
+      rc = out_dtype == KSQ_F16 ? launch_tile<F16, 2>(p, plan, partial, st) : launch_tile<BF16, 2>(p, plan, partial, st);
+    else if (plan.block_m == 128)
       rc = out_dtype == KSQ_F16 ? launch_tile<F16, 4>(p, plan, partial, st) : launch_tile<BF16, 4>(p, plan, partial, st);
     else
       rc = out_dtype == KSQ_F16 ? launch_tile<F16, 8>(p, plan, partial, st) : launch_tile<BF16, 8>(p, plan, partial, st);

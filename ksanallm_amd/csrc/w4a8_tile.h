@@ -2,7 +2,7 @@
 // (32*WM) x 256 output tile over a contiguous range of 128-deep k-blocks (= scale groups) on the fp8 matrix instruction.
 //
 //   - activations (e4m3 bytes) and weights (packed int4 codes) both go global -> LDS without touching registers
-//     (global_load_lds_dwordx4), one k-block per stage, three stages.  A 16-token x 128-byte activation operand is a
+//     (global_load_lds_dwordx4), one k-block per stage, three to six stages.  A 16-token x 128-byte activation operand is a
 //     2 KiB fragment filled by two loads of 64 contiguous bytes per row, its 16-byte pieces swizzled so that the
 //     read-back is free of bank conflicts; a weight fragment (16 columns x 128 k) is 1 KiB of codes, one contiguous
 //     load, read back 16 bytes per lane in lane order and expanded to the 32 operand bytes with one shift and two ANDs
@@ -36,10 +36,11 @@ struct W4A8TileParams {
 };
 
 constexpr int w4a8_tile_stage_bytes(int wm) { return (2 * wm) * 2048 + 16 * 1024; }
-constexpr int w4a8_tile_stages() { return 3; }
+// LDS stages: as many as 160 KiB hold.
+constexpr int w4a8_tile_stages(int wm) { return wm == 2 ? 6 : wm == 4 ? 4 : 3; }
 // per stage: operands, 1 KiB of group sums, 1 KiB of weight scales
 constexpr size_t w4a8_tile_lds_bytes(int wm) {
-  return static_cast<size_t>(w4a8_tile_stages()) * (w4a8_tile_stage_bytes(wm) + 2048);
+  return static_cast<size_t>(w4a8_tile_stages(wm)) * (w4a8_tile_stage_bytes(wm) + 2048);
 }
 
 __device__ __forceinline__ i32x8 w4a8_expand(i32x4 p) {
@@ -53,14 +54,14 @@ __device__ __forceinline__ i32x8 w4a8_expand(i32x4 p) {
   return r;
 }
 
-// WM = 8: 256-token tiles.  WM = 4: 128-token tiles.
+// WM = 8: 256-token tiles.  WM = 4: 128-token tiles.  WM = 2: 64-token tiles.
 // GROUP = 64 (128-token tiles only): a k-block holds two scale groups.  Its two rows of group sums and of weight scales
 // ride the same loads as the one row of GROUP = 128 (the lanes that repeat data there fetch the second row here), and
 // every MFMA is issued twice, once with the weight bytes of the upper 64 k cleared and once with the lower ones
 // cleared (this lane's 32 k lie in half lane / 32), each with its own addend and scales.
 template <typename TO, int WM, int GROUP = 128>
 __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
-  static_assert(WM == 8 || WM == 4, "256- or 128-token tiles");
+  static_assert(WM == 8 || WM == 4 || WM == 2, "256-, 128- or 64-token tiles");
   static_assert(GROUP == 128 || (GROUP == 64 && WM == 4), "group 64 runs on 128-token tiles");
   constexpr int GH = 128 / GROUP;
   constexpr int WAVES_N = 4;
@@ -72,7 +73,12 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
   constexpr int AFW = AF / 4;   // ... fetched by each of the wavefronts 0..3
   constexpr int STAGE_BYTES = w4a8_tile_stage_bytes(WM);
   constexpr int W_BASE = AF * FRAG;  // weight fragments of a stage start here
-  constexpr int NS = w4a8_tile_stages();
+  constexpr int NS = w4a8_tile_stages(WM);
+  // k-blocks between two barriers.  A k-block of the 64-token tile is 8 MFMAs per wavefront, about 512 of the 2000 cycles
+  // it takes: the rest is the chain barrier, LDS reads, code expansion, MFMA, scale FMAs, run by all wavefronts at once.
+  // Six stages in place of three alone left n = 25600, k = 5120 at 64 tokens at 29.8 us, two k-blocks per barrier
+  // bring it to 28.3: the wavefronts drift apart and fill each other's gaps.
+  constexpr uint32_t STEP = WM == 2 ? 2 : 1;
   constexpr int XS_BASE = NS * STAGE_BYTES;    // [NS][256] group sums
   constexpr int WS_BASE = XS_BASE + NS * 1024;  // [NS][256 fp16 (+ 512 bytes unused)] weight scales
 
@@ -199,6 +205,16 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
     }
     const uint32_t f0h = f0 + 1024 - 64;
     const uint32_t f1 = f0 + FRAG, f1h = f0h + FRAG;
+    if (AFW == 1) {  // one activation fragment per wavefront (64-token tiles)
+      asm volatile(
+          "s_nop 4\n\t"
+          "s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %3\n\t"
+          "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %3 offset:64"
+          :
+          : "v"(d_voff[0]), "s"(f0), "s"(f0h), "s"(src)
+          : "memory", "m0");
+      return;
+    }
     if (AFW == 2) {  // two activation fragments per wavefront (128-token tiles)
       asm volatile(
           "s_nop 4\n\t"
@@ -228,22 +244,23 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
           "s"(f2h), "s"(f3), "s"(f3h), "s"(src)
         : "memory", "m0");
   };
-  // Everything this wavefront issued has landed except the loads of the youngest stage (vmcnt retires in issue order;
+  // Everything this wavefront issued has landed except the loads of the youngest NS - 2 * STEP stages (vmcnt retires in issue order;
   // a wavefront issues the same loads every stage: 4 weight loads with or without the weight-scale load, or 2*AFW
   // activation loads with or without the group-sum load).
   // This wavefront's fragment reads of the stage have returned: behind the barrier other wavefronts refill the slot they
   // came from, and a bare s_barrier waits for nothing by itself.
   auto reads_done = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
   auto wait_stage = [&]() {
+    constexpr int AHEAD = NS - 2 * STEP;
     if (!stage_act) {
       if (wave == 4)
-        asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD * 5) : "memory");
       else
-        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD * 4) : "memory");
     } else if (has_xs_load) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * AFW + 1) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD * (2 * AFW + 1)) : "memory");
     } else {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * AFW) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD * 2 * AFW) : "memory");
     }
   };
 
@@ -367,19 +384,24 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
   // ---- schedule: stage c computes k-block c out of LDS slot c % NS and, right behind its first MFMA, issues the loads
   // of k-block c+NS-1 into the slot stage c-1 used (every wavefront left it at the previous barrier).  At the end of
   // the stage the loads of k-block c+1 have to have landed; the barrier makes them visible to all wavefronts.
-  load_scales(0);
-  load_operands(0);
-  load_scales(1);
-  load_operands(1);
+#pragma unroll
+  for (uint32_t c = 0; c < NS - STEP; ++c) {
+    load_scales(c);
+    load_operands(c);
+  }
   wait_stage();
   __syncthreads();
 
-  for (uint32_t c = 0; c < kb_count; ++c) {
-    if (idle) {
-      load_scales(c + NS - 1);
-      load_operands(c + NS - 1);
-    } else {
-      compute(c % NS, c + NS - 1);
+  for (uint32_t c = 0; c < kb_count; c += STEP) {
+#pragma unroll
+    for (uint32_t h = 0; h < STEP; ++h) {
+      if (h > 0 && c + h >= kb_count) break;  // (the last step of an odd number of k-blocks: only the drain below follows)
+      if (idle) {
+        load_scales(c + h + NS - STEP);
+        load_operands(c + h + NS - STEP);
+      } else {
+        compute((c + h) % NS, c + h + NS - STEP);
+      }
     }
     wait_stage();  // operands and scales of c+1
     reads_done();

@@ -138,6 +138,21 @@ def test_gemm_tile_kernel(ops, oracle, tile_kernels, out_dtype, m, n, k):
     H.check_gemm(out, ref, out_dtype, "w4a8 tile m=%d n=%d k=%d" % (m, n, k))
 
 
+# 64- and 128-token tiles keep five and three k-blocks of loads in flight: fewer k-blocks than that, as many, one more, parts
+# of four and five k-blocks; and every count of row tiles that hold tokens, with M % 4 == 0 and without
+@pytest.mark.parametrize("m,n,k", [(33, 272, 128), (48, 4112, 512), (49, 256, 640), (63, 528, 768), (64, 256, 896), (64, 272, 1152),
+                                   (65, 272, 256), (96, 256, 384), (127, 528, 512), (128, 256, 640)])
+def test_gemm_tile_kernel_few_tokens(ops, oracle, tile_kernels, m, n, k):
+    from ksanallm_amd import lib as L
+    assert L.select_tile(L.KIND_W4A8, m, n, k, H.BF16)["block_m"] == (64 if m <= 64 else 128)
+    w, scales = make_weight(n + k + m, k, n)
+    x = make_act(m * 3 + n, m, k, H.BF16)
+    xq, xsum = ops.w4a8_static_quant(x.cuda(), torch.tensor([0.05], dtype=torch.float32).cuda(), False)
+    out = ops.w4a8_gemm(xq, xsum, ops.w4a8_repack_weight(w.cuda()), scales.cuda(), 0.03, n, torch.bfloat16)
+    ref = oracle.w4a8_gemm(xq.cpu().numpy(), w.numpy().view(np.int8), H.bits_of(scales), 0.03)
+    H.check_gemm(out, ref, H.BF16, "w4a8 tile m=%d n=%d k=%d" % (m, n, k))
+
+
 @pytest.mark.parametrize("m,n,k", [(3, 8192, 512), (20, 8192, 512), (16, 16384, 256), (32, 16384, 256), (1, 4096, 1024)])
 def test_gemm_streaming_kernel_variants(ops, oracle, m, n, k):
     """The streaming kernel's other instantiations: four strips per workgroup with eight wavefronts (n = 8192) and with
