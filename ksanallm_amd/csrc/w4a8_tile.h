@@ -36,7 +36,9 @@ struct W4A8TileParams {
 };
 
 constexpr int w4a8_tile_stage_bytes(int wm) { return (2 * wm) * 2048 + 16 * 1024; }
-// LDS stages: as many as 160 KiB hold.
+// LDS stages: as many as 160 KiB hold (128-token tiles, four in place of three: n = 25600, k = 5120 at 128 tokens 41.5 ->
+// 39.7 us; 64-token tiles, six, with STEP below: n = 28672, k = 1024 at 64 tokens 26.0 -> 14.4, n = 14336, k = 8192
+// 29.7 -> 26.7).
 constexpr int w4a8_tile_stages(int wm) { return wm == 2 ? 6 : wm == 4 ? 4 : 3; }
 // per stage: operands, 1 KiB of group sums, 1 KiB of weight scales
 constexpr size_t w4a8_tile_lds_bytes(int wm) {
