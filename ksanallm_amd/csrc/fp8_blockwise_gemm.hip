@@ -360,7 +360,7 @@ int launch_fp8_tile_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s) 
   p.numel = q.numel;
   p.top_k = q.top_k;
   p.scale_rows = q.scale_rows;
-  p.deep_rows = deep ? 160 : 0;
+  p.deep_limit = deep ? 161 : 0;
   fp8_tile_kernel<TO, true, WM><<<p.tiles_m * p.tiles_n, 512, lds, s>>>(p);
   return KSQ_OK;
 }

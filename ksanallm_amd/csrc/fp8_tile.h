@@ -40,7 +40,7 @@ struct Fp8TileParams {
   const int32_t* num_post_pad;
   const float* topk_w;
   uint32_t numel, top_k, scale_rows;  // scale_rows = ceil(N/128): rows of one expert's b_s
-  uint32_t deep_rows;                 // 256-slot blocks of at most this many slots run on the three-stage tile
+  uint32_t deep_limit;                // 256-slot blocks that hold fewer slots run on the three-stage tile (0: none does)
 };
 
 __device__ __forceinline__ f32x4 mfma_fp8_k128(i32x8 a, i32x8 b, f32x4 c) {
@@ -465,7 +465,7 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   }
 }
 
-// A 256-slot block of the grouped form with at most 160 tokens (deep_rows) runs the 160-token tile's code: three stages
+// A 256-slot block of the grouped form with at most 160 tokens (deep_limit - 1) runs the 160-token tile's code: three stages
 // of 52 KiB instead of two of 64, because what bounds such a block is the stream of its weights, and only the activation
 // fragments that hold tokens are fetched.  160 is what the LDS has room for; that it lies above 128 matters: with 125
 // tokens per expert on average four experts in ten hold more than 128, and in 128-slot blocks each of those reads its
@@ -483,7 +483,9 @@ __global__ void __launch_bounds__(512, 1) fp8_tile_kernel(Fp8TileParams p) {
       const bool is_row = static_cast<uint32_t>(p.sorted_ids[m0 + h * 64 + (threadIdx.x & 63)]) < p.numel;
       rows += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(is_row)));
     }
-    if (__builtin_amdgcn_readfirstlane(rows) <= p.deep_rows) {
+    // (strictly below: where K leaves no room for three stages the limit is 0, and the launch has not asked for their LDS -
+    // a block without any token must then not come here either)
+    if (__builtin_amdgcn_readfirstlane(rows) < p.deep_limit) {
       fp8_tile_body<TO, true, 5, 256>(p, lds);
       return;
     }

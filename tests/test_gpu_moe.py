@@ -577,6 +577,33 @@ def test_grouped_fp8_tile_kernel_at_the_edges_of_the_three_stage_tile(ops, oracl
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
+def test_grouped_fp8_tile_kernel_where_three_stages_do_not_fit(ops, oracle):
+    """K > 28672 leaves no room in the LDS for three stages: every 256-slot block then runs on two, one without any token
+    (which the alignment never makes, but a caller's own permutation may) among them."""
+    n, k, rows = 272, 28800, [100, 0, 200, 160]
+    E, T = len(rows), sum(rows)
+    g = H.gen(7900)
+    bq, bs = _fp8_experts(oracle, 7910, E, n, k)
+    x = torch.randn((T, k), generator=g).to(torch.bfloat16)
+    q, s = ops.per_token_group_quant_fp8(x.cuda(), k, 128, False)
+    wp, wsc = ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda()
+    flat = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
+    sorted_ids = torch.full((E, 256), T, dtype=torch.int32)   # one block per expert, pad slots at the end
+    for e in range(E):
+        mine = torch.nonzero(flat == e).flatten().to(torch.int32)
+        sorted_ids[e, :mine.numel()] = mine
+    out = ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, None, sorted_ids.flatten().cuda(), torch.arange(E, dtype=torch.int32).cuda(),
+                                     torch.tensor([E * 256], dtype=torch.int32).cuda(), T, 1, 256, torch.bfloat16)
+    aligned = ops.moe_align_block_size(flat.reshape(T, 1).cuda(), E, 128)
+    short = ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, None, *aligned, T, 1, 128, torch.bfloat16)
+    assert torch.equal(out.view(torch.int16), short.view(torch.int16))
+    qh, sh = q.cpu().numpy(), s.cpu().numpy()
+    pick = [0, 15, 99, 100, 260, 299, 300, 459]   # the oracle on some rows of every expert
+    ref = np.stack([oracle.fp8_blockwise_gemm(qh[t:t + 1], np.ascontiguousarray(sh[t:t + 1]), bq[flat[t]], bs[flat[t]], False)[0]
+                    for t in pick])
+    H.check_gemm(out[pick], ref, H.BF16, "grouped fp8 tile kernel, K = %d" % k)
+
+
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
 @pytest.mark.parametrize("T,E,topk,hidden,inter", [(1, 8, 2, 256, 128), (48, 16, 4, 512, 256), (200, 8, 2, 384, 640),
                                                    (1200, 8, 2, 512, 256)])   # the last: 300 slots per expert, 256-slot blocks
