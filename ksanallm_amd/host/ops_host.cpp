@@ -4,13 +4,15 @@
 // for torch.cuda.current_stream(), 1.8 us for torch.empty), and a MoE block of one token 36 us.
 //
 // The library is not linked: bind() takes the addresses of its entry points from the ctypes binding, so that both sides
-// always call the same library.  Outputs and scratch come from torch's caching allocator on the current stream, per
-// call: nothing is shared between streams or threads, and nothing is kept.
+// always call the same library.  Outputs and scratch come from torch's caching allocator, per call: nothing is shared
+// between streams or threads, and nothing is kept.  A call runs on the device of its first tensor and on that device's
+// current stream, whatever device is current outside: the allocator hands scratch out, and takes it back, for that stream.
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
@@ -117,7 +119,15 @@ size_t dim(const at::Tensor& t, int64_t d, int64_t dims, const char* what) {
   return static_cast<size_t>(t.size(d));
 }
 
-// ------------------------------------------------------------------------------------------------ allocation, stream
+// ------------------------------------------------------------------------------------------------ device, allocation, stream
+// Makes the tensor's device the current one for the rest of the call.
+struct OnDevice {
+  c10::OptionalDeviceGuard guard;
+  explicit OnDevice(const at::Tensor& t) {
+    if (t.is_cuda()) guard.reset_device(t.device());
+  }
+};
+
 at::Tensor empty(std::initializer_list<size_t> shape, at::ScalarType dtype, const at::Tensor& like) {
   int64_t s[4];
   int n = 0;
@@ -143,6 +153,7 @@ struct Scratch {  // nullptr and 0 where nothing is needed
   }
 };
 
+// of the current device
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
 // fp32, flat, contiguous: the tensor itself when it is that already
@@ -154,6 +165,7 @@ at::Tensor flat(const at::Tensor& t, at::ScalarType dtype) {
 // ------------------------------------------------------------------------------------------------ the calls
 at::Tensor w4a16_gemm(const Args& a) {
   const at::Tensor &x = tensor(a.v[0]), &w = tensor(a.v[1]), &s = tensor(a.v[2]);
+  const OnDevice on(x);
   const at::Tensor* z = tensor_or_null(a.v[3]);
   const size_t n = size_arg(a.v[4]), k = size_arg(a.v[5]), group = size_arg(a.v[6]);
   const at::Tensor *given = tensor_or_null(a.v[7]), *ws = tensor_or_null(a.v[8]);
@@ -174,6 +186,7 @@ at::Tensor w4a16_gemm(const Args& a) {
 // codes and scales of per_token_group_quant_fp8
 std::pair<at::Tensor, at::Tensor> group_quant(const at::Tensor& x, size_t k, size_t group, bool column_major, bool fuse,
                                               const at::Tensor* q_given, const at::Tensor* s_given) {
+  const OnDevice on(x);
   const size_t m = x.dim() ? x.size(0) : 0;
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
   at::Tensor q = q_given ? *q_given : empty({m, k}, at::kByte, x);
@@ -187,6 +200,7 @@ std::pair<at::Tensor, at::Tensor> group_quant(const at::Tensor& x, size_t k, siz
 
 at::Tensor fp8_blockwise_gemm(const Args& a) {
   const at::Tensor &aq = tensor(a.v[0]), &as = tensor(a.v[1]), &b = tensor(a.v[2]), &bs = tensor(a.v[3]);
+  const OnDevice on(aq);
   const at::ScalarType odt = dtype_arg(a.v[4]);
   const at::Tensor *given = tensor_or_null(a.v[5]), *ws = tensor_or_null(a.v[6]);
   const size_t m = dim(aq, 0, 2, "fp8_blockwise_gemm: a_q"), k = aq.size(1), n = b.dim() ? b.size(0) : 0;
@@ -203,6 +217,7 @@ at::Tensor fp8_blockwise_gemm(const Args& a) {
 
 std::pair<at::Tensor, at::Tensor> w4a8_static_quant(const Args& a) {
   const at::Tensor &x = tensor(a.v[0]), &scale = tensor(a.v[1]);
+  const OnDevice on(x);
   const bool per_channel = bool_arg(a.v[2]), per_token = bool_arg(a.v[3]);
   const size_t group = size_arg(a.v[4]);
   const size_t m = dim(x, 0, 2, "w4a8_static_quant: x"), k = x.size(1);
@@ -218,6 +233,7 @@ std::pair<at::Tensor, at::Tensor> w4a8_static_quant(const Args& a) {
 
 at::Tensor w4a8_gemm(const Args& a) {
   const at::Tensor &aq = tensor(a.v[0]), &xsum = tensor(a.v[1]), &w = tensor(a.v[2]), &scales = tensor(a.v[3]);
+  const OnDevice on(aq);
   const double alpha = float_arg(a.v[4]);
   const size_t n = size_arg(a.v[5]);
   const at::ScalarType odt = dtype_arg(a.v[6]);
@@ -241,6 +257,7 @@ at::Tensor w4a8_gemm(const Args& a) {
 
 std::pair<at::Tensor, at::Tensor> moe_topk_softmax(const Args& a) {
   const at::Tensor& gating = tensor(a.v[0]);
+  const OnDevice on(gating);
   const size_t top_k = size_arg(a.v[1]);
   const int norm = bool_arg(a.v[2]);
   const float scaling = static_cast<float>(float_arg(a.v[3]));
@@ -254,6 +271,7 @@ std::pair<at::Tensor, at::Tensor> moe_topk_softmax(const Args& a) {
 
 std::pair<at::Tensor, at::Tensor> moe_grouped_topk(const Args& a) {
   const at::Tensor& gating = tensor(a.v[0]);
+  const OnDevice on(gating);
   const size_t top_k = size_arg(a.v[1]), groups = size_arg(a.v[2]), topk_group = size_arg(a.v[3]);
   const int sigmoid = bool_arg(a.v[4]);
   const at::Tensor* bias = tensor_or_null(a.v[5]);
@@ -305,6 +323,7 @@ struct Routed {  // the router's outputs, flat
 
 at::Tensor fused_moe_w4a16(const Args& a) {
   const at::Tensor &x = tensor(a.v[0]), &w13 = tensor(a.v[1]), &s13 = tensor(a.v[2]), &w2 = tensor(a.v[3]), &s2 = tensor(a.v[4]);
+  const OnDevice on(x);
   const Routed r(tensor(a.v[5]), tensor(a.v[6]));
   const size_t E = size_arg(a.v[7]), hidden = size_arg(a.v[8]), inter = size_arg(a.v[9]), group = size_arg(a.v[10]);
   const bool block_given = a.v[11] != Py_None;
@@ -364,6 +383,7 @@ at::Tensor fused_moe_w4a16(const Args& a) {
 
 at::Tensor fused_moe_fp8_blockwise(const Args& a) {
   const at::Tensor &x = tensor(a.v[0]), &w13 = tensor(a.v[1]), &s13 = tensor(a.v[2]), &w2 = tensor(a.v[3]), &s2 = tensor(a.v[4]);
+  const OnDevice on(x);
   const Routed r(tensor(a.v[5]), tensor(a.v[6]));
   const bool block_given = a.v[7] != Py_None;
   size_t block_m = block_given ? size_arg(a.v[7]) : 0;

@@ -2,8 +2,13 @@
 
 Each function names the ``Invoke*`` wrapper of the reference it stands for
 (src/ksana_llm/kernels/nvidia/basic_kernel_wrapper.h:32-115,295-336 and moe_kernel_wrapper.h:28-88) and forwards to
-the C-ABI of libksq_hip.so on the tensor's current stream.  Torch is used for device memory and streams only.
+the C-ABI of libksq_hip.so on the device of its first tensor and that device's current stream.  Torch is used for device
+memory and streams only.
 """
+import contextlib
+import functools
+import inspect
+
 import torch
 
 from . import lib as _l
@@ -38,6 +43,19 @@ def _stream():
     return _h.current_stream()
 
 
+def _on_device(fn):
+    """Runs fn with its first tensor's device current: its scratch then belongs to the stream that it launches on.  (The C++
+    side does the same for the hot calls.)"""
+    first = next(iter(inspect.signature(fn).parameters))
+
+    @functools.wraps(fn)
+    def call(*args, **kwargs):
+        t = args[0] if args else kwargs.get(first)
+        with torch.cuda.device_of(t) if isinstance(t, torch.Tensor) else contextlib.nullcontext():
+            return fn(*args, **kwargs)
+    return call
+
+
 def _ptr(t):
     if t is None:
         return None
@@ -54,6 +72,7 @@ def _need_bytes(t, nbytes, what):
         raise ValueError("%s: tensor holds %d bytes, the declared layout needs %d" % (what, have, nbytes))
 
 
+@_on_device
 def repack_weight(src, layout, E, K, N):
     """Checkpoint int4 weight -> CDNA4 tile layout (uint8 tensor of E*K*N/2 bytes)."""
     _need_bytes(src, E * K * N // 2, "repack_weight")
@@ -62,6 +81,7 @@ def repack_weight(src, layout, E, K, N):
     return dst
 
 
+@_on_device
 def unpack_weight(packed, layout, E, K, N):
     """Inverse of :func:`repack_weight`; returns the checkpoint layout as int32 (GPTQ/AWQ) or uint8/int8 bytes."""
     if layout == _l.SRC_GPTQ:
@@ -76,6 +96,7 @@ def unpack_weight(packed, layout, E, K, N):
     return dst
 
 
+@_on_device
 def repack_scales(src, layout, E, K, N, group):
     _need_bytes(src, E * (K // group) * N * src.element_size(), "repack_scales")
     dst = torch.empty(E * (K // group) * N, dtype=src.dtype, device=src.device)
@@ -83,6 +104,7 @@ def repack_scales(src, layout, E, K, N, group):
     return dst
 
 
+@_on_device
 def unpack_scales(packed, layout, E, K, N, group):
     G = K // group
     shape = ((E, G, N) if E > 1 else (G, N)) if layout == _l.SCALE_GN else (E, N, G)
@@ -91,6 +113,7 @@ def unpack_scales(packed, layout, E, K, N, group):
     return dst
 
 
+@_on_device
 def repack_zeros(src, layout, K, N, group):
     _need_bytes(src, (K // group) * N // (2 if layout == _l.ZERO_AWQ_PACKED else 1), "repack_zeros")
     dst = torch.empty((K // group) * N, dtype=torch.uint8, device=src.device)
@@ -98,6 +121,7 @@ def repack_zeros(src, layout, K, N, group):
     return dst
 
 
+@_on_device
 def unpack_zeros(packed, layout, K, N, group):
     G = K // group
     if layout == _l.ZERO_AWQ_PACKED:
@@ -123,6 +147,7 @@ def w4a16_gemm(x, w_packed, scales_packed, zeros_packed, n, k, group, out=None, 
     return _h.w4a16_gemm(x, w_packed, scales_packed, zeros_packed, n, k, group, out, workspace)
 
 
+@_on_device
 def w4a16_gemm_f32(x, w_packed, scales_packed, zeros_packed, n, k, group, workspace=None):
     """ksq_w4a16_gemm_f32: the same kernels and plan as w4a16_gemm with the fp32 sums stored unrounded (verification)."""
     m = x.shape[0]
@@ -150,6 +175,7 @@ def fp8_blockwise_gemm(a_q, a_s, b, b_s, out_dtype=torch.bfloat16, out=None, wor
     return _h.fp8_blockwise_gemm(a_q, a_s, b, b_s, out_dtype, out, workspace)
 
 
+@_on_device
 def fp8_blockwise_gemm_f32(a_q, a_s, b, b_s, workspace=None):
     """ksq_fp8_blockwise_gemm_f32: the same kernels and plan as fp8_blockwise_gemm with the fp32 sums stored unrounded."""
     m, k = a_q.shape
@@ -167,6 +193,7 @@ def fp8_blockwise_gemm_f32(a_q, a_s, b, b_s, workspace=None):
 
 
 # ----------------------------------------------------------------------------------------------- MoE
+@_on_device
 def moe_align_block_size(topk_ids, num_experts, block_m):
     """InvokeSglMoeAlignBlockSize / InvokeMoeAlignBlockSize: (sorted_ids, expert_ids, num_post_pad) int32 tensors."""
     ids = topk_ids.reshape(-1)
@@ -182,6 +209,7 @@ def moe_align_block_size(topk_ids, num_experts, block_m):
     return sorted_ids, expert_ids, num_post_pad
 
 
+@_on_device
 def moe_w4a16_gemm(x, w_packed, scales_packed, topk_w, sorted_ids, expert_ids, num_post_pad, numel, top_k, E, n, k,
                    group, block_m, out=None):
     """InvokeMoeWna16Gemm / InvokeFusedMoeGptqAwqKernel: out [numel, n]."""
@@ -196,6 +224,7 @@ def moe_w4a16_gemm(x, w_packed, scales_packed, topk_w, sorted_ids, expert_ids, n
     return out
 
 
+@_on_device
 def moe_w4a16_gate_up_silu(x, w_packed, scales_packed, sorted_ids, expert_ids, num_post_pad, numel, top_k, E, n, k, group,
                            block_m, out=None):
     """The first MoE GEMM with silu*mul in its epilogue (any block size of moe_w4a16_gemm): out [numel, n/2], bit for bit what
@@ -225,6 +254,7 @@ def moe_grouped_topk(gating, top_k, num_expert_group=1, topk_group=1, scoring_fu
                                routed_scaling_factor)
 
 
+@_on_device
 def silu_and_mul(x, out=None):
     """InvokeSiluAndMul: x [rows, 2*inter] -> [rows, inter]."""
     rows, two = x.shape
@@ -234,6 +264,7 @@ def silu_and_mul(x, out=None):
     return out
 
 
+@_on_device
 def moe_sum(x, out=None):
     """InvokeMoeSum: x [tokens, topk, d] -> [tokens, d]."""
     tokens, topk, d = x.shape
@@ -256,6 +287,7 @@ def fused_moe_w4a16(x, w13_packed, s13_packed, w2_packed, s2_packed, topk_ids, t
                               block_m, FEW_TOKENS)
 
 
+@_on_device
 def moe_fp8_blockwise_gemm(a_q, a_s, a_s_column_major, b, b_s, topk_w, sorted_ids, expert_ids, num_post_pad, numel,
                            top_k, block_m, out_dtype=torch.bfloat16, out=None):
     """fp8_w8a8 block-quantized fused_moe_kernel launch: a_q [rows,k] e4m3 bytes, b [E,n,k] packed by fp8_repack_weight,
@@ -279,6 +311,7 @@ def fused_moe_fp8_blockwise(x, w13, w13_scale, w2, w2_scale, topk_ids, topk_w, b
     return _h.fused_moe_fp8_blockwise(x, w13, w13_scale, w2, w2_scale, topk_ids, topk_w, block_m, FEW_TOKENS)
 
 
+@_on_device
 def fp8_e4m3_quantize(x, scale=None):
     """Fp8E4m3Quantize: x [channels, size] -> (codes uint8, scale fp32 [channels]); scale given = static."""
     channels, size = x.shape
@@ -289,6 +322,7 @@ def fp8_e4m3_quantize(x, scale=None):
     return q, s
 
 
+@_on_device
 def fp8_quantized_matmul(a_q, a_scale, b, b_scale, out_dtype=torch.bfloat16, out=None, workspace=None):
     """Fp8QuantizedMatMul: a_q [m,k] e4m3 bytes, b [n,k] packed by fp8_repack_weight, one fp32 device scale each."""
     m, k = a_q.shape
@@ -307,6 +341,7 @@ def sort_g_idx(g_idx):
     return torch.argsort(g_idx.to(torch.int64), stable=True).to(torch.int32)
 
 
+@_on_device
 def repack_weight_act_order(qweight, perm, K, N):
     """gptq_marlin_repack with a permutation: qweight [K/8, N] int32 (GPTQ), perm int32 [K] -> packed weight."""
     out = torch.empty(_lib.ksq_w4a16_packed_weight_bytes(1, K, N), dtype=torch.uint8, device=qweight.device)
@@ -314,6 +349,7 @@ def repack_weight_act_order(qweight, perm, K, N):
     return out
 
 
+@_on_device
 def permute_columns(x, perm, out=None):
     """out[r, j] = x[r, perm[j]]."""
     m, k = x.shape
@@ -323,6 +359,7 @@ def permute_columns(x, perm, out=None):
     return out
 
 
+@_on_device
 def moe_permute_columns(x, perm, topk_ids, top_k, out=None):
     """out[s, j] = x[s // top_k, perm[topk_ids[s], j]]: x [rows, k], perm int32 [E, k], topk_ids int32 [numel]."""
     k = x.shape[1]
@@ -334,6 +371,7 @@ def moe_permute_columns(x, perm, topk_ids, top_k, out=None):
     return out
 
 
+@_on_device
 def fp8_repack_weight(w):
     """Checkpoint-layout e4m3 weight [N, K] or [E, N, K] (uint8) -> the packed fragment layout the FP8 GEMMs read."""
     E = w.shape[0] if w.dim() == 3 else 1
@@ -343,6 +381,7 @@ def fp8_repack_weight(w):
     return out
 
 
+@_on_device
 def fp8_unpack_weight(packed):
     """Inverse of :func:`fp8_repack_weight` (the tensor keeps the logical shape [N, K] / [E, N, K])."""
     E = packed.shape[0] if packed.dim() == 3 else 1
@@ -353,6 +392,7 @@ def fp8_unpack_weight(packed):
 
 
 # ----------------------------------------------------------------------------------------------- W4A8
+@_on_device
 def w4a8_repack_weight(w):
     """W4A8 weight [K, N/2] (int8/uint8, two's-complement nibbles, low nibble = even column: the input of the
     reference's PreprocessWeightsForMixedGemm) -> the packed fragment layout ksq_w4a8_gemm reads."""
@@ -362,6 +402,7 @@ def w4a8_repack_weight(w):
     return out
 
 
+@_on_device
 def w4a8_unpack_weight(packed, K, N):
     """Inverse of :func:`w4a8_repack_weight`: uint8 [K, N/2]."""
     out = torch.empty((K, N // 2), dtype=torch.uint8, device=packed.device)
@@ -375,6 +416,7 @@ def w4a8_static_quant(x, scale, per_channel=False, per_token=False, group=128):
     return _h.w4a8_static_quant(x, scale, per_channel, per_token, group)
 
 
+@_on_device
 def w4a8_group_sums(a_q, group=128):
     """Group sums of activations that are e4m3 already (uint8 [m,k]) -> fp32 [k/group, m]; group 128 or 64."""
     m, k = a_q.shape
