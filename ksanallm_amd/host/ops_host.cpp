@@ -48,12 +48,20 @@ struct PyRaised {};
   throw PyRaised{};
 }
 
+// Lets other Python threads run: around the library's calls and around allocations, either of which may wait for the
+// device (an allocator that has to ask the driver, or to give memory back first).
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
 template <typename F>
 void call(F&& f) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
+  {
+    const WithoutGil no_gil;
+    rc = f();
+  }
   if (rc == 0) return;
   PyObject* r = PyObject_CallFunction(check_fn, "i", rc);
   Py_XDECREF(r);
@@ -133,6 +141,7 @@ at::Tensor empty(std::initializer_list<size_t> shape, at::ScalarType dtype, cons
   int n = 0;
   for (size_t v : shape) s[n++] = static_cast<int64_t>(v);
   const at::IntArrayRef sizes(s, n);
+  const WithoutGil no_gil;
   if (!like.is_cuda()) return at::empty(sizes, like.options().dtype(dtype));
   return at::Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));
 }

@@ -1,0 +1,42 @@
+"""The host side of ops.py's hot calls on a machine without a GPU: what is refused, and before which other step.  A call on CPU
+tensors goes through its size checks and the allocation of its outputs and is refused (AssertionError) before any launch."""
+import threading
+import time
+
+import pytest
+import torch
+
+
+def test_allocation_runs_without_the_interpreter_lock():
+    """An allocation that takes its time (here: outputs that torch is told to fill) does not stop the other Python threads."""
+    from ksanallm_amd import ops
+    before = torch.are_deterministic_algorithms_enabled(), torch.utils.deterministic.fill_uninitialized_memory, torch.get_num_threads()
+    stop, gaps = threading.Event(), []
+
+    def tick():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.001)
+            now = time.perf_counter()
+            gaps.append(now - last)
+            last = now
+    thread = threading.Thread(target=tick)
+    torch.use_deterministic_algorithms(True)
+    torch.utils.deterministic.fill_uninitialized_memory = True
+    torch.set_num_threads(1)
+    try:
+        thread.start()
+        time.sleep(0.02)
+        del gaps[:]
+        t0 = time.perf_counter()
+        with pytest.raises(AssertionError, match="device-resident"):
+            ops.moe_topk_softmax(torch.zeros((1, 8)), 1 << 28)   # two outputs of 1 GiB
+        took = time.perf_counter() - t0
+    finally:
+        stop.set()
+        thread.join()
+        torch.use_deterministic_algorithms(before[0])
+        torch.utils.deterministic.fill_uninitialized_memory = before[1]
+        torch.set_num_threads(before[2])
+    assert took > 0.05, "the allocation was over too soon to tell (%.3f s)" % took
+    assert max(gaps) < took / 3, "another thread stood still for %.3f of %.3f s" % (max(gaps), took)
