@@ -210,13 +210,12 @@ std::pair<at::Tensor, at::Tensor> group_quant(const at::Tensor& x, size_t k, siz
 at::Tensor fp8_blockwise_gemm(const Args& a) {
   const at::Tensor &aq = tensor(a.v[0]), &as = tensor(a.v[1]), &b = tensor(a.v[2]), &bs = tensor(a.v[3]);
   const OnDevice on(aq);
-  const at::ScalarType odt = dtype_arg(a.v[4]);
   const at::Tensor *given = tensor_or_null(a.v[5]), *ws = tensor_or_null(a.v[6]);
   const size_t m = dim(aq, 0, 2, "fp8_blockwise_gemm: a_q"), k = aq.size(1), n = b.dim() ? b.size(0) : 0;
   need_bytes(as, k / 128 * m * 4, "fp8_blockwise_gemm: activation scales");
   need_bytes(b, n * k, "fp8_blockwise_gemm: weight");
   need_bytes(bs, (n + 127) / 128 * (k / 128) * 4, "fp8_blockwise_gemm: weight scales");
-  at::Tensor out = given ? *given : empty({m, n}, odt, aq);
+  at::Tensor out = given ? *given : empty({m, n}, dtype_arg(a.v[4]), aq);
   const int d = dt(out, true);
   const Scratch scratch(ws, aq, ws ? 0 : lib.fp8_blockwise_workspace_size(m, n, k));
   void *po = ptr(out), *pa = ptr(aq), *pas = ptr(as), *pb = ptr(b), *pbs = ptr(bs), *st = stream();
@@ -245,7 +244,6 @@ at::Tensor w4a8_gemm(const Args& a) {
   const OnDevice on(aq);
   const double alpha = float_arg(a.v[4]);
   const size_t n = size_arg(a.v[5]);
-  const at::ScalarType odt = dtype_arg(a.v[6]);
   const at::Tensor *given = tensor_or_null(a.v[7]), *ws = tensor_or_null(a.v[8]);
   const size_t group = size_arg(a.v[9]);
   const size_t m = dim(aq, 0, 2, "w4a8_gemm: a_q"), k = aq.size(1);
@@ -254,7 +252,7 @@ at::Tensor w4a8_gemm(const Args& a) {
   need_bytes(w, n * k / 2, "w4a8_gemm: packed weight");
   need_bytes(scales, k / group * n * 2, "w4a8_gemm: scales");
   if (scales.scalar_type() != at::kHalf) raise(PyExc_AssertionError, "w4a8_gemm: scales must be float16");
-  at::Tensor out = given ? *given : empty({m, n}, odt, aq);
+  at::Tensor out = given ? *given : empty({m, n}, dtype_arg(a.v[6]), aq);
   const int d = dt(out);
   const Scratch scratch(ws, aq, ws ? 0 : lib.w4a8_workspace_size(m, n, k));
   void *po = ptr(out), *pa = ptr(aq), *pxs = ptr(xsum), *pw = ptr(w), *ps = ptr(scales), *st = stream();

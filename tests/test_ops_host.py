@@ -40,3 +40,18 @@ def test_allocation_runs_without_the_interpreter_lock():
         torch.set_num_threads(before[2])
     assert took > 0.05, "the allocation was over too soon to tell (%.3f s)" % took
     assert max(gaps) < took / 3, "another thread stood still for %.3f of %.3f s" % (max(gaps), took)
+
+
+def test_out_dtype_is_not_looked_at_where_out_is_given():
+    from ksanallm_amd import ops
+    m, n, k = 2, 32, 128
+    a, a_s = torch.zeros((m, k), dtype=torch.uint8), torch.zeros((1, m))
+    out = torch.zeros((m, n), dtype=torch.float16)
+    for bad in (None, "half"):
+        with pytest.raises(AssertionError, match="device-resident"):
+            ops.fp8_blockwise_gemm(a, a_s, torch.zeros((n, k), dtype=torch.uint8), torch.zeros((1, 1)), out_dtype=bad, out=out)
+        with pytest.raises(AssertionError, match="device-resident"):
+            ops.w4a8_gemm(a, a_s, torch.zeros(n * k // 2, dtype=torch.uint8), torch.zeros((1, n), dtype=torch.float16), 1.0, n,
+                          out_dtype=bad, out=out)
+        with pytest.raises(TypeError):   # without out it names the type to allocate
+            ops.fp8_blockwise_gemm(a, a_s, torch.zeros((n, k), dtype=torch.uint8), torch.zeros((1, 1)), out_dtype=bad)
