@@ -116,10 +116,21 @@ void* ptr(const at::Tensor& t) {
 void* ptr(const at::Tensor* t) { return t ? ptr(*t) : nullptr; }
 
 // The C-ABI takes bare pointers: a tensor that is smaller than the layout it is declared to hold would be read past
-// its end on the device, so the size is checked here.
+// its end on the device, so the size is checked here.  (`nbytes` of sizes that the caller states: by product() below.)
 void need_bytes(const at::Tensor& t, size_t nbytes, const char* what) {
   const size_t have = t.numel() * t.element_size();
   if (have < nbytes) raise(PyExc_ValueError, "%s: tensor holds %zu bytes, the declared layout needs %zu", what, have, nbytes);
+}
+
+// the product of sizes, or the largest size where it does not fit: a declared layout that no tensor can hold
+size_t product(std::initializer_list<size_t> factors) {
+  size_t p = 1;
+  bool over = false, zero = false;
+  for (size_t f : factors) {
+    zero |= f == 0;
+    over |= __builtin_mul_overflow(p, f, &p);
+  }
+  return zero ? 0 : over ? SIZE_MAX : p;
 }
 
 size_t dim(const at::Tensor& t, int64_t d, int64_t dims, const char* what) {
@@ -180,10 +191,10 @@ at::Tensor w4a16_gemm(const Args& a) {
   const at::Tensor *given = tensor_or_null(a.v[7]), *ws = tensor_or_null(a.v[8]);
   const size_t m = x.dim() ? x.size(0) : 0;
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
-  need_bytes(x, m * k * 2, "w4a16_gemm: x");
-  need_bytes(w, k * n / 2, "w4a16_gemm: packed weight");
-  need_bytes(s, k / group * n * 2, "w4a16_gemm: scales");
-  if (z) need_bytes(*z, k / group * n, "w4a16_gemm: zero points");
+  need_bytes(x, product({m, k, 2}), "w4a16_gemm: x");
+  need_bytes(w, product({k, n}) / 2, "w4a16_gemm: packed weight");
+  need_bytes(s, product({k / group, n, 2}), "w4a16_gemm: scales");
+  if (z) need_bytes(*z, product({k / group, n}), "w4a16_gemm: zero points");
   const int d = dt(x);
   at::Tensor out = given ? *given : empty({m, n}, x.scalar_type(), x);
   const Scratch scratch(ws, x, ws ? 0 : lib.w4a16_workspace_size(m, n, k, group, d));
@@ -212,9 +223,9 @@ at::Tensor fp8_blockwise_gemm(const Args& a) {
   const OnDevice on(aq);
   const at::Tensor *given = tensor_or_null(a.v[5]), *ws = tensor_or_null(a.v[6]);
   const size_t m = dim(aq, 0, 2, "fp8_blockwise_gemm: a_q"), k = aq.size(1), n = b.dim() ? b.size(0) : 0;
-  need_bytes(as, k / 128 * m * 4, "fp8_blockwise_gemm: activation scales");
-  need_bytes(b, n * k, "fp8_blockwise_gemm: weight");
-  need_bytes(bs, (n + 127) / 128 * (k / 128) * 4, "fp8_blockwise_gemm: weight scales");
+  need_bytes(as, product({k / 128, m, 4}), "fp8_blockwise_gemm: activation scales");
+  need_bytes(b, product({n, k}), "fp8_blockwise_gemm: weight");
+  need_bytes(bs, product({(n + 127) / 128, k / 128, 4}), "fp8_blockwise_gemm: weight scales");
   at::Tensor out = given ? *given : empty({m, n}, dtype_arg(a.v[4]), aq);
   const int d = dt(out, true);
   const Scratch scratch(ws, aq, ws ? 0 : lib.fp8_blockwise_workspace_size(m, n, k));
@@ -248,9 +259,9 @@ at::Tensor w4a8_gemm(const Args& a) {
   const size_t group = size_arg(a.v[9]);
   const size_t m = dim(aq, 0, 2, "w4a8_gemm: a_q"), k = aq.size(1);
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
-  need_bytes(xsum, k / group * m * 4, "w4a8_gemm: group sums");
-  need_bytes(w, n * k / 2, "w4a8_gemm: packed weight");
-  need_bytes(scales, k / group * n * 2, "w4a8_gemm: scales");
+  need_bytes(xsum, product({k / group, m, 4}), "w4a8_gemm: group sums");
+  need_bytes(w, product({n, k}) / 2, "w4a8_gemm: packed weight");
+  need_bytes(scales, product({k / group, n, 2}), "w4a8_gemm: scales");
   if (scales.scalar_type() != at::kHalf) raise(PyExc_AssertionError, "w4a8_gemm: scales must be float16");
   at::Tensor out = given ? *given : empty({m, n}, dtype_arg(a.v[6]), aq);
   const int d = dt(out);
@@ -324,7 +335,7 @@ struct Routed {  // the router's outputs, flat
     numel = tokens * top_k;
     w = flat(topk_w, at::kFloat);
     ids = flat(topk_ids, at::kInt);
-    need_bytes(w, numel * 4, "topk_w");
+    need_bytes(w, product({numel, 4}), "topk_w");
   }
 };
 
@@ -337,11 +348,11 @@ at::Tensor fused_moe_w4a16(const Args& a) {
   size_t block_m = block_given ? size_arg(a.v[11]) : 0;
   const size_t few_tokens = size_arg(a.v[12]);
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
-  need_bytes(x, r.tokens * hidden * 2, "fused_moe_w4a16: x");
-  need_bytes(w13, E * hidden * inter, "fused_moe_w4a16: packed gate / up weight");
-  need_bytes(s13, E * (hidden / group) * inter * 4, "fused_moe_w4a16: gate / up scales");
-  need_bytes(w2, E * hidden * inter / 2, "fused_moe_w4a16: packed down weight");
-  need_bytes(s2, E * (inter / group) * hidden * 2, "fused_moe_w4a16: down scales");
+  need_bytes(x, product({r.tokens, hidden, 2}), "fused_moe_w4a16: x");
+  need_bytes(w13, product({E, hidden, inter}), "fused_moe_w4a16: packed gate / up weight");
+  need_bytes(s13, product({E, hidden / group, inter, 4}), "fused_moe_w4a16: gate / up scales");
+  need_bytes(w2, product({E, hidden, inter}) / 2, "fused_moe_w4a16: packed down weight");
+  need_bytes(s2, product({E, inter / group, hidden, 2}), "fused_moe_w4a16: down scales");
   const int d = dt(x);
   const at::ScalarType t = x.scalar_type();
   void *st = stream(), *px = ptr(x), *pw13 = ptr(w13), *ps13 = ptr(s13), *pw2 = ptr(w2), *ps2 = ptr(s2), *ptw = ptr(r.w),
@@ -396,10 +407,10 @@ at::Tensor fused_moe_fp8_blockwise(const Args& a) {
   size_t block_m = block_given ? size_arg(a.v[7]) : 0;
   const size_t few_tokens = size_arg(a.v[8]);
   const size_t E = dim(w13, 0, 3, "fused_moe_fp8_blockwise: w13"), n1 = w13.size(1), hidden = w13.size(2), inter = n1 / 2;
-  need_bytes(x, r.tokens * hidden * x.element_size(), "fused_moe_fp8_blockwise: x");
-  need_bytes(w2, E * hidden * inter, "fused_moe_fp8_blockwise: down weight");
-  need_bytes(s13, E * ((n1 + 127) / 128) * (hidden / 128) * 4, "fused_moe_fp8_blockwise: gate / up scales");
-  need_bytes(s2, E * ((hidden + 127) / 128) * (inter / 128) * 4, "fused_moe_fp8_blockwise: down scales");
+  need_bytes(x, product({r.tokens, hidden, static_cast<size_t>(x.element_size())}), "fused_moe_fp8_blockwise: x");
+  need_bytes(w2, product({E, hidden, inter}), "fused_moe_fp8_blockwise: down weight");
+  need_bytes(s13, product({E, (n1 + 127) / 128, hidden / 128, 4}), "fused_moe_fp8_blockwise: gate / up scales");
+  need_bytes(s2, product({E, (hidden + 127) / 128, inter / 128, 4}), "fused_moe_fp8_blockwise: down scales");
   const int d = dt(x);
   const at::ScalarType t = x.scalar_type();
   void *st = stream(), *pw13 = ptr(w13), *ps13 = ptr(s13), *pw2 = ptr(w2), *ps2 = ptr(s2), *ptw = ptr(r.w), *pids = ptr(r.ids);

@@ -55,3 +55,22 @@ def test_out_dtype_is_not_looked_at_where_out_is_given():
                           out_dtype=bad, out=out)
         with pytest.raises(TypeError):   # without out it names the type to allocate
             ops.fp8_blockwise_gemm(a, a_s, torch.zeros((n, k), dtype=torch.uint8), torch.zeros((1, 1)), out_dtype=bad)
+
+
+HUGE = 1 << 60   # a size that a caller states beside its tensors: products with it leave 64 bits
+
+
+def test_declared_sizes_beyond_64_bits_do_not_pass_for_small_ones():
+    """The layout that n, k and the number of experts declare is compared with what the tensors hold as an exact number."""
+    from ksanallm_amd import ops
+    x, w, s = torch.zeros((16, 128), dtype=torch.float16), torch.zeros(16, dtype=torch.uint8), torch.zeros(16, dtype=torch.float16)
+    for n, k in ((16, HUGE), (HUGE, 16), (HUGE, HUGE), (1 << 62, 128), (1 << 63, 128)):
+        with pytest.raises((ValueError, OverflowError)):
+            ops.w4a16_gemm(x, w, s, None, n, k, 128, out=torch.zeros(1, dtype=torch.float16))
+    a, a_s = torch.zeros((16, 128), dtype=torch.uint8), torch.zeros((1, 16))
+    with pytest.raises(ValueError):
+        ops.w4a8_gemm(a, a_s, w, s, 1.0, HUGE, out=torch.zeros(1, dtype=torch.float16))
+    ids, tw = torch.zeros((8, 2), dtype=torch.int32), torch.zeros((8, 2))
+    for E, hidden, inter in ((HUGE, 128, 128), (16, HUGE, 128), (16, 128, HUGE), (1 << 32, 1 << 16, 1 << 16)):
+        with pytest.raises(ValueError):
+            ops.fused_moe_w4a16(x, w, s, w, s, ids, tw, E, hidden, inter, 128)
