@@ -133,6 +133,10 @@ size_t product(std::initializer_list<size_t> factors) {
   return zero ? 0 : over ? SIZE_MAX : p;
 }
 
+size_t rows(const at::Tensor& t) {
+  if (t.dim() == 0) raise(PyExc_IndexError, "a tensor without dimensions has no rows");
+  return static_cast<size_t>(t.size(0));
+}
 size_t dim(const at::Tensor& t, int64_t d, int64_t dims, const char* what) {
   if (t.dim() != dims) raise(PyExc_ValueError, "%s: a tensor of %d dimensions is required", what, static_cast<int>(dims));
   return static_cast<size_t>(t.size(d));
@@ -189,7 +193,7 @@ at::Tensor w4a16_gemm(const Args& a) {
   const at::Tensor* z = tensor_or_null(a.v[3]);
   const size_t n = size_arg(a.v[4]), k = size_arg(a.v[5]), group = size_arg(a.v[6]);
   const at::Tensor *given = tensor_or_null(a.v[7]), *ws = tensor_or_null(a.v[8]);
-  const size_t m = x.dim() ? x.size(0) : 0;
+  const size_t m = rows(x);
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
   need_bytes(x, product({m, k, 2}), "w4a16_gemm: x");
   need_bytes(w, product({k, n}) / 2, "w4a16_gemm: packed weight");
@@ -207,7 +211,7 @@ at::Tensor w4a16_gemm(const Args& a) {
 std::pair<at::Tensor, at::Tensor> group_quant(const at::Tensor& x, size_t k, size_t group, bool column_major, bool fuse,
                                               const at::Tensor* q_given, const at::Tensor* s_given) {
   const OnDevice on(x);
-  const size_t m = x.dim() ? x.size(0) : 0;
+  const size_t m = rows(x);
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
   at::Tensor q = q_given ? *q_given : empty({m, k}, at::kByte, x);
   at::Tensor s = s_given ? *s_given
@@ -222,7 +226,7 @@ at::Tensor fp8_blockwise_gemm(const Args& a) {
   const at::Tensor &aq = tensor(a.v[0]), &as = tensor(a.v[1]), &b = tensor(a.v[2]), &bs = tensor(a.v[3]);
   const OnDevice on(aq);
   const at::Tensor *given = tensor_or_null(a.v[5]), *ws = tensor_or_null(a.v[6]);
-  const size_t m = dim(aq, 0, 2, "fp8_blockwise_gemm: a_q"), k = aq.size(1), n = b.dim() ? b.size(0) : 0;
+  const size_t m = dim(aq, 0, 2, "fp8_blockwise_gemm: a_q"), k = aq.size(1), n = rows(b);
   need_bytes(as, product({k / 128, m, 4}), "fp8_blockwise_gemm: activation scales");
   need_bytes(b, product({n, k}), "fp8_blockwise_gemm: weight");
   need_bytes(bs, product({(n + 127) / 128, k / 128, 4}), "fp8_blockwise_gemm: weight scales");

@@ -74,3 +74,17 @@ def test_declared_sizes_beyond_64_bits_do_not_pass_for_small_ones():
     for E, hidden, inter in ((HUGE, 128, 128), (16, HUGE, 128), (16, 128, HUGE), (1 << 32, 1 << 16, 1 << 16)):
         with pytest.raises(ValueError):
             ops.fused_moe_w4a16(x, w, s, w, s, ids, tw, E, hidden, inter, 128)
+
+
+def test_a_tensor_without_dimensions_has_no_rows():
+    from ksanallm_amd import ops
+    nil = torch.zeros((), dtype=torch.float16)
+    out = torch.zeros((1, 16), dtype=torch.float16)
+    w, s = torch.zeros(16 * 128 // 2, dtype=torch.uint8), torch.zeros(16, dtype=torch.float16)
+    with pytest.raises(IndexError):
+        ops.w4a16_gemm(nil, w, s, None, 16, 128, 128, out=out)
+    with pytest.raises(IndexError):
+        ops.per_token_group_quant_fp8(nil, 128, q=torch.zeros(0, dtype=torch.uint8), s=torch.zeros(0))
+    with pytest.raises(IndexError):
+        ops.fp8_blockwise_gemm(torch.zeros((1, 128), dtype=torch.uint8), torch.zeros(1), torch.zeros((), dtype=torch.uint8),
+                               torch.zeros(1), out=out)
