@@ -200,6 +200,11 @@ at::Tensor w4a16_gemm(const Args& a) {
   need_bytes(s, product({k / group, n, 2}), "w4a16_gemm: scales");
   if (z) need_bytes(*z, product({k / group, n}), "w4a16_gemm: zero points");
   const int d = dt(x);
+  if (given) {
+    if (given->scalar_type() != x.scalar_type())
+      raise(PyExc_TypeError, "w4a16_gemm: out must be of x's type, got %s", at::toString(given->scalar_type()));
+    need_bytes(*given, product({m, n, 2}), "w4a16_gemm: out");
+  }
   at::Tensor out = given ? *given : empty({m, n}, x.scalar_type(), x);
   const Scratch scratch(ws, x, ws ? 0 : lib.w4a16_workspace_size(m, n, k, group, d));
   void *po = ptr(out), *px = ptr(x), *pw = ptr(w), *ps = ptr(s), *pz = ptr(z), *st = stream();
@@ -213,6 +218,9 @@ std::pair<at::Tensor, at::Tensor> group_quant(const at::Tensor& x, size_t k, siz
   const OnDevice on(x);
   const size_t m = rows(x);
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
+  need_bytes(x, product({m, k, static_cast<size_t>(x.element_size()), fuse ? size_t(2) : size_t(1)}), "fp8_group_quant: x");
+  if (q_given) need_bytes(*q_given, product({m, k}), "fp8_group_quant: q");
+  if (s_given) need_bytes(*s_given, product({m, k / group, 4}), "fp8_group_quant: s");
   at::Tensor q = q_given ? *q_given : empty({m, k}, at::kByte, x);
   at::Tensor s = s_given ? *s_given
                          : (column_major ? empty({k / group, m}, at::kFloat, x) : empty({m, k / group}, at::kFloat, x));
@@ -232,6 +240,7 @@ at::Tensor fp8_blockwise_gemm(const Args& a) {
   need_bytes(bs, product({(n + 127) / 128, k / 128, 4}), "fp8_blockwise_gemm: weight scales");
   at::Tensor out = given ? *given : empty({m, n}, dtype_arg(a.v[4]), aq);
   const int d = dt(out, true);
+  need_bytes(out, product({m, n, static_cast<size_t>(out.element_size())}), "fp8_blockwise_gemm: out");
   const Scratch scratch(ws, aq, ws ? 0 : lib.fp8_blockwise_workspace_size(m, n, k));
   void *po = ptr(out), *pa = ptr(aq), *pas = ptr(as), *pb = ptr(b), *pbs = ptr(bs), *st = stream();
   call([&] { return lib.fp8_blockwise_gemm(pa, pas, pb, pbs, po, m, n, k, d, scratch.p, scratch.bytes, st); });
@@ -245,6 +254,8 @@ std::pair<at::Tensor, at::Tensor> w4a8_static_quant(const Args& a) {
   const size_t group = size_arg(a.v[4]);
   const size_t m = dim(x, 0, 2, "w4a8_static_quant: x"), k = x.size(1);
   if (group == 0) raise(PyExc_ZeroDivisionError, "group size 0");
+  if (scale.scalar_type() != at::kFloat) raise(PyExc_ValueError, "w4a8_static_quant: scale must be fp32");
+  need_bytes(scale, product({per_channel ? k : (per_token ? m : 1), 4}), "w4a8_static_quant: scale");
   at::Tensor q = empty({m, k}, at::kByte, x), xsum = empty({k / group, m}, at::kFloat, x);
   int mode = per_channel ? KSQ_W4A8_PER_CHANNEL : (per_token ? KSQ_W4A8_PER_TOKEN : KSQ_W4A8_PER_TENSOR);
   if (group == 64) mode |= KSQ_W4A8_SUMS_PER_64;
@@ -269,6 +280,7 @@ at::Tensor w4a8_gemm(const Args& a) {
   if (scales.scalar_type() != at::kHalf) raise(PyExc_AssertionError, "w4a8_gemm: scales must be float16");
   at::Tensor out = given ? *given : empty({m, n}, dtype_arg(a.v[6]), aq);
   const int d = dt(out);
+  need_bytes(out, product({m, n, 2}), "w4a8_gemm: out");
   const Scratch scratch(ws, aq, ws ? 0 : lib.w4a8_workspace_size(m, n, k));
   void *po = ptr(out), *pa = ptr(aq), *pxs = ptr(xsum), *pw = ptr(w), *ps = ptr(scales), *st = stream();
   call([&] {
@@ -302,7 +314,10 @@ std::pair<at::Tensor, at::Tensor> moe_grouped_topk(const Args& a) {
   const size_t tokens = dim(gating, 0, 2, "moe_grouped_topk: gating"), E = gating.size(1);
   const int d = dt(gating, true);
   at::Tensor w = empty({tokens, top_k}, at::kFloat, gating), ids = empty({tokens, top_k}, at::kInt, gating);
-  if (bias && bias->scalar_type() != at::kFloat) raise(PyExc_ValueError, "e_bias must be fp32");
+  if (bias) {
+    if (bias->scalar_type() != at::kFloat) raise(PyExc_ValueError, "e_bias must be fp32");
+    need_bytes(*bias, product({E, 4}), "moe_grouped_topk: e_bias");
+  }
   void *pg = ptr(gating), *pb = ptr(bias), *pw = ptr(w), *pi = ptr(ids), *st = stream();
   call([&] {
     return lib.moe_grouped_topk(pg, pb, pw, pi, tokens, E, top_k, groups, topk_group, sigmoid, renormalize, scaling, d, st);

@@ -88,3 +88,40 @@ def test_a_tensor_without_dimensions_has_no_rows():
     with pytest.raises(IndexError):
         ops.fp8_blockwise_gemm(torch.zeros((1, 128), dtype=torch.uint8), torch.zeros(1), torch.zeros((), dtype=torch.uint8),
                                torch.zeros(1), out=out)
+
+
+def test_tensors_that_the_caller_gives_are_checked_against_what_the_call_reads_and_writes():
+    """Too small a tensor - outputs and the quantizers' arguments as much as weights - is refused by name, before any launch."""
+    from ksanallm_amd import ops
+    f16, u8, f32 = torch.float16, torch.uint8, torch.float32
+    m, n, k = 16, 32, 256
+    x, w, s = torch.zeros((m, k), dtype=f16), torch.zeros(n * k // 2, dtype=u8), torch.zeros((k // 128, n), dtype=f16)
+    a, a_s = torch.zeros((m, k), dtype=u8), torch.zeros((k // 128, m))
+    b, b_s = torch.zeros((n, k), dtype=u8), torch.zeros((1, k // 128))
+    good, short = torch.zeros((m, n), dtype=f16), torch.zeros((m, n - 1), dtype=f16)
+
+    def refused(match, fn, *args, **kw):
+        with pytest.raises((ValueError, TypeError), match=match):
+            fn(*args, **kw)
+
+    def passes_the_checks(fn, *args, **kw):
+        with pytest.raises(AssertionError, match="device-resident"):
+            fn(*args, **kw)
+    for out, check in ((short, refused), (good, None)):
+        for fn, args in ((ops.w4a16_gemm, (x, w, s, None, n, k, 128)), (ops.fp8_blockwise_gemm, (a, a_s, b, b_s)),
+                         (ops.w4a8_gemm, (a, a_s, w, s, 1.0, n))):
+            passes_the_checks(fn, *args, out=out) if check is None else refused("out", fn, *args, out=out)
+    refused("out", ops.w4a16_gemm, x, w, s, None, n, k, 128, out=good.to(torch.bfloat16))     # x is float16
+    passes_the_checks(ops.fp8_blockwise_gemm, a, a_s, b, b_s, out=good.float())
+    refused("x", ops.per_token_group_quant_fp8, x, 2 * k)
+    refused("x", ops.per_token_group_quant_fp8, x, k, fuse_silu_mul=True)                     # reads 2 k columns
+    passes_the_checks(ops.per_token_group_quant_fp8, x, k // 2, fuse_silu_mul=True)
+    refused("q", ops.per_token_group_quant_fp8, x, k, q=torch.zeros((m, k - 1), dtype=u8))
+    refused("s", ops.per_token_group_quant_fp8, x, k, s=torch.zeros((1, m)))
+    passes_the_checks(ops.per_token_group_quant_fp8, x, k, q=torch.zeros((m, k), dtype=u8), s=torch.zeros((k // 128, m)))
+    for kw, count in (({}, 1), ({"per_channel": True}, k), ({"per_token": True}, m)):
+        passes_the_checks(ops.w4a8_static_quant, x, torch.ones(count), **kw)
+        refused("scale", ops.w4a8_static_quant, x, torch.ones(count - 1), **kw)
+        refused("scale", ops.w4a8_static_quant, x, torch.ones(count, dtype=torch.float64), **kw)
+    refused("e_bias", ops.moe_grouped_topk, torch.zeros((m, 8)), 2, e_bias=torch.zeros(7))
+    passes_the_checks(ops.moe_grouped_topk, torch.zeros((m, 8)), 2, e_bias=torch.zeros(8))
