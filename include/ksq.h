@@ -398,7 +398,8 @@ typedef struct ksq_tile_desc {
 
 /* The descriptor describes group size 128.  Other group sizes of W4A16 keep the kernel and block shape but carry more
  * scales per k-tile; W4A8 with group 64 runs 128-token tiles whose K range is not cut (split_k and grid then differ
- * from what is reported here). */
+ * from what is reported here).  KSQ_KIND_MOE_W4A16 describes the grouped streaming launch of m slots of one expert, in
+ * blocks of 16 slots (m <= 16) or 32; the blocks of 128 and 256 slots run the tile kernel. */
 int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype, ksq_tile_desc* out_desc);
 
 /* Above 32 rows ksq_w4a16_gemm, ksq_fp8_blockwise_gemm and ksq_w4a8_gemm run the MFMA tile kernels, but for small

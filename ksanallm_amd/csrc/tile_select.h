@@ -16,6 +16,8 @@ struct SplitKChoice {
 SplitKChoice select_splitk(size_t m, size_t n, size_t k);
 // same rule for a grid of m_blocks row blocks of 16*mt rows each (MoE: one block per aligned expert segment)
 SplitKChoice select_splitk_blocks(int mt, size_t m_blocks, size_t n, size_t k);
+// grouped W4A16 launch over about `blocks` blocks of block_m (16 or 32) slots, numel of them routed; K is never cut over workgroups
+SplitKChoice select_splitk_grouped(size_t block_m, size_t blocks, size_t numel, size_t n, size_t k);
 
 // The decode-form kernels also serve small problems of more than 32 rows, in blocks of 32 rows; never more than this
 // many rows (the workspace queries walk every m up to it).

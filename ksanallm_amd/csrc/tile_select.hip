@@ -104,6 +104,26 @@ SplitKChoice select_splitk_blocks(int mt, size_t m_blocks, size_t n, size_t k) {
   return c;
 }
 
+// Activations through LDS (w4a16_splitk.h) as in the dense form: 2-3 % at E = 256, hidden 7168, inter 2048 from a few
+// tokens per expert on (64 tokens 813 -> 788 us, 512 tokens 1353 -> 1316 us for the whole block), not for a handful of
+// blocks (1 token: 50.1 -> 52.6 us).
+SplitKChoice select_splitk_grouped(size_t block_m, size_t blocks, size_t numel, size_t n, size_t k) {
+  SplitKChoice c = select_splitk_blocks(static_cast<int>(block_m / 16), blocks, n, k);
+  if ((n / 16) % 4 == 0 && numel >= 32) {
+    if (c.mt == 2 && c.nt == 8) {
+      c.waves = 4;
+      c.xc = 4;
+    } else if (c.mt == 2 && c.nt == 4) {
+      c.waves = 8;
+      c.xc = 8;
+    } else if (c.mt == 1 && c.nt >= 4) {
+      c.waves = 8;
+      c.xc = 8;
+    }
+  }
+  return c;
+}
+
 // Regime switch.  Up to 32 rows the split-K (decode) kernel; above, the MFMA tile kernel - except while the problem is
 // small: the tile kernel has a floor of 17-22 us (a workgroup's prologue, the fp32 partial tiles of the cut along K and
 // the pass that sums them), and the decode kernel run over blocks of 32 rows, each streaming the weights again (out of
@@ -335,7 +355,8 @@ KSQ_EXPORT int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype
         d->grid = static_cast<int32_t>(t.grid);
         return KSQ_OK;
       }
-      SplitKChoice c = select_splitk(m, n, k);
+      const size_t slots = m <= 16 ? 16 : 32;
+      const SplitKChoice c = kind == KSQ_KIND_W4A16 ? select_splitk(m, n, k) : select_splitk_grouped(slots, div_up(m, slots), m, n, k);
       d->kernel = KSQ_KERNEL_SPLITK_WAVE;
       d->block_m = 16 * c.mt;
       d->block_n = 16 * c.nt;
@@ -343,7 +364,7 @@ KSQ_EXPORT int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype
       d->waves = c.waves;
       d->split_k = c.waves * c.parts;
       d->grid = static_cast<int32_t>((n / 16 / c.nt) * div_up(m, 16 * c.mt) * c.parts);
-      d->x_chunk = kind == KSQ_KIND_W4A16 ? c.xc : 0;
+      d->x_chunk = c.xc;
       return KSQ_OK;
     }
     case KSQ_KIND_FP8_BLOCKWISE: {

@@ -476,26 +476,10 @@ int moe_w4a16_gemm_impl(const char* fn, bool fuse_silu, void* out, const void* x
   p.num_experts = static_cast<uint32_t>(E);
   p.x_bytes = static_cast<uint32_t>(x_rows * k * 2);
   // about numel/block_m + E/2 of the aligned blocks hold rows; K is never split across workgroups here
-  SplitKChoice c = select_splitk_blocks(static_cast<int>(block_m / 16),
-                                        few ? numel : std::min(cap_blocks, numel / block_m + E / 2 + 1), n, k);
+  SplitKChoice c = select_splitk_grouped(block_m, few ? numel : std::min(cap_blocks, numel / block_m + E / 2 + 1), numel, n, k);
   if (fuse_silu) {
     if (c.nt < 2) c.nt = 2;  // a workgroup holds gate and up tiles in pairs
     p.pair_tiles = static_cast<uint32_t>(n / 32);
-  }
-  // activations through LDS (w4a16_splitk.h) as in the dense form: 2-3 % at E = 256, hidden 7168, inter 2048 from a
-  // few tokens per expert on (64 tokens 813 -> 788 us, 512 tokens 1353 -> 1316 us for the whole block), not for a
-  // handful of blocks (1 token: 50.1 -> 52.6 us)
-  if ((n / 16) % 4 == 0 && numel >= 32) {
-    if (c.mt == 2 && c.nt == 8) {
-      c.waves = 4;
-      c.xc = 4;
-    } else if (c.mt == 2 && c.nt == 4) {
-      c.waves = 8;
-      c.xc = 8;
-    } else if (c.mt == 1 && c.nt >= 4) {
-      c.waves = 8;
-      c.xc = 8;
-    }
   }
   int rc = dtype == KSQ_F16 ? dispatch_tile<F16, true>(p, c, static_cast<uint32_t>(cap_blocks), group, as_stream(stream))
                             : dispatch_tile<BF16, true>(p, c, static_cast<uint32_t>(cap_blocks), group, as_stream(stream));

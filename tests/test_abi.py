@@ -77,3 +77,17 @@ def test_small_problem_rule_and_its_switch():
     finally:
         assert L.set_small_problem_rule(True) is False
     assert L.select_tile(L.KIND_W4A16, *small, L.BF16)["kernel"] == 0
+
+
+def test_descriptor_of_the_grouped_streaming_launch():
+    """KSQ_KIND_MOE_W4A16 describes the grouped streaming launch, which never cuts K over workgroups: its K slices are its
+    wavefronts, four of them while fewer than 32 slots are routed, and then, through LDS, as many as that form has."""
+    from ksanallm_amd import lib as L
+    for m, n, k in ((1, 4096, 14336), (20, 4096, 14336), (31, 1024, 16384), (16, 14336, 4096)):
+        d = L.select_tile(L.KIND_MOE_W4A16, m, n, k, L.BF16)
+        assert (d["kernel"], d["waves"], d["split_k"], d["x_chunk"]) == (0, 4, 4, 0)
+        assert d["block_m"] == (16 if m <= 16 else 32) and d["grid"] == n // d["block_n"]
+    for m, n, k, waves, chunk in ((32, 14336, 4096, 8, 8), (32, 57344, 8192, 4, 4), (64, 4096, 14336, 4, 0)):
+        d = L.select_tile(L.KIND_MOE_W4A16, m, n, k, L.BF16)
+        assert (d["block_m"], d["waves"], d["split_k"], d["x_chunk"]) == (32, waves, waves, chunk)
+        assert d["grid"] == n // d["block_n"] * (m // 32)
