@@ -63,11 +63,24 @@ SplitKChoice select_splitk(size_t m, size_t n, size_t k) {
   //   7.9 us in registers, 8.4 us through LDS), and with up to 8 rows four column tiles per wavefront beat eight
   //   (n = 57344, k = 8192, 1 row: 40.7 against 43.1 us).
   // - K cut over workgroups, 17 rows and more: x outweighs the weights there by construction (n = 4096, k = 14336: 20 rows
-  //   13.2 -> 12.9 us, 32 rows 15.8 -> 14.3, 64 rows 21.6 -> 19.0, 128 rows 36.7 -> 31.5; n = k = 5120 at 32 rows
-  //   12.7 -> 11.6; n = 5120, k = 25600 at 32 rows 34.4 -> 29.0; n = 2048, k = 8192 at 32 rows 11.5 -> 11.0).
+  //   13.2 -> 12.9 us, 32 rows 15.8 -> 14.3..15.2, 64 rows 21.6 -> 19.0, 128 rows 36.7 -> 31.5; n = k = 5120 at 32 rows
+  //   12.7 -> 11.6; n = 5120, k = 25600 at 32 rows 34.4 -> 29.0; n = 2048, k = 8192 at 32 rows 11.5 -> 11.0).  Eight
+  //   wavefronts are one workgroup per CU where the register form holds two, so with more workgroups than CUs a second
+  //   round begins and takes back what the traffic gave (n = 2112, k = 17024, 264 workgroups: 17 rows 16.6 -> 18.2 us,
+  //   26 rows 18.1 -> 18.9; n = 4544, k = 9600, 284: 20 rows 17.9 -> 18.9) until a workgroup has rows and k-tiles enough
+  //   (32 rows: n = 2112 19.4 -> 19.4, n = 4544 20.6 -> 20.3, n = 4992, k = 20480 30.9 -> 28.0; n = 2432, k = 9600 at 160 rows
+  //   30.3 -> 26.6; n = 1600, k = 5760 at 90 rows, 12 k-tiles a part: 15.8 -> 16.3).
+  //   With fewer than 32 rows a part of 9 to 11 k-tiles stays there too: two turns of eight wavefronts, the second one
+  //   nearly empty, against three turns of four (n = 1024, 64 workgroups, 9 k-tiles: 17 rows 8.2 -> 8.5 us, 24 rows 8.9 -> 9.2,
+  //   32 rows 9.5 -> 9.5; 10 and 11 at 32 rows 9.6 -> 9.4, 9.8 -> 9.5; 8 and 12 at 24 rows 7.8 -> 7.6, 9.4 -> 9.2).
   if (c.parts > 1 && mt == 2) {
-    c.waves = 8;
-    c.xc = 8;
+    const size_t kt = div_up(k / 128, c.parts);
+    const bool resident = strips / 4 * m_blocks * c.parts <= static_cast<size_t>(kNumCU);
+    const bool empty_turn = m < 32 && kt > 8 && kt < 12;
+    if (resident ? !empty_turn : m >= 32 && kt >= 16) {
+      c.waves = 8;
+      c.xc = 8;
+    }
   }
   if (c.parts == 1 && strips % 4 == 0) {
     if (mt == 2 && c.nt == 8) {

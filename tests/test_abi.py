@@ -91,3 +91,15 @@ def test_descriptor_of_the_grouped_streaming_launch():
         d = L.select_tile(L.KIND_MOE_W4A16, m, n, k, L.BF16)
         assert (d["block_m"], d["waves"], d["split_k"], d["x_chunk"]) == (32, waves, waves, chunk)
         assert d["grid"] == n // d["block_n"] * (m // 32)
+
+
+def test_decode_with_k_cut_over_workgroups_takes_x_through_lds_where_that_pays():
+    """x goes through LDS (one workgroup of eight wavefronts per CU) where every workgroup is resident at once, but for parts
+    of 9..11 k-tiles below 32 rows; with more workgroups than CUs only from 32 rows and 16 k-tiles per part on."""
+    from ksanallm_amd import lib as L
+    for m, n, k, waves, chunk in ((20, 2048, 17024, 8, 8), (20, 2112, 17024, 4, 0), (31, 4160, 9600, 4, 0), (32, 4160, 9600, 8, 8),
+                                  (90, 1600, 5760, 4, 0), (90, 2624, 8192, 8, 8), (160, 2432, 9600, 8, 8), (24, 1024, 4096, 8, 8), (24, 1024, 4608, 4, 0),
+                                  (24, 1024, 5632, 4, 0), (24, 1024, 6144, 8, 8), (32, 1024, 4608, 8, 8)):
+        d = L.select_tile(L.KIND_W4A16, m, n, k, L.BF16)
+        assert d["kernel"] == 0 and d["split_k"] > d["waves"]
+        assert (d["waves"], d["x_chunk"]) == (waves, chunk), (m, n, k)

@@ -305,6 +305,17 @@ def test_decode_k_parts_x_through_lds(ops, dtype, awq, M, N, K):
     H.check_gemm(y, H.w4a16_oracle(d), dtype, "decode K parts, x through LDS M=%d N=%d K=%d" % (M, N, K))
 
 
+# ... and in the register form: more workgroups than CUs with fewer than 32 rows or 16 k-tiles a part, parts of 9..11 k-tiles
+@pytest.mark.parametrize("dtype,awq,M,N,K", [(H.BF16, True, 18, 1024, 4608), (H.F16, False, 29, 2048, 5504), (H.F16, False, 17, 2112, 8192), (H.BF16, True, 31, 4160, 4224), (H.BF16, False, 90, 1600, 5760)])
+def test_decode_k_parts_x_in_registers(ops, dtype, awq, M, N, K):
+    from ksanallm_amd import lib as L
+    desc = L.select_tile(L.KIND_W4A16, M, N, K, dtype)
+    assert desc["kernel"] == 0 and desc["x_chunk"] == 0 and desc["waves"] == 4 and desc["split_k"] > 4
+    d = H.make_w4a16(4150 + M + N, M, N, K, 128, dtype, awq=awq, z_lo=0, z_hi=15)
+    y = run_case(ops, d)
+    H.check_gemm(y, H.w4a16_oracle(d), dtype, "decode K parts, x in registers M=%d N=%d K=%d" % (M, N, K))
+
+
 # decode regime with the activations staged through LDS (17..32 rows; up to 16 rows from 48 MB of weights): K that is
 # not a whole number of 4-k-tile loads, one chunk and several, ragged row counts, both dtypes, with and without zero points
 @pytest.mark.parametrize("dtype,awq", [(H.F16, False), (H.BF16, True), (H.F16, True), (H.BF16, False)])
