@@ -332,11 +332,17 @@ KSQ_EXPORT int ksq_moe_w4a16_down_sum(void* out, const void* x, const void* w_pa
   const bool two = (n / 16) % 2 == 0 && (n / 32) * tokens >= 192;
   p.magic2 = dtype == KSQ_F16 ? F16::kMagic2 : BF16::kMagic2;
   int rc;
-  // ... and eight wavefronts instead of four where their rings of two k-tiles fill: what bounds the kernel is the bytes a
-  // CU keeps in flight, and 224 workgroups of four wavefronts keep 24 KiB (whole one-token block, 8 of 256 experts, hidden
-  // 7168, inter 2048: 44.1 -> 42.4 us; 4 experts 26.2 -> 25.0; 2 experts of inter 1024, 16 k-tiles: 17.9 -> 17.4; four
-  // tokens 127.9 -> 127.0; eight wavefronts with a ring of three or four 0.4-0.9 us behind two)
-  const bool eight = two && top_k * k >= 16 * 128;
+  // ... and eight wavefronts instead of four where that does not multiply more: what bounds the kernel is the bytes a CU
+  // keeps in flight, and 224 workgroups of four wavefronts keep 24 KiB; but a turn of the main loop is 16 k-tiles for eight
+  // wavefronts (rings of two) and 12 for four (rings of three), and what K lacks of a whole turn is loaded and multiplied all
+  // the same.  Whole block, four -> eight wavefronts: 128 k-tiles (8 experts of inter 2048, hidden 7168, one token)
+  // 46.5 -> 43.8 us, 64 k-tiles 28.1 -> 26.8, 32 24.1 -> 23.8; 36 (6 of inter 768: 48 for 36) 27.2 -> 27.5, with four tokens
+  // 55.3 -> 57.9; 24 (32 for 24) with four tokens 36.6 -> 39.4; 60 (4 of inter 1920, hidden 4608, three tokens) 45.2 -> 45.6.
+  // The same number either way: eight where every workgroup is resident at once (90 k-tiles, hidden 1792, four tokens
+  // 37.5 -> 36.3), four above (40 k-tiles, hidden 3072, four tokens 33.6 -> 34.1).  Fewer than 16 k-tiles do not fill eight
+  // rings.  Eight wavefronts with a ring of three or four are 0.4-0.9 us behind two.
+  const size_t kt = top_k * k / 128, pad8 = round_up(kt, 16), pad4 = round_up(kt, 12);
+  const bool eight = two && kt >= 16 && (pad8 < pad4 || (pad8 == pad4 && (n / 32) * tokens <= 256));
   auto go = [&](auto t) {
     typedef decltype(t) T;
     const uint32_t rows = static_cast<uint32_t>(tokens);

@@ -364,10 +364,12 @@ def test_silu_over_every_input_of_the_type(ops, dtype):
     print("silu %s: %d of %d inputs one unit off the correctly rounded value (%.3f %%)" % (td, int((d > 0).sum()), n, 100 * share))
 
 
-@pytest.mark.parametrize("topk,k", [(5, 384), (4, 512), (17, 128), (2, 1024), (3, 1408)])
+@pytest.mark.parametrize("topk,k", [(5, 384), (4, 512), (17, 128), (2, 1024), (3, 1408), (4, 1024)])
 def test_down_sum_with_eight_wavefronts(topk, k):
-    """15 k-tiles run on four wavefronts, 16 and more on eight, one token (few workgroups) on the one-column form of four:
-    the same fp32 sum in another order, so an fp16 output differs by one unit (2^-10 of its value) at most."""
+    """15, 17 and 33 k-tiles run on four wavefronts, 16 and 32 on eight, one token (few workgroups) on the one-column form of
+    four.  Against 64 bits: an fp16 output is rounded once, which leaves at most 2^-11 of its value and 2^-11 / sqrt(3) in the
+    mean square; what the fp32 sum adds (about 1e-5 of the outputs' root mean square) gets 1e-3, a k-tile too few or too
+    many is 0.17 and more of it."""
     from ksanallm_amd import lib as L
     from ksanallm_amd import ops
     E, n, T = 24, 2048, 3
@@ -391,6 +393,14 @@ def test_down_sum_with_eight_wavefronts(topk, k):
     one = torch.cat([down(t, t + 1) for t in range(T)])
     assert torch.isfinite(one).all()
     assert float((whole - one).norm() / one.norm()) < 2.0 ** -10
+    wd = torch.stack([codes & 15, codes >> 4], -1).reshape(E, n, k).double() - 8
+    wd *= ops.unpack_scales(s, L.SCALE_NG, E, k, n, 128).cpu().double().repeat_interleave(128, -1)
+    ref = torch.stack([sum(float(tw[t, j]) * (wd[int(ids[t, j])] @ x[t * topk + j].cpu().double()) for j in range(topk)) for t in range(T)])
+    rms = float(ref.norm()) / ref.numel() ** 0.5
+    for y in (whole, one):
+        err = (y.cpu().double() - ref).abs()
+        assert float(err.norm() / ref.norm()) < 2.0 ** -11 / 3 ** 0.5 + 1e-4
+        assert bool((err <= 2.0 ** -11 * ref.abs() + 1e-3 * rms).all()), float((err - 2.0 ** -11 * ref.abs()).max() / rms)
 
 
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
