@@ -222,6 +222,26 @@ def test_blockwise_gemm_tile_kernel(ops, oracle, m, n, k, bm, tile_kernels):
         assert e.value.code == 3
 
 
+# the wavefront rows of a dense tile share the row tiles that hold tokens, evenly or not: every count of them in the last block
+@pytest.mark.parametrize("bm,n,k", [(128, 272, 384), (256, 2304, 384)])
+def test_blockwise_gemm_tile_kernel_every_count_of_live_row_tiles(ops, oracle, bm, n, k, tile_kernels):
+    from ksanallm_amd import lib as L
+    full = bm if bm == 128 else 1024 + bm
+    x, bq, bs = make_fp8_problem(oracle, 4460 + bm, full, n, k)
+    w, ws = packed(ops, bq), torch.from_numpy(bs).cuda()
+
+    def run(m):
+        assert L.select_tile(L.KIND_FP8_BLOCKWISE, m, n, k, H.BF16)["block_m"] == bm
+        q, s = ops.per_token_group_quant_fp8(x[:m].contiguous().cuda(), k, 128, True)
+        return ops.fp8_blockwise_gemm(q, s, w, ws, torch.bfloat16), q, s
+    whole, q, s = run(full)
+    ref = oracle.fp8_blockwise_gemm(q.cpu().numpy(), s.cpu().numpy(), bq[:128], bs[:1], True)
+    H.check_gemm(whole[:, :128], ref, H.BF16, "fp8 tile, first 128 columns")
+    for m in range(full - bm + 11, full, 16):
+        if m > 32:
+            assert torch.equal(run(m)[0].view(torch.int16), whole[:m].view(torch.int16)), m
+
+
 # small problems of more than 32 tokens (ceil(m / 32) * n * k <= 5 * 2^24, m <= 512): the streaming kernel over blocks of
 # 32 tokens, ragged last block included
 @pytest.mark.parametrize("m,n,k", [(65, 256, 128), (100, 272, 384), (128, 4096, 4096), (300, 2320, 1152), (500, 768, 640),
