@@ -63,6 +63,17 @@ constexpr size_t fp8_tile_lds_bytes(int wm, size_t kb_max) {
   return static_cast<size_t>(fp8_tile_stages(wm)) * (fp8_tile_stage_bytes(wm) + fp8_tile_scale_bytes(wm)) + 2 * kb_max * 4;
 }
 
+// Grouped form: the row blocks that hold slots, of the p.tiles_m that the grid was sized for (the largest number an
+// alignment can make).  The work order runs over these alone and the workgroups past them leave.  Over all of p.tiles_m
+// the blocks without slots sit at the end of every band of eight column tiles, and by how a band divides by 256 some XCDs
+// got them all: 32 experts of 96 slots, n = 4096, k = 1152 in 256-slot blocks, 512 tiles of 704, were 76 tiles each on five
+// XCDs and 44 on three (67.2 us; 128-slot blocks, 512 of 880, happened to give 64 each: 50.2).
+template <int BLOCK>
+__device__ __forceinline__ uint32_t fp8_live_blocks(const Fp8TileParams& p) {
+  const uint32_t blocks = (static_cast<uint32_t>(p.num_post_pad[0]) + (BLOCK - 1)) / BLOCK;
+  return __builtin_amdgcn_readfirstlane(blocks < p.tiles_m ? blocks : p.tiles_m);
+}
+
 // BLOCK: slots between consecutive row blocks (tile_m * BLOCK is the block's first slot): the tile's own 32 * WM rows, or
 // - grouped form - 256 for a 160-token tile that serves a 256-slot block with at most 160 tokens.
 template <typename TO, bool GROUPED, int WM, int BLOCK>
@@ -88,7 +99,9 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
 
   // ---- work id (tile_work.h): output tile and the part of K this workgroup computes
   // (the divisions inside run on the vector unit: readfirstlane brings the wave-uniform results back to scalars)
-  const TileWork work = tile_work(blockIdx.x, p.tiles_m, p.tiles_n, p.main_items, p.splits, GROUPED);
+  const uint32_t tiles_m = GROUPED ? fp8_live_blocks<BLOCK>(p) : p.tiles_m;
+  if (GROUPED && blockIdx.x >= tiles_m * p.tiles_n) return;  // uniform: the whole workgroup leaves
+  const TileWork work = tile_work(blockIdx.x, tiles_m, p.tiles_n, p.main_items, p.splits, GROUPED);
   const uint32_t tile_m = __builtin_amdgcn_readfirstlane(work.tile_m), tile_n = __builtin_amdgcn_readfirstlane(work.tile_n);
   const uint32_t part = __builtin_amdgcn_readfirstlane(work.part), slot = __builtin_amdgcn_readfirstlane(work.slot);
   const bool direct = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(work.direct)) != 0;
@@ -113,7 +126,6 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
     live_tiles = rows < static_cast<uint32_t>(BM) ? (rows + 15) / 16 : AF;
   }
   if (GROUPED) {
-    if (m0 >= static_cast<uint32_t>(p.num_post_pad[0])) return;  // uniform: the whole workgroup leaves
     expert = static_cast<size_t>(__builtin_amdgcn_readfirstlane(p.expert_ids[tile_m]));
     uint32_t rows = 0;
 #pragma unroll
@@ -480,9 +492,10 @@ template <typename TO, bool GROUPED = false, int WM = 8>
 __global__ void __launch_bounds__(512, 1) fp8_tile_kernel(Fp8TileParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];  // fp8_tile_lds_bytes (the larger of both forms)
   if constexpr (GROUPED && WM == 8) {
-    const TileWork work = tile_work(blockIdx.x, p.tiles_m, p.tiles_n, p.main_items, p.splits, true);
+    const uint32_t tiles_m = fp8_live_blocks<256>(p);
+    if (blockIdx.x >= tiles_m * p.tiles_n) return;  // uniform: the whole workgroup leaves
+    const TileWork work = tile_work(blockIdx.x, tiles_m, p.tiles_n, p.main_items, p.splits, true);
     const uint32_t m0 = __builtin_amdgcn_readfirstlane(work.tile_m) * 256;
-    if (m0 >= static_cast<uint32_t>(p.num_post_pad[0])) return;  // uniform: the whole workgroup leaves
     uint32_t rows = 0;
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
