@@ -41,6 +41,13 @@ def make_w4a16(seed, M, N, K, group, dtype, awq, x_std=1.0, s_lo=0.004, s_hi=0.0
     return d
 
 
+def last_columns(d, n, first_row=0):
+    """What the oracle needs of a dense case for its last n columns and its rows from first_row on."""
+    return dict(d, N=n, x=d["x"][first_row:].contiguous(), codes=np.ascontiguousarray(d["codes"][:, -n:]),
+                scales=d["scales"][:, -n:].contiguous(),
+                zeros=None if d["zeros"] is None else np.ascontiguousarray(d["zeros"][:, -n:]))
+
+
 def w4a16_oracle(d):
     return orc.w4a16_gemm(bits_of(d["x"]), d["codes"], bits_of(d["scales"]), d["zeros"], d["group"], d["dtype"])
 

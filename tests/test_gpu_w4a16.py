@@ -112,21 +112,28 @@ def test_prefill_256_row_tiles(ops, dtype, awq, M, N, K, tile_kernels):
                  weights_rounded=True)
 
 
-# the main loop of the tile kernel exists once per number of row tiles that hold rows: every count, 128- and 256-row tiles
+# The main loop of the tile kernel exists once per number of row tiles that hold rows: every count from four (fewer run that
+# instance) in the last block of a 128- and of a 256-row tile.  A turn of the loop is six stages of half a k-tile: three whole
+# turns (9 k-tiles), turns and a part of one (7 and 8 k-tiles), less than one.
 @pytest.mark.parametrize("awq", [False, True])
-@pytest.mark.parametrize("M,N,K", [(m, 8448, 128) for m in (129, 145, 161, 177, 193, 209, 225, 241)] +
-                         [(m, 272, 384) for m in (33, 65, 81, 97, 113)])
+@pytest.mark.parametrize("M,N,K", [(m, 8448, k) for m, k in ((129, 1152), (145, 1024), (161, 896), (177, 1152), (193, 1024), (209, 896),
+                                                             (225, 1152), (241, 1024), (161, 128), (241, 128))] +
+                         [(1024 + m, 2304, k) for m, k in ((17, 896), (65, 1024), (81, 896), (97, 1152), (113, 1024))] +
+                         [(m, 272, k) for m, k in ((33, 1152), (65, 1024), (81, 896), (97, 1152), (113, 1024), (113, 384))])
 def test_prefill_every_row_tile_count(ops, awq, M, N, K, tile_kernels):
     from ksanallm_amd import lib as L
-    full = 256 if M > 128 else 128
-    assert L.select_tile(L.KIND_W4A16, M, N, K, H.BF16)["block_m"] == full
+    block = 256 if M > 128 else 128
+    full = -(-M // block) * block
+    desc = L.select_tile(L.KIND_W4A16, M, N, K, H.BF16)
+    assert desc["kernel"] == 1 and desc["block_m"] == block and desc["split_k"] == 1
     d = H.make_w4a16(3500 + M, full, N, K, 128, H.BF16, awq=awq, x_std=0.5, s_lo=0.002, s_hi=0.01, z_lo=0, z_hi=15)
     y = run_case(ops, d)
     short = run_case(ops, dict(d, M=M, x=d["x"][:M].contiguous()))
     assert (short == y[:M]).all(), "a row's sum depends on how many rows the tile holds"
-    n = 64   # the oracle on the first columns: what a wrong row tile would show in every column
-    sub = H.w4a16_oracle(d)[:M, :n]
-    H.check_gemm(short[:, :n], sub, H.BF16, "row tiles M=%d" % M, weights_rounded=True)
+    # the oracle on the last columns of the last block: what a wrong row tile would show in every column
+    r0 = full - block
+    sub = H.w4a16_oracle(H.last_columns(d, 64, r0))[:M - r0]
+    H.check_gemm(short[r0:, -64:], sub, H.BF16, "row tiles M=%d K=%d" % (M, K), weights_rounded=True)
 
 
 # few output tiles: K is split over workgroups, fp32 partials go through the workspace and a second kernel sums them
