@@ -33,14 +33,14 @@ bool small_w4a16_problem(size_t m, size_t n, size_t k, size_t group);
 // are computed whole, the others in `splits` parts of kt_per_split k-steps whose fp32 partial tiles go through the
 // workspace.  main_items == 0 and splits > 1: every tile is cut (grids far smaller than the chip).
 struct TilePlan {
-  int block_m;  // 128 or 256
+  int block_m;  // 64 (W4A8), 128 or 256
   unsigned tiles_m, tiles_n, main_items, splits, kt_per_split, grid;
   size_t workspace_bytes;
 };
 TilePlan plan_mfma_tile(size_t m, size_t n, size_t k);
 
 // Blockwise FP8: whether the MFMA tile kernel replaces the split-K wavefront kernel (above 32 tokens, but for small problems),
-// and its grid (block_m is always 256; kt_per_split counts 128-deep k-blocks).
+// and its grid (kt_per_split counts 128-deep k-blocks).
 bool use_fp8_tile(size_t m, size_t n, size_t k);
 TilePlan plan_fp8_tile(size_t m, size_t n, size_t k);
 // W4A8 (w4a8_tile.h): the same regime rule with its own size limit, the same tile shapes with its own costs of a cut along K

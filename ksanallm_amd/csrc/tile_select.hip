@@ -278,12 +278,17 @@ TilePlan plan_fp8_tile(size_t m, size_t n, size_t k) {
 // W4A8: the blockwise-FP8 tile shapes; a k-step moves three quarters of the bytes and its prologue is shorter, so a
 // cut along K pays earlier (measured at n = 25600, k = 5120: with the FP8 costs 64 / 128 / 256 tokens ran whole tiles
 // on 100 of the 256 CUs in 38 / 51 / 83 us, with these they are cut in two or three: 28 / 38 / 60 us)
-// Up to 64 tokens, 64-token tiles: the two wavefront rows share the row tiles (of a 128-token tile the lower one would
-// stand idle) and a barrier comes every two k-blocks (n = 25600, k = 5120 at 64 tokens, quantizer included:
-// 29.65 -> 28.3 us).
+// Up to 64 tokens, 64-token tiles where K is whole or cut into parts of at least 32 k-blocks: the two wavefront rows share
+// the row tiles (of a 128-token tile the lower one stands idle) and a barrier comes every two k-blocks.  Whole tiles, 128-
+// against 64-token: n = 28672, k = 1024 at 64 tokens 13.1 / 12.4 us, n = 25600, k = 3072 24.4 / 23.2, n = 8192, k = 1024
+// 12.0 / 10.8.  Shorter parts run on 128-token tiles: K is cut until (nearly) every CU has a workgroup, all of them fill
+// their rings out of HBM at once, and a form that begins, and goes on, only when two k-blocks have landed starts later than
+// one that waits for one (n = 16224, k = 3968 at 40 tokens, parts of 8: 17.3 / 18.0 us; n = 8192, k = 14336, parts of 14:
+// 22.5 / 23.8; n = 4352, k = 20480 at 64 tokens, parts of 11: 23.8 / 24.7; parts of 20..24 at 40 tokens 27.4 / 28.4 and
+// 29.7 / 30.3; parts of 32 at 64 tokens 38.2 / 37.2, 35.3 / 35.3 and 37.1 / 36.6).
 TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k) {
   TilePlan t{};
-  t.block_m = m <= 64 ? 64 : (m <= 128 || (m < 1024 && (m - 1) % 256 < 128)) ? 128 : 256;
+  t.block_m = (m <= 128 || (m < 1024 && (m - 1) % 256 < 128)) ? 128 : 256;
   // as in plan_mfma_tile: at most 32 tiles of 256 tokens are better served by 128-token tiles and half the cut along K
   // (n = k = 5120 at 256 tokens: 31 -> 25 us; n = k = 4096 at 512 tokens: 33 -> 27 us)
   if (t.block_m == 256 && div_up(m, 256) * div_up(n, 256) <= 32 && k <= 16384) t.block_m = 128;
@@ -291,6 +296,7 @@ TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k) {
   t.tiles_n = static_cast<unsigned>(div_up(n, 256));
   static const SpreadCost cost{6.0, 4.0, 3.0, 0.03};
   spread_tiles(t.tiles_m * t.tiles_n, static_cast<unsigned>(k / 128), cost, &t);
+  if (m <= 64 && (t.splits == 1 || t.kt_per_split >= 32)) t.block_m = 64;  // (one row block either way)
   finish_plan(&t);
   return t;
 }

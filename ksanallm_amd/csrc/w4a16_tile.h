@@ -309,10 +309,10 @@ __global__ void __launch_bounds__(512, 1) w4a16_tile_kernel(TileParams p) {
   };
   auto wait_only = [&](auto n) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory"); };
 
-  // Everything from here to the end of the main loop exists once per number of row tiles that are multiplied (WMV):
-  // all WM of them, or - block at most half full - the lower WM/2 only.  The choice is made once per
-  // workgroup, outside the scheduled loop; guarding single row tiles inside it would split the loop body into basic
-  // blocks and lose the interleaving of LDS reads, conversions and MFMAs (measured: 20 % slower, not faster).
+  // Everything from here to the end of the main loop exists once per number of row tiles that are multiplied (WMV): which
+  // ones exist stands at the choice, below the lambda.  The choice is made once per workgroup, outside the scheduled loop;
+  // guarding single row tiles inside it would split the loop body into basic blocks and lose the interleaving of LDS reads,
+  // conversions and MFMAs (measured: 20 % slower, not faster).
   auto run = [&](auto wmv_c) {
     constexpr int WMV = decltype(wmv_c)::value;
     // Fragments this wavefront stages per x stage.  A 256-row block of which at most the lower eight row tiles hold

@@ -36,9 +36,10 @@ struct W4A8TileParams {
 };
 
 constexpr int w4a8_tile_stage_bytes(int wm) { return (2 * wm) * 2048 + 16 * 1024; }
-// LDS stages: as many as 160 KiB hold (128-token tiles, four in place of three: n = 25600, k = 5120 at 128 tokens 41.5 ->
-// 39.7 us; 64-token tiles, six, with STEP below: n = 28672, k = 1024 at 64 tokens 26.0 -> 14.4, n = 14336, k = 8192
-// 29.7 -> 26.7).
+// LDS stages: as many as 160 KiB hold.  The launch alone, weights out of HBM: 128-token tiles, four in place of three:
+// n = 25600, k = 5120 at 128 tokens 38.6 -> 36.6 us, n = 14336, k = 8192 34.0 -> 32.7, n = 28672, k = 1024 17.5 -> 16.8;
+// 64-token tiles, six, with STEP below: n = 28672, k = 1024 at 64 tokens 12.4 us (128-token tiles: 13.6 with three, 13.1
+// with four).
 constexpr int w4a8_tile_stages(int wm) { return wm == 2 ? 6 : wm == 4 ? 4 : 3; }
 // per stage: operands, 1 KiB of group sums, 1 KiB of weight scales
 constexpr size_t w4a8_tile_lds_bytes(int wm) {
@@ -78,8 +79,8 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
   constexpr int NS = w4a8_tile_stages(WM);
   // k-blocks between two barriers.  A k-block of the 64-token tile is 8 MFMAs per wavefront, about 512 of the 2000 cycles
   // it takes: the rest is the chain barrier, LDS reads, code expansion, MFMA, scale FMAs, run by all wavefronts at once.
-  // Six stages in place of three alone left n = 25600, k = 5120 at 64 tokens at 29.8 us, two k-blocks per barrier
-  // bring it to 28.3: the wavefronts drift apart and fill each other's gaps.
+  // Six stages in place of three alone left n = 25600, k = 5120 at 64 tokens, cut in two, at 29.8 us (quantizer included),
+  // two k-blocks per barrier brought it to 28.3: the wavefronts drift apart and fill each other's gaps.
   constexpr uint32_t STEP = WM == 2 ? 2 : 1;
   constexpr int XS_BASE = NS * STAGE_BYTES;    // [NS][256] group sums
   constexpr int WS_BASE = XS_BASE + NS * 1024;  // [NS][256 fp16 (+ 512 bytes unused)] weight scales
@@ -246,7 +247,7 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
           "s"(f2h), "s"(f3), "s"(f3h), "s"(src)
         : "memory", "m0");
   };
-  // Everything this wavefront issued has landed except the loads of the youngest NS - 2 * STEP stages (vmcnt retires in issue order;
+  // Everything this wavefront issued has landed except the loads of the youngest NS - 2*STEP stages (vmcnt retires in issue order;
   // a wavefront issues the same loads every stage: 4 weight loads with or without the weight-scale load, or 2*AFW
   // activation loads with or without the group-sum load).
   // This wavefront's fragment reads of the stage have returned: behind the barrier other wavefronts refill the slot they
@@ -383,9 +384,11 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
     }
   };
 
-  // ---- schedule: stage c computes k-block c out of LDS slot c % NS and, right behind its first MFMA, issues the loads
-  // of k-block c+NS-1 into the slot stage c-1 used (every wavefront left it at the previous barrier).  At the end of
-  // the stage the loads of k-block c+1 have to have landed; the barrier makes them visible to all wavefronts.
+  // ---- schedule, in steps of STEP k-blocks between two barriers: k-block c is computed out of LDS slot c % NS and, right
+  // behind its first MFMA, the loads of k-block c+NS-STEP go out into the slot that k-block c-STEP used - the step before,
+  // whose reads had returned in every wavefront at the last barrier.  The wait at the end of a step leaves the loads of the
+  // NS-2*STEP youngest k-blocks in flight: those of the next step's k-blocks have landed, and the barrier makes them visible
+  // to all wavefronts.
 #pragma unroll
   for (uint32_t c = 0; c < NS - STEP; ++c) {
     load_scales(c);
@@ -405,7 +408,7 @@ __global__ void __launch_bounds__(512, 1) w4a8_tile_kernel(W4A8TileParams p) {
         compute((c + h) % NS, c + h + NS - STEP);
       }
     }
-    wait_stage();  // operands and scales of c+1
+    wait_stage();  // operands and scales of the next step
     reads_done();
     __builtin_amdgcn_s_barrier();
   }

@@ -79,6 +79,22 @@ def test_small_problem_rule_and_its_switch():
     assert L.select_tile(L.KIND_W4A16, *small, L.BF16)["kernel"] == 0
 
 
+def test_w4a8_64_token_tiles_serve_whole_tiles_and_long_parts():
+    """Up to 64 tokens: 64-token tiles while K is whole or its parts have 32 k-blocks, 128-token tiles over shorter parts."""
+    from ksanallm_amd import lib as L
+    L.set_small_problem_rule(False)
+    try:
+        for m, n, k, bm, cut in ((64, 28672, 1024, 64, 1), (33, 8192, 1536, 64, 1), (64, 25600, 3072, 64, 1), (64, 25600, 8192, 64, 2),
+                                 (48, 25600, 7936, 128, 2), (40, 16224, 3968, 128, 4), (64, 8192, 14336, 128, 8),
+                                 (33, 4352, 20480, 128, 15), (65, 28672, 1024, 128, 1)):
+            d = L.select_tile(L.KIND_W4A8, m, n, k, L.BF16)
+            assert (d["kernel"], d["block_m"], d["split_k"]) == (1, bm, cut), (m, n, k, d)
+            need = L.load().ksq_w4a8_workspace_size(m, n, k)
+            assert need >= (d["grid"] * bm * 256 * 4 if cut > 1 else 0)
+    finally:
+        L.set_small_problem_rule(True)
+
+
 def test_descriptor_of_the_grouped_streaming_launch():
     """KSQ_KIND_MOE_W4A16 describes the grouped streaming launch, which never cuts K over workgroups: its K slices are its
     wavefronts, four of them while fewer than 32 slots are routed, and then, through LDS, as many as that form has."""

@@ -139,19 +139,21 @@ def test_gemm_tile_kernel(ops, oracle, tile_kernels, out_dtype, m, n, k):
 
 
 # 64- and 128-token tiles keep four and three k-blocks of loads in flight: fewer k-blocks than that, as many, one more; parts of
-# K of one to five k-blocks, even and odd (`parts`: k-blocks of a part, and of the last one); and every count of row tiles that
-# hold tokens, with M % 4 == 0 and without
+# K (`parts`: k-blocks of a part, and of the last one) of one to five k-blocks on the 128-token tile and of 18 to 33, even and
+# odd, on the 64-token tile, which takes parts of 32 and more; and every count of row tiles that hold tokens, with M % 4 == 0 and
+# without
 @pytest.mark.parametrize("m,n,k,parts", [
     (33, 272, 128, None), (48, 4112, 512, None), (49, 256, 640, None), (63, 528, 768, None), (64, 256, 896, None), (64, 272, 1152, None),
     (65, 272, 256, None), (96, 256, 384, None), (127, 528, 512, None), (128, 256, 640, None),
     (64, 256, 1536, (4, 4)), (61, 272, 1664, (4, 1)), (33, 272, 1792, (4, 2)), (47, 272, 2432, (4, 3)), (64, 272, 8320, (5, 5)),
-    (50, 272, 8576, (5, 2)), (128, 256, 1536, (4, 4)), (99, 272, 1664, (4, 1)), (100, 272, 8320, (5, 5))])
+    (50, 272, 8576, (5, 2)), (128, 256, 1536, (4, 4)), (99, 272, 1664, (4, 1)), (100, 272, 8320, (5, 5)),
+    (64, 272, 65664, (33, 18)), (61, 272, 63744, (32, 18)), (33, 256, 67584, (33, 33)), (47, 256, 65536, (32, 32))])
 def test_gemm_tile_kernel_few_tokens(ops, oracle, tile_kernels, m, n, k, parts):
     from ksanallm_amd import lib as L
     desc = L.select_tile(L.KIND_W4A8, m, n, k, H.BF16)
-    assert desc["block_m"] == (64 if m <= 64 else 128)
     kb, cut = k // 128, desc["split_k"]
     per = -(-kb // cut)
+    assert desc["block_m"] == (64 if m <= 64 and (cut == 1 or per >= 32) else 128)
     assert (cut == 1) if parts is None else (cut > 1 and (per, kb - (cut - 1) * per) == parts)
     w, scales = make_weight(n + k + m, k, n)
     x = make_act(m * 3 + n, m, k, H.BF16)
