@@ -1,6 +1,7 @@
 // Per-shape tile selection: closed-form rules of (kind, m, n, k, dtype) for a 256-CU, 8-XCD MI355X.
 // Host code only; no timing and no device queries, so the answer is the same at load time and at run time.
 #include <atomic>
+#include <cmath>
 
 #include "ksq_common.h"
 #include "tile_select.h"
@@ -328,13 +329,36 @@ using namespace ksq;
 // hidden 7168, inter 2048, top-8, whole call with 16- / 32- / 128- / 256-row blocks: 1.50 / 1.49 / 1.61 / - ms at 2 rows
 // per expert, 1.85 / 1.84 / 1.95 / - at 8, - / 1.95 / 1.98 / 2.02 at 12, - / 2.06 / 2.00 / 2.04 at 16, - / 3.18 / 2.12 /
 // 2.12 at 32, - / - / 2.31 / 2.33 at 64, - / - / 2.56 / 2.60 at 96, - / - / 2.85 / 2.75 at 112, - / - / 3.22 / 2.87 at 125,
-// - / - / 3.29 / 2.91 at 128, - / - / 3.85 / 3.40 at 160, - / - / 5.45 / 4.92 at 256.
+// - / - / 3.29 / 2.91 at 128, - / - / 3.85 / 3.40 at 160, - / - / 5.45 / 4.92 at 256.  (Other sizes: ksq_moe_fp8_block_m_sized.)
 KSQ_EXPORT size_t ksq_moe_fp8_block_m(size_t numel, size_t E) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E;
   if (per_expert >= 104) return 256;
   if (per_expert >= 16) return 128;
   return per_expert < 2 ? 16 : 32;
+}
+
+// The same where the experts' sizes are known.  Between 104 and 127 slots per expert the larger block pays by the rounds of
+// workgroups that it saves: in 128-slot blocks, experts of more than 128 slots bring a second row block - their expected
+// number under even routing, 128.5 - mean in standard deviations of a binomial -, and where those start another round of the
+// 256 CUs in either GEMM, 256-slot blocks are up to a quarter faster; where they do not, a block of up to 160 slots is a
+// longer chain than two of 128 and 1-7 % slower.  Whole call with 128- / 256-slot blocks, us, the faster one chosen: 32
+// experts, hidden 2048, inter 1024 (256 workgroups) at 112 slots 122.9 / 92.9; 64, 1024, 512 (256) at 120 97.8 / 79.1; 16,
+// 7168, 2048 at 112 266.7 / 231.9; 24, 2048, 1024 (192) at 120 86.2 / 90.7, at 127 104.4 / 90.4; 32, 1024, 512 (128) at
+// 120 61.4 / 65.0; 16, 1152, 512 at 120 78.9 / 82.2; 8, 7168, 2048 at 112 134.9 / 138.6, at 127 156.1 / 143.1.  Over 92
+// sizes of 4 to 160 experts the choice was at most 4.5 % behind the other one, the constant line at 104 slots 7 %.
+// (From 128 slots on every second expert has a second row block, and the line is the one above.)
+KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidden, size_t inter) {
+  const size_t block_m = ksq_moe_fp8_block_m(numel, E);
+  if (block_m != 256 || numel / E >= 128) return block_m;
+  const double mean = static_cast<double>(numel) / E, variance = mean * (1.0 - 1.0 / E);
+  const double share = variance > 0 ? 0.5 * std::erfc((128.5 - mean) / std::sqrt(2.0 * variance)) : 0.0;
+  const size_t blocks = E + static_cast<size_t>(std::ceil(share * E));
+  for (size_t n : {2 * inter, hidden}) {
+    const size_t tiles = div_up(n, 256);
+    if (div_up(blocks * tiles, kNumCU) > div_up(E * tiles, kNumCU)) return 256;
+  }
+  return 128;
 }
 
 // Rows per expert block for numel routed (token, slot) pairs over E experts.  Replaces the M thresholds of

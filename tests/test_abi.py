@@ -95,6 +95,23 @@ def test_w4a8_64_token_tiles_serve_whole_tiles_and_long_parts():
         L.set_small_problem_rule(True)
 
 
+def test_block_fp8_expert_blocks_follow_the_rounds_of_workgroups():
+    """Slots per expert below 104 or from 128 on: the rule of unknown sizes.  Between: 256-slot blocks where the experts that
+    need a second 128-slot block start another round of 256 workgroups in either GEMM."""
+    from ksanallm_amd import lib as L
+    lib = L.load()
+    for per in (0, 1, 2, 15, 16, 103, 128, 400):
+        for E, hidden, inter in ((1, 7168, 2048), (16, 1152, 512), (256, 7168, 2048)):
+            numel = per * E + E // 2
+            assert lib.ksq_moe_fp8_block_m_sized(numel, E, hidden, inter) == lib.ksq_moe_fp8_block_m(numel, E)
+    assert lib.ksq_moe_fp8_block_m_sized(100, 0, 1024, 512) == 16
+    for E, hidden, inter, per, bm in ((32, 2048, 1024, 104, 256), (64, 1024, 512, 120, 256), (256, 7168, 2048, 104, 256),
+                                      (16, 7168, 2048, 112, 256), (24, 2048, 1024, 120, 128), (24, 2048, 1024, 127, 256),
+                                      (32, 1024, 512, 127, 128), (16, 1152, 512, 120, 128), (8, 7168, 2048, 112, 128),
+                                      (8, 7168, 2048, 127, 256), (1, 7168, 2048, 120, 128)):
+        assert lib.ksq_moe_fp8_block_m_sized(per * E, E, hidden, inter) == bm, (E, hidden, inter, per)
+
+
 def test_descriptor_of_the_grouped_streaming_launch():
     """KSQ_KIND_MOE_W4A16 describes the grouped streaming launch, which never cuts K over workgroups: its K slices are its
     wavefronts, four of them while fewer than 32 slots are routed, and then, through LDS, as many as that form has."""
