@@ -13,10 +13,13 @@
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <utility>
 
 #include "ksq.h"
 
@@ -37,10 +40,27 @@ struct Library {
 } lib;
 PyObject* check_fn = nullptr;  // ksanallm_amd.lib.check: raises KsqError with the library's message
 
+// Lets other Python threads run from the first allocation of a call on, to its end (its arguments are read before):
+// allocations and the library's calls may wait for the device (an allocator that has to ask the driver, or to give memory
+// back first).  One hand-over per call: with one per allocation and launch, and the device set and reset beside it, the
+// smallest call took 4.46 us, 4.28 before that and 4.0 to 4.1 now.  The state is this thread's; an entry point puts an outer
+// call's aside (a Python allocator or dispatch mode may call back).
+thread_local PyThreadState* without_gil = nullptr;
+void release_gil() {
+  if (!without_gil) without_gil = PyEval_SaveThread();
+}
+void hold_gil() {
+  if (PyThreadState* state = without_gil) {
+    without_gil = nullptr;
+    PyEval_RestoreThread(state);
+  }
+}
+
 // A Python exception is set; unwinds to the entry point.
 struct PyRaised {};
 
 [[noreturn]] void raise(PyObject* type, const char* fmt, ...) {
+  hold_gil();
   va_list ap;
   va_start(ap, fmt);
   PyErr_FormatV(type, fmt, ap);
@@ -48,21 +68,12 @@ struct PyRaised {};
   throw PyRaised{};
 }
 
-// Lets other Python threads run: around the library's calls and around allocations, either of which may wait for the
-// device (an allocator that has to ask the driver, or to give memory back first).
-struct WithoutGil {
-  PyThreadState* state = PyEval_SaveThread();
-  ~WithoutGil() { PyEval_RestoreThread(state); }
-};
-
 template <typename F>
 void call(F&& f) {
-  int rc;
-  {
-    const WithoutGil no_gil;
-    rc = f();
-  }
+  release_gil();
+  const int rc = f();
   if (rc == 0) return;
+  hold_gil();
   PyObject* r = PyObject_CallFunction(check_fn, "i", rc);
   Py_XDECREF(r);
   if (!PyErr_Occurred()) PyErr_Format(PyExc_RuntimeError, "ksq status %d", rc);
@@ -143,11 +154,11 @@ size_t dim(const at::Tensor& t, int64_t d, int64_t dims, const char* what) {
 }
 
 // ------------------------------------------------------------------------------------------------ device, allocation, stream
-// Makes the tensor's device the current one for the rest of the call.
+// Makes the tensor's device the current one for the rest of the call, where it is not that already.
 struct OnDevice {
   c10::OptionalDeviceGuard guard;
   explicit OnDevice(const at::Tensor& t) {
-    if (t.is_cuda()) guard.reset_device(t.device());
+    if (t.is_cuda() && t.device().index() != c10::hip::current_device()) guard.reset_device(t.device());
   }
 };
 
@@ -156,7 +167,7 @@ at::Tensor empty(std::initializer_list<size_t> shape, at::ScalarType dtype, cons
   int n = 0;
   for (size_t v : shape) s[n++] = static_cast<int64_t>(v);
   const at::IntArrayRef sizes(s, n);
-  const WithoutGil no_gil;
+  release_gil();
   if (!like.is_cuda()) return at::empty(sizes, like.options().dtype(dtype));
   return at::Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));
 }
@@ -177,13 +188,18 @@ struct Scratch {  // nullptr and 0 where nothing is needed
   }
 };
 
-// of the current device
-void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+// the stream that is current on the tensor's device (without one: on the current device)
+void* stream(const at::Tensor* t = nullptr) {
+  return c10::hip::getCurrentHIPStream(t && t->is_cuda() ? t->device().index() : -1).stream();
+}
 
 // fp32, flat, contiguous: the tensor itself when it is that already
 at::Tensor flat(const at::Tensor& t, at::ScalarType dtype) {
   if (t.scalar_type() == dtype && t.is_contiguous()) return t;
-  return t.reshape({-1}).to(dtype).contiguous();
+  release_gil();
+  at::Tensor r = t.reshape({-1}).to(dtype).contiguous();
+  hold_gil();  // further arguments are read after it
+  return r;
 }
 
 // ------------------------------------------------------------------------------------------------ the calls
@@ -207,7 +223,7 @@ at::Tensor w4a16_gemm(const Args& a) {
   }
   at::Tensor out = given ? *given : empty({m, n}, x.scalar_type(), x);
   const Scratch scratch(ws, x, ws ? 0 : lib.w4a16_workspace_size(m, n, k, group, d));
-  void *po = ptr(out), *px = ptr(x), *pw = ptr(w), *ps = ptr(s), *pz = ptr(z), *st = stream();
+  void *po = ptr(out), *px = ptr(x), *pw = ptr(w), *ps = ptr(s), *pz = ptr(z), *st = stream(&x);
   call([&] { return lib.w4a16_gemm(po, px, pw, ps, pz, scratch.p, scratch.bytes, m, n, k, group, d, st); });
   return out;
 }
@@ -225,7 +241,7 @@ std::pair<at::Tensor, at::Tensor> group_quant(const at::Tensor& x, size_t k, siz
   at::Tensor s = s_given ? *s_given
                          : (column_major ? empty({k / group, m}, at::kFloat, x) : empty({m, k / group}, at::kFloat, x));
   const int d = dt(x, true);
-  void *px = ptr(x), *pq = ptr(q), *ps = ptr(s), *st = stream();
+  void *px = ptr(x), *pq = ptr(q), *ps = ptr(s), *st = stream(&x);
   call([&] { return lib.fp8_group_quant(px, pq, ps, m, k, group, column_major, fuse, d, st); });
   return {std::move(q), std::move(s)};
 }
@@ -242,7 +258,7 @@ at::Tensor fp8_blockwise_gemm(const Args& a) {
   const int d = dt(out, true);
   need_bytes(out, product({m, n, static_cast<size_t>(out.element_size())}), "fp8_blockwise_gemm: out");
   const Scratch scratch(ws, aq, ws ? 0 : lib.fp8_blockwise_workspace_size(m, n, k));
-  void *po = ptr(out), *pa = ptr(aq), *pas = ptr(as), *pb = ptr(b), *pbs = ptr(bs), *st = stream();
+  void *po = ptr(out), *pa = ptr(aq), *pas = ptr(as), *pb = ptr(b), *pbs = ptr(bs), *st = stream(&aq);
   call([&] { return lib.fp8_blockwise_gemm(pa, pas, pb, pbs, po, m, n, k, d, scratch.p, scratch.bytes, st); });
   return out;
 }
@@ -260,7 +276,7 @@ std::pair<at::Tensor, at::Tensor> w4a8_static_quant(const Args& a) {
   int mode = per_channel ? KSQ_W4A8_PER_CHANNEL : (per_token ? KSQ_W4A8_PER_TOKEN : KSQ_W4A8_PER_TENSOR);
   if (group == 64) mode |= KSQ_W4A8_SUMS_PER_64;
   const int d = dt(x);
-  void *px = ptr(x), *psc = ptr(scale), *pq = ptr(q), *pxs = ptr(xsum), *st = stream();
+  void *px = ptr(x), *psc = ptr(scale), *pq = ptr(q), *pxs = ptr(xsum), *st = stream(&x);
   call([&] { return lib.w4a8_static_quant(px, psc, pq, pxs, m, k, mode, d, st); });
   return {std::move(q), std::move(xsum)};
 }
@@ -282,7 +298,7 @@ at::Tensor w4a8_gemm(const Args& a) {
   const int d = dt(out);
   need_bytes(out, product({m, n, 2}), "w4a8_gemm: out");
   const Scratch scratch(ws, aq, ws ? 0 : lib.w4a8_workspace_size(m, n, k));
-  void *po = ptr(out), *pa = ptr(aq), *pxs = ptr(xsum), *pw = ptr(w), *ps = ptr(scales), *st = stream();
+  void *po = ptr(out), *pa = ptr(aq), *pxs = ptr(xsum), *pw = ptr(w), *ps = ptr(scales), *st = stream(&aq);
   call([&] {
     return lib.w4a8_gemm(pa, pxs, pw, ps, static_cast<float>(alpha), po, m, n, k, group, d, scratch.p, scratch.bytes, st);
   });
@@ -298,7 +314,7 @@ std::pair<at::Tensor, at::Tensor> moe_topk_softmax(const Args& a) {
   const size_t tokens = dim(gating, 0, 2, "moe_topk_softmax: gating"), E = gating.size(1);
   const int d = dt(gating, true);
   at::Tensor w = empty({tokens, top_k}, at::kFloat, gating), ids = empty({tokens, top_k}, at::kInt, gating);
-  void *pg = ptr(gating), *pw = ptr(w), *pi = ptr(ids), *st = stream();
+  void *pg = ptr(gating), *pw = ptr(w), *pi = ptr(ids), *st = stream(&gating);
   call([&] { return lib.moe_topk_softmax(pg, pw, pi, tokens, E, top_k, norm, scaling, d, st); });
   return {std::move(w), std::move(ids)};
 }
@@ -318,7 +334,7 @@ std::pair<at::Tensor, at::Tensor> moe_grouped_topk(const Args& a) {
     if (bias->scalar_type() != at::kFloat) raise(PyExc_ValueError, "e_bias must be fp32");
     need_bytes(*bias, product({E, 4}), "moe_grouped_topk: e_bias");
   }
-  void *pg = ptr(gating), *pb = ptr(bias), *pw = ptr(w), *pi = ptr(ids), *st = stream();
+  void *pg = ptr(gating), *pb = ptr(bias), *pw = ptr(w), *pi = ptr(ids), *st = stream(&gating);
   call([&] {
     return lib.moe_grouped_topk(pg, pb, pw, pi, tokens, E, top_k, groups, topk_group, sigmoid, renormalize, scaling, d, st);
   });
@@ -374,7 +390,7 @@ at::Tensor fused_moe_w4a16(const Args& a) {
   need_bytes(s2, product({E, inter / group, hidden, 2}), "fused_moe_w4a16: down scales");
   const int d = dt(x);
   const at::ScalarType t = x.scalar_type();
-  void *st = stream(), *px = ptr(x), *pw13 = ptr(w13), *ps13 = ptr(s13), *pw2 = ptr(w2), *ps2 = ptr(s2), *ptw = ptr(r.w),
+  void *st = stream(&x), *px = ptr(x), *pw13 = ptr(w13), *ps13 = ptr(s13), *pw2 = ptr(w2), *ps2 = ptr(s2), *ptw = ptr(r.w),
        *pids = ptr(r.ids);
   if (!block_given && r.tokens <= few_tokens && r.numel <= 64 && r.top_k <= 32 && (2 * inter) % 32 == 0) {
     // a few decode tokens: two launches - the first GEMM with every slot a block of its own (no aligned permutation) and
@@ -432,7 +448,7 @@ at::Tensor fused_moe_fp8_blockwise(const Args& a) {
   need_bytes(s2, product({E, (hidden + 127) / 128, inter / 128, 4}), "fused_moe_fp8_blockwise: down scales");
   const int d = dt(x);
   const at::ScalarType t = x.scalar_type();
-  void *st = stream(), *pw13 = ptr(w13), *ps13 = ptr(s13), *pw2 = ptr(w2), *ps2 = ptr(s2), *ptw = ptr(r.w), *pids = ptr(r.ids);
+  void *st = stream(&x), *pw13 = ptr(w13), *ps13 = ptr(s13), *pw2 = ptr(w2), *ps2 = ptr(s2), *ptw = ptr(r.w), *pids = ptr(r.ids);
   const bool few = !block_given && r.tokens <= few_tokens && r.numel <= 64 && r.top_k <= 32;
   if (!block_given && !few) block_m = lib.moe_fp8_block_m_sized(r.numel, E, hidden, inter);
   if (!few && block_m == 0) raise(PyExc_ZeroDivisionError, "block size 0");
@@ -493,15 +509,22 @@ PyObject* entry(PyObject*, PyObject* const* v, Py_ssize_t n) {
     PyErr_SetString(PyExc_RuntimeError, "bind() has not been called");
     return nullptr;
   }
+  PyThreadState* const outer = std::exchange(without_gil, nullptr);
+  PyObject* r = nullptr;
   try {
-    return wrap(F(Args{v, n}));
-  } catch (const PyRaised&) {
+    auto result = F(Args{v, n});
+    hold_gil();
+    r = wrap(std::move(result));
+  } catch (const PyRaised&) {  // (raise() holds the lock)
   } catch (const std::bad_alloc&) {
+    hold_gil();
     PyErr_NoMemory();
   } catch (const std::exception& e) {  // out of device memory, among others: torch's own exception types
+    hold_gil();
     torch::translate_exception_to_python(std::current_exception());
   }
-  return nullptr;
+  without_gil = outer;
+  return r;
 }
 
 PyObject* current_stream(PyObject*, PyObject*) {
