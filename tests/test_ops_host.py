@@ -8,18 +8,17 @@ import torch
 
 
 def test_allocation_runs_without_the_interpreter_lock():
-    """An allocation that takes its time (here: outputs that torch is told to fill) does not stop the other Python threads."""
+    """An allocation that takes its time (here: outputs that torch is told to fill) does not stop the other Python threads: one
+    that wakes every millisecond goes on waking.  Under the lock it would wake at most between the call's two allocations and
+    around them, however long these take."""
     from ksanallm_amd import ops
     before = torch.are_deterministic_algorithms_enabled(), torch.utils.deterministic.fill_uninitialized_memory, torch.get_num_threads()
-    stop, gaps = threading.Event(), []
+    stop, ticks = threading.Event(), []
 
     def tick():
-        last = time.perf_counter()
         while not stop.is_set():
             time.sleep(0.001)
-            now = time.perf_counter()
-            gaps.append(now - last)
-            last = now
+            ticks.append(time.perf_counter())
     thread = threading.Thread(target=tick)
     torch.use_deterministic_algorithms(True)
     torch.utils.deterministic.fill_uninitialized_memory = True
@@ -27,19 +26,19 @@ def test_allocation_runs_without_the_interpreter_lock():
     try:
         thread.start()
         time.sleep(0.02)
-        del gaps[:]
         t0 = time.perf_counter()
         with pytest.raises(AssertionError, match="device-resident"):
             ops.moe_topk_softmax(torch.zeros((1, 8)), 1 << 26)   # two outputs of 256 MiB
-        took = time.perf_counter() - t0
+        t1 = time.perf_counter()
     finally:
         stop.set()
         thread.join()
         torch.use_deterministic_algorithms(before[0])
         torch.utils.deterministic.fill_uninitialized_memory = before[1]
         torch.set_num_threads(before[2])
-    assert took > 0.05, "the allocation was over too soon to tell (%.3f s)" % took
-    assert max(gaps) < took / 3, "another thread stood still for %.3f of %.3f s" % (max(gaps), took)
+    assert t1 - t0 > 0.02, "the allocation was over too soon to tell (%.3f s)" % (t1 - t0)
+    woke = sum(t0 < t < t1 for t in ticks)
+    assert woke >= 8, "another thread ran %d times in %.3f s" % (woke, t1 - t0)
 
 
 def test_out_dtype_is_not_looked_at_where_out_is_given():
