@@ -141,8 +141,9 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   // so that a stage's weight loads go out at its start and not behind an MFMA (n = 12480, k = 6912: 385 tokens, nine row tiles
   // in the second block, 69.7 us shared evenly and 64.8 as 8 and 1; 1121, seven in the last, 109.1 and 103.1; ten row tiles
   // the same either way, twelve 69.3 and 70.3).  A 128-token tile shares evenly at every count (52 tokens, four row tiles,
-  // n = 13856, k = 1152: 14.9 and 17.2 us; six row tiles as 4 and 2 would be 1-3 % ahead, but the same rule in that instance
-  // cost its full tiles 1-5 %).
+  // n = 13856, k = 1152: 14.9 and 17.2 us), though a last block of few row tiles behind full ones loses up to 2 % by it (523
+  // tokens, n = 6656, k = 10752: 88.9 and 87.7) and six row tiles as 4 and 2 would be 1-3 % ahead: the rule of the 256-token
+  // tile in that instance cost its full tiles 1-5 %.
   const uint32_t per_wave = !GROUPED && WM == 8 && live_tiles <= 9 ? WM : (live_tiles + 1) / 2;  // row tiles a wavefront covers
   const uint32_t rt0 = wm * per_wave;              // its first row tile
   const uint32_t mine = live_tiles > rt0 ? (live_tiles - rt0 < per_wave ? live_tiles - rt0 : per_wave) : 0;

@@ -64,7 +64,7 @@ SplitKChoice select_splitk(size_t m, size_t n, size_t k) {
   //   7.9 us in registers, 8.4 us through LDS), and with up to 8 rows four column tiles per wavefront beat eight
   //   (n = 57344, k = 8192, 1 row: 40.7 against 43.1 us).
   // - K cut over workgroups, 17 rows and more: x outweighs the weights there by construction (n = 4096, k = 14336: 20 rows
-  //   13.2 -> 12.9 us, 32 rows 15.8 -> 14.3..15.2, 64 rows 21.6 -> 19.0, 128 rows 36.7 -> 31.5; n = k = 5120 at 32 rows
+  //   13.2 -> 12.9 us, 32 rows 15.8 -> 14.3..15.2, 64 rows 21.6 -> 19.0; n = k = 5120 at 32 rows
   //   12.7 -> 11.6; n = 5120, k = 25600 at 32 rows 34.4 -> 29.0; n = 2048, k = 8192 at 32 rows 11.5 -> 11.0).  Eight
   //   wavefronts are one workgroup per CU where the register form holds two, so with more workgroups than CUs a second
   //   round begins and takes back what the traffic gave (n = 2112, k = 17024, 264 workgroups: 17 rows 16.6 -> 18.2 us,
@@ -148,7 +148,9 @@ SplitKChoice select_splitk_grouped(size_t block_m, size_t blocks, size_t numel, 
 // 11.3 / 26.4, at 512 rows 29.2 / 40.1; n = k = 8192 at 64 rows 18.1 / 24.1, at 128 rows 30.6 / 32.0, at 192 rows
 // 44.4 / 41.3; n = 14336, k = 4096 at 64 rows 17.9 / 23.1, at 128 rows 26.4 / 30.3, at 384 rows 75.1 / 56.3; n = 4096,
 // k = 14336 at 128 rows 27.9 / 32.1, at 192 rows 48.4 / 38.9; n = 25600, k = 5120 at 64 rows 33.5 / 37.6, at 96 rows
-// 48.6 / 46.1; n = 4096, k = 28672 at 64 rows 35.8 / 34.4; n = 5120, k = 25600 at 64 rows 61.7 / 36.6.
+// 48.6 / 46.1; n = 4096, k = 28672 at 64 rows 35.8 / 34.4; n = 5120, k = 25600 at 64 rows 61.7 / 36.6.  With the tile kernel's
+// instances per number of live row tiles the line stays: n = k = 8192 at 128 rows 32.6 / 32.0, n = 25600, k = 5120 at 64 rows
+// 35.1 / 36.1, n = 14336, k = 4096 at 128 rows 28.5 / 30.3, n = 4096, k = 14336 at 128 rows 29.4 / 32.1.
 // (Group 128 only: the wide decode instances exist for that group.)
 bool small_w4a16_problem(size_t m, size_t n, size_t k, size_t group) {
   const size_t limit = k >= 4 * n ? (size_t(1) << 27) : (size_t(1) << 28);
@@ -234,8 +236,8 @@ TilePlan plan_mfma_tile(size_t m, size_t n, size_t k) {
 // tokens 28.5 / 23.8; n = 2048, k = 7168 at 128 tokens 16.0 / 23.1, at 256 tokens 16.0 / 22.2, at 384 tokens 29.2 / 23.4;
 // n = 7168, k = 2048 at 192 tokens 18.9 / 23.6, at 256 tokens 24.0 / 23.6; n = 4608, k = 7168 at 64 tokens 17.1 / 18.7, at
 // 128 tokens 31.9 / 22.3; n = 7168, k = 4608 at 64 tokens 13.6 / 18.0, at 96 tokens 25.0 / 20.0; n = k = 7168 at 64 tokens
-// 18.2 / 21.0, at 96 tokens 33.6 / 22.9; n = 24576, k = 1536 at 64 tokens 22.0 / 19.6; n = 18432, k = 7168 at 48 tokens
-// 52.9 / 32.1.
+// 18.2 / 20.5, at 96 tokens 33.6 / 23.1; n = 24576, k = 1536 at 64 tokens 22.0 / 16.6; n = 18432, k = 7168 at 48 tokens
+// 52.9 / 31.8.
 bool use_fp8_tile(size_t m, size_t n, size_t k) {
   if (m <= 32) return false;
   if (g_small_problem_rule.load(std::memory_order_relaxed) && m <= kRowBlockMaxM && n <= 4 * k &&
@@ -249,7 +251,7 @@ bool use_fp8_tile(size_t m, size_t n, size_t k) {
 // tokens 10.5 / 24.1, at 256 tokens 15.3 / 24.1, at 512 tokens 35.0 / 26.0; n = k = 5120 at 96 tokens 11.7 / 22.8, at 192
 // tokens 18.7 / 23.6, at 256 tokens 28.5 / 24.6; n = 8192, k = 2048 at 128 tokens 10.3 / 23.6; n = 2048, k = 7168 at 256
 // tokens 16.4 / 22.0; n = k = 8192 at 64 tokens 18.1 / 20.0, at 96 tokens 26.1 / 24.7; n = 14336, k = 4096 at 64 tokens
-// 15.6 / 18.7, at 96 tokens 23.7 / 23.7; n = 25600, k = 5120 at 48 tokens 32.8 / 27.1.
+// 15.6 / 18.6, at 96 tokens 23.7 / 23.4; n = 25600, k = 5120 at 48 tokens 32.8 / 25.6.
 bool use_w4a8_tile(size_t m, size_t n, size_t k) {
   if (m <= 32) return false;
   if (g_small_problem_rule.load(std::memory_order_relaxed) && m <= kRowBlockMaxM && n <= 4 * k &&

@@ -485,7 +485,9 @@ __global__ void __launch_bounds__(512, 1) w4a16_tile_kernel(TileParams p) {
   // to those over 8 and 12 took a tenth off the whole call.  Dense form: a prompt or a batch of 129..255 rows is one
   // 256-row tile, all of which was multiplied as soon as more than half of it held rows (n = 14336, k = 4096, 150 rows,
   // bf16 with zero points: 40.9 -> 34.6 us with ten of sixteen row tiles multiplied).
-  // (groups of 64 and 32 rows, dense: half of the tile or all of it)
+  // (groups of 64 and 32 rows, dense: half of the tile or all of it.  The loop would serve every count there too; those
+  // formats are rare and each instance is another copy of the loop, so these are not built, and what they would give is not
+  // measured.)
   if constexpr (GROUPED || GROUP == 128) {
     for_tile_count<4, WM>(live_tiles, run);
   } else if (live_tiles <= WM / 2) {
