@@ -363,6 +363,22 @@ KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidde
   return 128;
 }
 
+// The block size of a whole block-fp8 expert block (both GEMMs and their alignment), the streaming tile kernel
+// (fp8_stream.h) counted in.  From four slots per expert on its row blocks beat the 32-row blocks of the decode form where
+// the experts give at least every other CU a 256-column tile in both GEMMs, us in 32-slot / 128-slot blocks at 4 and 8 slots:
+// 256 experts, hidden 7168, inter 2048 1748 / 1691 and 1848 / 1758; 256, 1024, 512 131 / 102 and 147 / 110; 64, 1024, 512 49 / 39 and
+// 53 / 40; 16, 4096, 2048 87 / 83 and 89 / 84; 32, 1024, 512 (128 tiles) 32.5 / 31.4 and 34.2 / 32.5; 16, 2048, 1408 (128) 47.5 /
+// 45.3 and 49.5 / 46.2; but 8, 4096, 1536 (96) 48.2 / 51.2 and 49.9 / 52.2, 16, 1024, 512 (64) 25.2 / 28.9 and 25.6 / 29.2.  (Below
+// four: 32, 4096, 2048 at 1 and 2 slots 106 / 118 and 138 / 139, 128, 2944, 768 at 1 118 / 122.)  From 64 slots on 256-slot
+// blocks, so that few experts need two (32, 4096, 2048 at 110, 128- / 256-slot blocks 240 / 205; 256, 7168, 2048 at 112 2449 / 2329).
+KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {
+  if (E == 0) return 16;
+  const size_t per_expert = numel / E, tiles = E * div_up(2 * inter < hidden ? 2 * inter : hidden, 256);
+  if (per_expert >= 64) return 256;
+  if (per_expert >= 16 || (per_expert >= 4 && tiles >= static_cast<size_t>(kNumCU) / 2)) return 128;
+  return ksq_moe_fp8_block_m(numel, E);
+}
+
 // Rows per expert block for numel routed (token, slot) pairs over E experts.  Replaces the M thresholds of
 // InvokeFusedMoe (16 / 32 / 64 rows by token count): below about 40 rows per expert the weights are streamed once per
 // 16- or 32-row block (HBM-bound); above, the MFMA tile kernel takes 256-row blocks, of which it multiplies the row

@@ -29,7 +29,7 @@ namespace {
 #define KSQ_FOR_EACH_FN(F) \
   F(w4a16_workspace_size) F(w4a16_gemm) F(fp8_group_quant) F(fp8_blockwise_workspace_size) F(fp8_blockwise_gemm) \
   F(w4a8_static_quant) F(w4a8_workspace_size) F(w4a8_gemm) F(moe_topk_softmax) F(moe_grouped_topk) \
-  F(moe_align_capacity) F(moe_align_scratch_bytes) F(moe_align) F(moe_block_m) F(moe_fp8_block_m_sized) F(moe_w4a16_gemm) \
+  F(moe_align_capacity) F(moe_align_scratch_bytes) F(moe_align) F(moe_block_m) F(moe_fp8_row_block) F(moe_w4a16_gemm) \
   F(moe_w4a16_gate_up_silu) F(moe_w4a16_down_sum) F(moe_fp8_blockwise_gemm) F(moe_fp8_down_sum) F(moe_silu_mul) \
   F(moe_sum)
 
@@ -450,7 +450,7 @@ at::Tensor fused_moe_fp8_blockwise(const Args& a) {
   const at::ScalarType t = x.scalar_type();
   void *st = stream(&x), *pw13 = ptr(w13), *ps13 = ptr(s13), *pw2 = ptr(w2), *ps2 = ptr(s2), *ptw = ptr(r.w), *pids = ptr(r.ids);
   const bool few = !block_given && r.tokens <= few_tokens && r.numel <= 64 && r.top_k <= 32;
-  if (!block_given && !few) block_m = lib.moe_fp8_block_m_sized(r.numel, E, hidden, inter);
+  if (!block_given && !few) block_m = lib.moe_fp8_row_block(r.numel, E, hidden, inter);
   if (!few && block_m == 0) raise(PyExc_ZeroDivisionError, "block size 0");
   Aligned al;
   if (!few) al = moe_align(r.ids, E, block_m, st);

@@ -36,7 +36,7 @@ class MoeLayer : public BaseLayer {
   // rows per expert, which changes no result)
   size_t BlockM(size_t tokens) const {
     if (IsFp8())
-      return ksq_moe_fp8_block_m_sized(tokens * expert_topk_, expert_num_per_node_, expert_hidden_size_, expert_inter_size_);
+      return ksq_moe_fp8_row_block(tokens * expert_topk_, expert_num_per_node_, expert_hidden_size_, expert_inter_size_);
     return ksq_moe_block_m(tokens * expert_topk_, expert_num_per_node_);
   }
   bool IsFp8() const { return compute_dtype_ == TYPE_BLOCK_FP8_E4M3; }

@@ -66,6 +66,7 @@ SIGNATURES = {
     "ksq_moe_block_m": (c_sz, [c_sz, c_sz]),
     "ksq_moe_fp8_block_m": (c_sz, [c_sz, c_sz]),
     "ksq_moe_fp8_block_m_sized": (c_sz, [c_sz, c_sz, c_sz, c_sz]),
+    "ksq_moe_fp8_row_block": (c_sz, [c_sz, c_sz, c_sz, c_sz]),
     "ksq_moe_fp8_blockwise_gemm": (c_i, [c_p, c_p, c_p, c_i, c_sz, c_p, c_p, c_p, c_p, c_p, c_p, c_sz, c_sz, c_sz, c_sz,
                                          c_sz, c_sz, c_i, c_p]),
     "ksq_moe_fp8_down_sum": (c_i, [c_p, c_p, c_p, c_p, c_p, c_p, c_p, c_sz, c_sz, c_sz, c_sz, c_sz, c_i, c_p]),

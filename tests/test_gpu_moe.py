@@ -587,6 +587,34 @@ def test_grouped_fp8_tile_kernel_at_the_edges_of_the_three_stage_tile(ops, oracl
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("kb", [1, 2, 3, 4, 5, 6, 7, 8, 9, 13])
+@pytest.mark.parametrize("bm,rows", [(128, [1, 128, 65, 17]), (256, [208, 256, 131, 16, 209])])
+def test_grouped_fp8_streaming_tile_over_its_ring(ops, oracle, bm, rows, kb):
+    """Every remainder of the k-blocks over the rings of the streaming tile kernel (four, three and two k-blocks deep by the
+    number of row tiles), with the scales of four k-blocks in one piece (kb % 4 == 0) and without, and a ragged last column
+    tile."""
+    E, T, topk, n, k = len(rows), sum(rows) // 2, 2, 272, 128 * kb
+    g = H.gen(8000 + kb + bm)
+    bq, bs = _fp8_experts(oracle, 8010 + kb, E, n, k)
+    x = torch.randn((T, k), generator=g).to(torch.bfloat16)
+    ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])[:T * topk]
+    ids = ids[torch.randperm(T * topk, generator=g)].reshape(T, topk).contiguous()
+    tw = torch.rand((T, topk), generator=g) + 0.1
+    q, s = ops.per_token_group_quant_fp8(x.cuda(), k, 128, False)
+    sorted_ids, expert_ids, npp = ops.moe_align_block_size(ids.cuda(), E, bm)
+    assert T * topk <= bm * E
+    out = ops.moe_fp8_blockwise_gemm(q, s, False, ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda(),
+                                     tw.reshape(-1).cuda(), sorted_ids, expert_ids, npp, T * topk, topk, bm, torch.bfloat16)
+    qh, sh = q.cpu().numpy(), s.cpu().numpy()
+    ref = np.zeros((T * topk, n), np.float32)
+    flat = ids.reshape(-1).numpy()
+    for e in range(E):
+        slots = np.nonzero(flat == e)[0]
+        ref[slots] = oracle.fp8_blockwise_gemm(qh[slots // topk], np.ascontiguousarray(sh[slots // topk]), bq[e], bs[e], False)
+    ref *= tw.reshape(-1, 1).numpy()
+    H.check_gemm(out, ref, H.BF16, "fp8 streaming tile kernel, %d k-blocks" % kb)
+
+
 def test_grouped_fp8_tile_kernel_where_three_stages_do_not_fit(ops, oracle):
     """K > 28672 leaves no room in the LDS for three stages: every 256-slot block then runs on two, one without any token
     (which the alignment never makes, but a caller's own permutation may) among them."""
