@@ -335,6 +335,19 @@ int ksq_moe_fp8_blockwise_gemm(void* out, const void* a_q, const void* a_s, int 
                                const void* b_s, const void* topk_w, const void* sorted_ids, const void* expert_ids,
                                const void* num_post_pad, size_t numel, size_t top_k, size_t E, size_t n, size_t k,
                                size_t block_m, int out_dtype, void* stream);
+/* The first GEMM of block-fp8 experts with silu * mul and the second quantization in its epilogue: weights b [E, 2 * inter, k]
+ * (n = 2 * inter, gate rows in front), results q [numel, inter] e4m3 and s fp32 [numel, inter / 128], the bits that
+ * ksq_moe_fp8_blockwise_gemm into `dtype` followed by ksq_fp8_group_quant with the fused activation give, without the
+ * [numel, 2 * inter] buffer in between.  ksq_moe_fp8_fused_quant() tells whether it serves a call (1) or not (0, and the call
+ * returns KSQ_ERR_UNSUPPORTED): the streaming tile kernel has to take it and n has to be a multiple of 256.
+ * Replaces the fused_moe_kernel launch, InvokeSiluAndMul and InvokePerTokenGroupQuantFp8E4m3 of InvokeFusedMoe
+ * (S/kernels/nvidia/moe_kernel_wrapper.cpp:498-560). */
+int ksq_moe_fp8_fused_quant(size_t numel, size_t E, size_t n, size_t k, size_t block_m);
+int ksq_moe_fp8_gate_up_quant(void* q, void* s, const void* a_q, const void* a_s, int a_s_column_major, size_t a_rows,
+                              const void* b, const void* b_s, const void* sorted_ids, const void* expert_ids,
+                              const void* num_post_pad, size_t numel, size_t top_k, size_t E, size_t n, size_t k, size_t block_m,
+                              int dtype, void* stream);
+
 /* ksq_moe_w4a16_down_sum for block-quantized fp8 experts: the second GEMM and the sum over top-k in one launch, for up
  * to 8 tokens.  a_q [tokens * top_k, k] e4m3 with scales a_s [tokens * top_k, k/128] row-major (the second
  * quantization's output), b / b_s the experts' packed weights and block scales, topk_w / topk_ids [tokens, top_k];

@@ -368,11 +368,12 @@ int launch_fp8_tile_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s) 
 }
 
 // grouped (MoE) form of the streaming tile kernel: one block of 16 * RT_MAX slots per row tile
-template <typename TO, int RT_MAX>
-int launch_fp8_stream_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s) {
+// (out_s given: the paired form)
+template <typename TO, int RT_MAX, bool PAIRED = false>
+int launch_fp8_stream_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s, float* out_s = nullptr) {
   // more dynamic LDS than a kernel may use without asking: once per device
   static std::atomic<uint64_t> configured{0};
-  if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&fp8_stream_tile_kernel<TO, RT_MAX>), kFp8StreamLdsMax)) return rc;
+  if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&fp8_stream_tile_kernel<TO, RT_MAX, PAIRED>), kFp8StreamLdsMax)) return rc;
   Fp8StreamParams p{};
   p.a = q.a;
   p.a_s = q.a_s;
@@ -394,7 +395,8 @@ int launch_fp8_stream_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s
   p.numel = q.numel;
   p.top_k = q.top_k;
   p.scale_rows = q.scale_rows;
-  fp8_stream_tile_kernel<TO, RT_MAX><<<p.tiles_m * p.tiles_n, 512, fp8_stream_lds_bytes(RT_MAX, q.K / 128), s>>>(p);
+  p.out_s = out_s;
+  fp8_stream_tile_kernel<TO, RT_MAX, PAIRED><<<p.tiles_m * p.tiles_n, 512, fp8_stream_lds_bytes(RT_MAX, q.K / 128), s>>>(p);
   return KSQ_OK;
 }
 
@@ -492,11 +494,53 @@ KSQ_EXPORT int ksq_fp8_blockwise_gemm_f32(const void* a_q, const void* a_s, cons
                                  workspace_bytes, stream, out);
 }
 
+namespace {
+// The streaming tile kernel takes row blocks of 128 and 256 slots while an expert has one of them on average: its weights are
+// read once, and the kernel that streams them is the faster one (256 experts, hidden 7168, inter 2048, whole block,
+// fp8_tile.h / fp8_stream.h: 2.74 / 2.33 ms at 112 slots per expert, 4.05 / 3.78 at 224; 64, 2048, 1408: 0.258 / 0.243 at 200,
+// but 0.410 / 0.433 at 375, where weights are shared).
+bool use_fp8_stream(size_t numel, size_t E, size_t k, size_t block_m) {
+  return (block_m == 128 || block_m == 256) && numel <= block_m * E &&
+         fp8_stream_lds_bytes(block_m == 128 ? 8 : 16, k / 128) <= static_cast<size_t>(kFp8StreamLdsMax);
+}
+
+// out_s given: the gate / up GEMM with the activation and the second quantization in its epilogue
+int moe_fp8_gemm_impl(const char* fn, void* out, float* out_s, const void* a_q, const void* a_s, int a_s_column_major, size_t a_rows,
+                      const void* b, const void* b_s, const void* topk_w, const void* sorted_ids, const void* expert_ids,
+                      const void* num_post_pad, size_t numel, size_t top_k, size_t E, size_t n, size_t k, size_t block_m,
+                      int out_dtype, void* stream);
+}  // namespace
+
+KSQ_EXPORT int ksq_moe_fp8_fused_quant(size_t numel, size_t E, size_t n, size_t k, size_t block_m) {
+  return n % 256 == 0 && k % 128 == 0 && use_fp8_stream(numel, E, k, block_m);
+}
+
+KSQ_EXPORT int ksq_moe_fp8_gate_up_quant(void* q, void* s, const void* a_q, const void* a_s, int a_s_column_major, size_t a_rows,
+                                         const void* b, const void* b_s, const void* sorted_ids, const void* expert_ids,
+                                         const void* num_post_pad, size_t numel, size_t top_k, size_t E, size_t n, size_t k,
+                                         size_t block_m, int dtype, void* stream) {
+  const char* fn = "ksq_moe_fp8_gate_up_quant";
+  if (!s || !sorted_ids) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
+  if (reinterpret_cast<uintptr_t>(s) & 3u) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: scales must be 4-byte aligned", fn);
+  if (numel != 0 && !ksq_moe_fp8_fused_quant(numel, E, n, k, block_m))
+    return fail(KSQ_ERR_UNSUPPORTED, "%s: n=%zu k=%zu block_m=%zu for %zu slots of %zu experts (ksq_moe_fp8_fused_quant)", fn, n, k, block_m, numel, E);
+  return moe_fp8_gemm_impl(fn, q, static_cast<float*>(s), a_q, a_s, a_s_column_major, a_rows, b, b_s, nullptr, sorted_ids, expert_ids,
+                           num_post_pad, numel, top_k, E, n, k, block_m, dtype, stream);
+}
+
 KSQ_EXPORT int ksq_moe_fp8_blockwise_gemm(void* out, const void* a_q, const void* a_s, int a_s_column_major, size_t a_rows, const void* b,
                                           const void* b_s, const void* topk_w, const void* sorted_ids,
                                           const void* expert_ids, const void* num_post_pad, size_t numel, size_t top_k,
                                           size_t E, size_t n, size_t k, size_t block_m, int out_dtype, void* stream) {
-  const char* fn = "ksq_moe_fp8_blockwise_gemm";
+  return moe_fp8_gemm_impl("ksq_moe_fp8_blockwise_gemm", out, nullptr, a_q, a_s, a_s_column_major, a_rows, b, b_s, topk_w, sorted_ids,
+                           expert_ids, num_post_pad, numel, top_k, E, n, k, block_m, out_dtype, stream);
+}
+
+namespace {
+int moe_fp8_gemm_impl(const char* fn, void* out, float* out_s, const void* a_q, const void* a_s, int a_s_column_major, size_t a_rows,
+                      const void* b, const void* b_s, const void* topk_w, const void* sorted_ids, const void* expert_ids,
+                      const void* num_post_pad, size_t numel, size_t top_k, size_t E, size_t n, size_t k, size_t block_m,
+                      int out_dtype, void* stream) {
   if (!a_q || !a_s || !b || !b_s || !out) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
   // sorted_ids == NULL: a handful of slots, one per 16-row block, with the router's ids in expert_ids
   const bool few = !sorted_ids;
@@ -539,11 +583,14 @@ KSQ_EXPORT int ksq_moe_fp8_blockwise_gemm(void* out, const void* a_q, const void
   if (block_m >= 128) {  // prefill regime: MFMA tile kernel, rows gathered / scattered through the permutation
     if (a_rows * k > 0xffffffffull || a_rows * (k / 128) * 4 > 0xffffffffull)
       return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: activations too large", fn);
-    // An expert has one row block on average: its weights are read once, and the kernel that streams them is the faster one
-    // (256 experts, hidden 7168, inter 2048, whole block, fp8_tile.h / fp8_stream.h: 2.74 / 2.33 ms at 112 slots per expert,
-    // 4.05 / 3.78 at 224; 64, 2048, 1408: 0.258 / 0.243 at 200, but 0.410 / 0.433 at 375, where weights are shared).
-    const bool streamed = numel <= block_m * E && fp8_stream_lds_bytes(block_m == 128 ? 8 : 16, k / 128) <= kFp8StreamLdsMax;
-    if (streamed && block_m == 128)
+    const bool streamed = use_fp8_stream(numel, E, k, block_m);
+    if (out_s && block_m == 128)
+      rc = out_dtype == KSQ_F16 ? launch_fp8_stream_grouped<F16, 8, true>(p, blocks, as_stream(stream), out_s)
+                                : launch_fp8_stream_grouped<BF16, 8, true>(p, blocks, as_stream(stream), out_s);
+    else if (out_s)
+      rc = out_dtype == KSQ_F16 ? launch_fp8_stream_grouped<F16, 16, true>(p, blocks, as_stream(stream), out_s)
+                                : launch_fp8_stream_grouped<BF16, 16, true>(p, blocks, as_stream(stream), out_s);
+    else if (streamed && block_m == 128)
       rc = out_dtype == KSQ_F16 ? launch_fp8_stream_grouped<F16, 8>(p, blocks, as_stream(stream))
                                 : launch_fp8_stream_grouped<BF16, 8>(p, blocks, as_stream(stream));
     else if (streamed)
@@ -562,6 +609,7 @@ KSQ_EXPORT int ksq_moe_fp8_blockwise_gemm(void* out, const void* a_q, const void
   if (rc) return rc;
   return check_launch(fn);
 }
+}  // namespace
 
 KSQ_EXPORT int ksq_moe_fp8_down_sum(void* out, const void* a_q, const void* a_s, const void* b, const void* b_s,
                                     const void* topk_w, const void* topk_ids, size_t tokens, size_t top_k, size_t E, size_t n,

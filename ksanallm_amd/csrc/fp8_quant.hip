@@ -15,27 +15,11 @@
 #include <type_traits>
 
 #include "exact_div.h"
+#include "fp8_encode.h"
 #include "ksq_common.h"
 
 namespace ksq {
 namespace {
-
-__device__ __forceinline__ uint32_t cvt2_e4m3(float a, float b, uint32_t old, bool hi) {
-  // v_cvt_pk_fp8_f32 rounds to nearest even; inputs are clamped to +-448 first so the result never leaves the
-  // finite range (NaN passes through and encodes as NaN).
-  float ca = fminf(fmaxf(a, -448.0f), 448.0f);
-  float cb = fminf(fmaxf(b, -448.0f), 448.0f);
-  ca = (a != a) ? a : ca;
-  cb = (b != b) ? b : cb;
-  return hi ? static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(ca, cb, static_cast<int>(old), true))
-            : static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(ca, cb, static_cast<int>(old), false));
-}
-
-// two quotients that are known to lie within +-448 * (1 + 2^-23), or NaN: no clamp in front of the conversion
-__device__ __forceinline__ uint32_t cvt2_e4m3_in_range(float a, float b, uint32_t old, bool hi) {
-  return hi ? static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(a, b, static_cast<int>(old), true))
-            : static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(a, b, static_cast<int>(old), false));
-}
 
 // fp32 activations (the reference instantiates its quantizer for float as well): the same kernel with 32-byte loads and
 // IEEE divisions throughout - the reciprocal-and-correction form above is proven for inputs of at most 11 significant
@@ -110,38 +94,15 @@ __global__ void __launch_bounds__(BLOCK) fp8_group_quant_kernel(const void* __re
 #pragma unroll
   for (int off = LPG / 2; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, LPG));
 
-  // amax / 448, correctly rounded, by the same reciprocal-and-correction (amax has at most 11 significant bits, or is
-  // the floor 1e-10, whose quotient is a constant)
-  float scale;
-  {
-    constexpr float y448 = 1.0f / 448.0f;
-    const float q0 = amax * y448;
-    const float r = __builtin_fmaf(-q0, 448.0f, amax);
-    scale = __builtin_fmaf(r, y448, q0);
-    scale = amax == 1e-10f ? 1e-10f / 448.0f : scale;
-    scale = (!kF32 && amax >= 0x1p-60f && amax <= 0x1p100f) ? scale : amax / 448.0f;
-  }
+  const float scale = fp8_group_scale<kF32>(amax);
   if (!live) return;
   if ((threadIdx.x % LPG) == 0) {
     const uint32_t g = col / GROUP;
     const uint32_t ng = k / GROUP;
     s[COLMAJOR ? static_cast<size_t>(g) * m + t : static_cast<size_t>(t) * ng + g] = scale;
   }
-  u32x2 out{0u, 0u};
   const ExactDiv div(scale);
-  if (!kF32 && div.fast) {
-    // every |v| <= amax (an infinite v makes amax, hence the scale, infinite: not this branch), so the quotients stay
-    // within 448 * (1 + 2^-23), which the conversion rounds to 448 by itself
-    out.x = cvt2_e4m3_in_range(div(v[0]), div(v[1]), out.x, false);
-    out.x = cvt2_e4m3_in_range(div(v[2]), div(v[3]), out.x, true);
-    out.y = cvt2_e4m3_in_range(div(v[4]), div(v[5]), out.y, false);
-    out.y = cvt2_e4m3_in_range(div(v[6]), div(v[7]), out.y, true);
-  } else {
-    out.x = cvt2_e4m3(v[0] / scale, v[1] / scale, out.x, false);
-    out.x = cvt2_e4m3(v[2] / scale, v[3] / scale, out.x, true);
-    out.y = cvt2_e4m3(v[4] / scale, v[5] / scale, out.y, false);
-    out.y = cvt2_e4m3(v[6] / scale, v[7] / scale, out.y, true);
-  }
+  const u32x2 out{fp8_encode4<kF32>(div, v), fp8_encode4<kF32>(div, v + 4)};
   *reinterpret_cast<u32x2*>(q + e0) = out;
 }
 

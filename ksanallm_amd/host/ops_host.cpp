@@ -19,6 +19,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <tuple>
 #include <utility>
 
 #include "ksq.h"
@@ -30,8 +31,8 @@ namespace {
   F(w4a16_workspace_size) F(w4a16_gemm) F(fp8_group_quant) F(fp8_blockwise_workspace_size) F(fp8_blockwise_gemm) \
   F(w4a8_static_quant) F(w4a8_workspace_size) F(w4a8_gemm) F(moe_topk_softmax) F(moe_grouped_topk) \
   F(moe_align_capacity) F(moe_align_scratch_bytes) F(moe_align) F(moe_block_m) F(moe_fp8_row_block) F(moe_w4a16_gemm) \
-  F(moe_w4a16_gate_up_silu) F(moe_w4a16_down_sum) F(moe_fp8_blockwise_gemm) F(moe_fp8_down_sum) F(moe_silu_mul) \
-  F(moe_sum)
+  F(moe_w4a16_gate_up_silu) F(moe_w4a16_down_sum) F(moe_fp8_blockwise_gemm) F(moe_fp8_fused_quant) F(moe_fp8_gate_up_quant) \
+  F(moe_fp8_down_sum) F(moe_silu_mul) F(moe_sum)
 
 struct Library {
 #define KSQ_FN(name) decltype(&::ksq_##name) name;
@@ -458,13 +459,26 @@ at::Tensor fused_moe_fp8_blockwise(const Args& a) {
   void *ps = few ? nullptr : ptr(al.sorted_ids), *pe = few ? pids : ptr(al.expert_ids), *pn = few ? nullptr : ptr(al.num_post_pad);
   if (few) block_m = 16;
   auto [q1, q1s] = group_quant(x, hidden, 128, false, false, nullptr, nullptr);
-  at::Tensor c1 = empty({r.numel, n1}, t, x);
-  void *pq1 = ptr(q1), *pq1s = ptr(q1s), *p1 = ptr(c1);
-  call([&] {
-    return lib.moe_fp8_blockwise_gemm(p1, pq1, pq1s, 0, r.tokens, pw13, ps13, nullptr, ps, pe, pn, r.numel, r.top_k, E, n1, hidden,
-                                      block_m, d, st);
-  });
-  auto [q2, q2s] = group_quant(c1, inter, 128, false, true, nullptr, nullptr);
+  void *pq1 = ptr(q1), *pq1s = ptr(q1s);
+  at::Tensor q2, q2s;
+  if (!few && lib.moe_fp8_fused_quant(r.numel, E, n1, hidden, block_m)) {
+    // the activation and the second quantization run in the first GEMM's epilogue
+    q2 = empty({r.numel, inter}, at::kByte, x);
+    q2s = empty({r.numel, inter / 128}, at::kFloat, x);
+    void *pq = ptr(q2), *pqs = ptr(q2s);
+    call([&] {
+      return lib.moe_fp8_gate_up_quant(pq, pqs, pq1, pq1s, 0, r.tokens, pw13, ps13, ps, pe, pn, r.numel, r.top_k, E, n1, hidden, block_m,
+                                       d, st);
+    });
+  } else {
+    at::Tensor c1 = empty({r.numel, n1}, t, x);
+    void* p1 = ptr(c1);
+    call([&] {
+      return lib.moe_fp8_blockwise_gemm(p1, pq1, pq1s, 0, r.tokens, pw13, ps13, nullptr, ps, pe, pn, r.numel, r.top_k, E, n1, hidden,
+                                        block_m, d, st);
+    });
+    std::tie(q2, q2s) = group_quant(c1, inter, 128, false, true, nullptr, nullptr);
+  }
   void *pq2 = ptr(q2), *pq2s = ptr(q2s);
   if (few) {
     at::Tensor out = empty({r.tokens, hidden}, t, x);

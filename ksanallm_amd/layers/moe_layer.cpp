@@ -228,10 +228,17 @@ Status MoeLayer::Forward(const std::vector<Tensor>& input_tensors, std::vector<T
                  "MoeLayer");
         continue;
       }
-      KsqCheck(ksq_moe_fp8_blockwise_gemm(cache1, a1, a1_s, 0, tokens, w1, w1_scale, nullptr, sorted_ids, expert_ids,
-                                          num_post_pad, numel, topk, E, 2 * inter, hidden_size, block_m, dtype, stream),
-               "MoeLayer");
-      KsqCheck(ksq_fp8_group_quant(cache1, cache2, a2_s, numel, inter, 128, 0, 1, dtype, stream), "MoeLayer");
+      if (ksq_moe_fp8_fused_quant(numel, E, 2 * inter, hidden_size, block_m)) {
+        // the activation and the second quantization run in the first GEMM's epilogue
+        KsqCheck(ksq_moe_fp8_gate_up_quant(cache2, a2_s, a1, a1_s, 0, tokens, w1, w1_scale, sorted_ids, expert_ids, num_post_pad,
+                                           numel, topk, E, 2 * inter, hidden_size, block_m, dtype, stream),
+                 "MoeLayer");
+      } else {
+        KsqCheck(ksq_moe_fp8_blockwise_gemm(cache1, a1, a1_s, 0, tokens, w1, w1_scale, nullptr, sorted_ids, expert_ids,
+                                            num_post_pad, numel, topk, E, 2 * inter, hidden_size, block_m, dtype, stream),
+                 "MoeLayer");
+        KsqCheck(ksq_fp8_group_quant(cache1, cache2, a2_s, numel, inter, 128, 0, 1, dtype, stream), "MoeLayer");
+      }
       KsqCheck(ksq_moe_fp8_blockwise_gemm(cache3, cache2, a2_s, 0, numel, w2, w2_scale, weights, sorted_ids, expert_ids,
                                           num_post_pad, numel, 1, E, hidden_size, inter, block_m, dtype, stream),
                "MoeLayer");

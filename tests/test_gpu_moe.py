@@ -615,6 +615,43 @@ def test_grouped_fp8_streaming_tile_over_its_ring(ops, oracle, bm, rows, kb):
     H.check_gemm(out, ref, H.BF16, "fp8 streaming tile kernel, %d k-blocks" % kb)
 
 
+@pytest.mark.parametrize("dtype", [H.F16, H.BF16])
+@pytest.mark.parametrize("bm,rows,k,inter", [(128, [1, 16, 17, 127, 128, 65], 128, 128), (128, [5, 33, 100, 2], 640, 384),
+                                             (256, [129, 256, 208, 209, 16, 0], 512, 256), (256, [250, 7], 1152, 640)])
+def test_fp8_gate_up_gemm_with_the_second_quantization(ops, oracle, dtype, bm, rows, k, inter):
+    """The activation and the second quantization in the first GEMM's epilogue: the codes and scales of the two launches, bit
+    for bit, over row tile counts of every ring depth, with rows of zeros, of infinite and of NaN sums among them."""
+    from ksanallm_amd import lib as L
+    E, T, topk, n = len(rows), sum(rows), 1, 2 * inter
+    t = H.TORCH_DT[dtype]
+    g = H.gen(8100 + bm + k)
+    bq, bs = _fp8_experts(oracle, 8110 + k, E, n, k)
+    x = (torch.randn((T, k), generator=g) * 2).to(t)
+    x[T // 2] = 0
+    ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
+    ids = ids[torch.randperm(T, generator=g)].reshape(T, 1).contiguous().cuda()
+    q, s = ops.per_token_group_quant_fp8(x.cuda(), k, 128, False)
+    s[T // 3] = float("inf")   # an infinite scale: the row's sums are infinite or NaN
+    s[T // 4] *= 2.0 ** 30     # sums past fp16's range
+    aligned = ops.moe_align_block_size(ids, E, bm)
+    w, ws = ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda()
+    lib = L.load()
+    assert lib.ksq_moe_fp8_fused_quant(T, E, n, k, bm) == 1
+    gu = ops.moe_fp8_blockwise_gemm(q, s, False, w, ws, None, *aligned, T, topk, bm, t)
+    q0 = torch.empty((T, inter), dtype=torch.uint8, device="cuda")
+    s0 = torch.empty((T, inter // 128), dtype=torch.float32, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    L.check(lib.ksq_fp8_group_quant(gu.data_ptr(), q0.data_ptr(), s0.data_ptr(), T, inter, 128, 0, 1, dtype, st))
+    q1, s1 = torch.full_like(q0, 0x55), torch.full_like(s0, -1.0)
+    L.check(lib.ksq_moe_fp8_gate_up_quant(q1.data_ptr(), s1.data_ptr(), q.data_ptr(), s.data_ptr(), 0, T, w.data_ptr(), ws.data_ptr(),
+                                          *(a.data_ptr() for a in aligned), T, topk, E, n, k, bm, dtype, st))
+    assert torch.equal(s0.view(torch.int32), s1.view(torch.int32)) and torch.equal(q0, q1)
+    assert lib.ksq_moe_fp8_fused_quant(bm * E + 1, E, n, k, bm) == 0
+    with pytest.raises(L.KsqError):
+        L.check(lib.ksq_moe_fp8_gate_up_quant(q1.data_ptr(), s1.data_ptr(), q.data_ptr(), s.data_ptr(), 0, T, w.data_ptr(), ws.data_ptr(),
+                                              *(a.data_ptr() for a in aligned), T, topk, E, n, k, 32, dtype, st))
+
+
 def test_grouped_fp8_tile_kernel_where_three_stages_do_not_fit(ops, oracle):
     """K > 28672 leaves no room in the LDS for three stages: every 256-slot block then runs on two, one without any token
     (which the alignment never makes, but a caller's own permutation may) among them."""
