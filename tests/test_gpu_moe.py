@@ -88,6 +88,23 @@ def test_topk_softmax(ops, oracle, T, E, topk):
     np.testing.assert_array_equal(ids.cpu().numpy(), io)
 
 
+@pytest.mark.parametrize("E,topk", [(1, 1), (2, 2), (63, 6), (64, 8), (65, 32), (255, 8), (256, 32), (257, 8), (1024, 32)])
+def test_topk_softmax_among_ties(ops, oracle, E, topk):
+    """Logits of three values and -inf: almost every round ends in a tie, which the lowest id wins, also where the remaining
+    probabilities are zero."""
+    g = H.gen(E + topk)
+    logits = torch.randint(-1, 2, (9, E), generator=g).float()
+    logits[torch.rand((9, E), generator=g) < 0.4] = float("-inf")
+    logits[:, E // 2] = 0.0
+    logits[7] = 0.0
+    logits[8] = float("-inf")
+    logits[8, E - 1] = 3.0   # one expert with all of the probability
+    w, ids = ops.moe_topk_softmax(logits.cuda(), topk, True, 1.0)
+    wo, io = oracle.moe_topk_softmax(logits.numpy(), topk, True, 1.0, 2)
+    np.testing.assert_array_equal(ids.cpu().numpy(), io)
+    np.testing.assert_allclose(w.cpu().numpy(), wo, rtol=2e-6, atol=1e-9)
+
+
 def _check_routing(w, ids, wo, io, choose_gap_ok):
     """ids equal as sets per token; where they differ (expf on the GPU and on the host may round differently and swap
     two near-equal scores) the two experts' weights must agree to 3e-4, the reference test's own allowance."""
