@@ -478,6 +478,11 @@ __global__ void __launch_bounds__(512, 1) w4a16_tile_kernel(TileParams p) {
       stage(std::integral_constant<int, 4>{}, base);
       stage(std::integral_constant<int, 5>{}, base);
     }
+    // Drain the clamped prefetches before the LDS is released - and before their registers are: nothing reads what the last
+    // weight loads bring (those of the turn's last stage, into ring[1]; the ones before were waited for at the sync of its fifth),
+    // so without a use behind the wait the compiler may hand a register that a load is still on its way to to the
+    // epilogue's address arithmetic, which it places in front of the wait.
+    wait_tie(std::integral_constant<int, 0>{}, ring[1]);
   };
   // An instance of the main loop for every number of row tiles that hold rows, from four (the depth of the fragment
   // prefetch) to all of them.  Expert blocks: what a padded row tile costs is not so much time in the loop as power - its
@@ -495,7 +500,6 @@ __global__ void __launch_bounds__(512, 1) w4a16_tile_kernel(TileParams p) {
   } else {
     run(std::integral_constant<int, WM>{});
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // drain the clamped prefetches before the LDS is released
 
   // ---- store: lane holds row m = l%16 of the 16x16 tile and columns 4*(l/16) .. +3
   // Grouped form: the slot ids of all row tiles, then their routing weights, are fetched before the first store.  Read

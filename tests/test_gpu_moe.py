@@ -512,6 +512,28 @@ def test_few_tokens_form_drops_ids_outside_the_experts_and_rejects_what_it_canno
                                   idf.data_ptr(), None, numel, 1, E, hidden, inter, 128, 32, H.BF16, stream) == 1
 
 
+@pytest.mark.parametrize("dtype", [H.F16, H.BF16])
+@pytest.mark.parametrize("kt", [1, 2, 3, 4, 5, 11, 16])
+def test_grouped_tile_kernel_ends_over_k_tiles(ops, dtype, kt):
+    """The loads that are on their way when the main loop ends (its turns are three k-tiles long, and it prefetches past the
+    end of K) leave the epilogue's registers alone: experts with every row tile count, in 256- and 128-row blocks, which sum in
+    the same order - the same bits."""
+    from ksanallm_amd import lib as L
+    rows = [16 * c - 3 for c in range(1, 17)] * 4
+    E, T, n, k = len(rows), sum(rows), 512, 128 * kt
+    g = torch.Generator(device="cuda")
+    g.manual_seed(8200 + kt)
+    w = ops.repack_weight(torch.randint(0, 256, (E, n, k // 2), generator=g, device="cuda", dtype=torch.uint8), L.SRC_MOE_NK, E, k, n)
+    sc = (torch.rand((E, n, kt), generator=g, device="cuda") * 0.01 + 0.002).to(H.TORCH_DT[dtype])
+    sp = ops.repack_scales(sc, L.SCALE_NG, E, k, n, 128)
+    x = torch.randn((T, k), generator=g, device="cuda").to(H.TORCH_DT[dtype])
+    ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)]).cuda()
+    ids = ids[torch.randperm(T, generator=g, device="cuda")].reshape(T, 1).contiguous()
+    outs = [ops.moe_w4a16_gemm(x, w, sp, None, *ops.moe_align_block_size(ids, E, bm), T, 1, E, n, k, 128, bm) for bm in (256, 128)]
+    assert torch.isfinite(outs[0].float()).all()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 # ---- block-quantized fp8 experts -------------------------------------------------------------------------------------
 
 def _fp8_experts(oracle, seed, E, n, k):
