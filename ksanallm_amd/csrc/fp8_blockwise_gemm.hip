@@ -400,6 +400,43 @@ int launch_fp8_stream_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s
   return KSQ_OK;
 }
 
+// dense form of the streaming tile kernel: one block of 129..240 rows
+template <typename TO>
+int launch_fp8_stream_dense(const Fp8Params& q, const TilePlan& plan, float* partial, hipStream_t s) {
+  const size_t kb_max = (plan.main_items || plan.splits == 1) ? q.K / 128 : plan.kt_per_split;  // whole tiles span all of K
+  constexpr int RT_MAX = 16;
+  // more dynamic LDS than a kernel may use without asking: once per device
+  static std::atomic<uint64_t> configured{0};
+  if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&fp8_stream_tile_kernel<TO, RT_MAX, false, true>), kFp8StreamLdsMax)) return rc;
+  Fp8StreamParams p{};
+  p.a = q.a;
+  p.a_s = q.a_s;
+  p.b = q.b;
+  p.b_s = q.b_s;
+  p.out = q.out;
+  p.out32 = q.out32;
+  p.partial = partial;
+  p.N = q.N;
+  p.K = q.K;
+  p.block = 16 * RT_MAX;
+  p.tiles_m = plan.tiles_m;
+  p.tiles_n = plan.tiles_n;
+  p.main_items = plan.main_items;
+  p.splits = plan.splits;
+  p.kb_per_split = plan.kt_per_split;
+  p.as_row_bytes = 4;
+  p.as_kb_bytes = 4 * q.M;
+  p.numel = q.M;
+  p.top_k = 1;
+  fp8_stream_tile_kernel<TO, RT_MAX, false, true><<<plan.grid, 512, fp8_stream_lds_bytes(RT_MAX, kb_max), s>>>(p);
+  if (plan.splits > 1) {
+    const unsigned cut = plan.tiles_m * plan.tiles_n - plan.main_items;
+    splitk_reduce_kernel<TO, 16 * RT_MAX><<<cut * (2 * RT_MAX), 256, 0, s>>>(partial, static_cast<uint16_t*>(p.out), q.M, p.N, p.tiles_m,
+                                                                            p.tiles_n, p.main_items, p.splits, p.out32);
+  }
+  return KSQ_OK;
+}
+
 // per-tensor scales spread into the blockwise layouts
 __global__ void __launch_bounds__(256) fp8_expand_scales_kernel(const float* __restrict__ a_scale, const float* __restrict__ b_scale,
                                                                 float* __restrict__ a_s, size_t na, float* __restrict__ b_s,
@@ -431,6 +468,24 @@ KSQ_EXPORT size_t ksq_fp8_blockwise_workspace_size(size_t max_m, size_t n, size_
 }
 
 namespace {
+// One 256-row block of 129..240 rows: every weight is read once, by one workgroup, and the streaming tile kernel takes the tile
+// kernel's plan with three (to 13 row tiles) or two k-blocks of weights in flight, activation slots for the row tiles that hold
+// rows alone and eight wavefronts that share no weights.  fp8_tile.h / fp8_stream.h in us, GEMM alone, same bits: n = 18432,
+// k = 7168 at 129, 150, 200, 224 rows 50.7 / 44.3, 55.7 / 47.3, 59.8 / 55.2, 61.6 / 59.8; n = 7168, k = 18432 49.5 / 41.7, 51.8 /
+// 44.2, 55.3 / 52.3, 58.5 / 54.7; n = 24576, k = 1536, six k-blocks a workgroup, 27.9 / 22.2, 28.9 / 23.7, 30.7 / 27.7, 31.5 / 28.2;
+// n = k = 14336 68.8 / 58.0, 73.6 / 61.3, 78.8 / 75.7, 81.1 / 77.2.  With all sixteen row tiles the two cross (n = 28672, k = 4096
+// at 256 rows 60.5 / 62.8, n = k = 14336 84.9 / 84.9, n = 24576, k = 1536 33.4 / 30.7), and a few column tiles cut very often spend
+// their time on partial sums (n = 1040, k = 28672: 129 rows 31.6 / 32.6, 150 36.4 / 33.7, 200 37.5 / 38.2); n = 5120, k = 25600, 20
+// column tiles, at 129 and 200 rows 48.8 / 41.0, 55.1 / 50.6.  Workgroups of fewer than six k-blocks are not measured.
+// Blocks of 128 rows stay on fp8_tile.h: n = 28672, k = 4096 at 33 and 100 rows 29.1 / 30.9, 35.8 / 39.0, n = 4096, k = 7168 at
+// 100 rows 19.2 / 26.0; ahead by 4 to 6 % at n = k = 14336 only.
+bool use_fp8_stream_dense(const TilePlan& plan, size_t m, size_t k) {
+  const size_t kb_max = (plan.main_items || plan.splits == 1) ? k / 128 : plan.kt_per_split;
+  const size_t kb_min = plan.splits == 1 ? k / 128 : plan.kt_per_split;
+  return plan.tiles_m == 1 && plan.block_m == 256 && m <= 16 * kFp8StreamDenseTiles && plan.tiles_n >= 20 && kb_min >= 6 &&
+         fp8_stream_lds_bytes(16, kb_max) <= static_cast<size_t>(kFp8StreamLdsMax);
+}
+
 // out32 given (verification entry point): the same kernels under the same plan, with the fp32 sums stored to out32
 // [m, n] instead of rounded into out (which is then not touched)
 int fp8_blockwise_gemm_impl(const char* fn, const void* a_q, const void* a_s, const void* b, const void* b_s, void* out,
@@ -463,7 +518,10 @@ int fp8_blockwise_gemm_impl(const char* fn, const void* a_q, const void* a_s, co
                   n, k, plan.workspace_bytes, workspace ? workspace_bytes : size_t(0));
     if (256 * k > 0xffffffffull) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: k too large", fn);
     float* partial = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
-    if (plan.block_m == 128)
+    if (use_fp8_stream_dense(plan, m, k))
+      rc = out_dtype == KSQ_F16 ? launch_fp8_stream_dense<F16>(p, plan, partial, as_stream(stream))
+                                : launch_fp8_stream_dense<BF16>(p, plan, partial, as_stream(stream));
+    else if (plan.block_m == 128)
       rc = out_dtype == KSQ_F16 ? launch_fp8_tile<F16, 4>(p, plan, partial, as_stream(stream))
                                 : launch_fp8_tile<BF16, 4>(p, plan, partial, as_stream(stream));
     else

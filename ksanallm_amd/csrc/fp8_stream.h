@@ -41,6 +41,10 @@ struct Fp8StreamParams {
   const float* topk_w;
   uint32_t numel, top_k, scale_rows;  // scale_rows = ceil(N/128): rows of one expert's b_s
   float* out_s;               // PAIRED: scales [numel, N / 256] of the codes out [numel, N / 2]
+  // DENSE: a plain GEMM of numel rows (top_k 1, no slot ids), whose tiles may be cut along K
+  float* out32;               // verification only: the fp32 sums go here, [numel, N], and nothing is rounded to TO
+  float* partial;             // [slot][part][block][256] fp32 tiles of the workgroups that compute a part of K
+  uint32_t main_items, splits, kb_per_split;  // tile_work.h
 };
 
 constexpr int kFp8StreamLdsMax = 160 * 1024;
@@ -52,6 +56,7 @@ constexpr int fp8_stream_area(int rt) {
   const int d = fp8_stream_depth(rt);
   return d * rt * 2048 + (2 * fp8_stream_scale_slot4(rt) > d * 1024 ? 2 * fp8_stream_scale_slot4(rt) : d * 1024);
 }
+constexpr int kFp8StreamDenseTiles = 15;          // row tiles of a dense block, at most
 constexpr int kFp8StreamOutTiles = 8;             // row tiles whose results pass through LDS at a time
 constexpr int kFp8StreamOutPitch = 256 * 2 + 16;  // bytes of a row of them
 constexpr int fp8_stream_area_max(int rt_max) {
@@ -76,7 +81,11 @@ __device__ __forceinline__ P* scalar_ptr(P* ptr) {
 // the activation in front, without [numel, 2 * inter] through memory and without the quantizer's launch (256 experts, hidden
 // 7168, inter 2048, whole block: 512 tokens 1.86 -> 1.78 ms, 4000 tokens, where the activation of a tile stands for 5 us at
 // the end of its workgroup, 2.58 -> 2.55; 64 experts, hidden 2048, inter 1408, 48 tokens 115 -> 111 us).
-template <typename TO, int RT_MAX, bool PAIRED>
+//
+// DENSE: tile m holds rows m * block .., results go to their rows or, from a workgroup that computes a part of K, to fp32
+// partial tiles (splitk_reduce.h).  200 rows, n = 18432, k = 7168: 59.8 us with fp8_tile.h, 55.2 with this form (2.4 TB/s of
+// weights; 150 rows 55.7 -> 47.3): the MFMAs of 13 row tiles in whole waves of 32 columns and the partial sums are the rest.
+template <typename TO, int RT_MAX, bool PAIRED, bool DENSE = false>
 __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];  // fp8_stream_lds_bytes
   constexpr int WAVES = 8;
@@ -88,25 +97,38 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
   const int lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lrow = lane & 15, lq = lane >> 4;
-  const uint32_t KB = p.K / 128;
+  const uint32_t k_blocks = p.K / 128;
 
   // ---- work item (tile_work.h): over the row blocks that hold slots, those past them leave
-  const uint32_t filled = (static_cast<uint32_t>(p.num_post_pad[0]) + p.block - 1) / p.block;
-  const uint32_t tiles_m = __builtin_amdgcn_readfirstlane(filled < p.tiles_m ? filled : p.tiles_m);
-  if (blockIdx.x >= tiles_m * p.tiles_n) return;  // uniform: the whole workgroup leaves
-  const TileWork work = tile_work(blockIdx.x, tiles_m, p.tiles_n, 0, 1, true);
+  uint32_t tiles_m = p.tiles_m;
+  if constexpr (!DENSE) {
+    const uint32_t filled = (static_cast<uint32_t>(p.num_post_pad[0]) + p.block - 1) / p.block;
+    tiles_m = __builtin_amdgcn_readfirstlane(filled < p.tiles_m ? filled : p.tiles_m);
+    if (blockIdx.x >= tiles_m * p.tiles_n) return;  // uniform: the whole workgroup leaves
+  }
+  const TileWork work = tile_work(blockIdx.x, tiles_m, p.tiles_n, DENSE ? p.main_items : 0, DENSE ? p.splits : 1, !DENSE);
   const uint32_t tile_m = __builtin_amdgcn_readfirstlane(work.tile_m), tile_n = __builtin_amdgcn_readfirstlane(work.tile_n);
   const uint32_t m0 = tile_m * p.block, n0 = tile_n * BN;
+  const uint32_t part = __builtin_amdgcn_readfirstlane(work.part), out_slot = __builtin_amdgcn_readfirstlane(work.slot);
+  const bool direct = !DENSE || __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(work.direct)) != 0;
+  // the k-blocks of this workgroup: kb0 .. kb0 + KB - 1
+  const uint32_t kb0 = __builtin_amdgcn_readfirstlane(direct ? 0 : part * p.kb_per_split);
+  const uint32_t KB = __builtin_amdgcn_readfirstlane(direct || k_blocks - kb0 < p.kb_per_split ? k_blocks - kb0 : p.kb_per_split);
 
   // ---- slots of this block: their ids go to LDS (rows past the block hold no slot)
-  const size_t expert = static_cast<size_t>(__builtin_amdgcn_readfirstlane(p.expert_ids[tile_m]));
+  const size_t expert = DENSE ? 0 : static_cast<size_t>(__builtin_amdgcn_readfirstlane(p.expert_ids[tile_m]));
   uint32_t* ids = reinterpret_cast<uint32_t*>(lds + IDS_BASE);
-  if (threadIdx.x < 256) ids[threadIdx.x] = threadIdx.x < p.block ? static_cast<uint32_t>(p.sorted_ids[m0 + threadIdx.x]) : p.numel;
+  if (threadIdx.x < 256) {
+    if constexpr (DENSE)
+      ids[threadIdx.x] = threadIdx.x < p.block && m0 + threadIdx.x < p.numel ? m0 + threadIdx.x : p.numel;
+    else
+      ids[threadIdx.x] = threadIdx.x < p.block ? static_cast<uint32_t>(p.sorted_ids[m0 + threadIdx.x]) : p.numel;
+  }
   // the weight scales of the tile's two blocks of 128 weight rows
   for (uint32_t t = threadIdx.x; t < 2 * KB; t += 512) {
     const uint32_t blk = t / KB, kb = t - blk * KB, nb_last = (p.N - 1) / 128;
     const uint32_t nb = PAIRED ? tile_n + blk * (p.N / 256) : n0 / 128 + blk < nb_last ? n0 / 128 + blk : nb_last;
-    reinterpret_cast<float*>(lds + BS_BASE)[t] = p.b_s[(expert * p.scale_rows + nb) * KB + kb];
+    reinterpret_cast<float*>(lds + BS_BASE)[t] = p.b_s[(expert * p.scale_rows + nb) * k_blocks + kb0 + kb];
   }
   __syncthreads();
   uint32_t rows = 0;
@@ -116,11 +138,11 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
   auto row_of = [&](uint32_t r) -> uint32_t {  // activation row of slot r of the block; a row without a slot reads some valid one
     uint32_t sid = ids[r];
     sid = sid < p.numel ? sid : p.numel - 1;
-    return sid / p.top_k;
+    return DENSE ? sid : sid / p.top_k;
   };
 
-  const uint8_t* a_base = p.a;
-  const char* s_base = reinterpret_cast<const char*>(p.a_s);
+  const uint8_t* a_base = scalar_ptr(p.a + static_cast<size_t>(kb0) * 128);
+  const char* s_base = scalar_ptr(reinterpret_cast<const char*>(p.a_s) + static_cast<size_t>(kb0) * p.as_kb_bytes);
   const uint32_t s_voff = row_of((wave & 3) * 64 + lane) * p.as_row_bytes;
   const uint32_t w_voff = lane * 16;
   const uint32_t strips = p.N / 16;
@@ -128,7 +150,7 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const uint32_t strip = PAIRED ? tile_n * 8 + wave + t * (strips / 2) : n0 / 16 + wave * 2 + t;
-    w_base[t] = scalar_ptr(p.b + ((expert * strips + (strip < strips ? strip : strips - 1)) * KB) * FRAG);
+    w_base[t] = scalar_ptr(p.b + ((expert * strips + (strip < strips ? strip : strips - 1)) * k_blocks + kb0) * FRAG);
   }
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) char*)lds));
   // An activation fragment (16 rows x 128 bytes) is two loads of 8 rows: eight lanes take the eight 16-byte pieces of a
@@ -340,13 +362,31 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
       }
       return;
     }
+    if constexpr (DENSE) {
+      if (!direct || p.out32) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          const uint32_t r = i * 16 + lrow;
+          if (ids[r] < p.numel) {
+            float* const dst = direct ? p.out32 + static_cast<size_t>(m0 + r) * p.N + n0
+                                      : p.partial + ((static_cast<size_t>(out_slot) * p.splits + part) * p.block + r) * BN;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+              const uint32_t col = wave * 32 + t * 16 + 4 * lq;
+              if (n0 + col < p.N) *reinterpret_cast<f32x4*>(dst + col) = acc[t][i];
+            }
+          }
+        }
+        return;
+      }
+    }
     // Rounded results go through LDS (whose slots nothing reads any more), so that a row's 256 columns leave in
     // 16-byte pieces of consecutive lanes.
     float rws[RT];
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
       const uint32_t sid = ids[i * 16 + lrow];
-      rws[i] = (sid < p.numel && p.topk_w) ? p.topk_w[sid] : 1.0f;
+      rws[i] = (!DENSE && sid < p.numel && p.topk_w) ? p.topk_w[sid] : 1.0f;
     }
     constexpr int PITCH = kFp8StreamOutPitch;
     constexpr int PIECES = BN / 8;  // 16-byte pieces of a row
@@ -376,7 +416,7 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
       }
     }
   };
-  for_tile_count<1, RT_MAX>(live_tiles, run);
+  for_tile_count<DENSE ? 9 : 1, DENSE ? kFp8StreamDenseTiles : RT_MAX>(live_tiles, run);  // (dense: 129..240 rows)
 }
 
 }  // namespace ksq

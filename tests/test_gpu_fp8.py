@@ -242,6 +242,29 @@ def test_blockwise_gemm_tile_kernel_every_count_of_live_row_tiles(ops, oracle, b
             assert torch.equal(run(m)[0].view(torch.int16), whole[:m].view(torch.int16)), m
 
 
+# one block of 129..256 rows: every count of row tiles on the kernel that streams the weights, with whole tiles of seven k-blocks
+# and with parts of K, 16 columns in the last tile; two k-blocks and more than 240 rows stay on the other kernel
+@pytest.mark.parametrize("n,k,cut", [(8464, 256, False), (8464, 896, False), (8464, 3328, True)])
+def test_blockwise_gemm_one_block_of_129_to_256_rows(ops, oracle, n, k, cut):
+    from ksanallm_amd import lib as L
+    x, bq, bs = make_fp8_problem(oracle, 4470 + k, 256, n, k)
+    w, ws = packed(ops, bq), torch.from_numpy(bs).cuda()
+    ref = None
+    for m in (256, 129, 144, 145, 160, 176, 177, 193, 208, 224, 225, 240, 241):
+        d = L.select_tile(L.KIND_FP8_BLOCKWISE, m, n, k, H.BF16)
+        assert d["block_m"] == 256 and (d["split_k"] > 1) == cut
+        q, s = ops.per_token_group_quant_fp8(x[:m].contiguous().cuda(), k, 128, True)
+        if ref is None:
+            qc, sc = q.cpu().numpy(), s.cpu().numpy()
+            ref = [oracle.fp8_blockwise_gemm(qc, sc, bq[c:], bs[c // 128:], True) if c else
+                   oracle.fp8_blockwise_gemm(qc, sc, bq[:256], bs[:2], True) for c in (0, n - 16)]
+        y32 = ops.fp8_blockwise_gemm_f32(q, s, w, ws)
+        H.check_gemm_f32(y32[:, :256], ref[0][:m], "fp8 m=%d n=%d k=%d, first columns" % (m, n, k))
+        H.check_gemm_f32(y32[:, n - 16:], ref[1][:m], "fp8 m=%d n=%d k=%d, last columns" % (m, n, k))
+        for dt in (torch.float16, torch.bfloat16):
+            assert torch.equal(ops.fp8_blockwise_gemm(q, s, w, ws, dt).view(torch.int16), y32.to(dt).view(torch.int16)), m
+
+
 # small problems of more than 32 tokens (ceil(m / 32) * n * k <= 5 * 2^24, m <= 512): the streaming kernel over blocks of
 # 32 tokens, ragged last block included
 @pytest.mark.parametrize("m,n,k", [(65, 256, 128), (100, 272, 384), (128, 4096, 4096), (300, 2320, 1152), (500, 768, 640),
