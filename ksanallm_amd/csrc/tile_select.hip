@@ -369,14 +369,15 @@ KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidde
 // 256 experts, hidden 7168, inter 2048 1748 / 1691 and 1848 / 1758; 256, 1024, 512 131 / 102 and 147 / 110; 64, 1024, 512 49 / 39 and
 // 53 / 40; 16, 4096, 2048 87 / 83 and 89 / 84; 32, 1024, 512 (128 tiles) 32.5 / 31.4 and 34.2 / 32.5; 16, 2048, 1408 (128) 47.5 /
 // 45.3 and 49.5 / 46.2; but 8, 4096, 1536 (96) 48.2 / 51.2 and 49.9 / 52.2, 16, 1024, 512 (64) 25.2 / 28.9 and 25.6 / 29.2.  (Below
-// four: 32, 4096, 2048 at 1 and 2 slots 106 / 118 and 138 / 139, 128, 2944, 768 at 1 118 / 122.)  From 64 slots on 256-slot
-// blocks, so that few experts need two (32, 4096, 2048 at 110, 128- / 256-slot blocks 240 / 205; 256, 7168, 2048 at 112 2449 / 2329).
+// four: 32, 4096, 2048 at 1 and 2 slots 106 / 118 and 138 / 139, 128, 2944, 768 at 1 118 / 122.)  From 16 slots on the lines are
+// those of the tile kernel, for both kernels: 256-slot blocks gain nothing at 64 slots where the routing is even (16, 4096,
+// 2048 97.8 / 97.8) and leave half as many workgroups where it is not (logits with a spread of 0.7 per expert, 128- / 256-slot
+// blocks at 64 slots: 16, 2048, 1408 69 / 94; 8, 4096, 1536 81 / 105).
 KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E, tiles = E * div_up(2 * inter < hidden ? 2 * inter : hidden, 256);
-  if (per_expert >= 64) return 256;
-  if (per_expert >= 16 || (per_expert >= 4 && tiles >= static_cast<size_t>(kNumCU) / 2)) return 128;
-  return ksq_moe_fp8_block_m(numel, E);
+  if (per_expert >= 4 && per_expert < 16 && tiles >= static_cast<size_t>(kNumCU) / 2) return 128;
+  return ksq_moe_fp8_block_m_sized(numel, E, hidden, inter);
 }
 
 // Rows per expert block for numel routed (token, slot) pairs over E experts.  Replaces the M thresholds of
