@@ -113,12 +113,12 @@ def test_block_fp8_expert_blocks_follow_the_rounds_of_workgroups():
 
 
 def test_block_fp8_expert_row_blocks():
-    """From 4 to 15 slots per expert the row blocks of the streaming tile kernel where the experts make 128 tiles of 256 columns
-    in both GEMMs, the decode form's where they do not; otherwise the lines of the tile kernel."""
+    """From 4 to 15 slots per expert the row blocks of the streaming tile kernel where 16 experts or more make 128 tiles of 256
+    columns in both GEMMs, the decode form's where they do not; otherwise the lines of the tile kernel."""
     from ksanallm_amd import lib as L
     lib = L.load()
-    sizes = ((256, 7168, 2048, True), (32, 1024, 512, True), (32, 2048, 384, False), (31, 1024, 512, False), (8, 7168, 2048, True),
-             (7, 7168, 2048, False))
+    sizes = ((256, 7168, 2048, True), (32, 1024, 512, True), (32, 2048, 384, False), (31, 1024, 512, False), (16, 7168, 2048, True),
+             (15, 7168, 2048, False), (8, 7168, 2048, False))
     for per, many, few in ((0, 16, 16), (1, 16, 16), (2, 32, 32), (3, 32, 32), (4, 128, 32), (15, 128, 32), (16, 128, 128),
                            (63, 128, 128), (64, 128, 128), (103, 128, 128), (128, 256, 256), (1000, 256, 256)):
         for E, hidden, inter, enough in sizes:
