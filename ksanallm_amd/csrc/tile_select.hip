@@ -383,7 +383,10 @@ KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidde
 KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E, tiles = E * div_up(2 * inter < hidden ? 2 * inter : hidden, 256);
-  if (per_expert >= 4 && per_expert < 16 && E >= 16 && tiles >= static_cast<size_t>(kNumCU) / 2) return 128;
+  // (the row blocks of 128 slots hold 32-bit offsets into the activations, and the weight scales of all of K in the LDS)
+  const size_t longest = hidden > inter ? hidden : inter;
+  const bool fits = longest <= (size_t(1) << 20) && numel * longest <= 0xffffffffull;
+  if (per_expert >= 4 && per_expert < 16 && E >= 16 && tiles >= static_cast<size_t>(kNumCU) / 2 && fits) return 128;
   return ksq_moe_fp8_block_m_sized(numel, E, hidden, inter);
 }
 

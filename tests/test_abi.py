@@ -127,6 +127,12 @@ def test_block_fp8_expert_row_blocks():
         for E, hidden, inter, _ in sizes:
             assert lib.ksq_moe_fp8_row_block(per * E, E, hidden, inter) == lib.ksq_moe_fp8_block_m_sized(per * E, E, hidden, inter)
     assert lib.ksq_moe_fp8_row_block(100, 0, 1024, 512) == 16
+    # what the 128-slot launch refuses (activations of 4 GiB, K whose weight scales do not fit the LDS) stays with the decode form
+    for per, E, hidden, inter, bm in ((8, 1024, 524160, 128, 128), (8, 1024, 524416, 128, 32), (15, 256, 1048576, 128, 128),
+                                      (15, 256, 1048704, 128, 32), (4, 16, 1572864, 2048, 32), (4, 1024, 256, 1048576, 32)):
+        assert lib.ksq_moe_fp8_row_block(per * E, E, hidden, inter) == bm, (per, E, hidden, inter)
+        if bm == 128:
+            assert per * E * max(hidden, inter) <= 0xffffffff
 
 
 def test_descriptor_of_the_grouped_streaming_launch():
