@@ -3,9 +3,9 @@
 //
 // What bounds it is the stream of the weights out of HBM and what stands in its way in each CU's one vector memory path:
 //   - weights never touch LDS: every fragment belongs to one wavefront (two strips of 16 columns each), which loads it from
-//     its packed 2 KiB form (ksq_fp8_repack_weight) straight into a register ring of D k-blocks, non-temporally: they are
-//     read once, and cached they turn the L2 over (256 experts, hidden 7168, inter 2048, 512 tokens, whole block: 2.05 ->
-//     1.88 ms, 6.0 TB/s of weights; where several row blocks share weights it costs up to 10 %, and fp8_tile.h is taken).
+//     its packed 2 KiB form (ksq_fp8_repack_weight) straight into a register ring of D k-blocks, non-temporally unless the
+//     block is full: they are read once, and cached they turn the L2 over (256 experts, hidden 7168, inter 2048, 512 tokens,
+//     whole block: 2.05 -> 1.88 ms, 6.0 TB/s of weights).
 //   - activations go global -> LDS (global_load_lds_dwordx4, whole 128-byte lines) into D slots that hold only the row tiles
 //     with tokens; all eight wavefronts read them from there.  Four wavefronts and 128 columns, two workgroups to a CU,
 //     overlap a workgroup's ends with the other's stream but fetch the activations twice as often: 4000 tokens 2.79 against
@@ -171,6 +171,11 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
     constexpr int SLOT = RT * FRAG;
     constexpr int SC_BASE = D * SLOT;
     constexpr int SC4 = fp8_stream_scale_slot4(RT);
+    // A full block's expert most likely has another block, which reads the same weights: cached.  us, whole block in 128-slot
+    // blocks, logits with a spread of 1.5 per expert, non-temporally / cached (and with fp8_tile.h): 256 experts, hidden 7168,
+    // inter 2048 at 80 slots 2190 / 1928 (2107); 64, 7168, 2048 at 104 663 / 597 (626); 128, 2944, 768 at 80 291 / 257 (274).
+    // Even routing, where a full block is its expert's only one: level (2182 / 2198, 610 / 625, 261 / 261).
+    constexpr bool SHARED = !DENSE && RT == RT_MAX;
     const uint32_t sv = s_voff, wv = w_voff;  // (an assembly operand in a lambda inside a generic lambda is no capture)
     static_assert(D * (GROUP_LOADS + 1) < 64, "vmcnt is a 6-bit counter");
 
@@ -216,15 +221,26 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
     auto load_w = [&](uint32_t kb, i32x4 (&dst)[2][2]) {
       const uint8_t* w0 = w_base[0] + static_cast<size_t>(kb) * FRAG;
       const uint8_t* w1 = w_base[1] + static_cast<size_t>(kb) * FRAG;
-      asm volatile(
-          "s_nop 4\n\t"
-          "global_load_dwordx4 %0, %4, %5 nt\n\t"
-          "global_load_dwordx4 %1, %4, %5 offset:1024 nt\n\t"
-          "global_load_dwordx4 %2, %4, %6 nt\n\t"
-          "global_load_dwordx4 %3, %4, %6 offset:1024 nt"
-          : "=&v"(dst[0][0]), "=&v"(dst[0][1]), "=&v"(dst[1][0]), "=&v"(dst[1][1])
-          : "v"(wv), "s"(w0), "s"(w1)
-          : "memory");
+      if constexpr (SHARED)
+        asm volatile(
+            "s_nop 4\n\t"
+            "global_load_dwordx4 %0, %4, %5\n\t"
+            "global_load_dwordx4 %1, %4, %5 offset:1024\n\t"
+            "global_load_dwordx4 %2, %4, %6\n\t"
+            "global_load_dwordx4 %3, %4, %6 offset:1024"
+            : "=&v"(dst[0][0]), "=&v"(dst[0][1]), "=&v"(dst[1][0]), "=&v"(dst[1][1])
+            : "v"(wv), "s"(w0), "s"(w1)
+            : "memory");
+      else
+        asm volatile(
+            "s_nop 4\n\t"
+            "global_load_dwordx4 %0, %4, %5 nt\n\t"
+            "global_load_dwordx4 %1, %4, %5 offset:1024 nt\n\t"
+            "global_load_dwordx4 %2, %4, %6 nt\n\t"
+            "global_load_dwordx4 %3, %4, %6 offset:1024 nt"
+            : "=&v"(dst[0][0]), "=&v"(dst[0][1]), "=&v"(dst[1][0]), "=&v"(dst[1][1])
+            : "v"(wv), "s"(w0), "s"(w1)
+            : "memory");
     };
     auto wait = [&](auto n) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory"); };
     // the registers of k-block h became valid with the wait in front of this statement (volatile statements keep their order)
