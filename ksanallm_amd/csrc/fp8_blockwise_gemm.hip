@@ -396,7 +396,13 @@ int launch_fp8_stream_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s
   p.top_k = q.top_k;
   p.scale_rows = q.scale_rows;
   p.out_s = out_s;
-  fp8_stream_tile_kernel<TO, RT_MAX, PAIRED><<<p.tiles_m * p.tiles_n, 512, fp8_stream_lds_bytes(RT_MAX, q.K / 128), s>>>(p);
+  size_t lds = fp8_stream_lds_bytes(RT_MAX, q.K / 128);
+  const size_t tile_lds = fp8_tile_lds_bytes(8, q.K / 128);
+  if (RT_MAX == 16 && tile_lds <= static_cast<size_t>(kFp8StreamLdsMax)) {
+    p.tile_full = 1;
+    lds = std::max(lds, tile_lds);
+  }
+  fp8_stream_tile_kernel<TO, RT_MAX, PAIRED><<<p.tiles_m * p.tiles_n, 512, lds, s>>>(p);
   return KSQ_OK;
 }
 

@@ -13,7 +13,7 @@
 //   - a row's scales of four k-blocks are one 16-byte piece, fetched once: a load of one scale per row touches 64 lines for
 //     256 bytes, and one per k-block was 7 % of the call.
 //   - results leave through LDS as whole rows of the tile, non-temporally (8-byte stores of 32 bytes a row: 2.71 against 2.60 ms).
-//   - a loop instance per number of row tiles, chosen once per workgroup.
+//   - a loop instance per number of row tiles, chosen once per workgroup; full 256-slot blocks run fp8_tile.h's code.
 // Whole block at 4000 tokens, bf16: 2.87 ms with fp8_tile.h's grouped form, 2.60 with this one.
 #pragma once
 
@@ -45,6 +45,7 @@ struct Fp8StreamParams {
   float* out32;               // verification only: the fp32 sums go here, [numel, N], and nothing is rounded to TO
   float* partial;             // [slot][part][block][256] fp32 tiles of the workgroups that compute a part of K
   uint32_t main_items, splits, kb_per_split;  // tile_work.h
+  uint32_t tile_full;         // full 256-slot blocks run the code of fp8_tile.h (0: its stages do not fit beside K's weight scales)
 };
 
 constexpr int kFp8StreamLdsMax = 160 * 1024;
@@ -117,13 +118,58 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
 
   // ---- slots of this block: their ids go to LDS (rows past the block hold no slot)
   const size_t expert = DENSE ? 0 : static_cast<size_t>(__builtin_amdgcn_readfirstlane(p.expert_ids[tile_m]));
-  uint32_t* ids = reinterpret_cast<uint32_t*>(lds + IDS_BASE);
-  if (threadIdx.x < 256) {
+  constexpr int CHUNKS = RT_MAX / 4;  // of 64 slots
+  uint32_t sids[CHUNKS], rows = 0;
+#pragma unroll
+  for (int h = 0; h < CHUNKS; ++h) {
+    const uint32_t r = m0 + h * 64 + lane;
     if constexpr (DENSE)
-      ids[threadIdx.x] = threadIdx.x < p.block && m0 + threadIdx.x < p.numel ? m0 + threadIdx.x : p.numel;
+      sids[h] = r < p.numel ? r : p.numel;
     else
-      ids[threadIdx.x] = threadIdx.x < p.block ? static_cast<uint32_t>(p.sorted_ids[m0 + threadIdx.x]) : p.numel;
+      sids[h] = static_cast<uint32_t>(p.sorted_ids[r]);
+    rows += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(sids[h] < p.numel)));
   }
+  const uint32_t live_tiles = __builtin_amdgcn_readfirstlane((rows + 15) / 16);
+  // A full 256-slot block is bound by the LDS here (eight wavefronts that each read all sixteen activation fragments keep it
+  // busy as long as the MFMAs take) and runs the tile kernel's code, 2 x 4 wavefronts, in the same launch with the same bits.  us,
+  // whole block in 256-slot blocks, fp8_tile.h alone / fp8_stream.h alone / this: logits with a spread of 1.5 per expert, 256
+  // experts, hidden 7168, inter 2048 at 160 slots 3198 / 3287 / 3114; 64, 2048, 1408 257 / 271 / 250; 32, 4096, 2048 at 208 365 / 372 /
+  // 361; every token on the same sixteenth of the experts, 64, 7168, 2048 at 128 452 / 473 / 449; 8, 4096, 1536 108 / 126 / 106.  Even
+  // routing at 208 slots 3777 / 3497 / 3501, 261 / 249 / 249.  Blocks of 209 to 240 slots stay here, for the even routing: with
+  // few experts that most tokens prefer they are up to 5 % behind (8, 4096, 1536 at 232, the latter routing, 141 / 159 / 150).
+  if constexpr (!DENSE && RT_MAX == 16) {
+    if (live_tiles == RT_MAX && p.tile_full) {  // uniform: the whole workgroup
+      Fp8TileParams t{};
+      t.a = p.a;
+      t.a_s = p.a_s;
+      t.b = p.b;
+      t.b_s = p.b_s;
+      t.out = p.out;
+      t.out_s = p.out_s;
+      t.M = p.tiles_m * p.block;
+      t.N = p.N;
+      t.K = p.K;
+      t.tiles_m = p.tiles_m;
+      t.tiles_n = p.tiles_n;
+      t.splits = 1;
+      t.kb_per_split = k_blocks;
+      t.as_row_bytes = p.as_row_bytes;
+      t.as_kb_bytes = p.as_kb_bytes;
+      t.sorted_ids = p.sorted_ids;
+      t.expert_ids = p.expert_ids;
+      t.num_post_pad = p.num_post_pad;
+      t.topk_w = p.topk_w;
+      t.numel = p.numel;
+      t.top_k = p.top_k;
+      t.scale_rows = p.scale_rows;
+      fp8_tile_body<TO, true, 8, 256, true, PAIRED>(t, lds);
+      return;
+    }
+  }
+  uint32_t* ids = reinterpret_cast<uint32_t*>(lds + IDS_BASE);
+#pragma unroll
+  for (int h = 0; h < 4; ++h)
+    if (wave == static_cast<uint32_t>(h)) ids[h * 64 + lane] = h < CHUNKS ? sids[h < CHUNKS ? h : 0] : p.numel;
   // the weight scales of the tile's two blocks of 128 weight rows
   for (uint32_t t = threadIdx.x; t < 2 * KB; t += 512) {
     const uint32_t blk = t / KB, kb = t - blk * KB, nb_last = (p.N - 1) / 128;
@@ -131,10 +177,6 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
     reinterpret_cast<float*>(lds + BS_BASE)[t] = p.b_s[(expert * p.scale_rows + nb) * k_blocks + kb0 + kb];
   }
   __syncthreads();
-  uint32_t rows = 0;
-#pragma unroll
-  for (int h = 0; h < 4; ++h) rows += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(ids[h * 64 + lane] < p.numel)));
-  const uint32_t live_tiles = __builtin_amdgcn_readfirstlane((rows + 15) / 16);
   auto row_of = [&](uint32_t r) -> uint32_t {  // activation row of slot r of the block; a row without a slot reads some valid one
     uint32_t sid = ids[r];
     sid = sid < p.numel ? sid : p.numel - 1;
@@ -174,7 +216,8 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
     // A full block's expert most likely has another block, which reads the same weights: cached.  us, whole block in 128-slot
     // blocks, logits with a spread of 1.5 per expert, non-temporally / cached (and with fp8_tile.h): 256 experts, hidden 7168,
     // inter 2048 at 80 slots 2190 / 1928 (2107); 64, 7168, 2048 at 104 663 / 597 (626); 128, 2944, 768 at 80 291 / 257 (274).
-    // Even routing, where a full block is its expert's only one: level (2182 / 2198, 610 / 625, 261 / 261).
+    // Even routing, where a full block is its expert's only one: level (2182 / 2198, 610 / 625, 261 / 261).  (Full 256-slot blocks
+    // come here where tile_full is 0.)
     constexpr bool SHARED = !DENSE && RT == RT_MAX;
     const uint32_t sv = s_voff, wv = w_voff;  // (an assembly operand in a lambda inside a generic lambda is no capture)
     static_assert(D * (GROUP_LOADS + 1) < 64, "vmcnt is a 6-bit counter");

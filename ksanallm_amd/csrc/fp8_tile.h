@@ -17,6 +17,7 @@
 //     `s_waitcnt vmcnt(0)` + barrier per stage makes them visible and releases the LDS slot that was just consumed.
 #pragma once
 
+#include "fp8_encode.h"
 #include "ksq_common.h"
 #include "tile_work.h"
 
@@ -41,6 +42,7 @@ struct Fp8TileParams {
   const float* topk_w;
   uint32_t numel, top_k, scale_rows;  // scale_rows = ceil(N/128): rows of one expert's b_s
   uint32_t deep_limit;                // 256-slot blocks that hold fewer slots run on the three-stage tile (0: none does)
+  float* out_s;                       // PAIRED: scales [numel, N / 256] of the codes out [numel, N / 2]
 };
 
 __device__ __forceinline__ f32x4 mfma_fp8_k128(i32x8 a, i32x8 b, f32x4 c) {
@@ -76,8 +78,11 @@ __device__ __forceinline__ uint32_t fp8_live_blocks(const Fp8TileParams& p) {
 
 // BLOCK: slots between consecutive row blocks (tile_m * BLOCK is the block's first slot): the tile's own 32 * WM rows, or
 // - grouped form - 256 for a 160-token tile that serves a 256-slot block with at most 160 tokens.
-template <typename TO, bool GROUPED, int WM, int BLOCK>
+// FULL: the caller has found every row tile of the block to hold slots.  PAIRED: fp8_stream.h's form of that name - a tile
+// holds 128 gate rows of the weights and the matching 128 up rows, and the results are the second GEMM's codes and scales.
+template <typename TO, bool GROUPED, int WM, int BLOCK, bool FULL = false, bool PAIRED = false>
 __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds) {
+  static_assert(!PAIRED || (GROUPED && FULL && WM == 8), "the paired epilogue is written for whole 256-slot blocks");
   static_assert(WM == 8 || WM == 5 || WM == 4, "256-, 160- or 128-token tiles");
   static_assert(BLOCK == 2 * WM * 16 || (GROUPED && WM == 5 && BLOCK == 256), "block stride");
   constexpr int WAVES_N = 4;
@@ -125,8 +130,8 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
     const uint32_t rows = p.M - m0;
     live_tiles = rows < static_cast<uint32_t>(BM) ? (rows + 15) / 16 : AF;
   }
-  if (GROUPED) {
-    expert = static_cast<size_t>(__builtin_amdgcn_readfirstlane(p.expert_ids[tile_m]));
+  if (GROUPED) expert = static_cast<size_t>(__builtin_amdgcn_readfirstlane(p.expert_ids[tile_m]));
+  if (GROUPED && !FULL) {
     uint32_t rows = 0;
 #pragma unroll
     for (int h = 0; h < BLOCK / 64; ++h) {
@@ -159,7 +164,8 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   // it lies in memory - MFMA lane l then reads 16 bytes at 16l of each half, consecutive lanes consecutive addresses,
   // the one pattern the LDS serves at its full rate.
   const uint32_t k_step = stage_act ? 128u : 2048u;  // bytes from one k-block to the next
-  const uint32_t strip0 = n0 / 16;
+  // (paired: wavefronts 4 and 5 fetch the gate strips of the tile, 6 and 7 the up strips, which lie N / 32 strips further)
+  const uint32_t strip0 = PAIRED ? tile_n * 8 + (frag0 & 7) + (frag0 < 8 ? 0 : p.N / 32) : n0 / 16;
   const uint8_t* g_tile = stage_act ? p.a + static_cast<size_t>(GROUPED ? 0 : m0) * p.K
                                     : p.b + ((expert * (p.N / 16) + strip0) * KB) * 2048;
   g_tile += static_cast<size_t>(kb_begin) * k_step;
@@ -193,7 +199,7 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
       d_voff[f] = row * p.K + 16 * ((lane & 3) ^ (lane >> 4));
       d_voff_hi[f] = d_voff[f];
     } else {
-      uint32_t strip = strip0 + frag0 + f;
+      uint32_t strip = strip0 + (PAIRED ? 0 : frag0) + f;
       strip = strip < p.N / 16 ? strip : p.N / 16 - 1;  // strips past N repeat the last one; their results are dropped
       d_voff[f] = (strip - strip0) * KB * 2048 + 16 * lane;
       d_voff_hi[f] = d_voff[f] + 1024 - 64;
@@ -231,12 +237,12 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
     const uint32_t nb_last = (p.N - 1) / 128;
     for (uint32_t t = threadIdx.x; t < 2 * kb_count; t += 512) {
       const uint32_t blk = t / kb_count, kb = t - blk * kb_count;
-      uint32_t nb = n0 / 128 + blk;
+      uint32_t nb = PAIRED ? tile_n + blk * (p.N / 256) : n0 / 128 + blk;
       nb = nb < nb_last ? nb : nb_last;
       reinterpret_cast<float*>(lds + BS_BASE)[t] = p.b_s[(expert * p.scale_rows + nb) * KB + kb_begin + kb];
     }
   }
-  const float* bs_lds = reinterpret_cast<const float*>(lds + BS_BASE) + (wn >> 1) * kb_count;
+  const float* bs_lds = reinterpret_cast<const float*>(lds + BS_BASE) + (PAIRED ? 0 : (wn >> 1) * kb_count);
   const float* as_lds = reinterpret_cast<const float*>(lds + SCALE_BASE) + rt0 * 16 + lrow;
 
   // Every group of loads is one assembly statement opening with `s_nop 4`: its scalar operands are in place before
@@ -366,19 +372,19 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
   auto compute = [&](auto wmv_c, uint32_t slot, uint32_t kb, uint32_t next) {
     constexpr int WMV = decltype(wmv_c)::value;
     float sc[WMV];
-    {
-      const float bs = bs_lds[kb];
+    const float bs = bs_lds[kb], bs_up = PAIRED ? bs_lds[kb_count + kb] : bs;
 #pragma unroll
-      for (int i = 0; i < WMV; ++i) sc[i] = as_lds[slot * (SCALE_SLOT / 4) + i * 16] * bs;
-    }
+    for (int i = 0; i < WMV; ++i) sc[i] = PAIRED ? as_lds[slot * (SCALE_SLOT / 4) + i * 16] : as_lds[slot * (SCALE_SLOT / 4) + i * 16] * bs;
     const char* act = lds + slot * STAGE_BYTES + rt0 * FRAG;
-    const char* wgt = lds + slot * STAGE_BYTES + (W_FRAG0 + wn * WN) * FRAG;
+    // (paired: two gate strips, then the two up strips of the same channels)
+    const char* wgt = lds + slot * STAGE_BYTES + (W_FRAG0 + wn * (PAIRED ? 2 : WN)) * FRAG;
+    auto wfrag_at = [](int t) { return (PAIRED ? (t & 1) + (t >> 1) * 8 : t) * FRAG; };
     i32x8 wf[WN];
     i32x8 af[2];
     wf[0] = read_wfrag(wgt);
     af[0] = read_frag(act);
 #pragma unroll
-    for (int t = 1; t < WN; ++t) wf[t] = read_wfrag(wgt + t * FRAG);
+    for (int t = 1; t < WN; ++t) wf[t] = read_wfrag(wgt + wfrag_at(t));
     __builtin_amdgcn_sched_barrier(0x4);
     f32x4 tmp[3];
     const f32x4 zero{0.f, 0.f, 0.f, 0.f};
@@ -393,8 +399,9 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
       if (j >= 2) {  // the MFMA issued two places earlier has left the pipeline by now
         const int pi = (j - 2) / WN, pt = (j - 2) % WN;
         const f32x4 r = tmp[(j - 2) % 3];
+        const float f = PAIRED ? sc[pi] * (pt < WN / 2 ? bs : bs_up) : sc[pi];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[pt][pi][e] = __builtin_fmaf(r[e], sc[pi], acc[pt][pi][e]);
+        for (int e = 0; e < 4; ++e) acc[pt][pi][e] = __builtin_fmaf(r[e], f, acc[pt][pi][e]);
       }
       __builtin_amdgcn_sched_barrier(0x4);  // keep MFMAs, FMAs and LDS reads in this order (scalar ALU may move)
       if (j == 0) {  // right behind the first MFMA: the longest flight time the two LDS stages allow
@@ -427,7 +434,7 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
       __builtin_amdgcn_s_barrier();
     }
   } else {
-    for_tile_count<1, WM>(mine, [&](auto wmv_c) {
+    for_tile_count<FULL ? WM : 1, WM>(mine, [&](auto wmv_c) {
       for (uint32_t c = 0; c < kb_count; ++c) {
         compute(wmv_c, c % NS, c, c + NS - 1);
         wait_stage();  // operands and scales of c+1
@@ -437,6 +444,55 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
     });
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // drain the clamped prefetches before the LDS is released
+
+  if constexpr (PAIRED) {
+    __syncthreads();  // every wavefront's prefetches have landed: the stages are free
+    // LDS: the largest value of each row in each of the four wavefronts' 32 channels, the slot ids, the codes, 128 to a row
+    float* const row_max = reinterpret_cast<float*>(lds);
+    uint32_t* const ids = reinterpret_cast<uint32_t*>(lds + BM * 16);
+    char* const codes = lds + BM * 20;
+    constexpr int PITCH = 128 + 16;
+    if (threadIdx.x < BM) ids[threadIdx.x] = static_cast<uint32_t>(p.sorted_ids[m0 + threadIdx.x]);
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      float amax = 0.f;
+#pragma unroll
+      for (int t = 0; t < WN / 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = TO::to_float(TO::from_float(
+              silu_mul_f32(TO::to_float(TO::from_float(acc[t][i][e])), TO::to_float(TO::from_float(acc[t + WN / 2][i][e])))));
+          acc[t][i][e] = v;
+          amax = fmaxf(amax, fabsf(v));
+        }
+      amax = fmaxf(amax, __shfl_xor(amax, 16));
+      amax = fmaxf(amax, __shfl_xor(amax, 32));
+      if (lq == 0) row_max[((rt0 + i) * 16 + lrow) * WAVES_N + wn] = amax;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+      const uint32_t r = (rt0 + i) * 16 + lrow;
+      const f32x4 m = *reinterpret_cast<const f32x4*>(row_max + r * WAVES_N);
+      const float scale = fp8_group_scale<false>(fmaxf(fmaxf(fmaxf(1e-10f, m[0]), fmaxf(m[1], m[2])), m[3]));
+      const ExactDiv div(scale);
+#pragma unroll
+      for (int t = 0; t < WN / 2; ++t) {
+        const float v[4] = {acc[t][i][0], acc[t][i][1], acc[t][i][2], acc[t][i][3]};
+        *reinterpret_cast<uint32_t*>(codes + r * PITCH + wn * 32 + t * 16 + 4 * lq) = fp8_encode4<false>(div, v);
+      }
+      const uint32_t row = ids[r];
+      if (wn == (static_cast<uint32_t>(i) & 3) && lq == 0 && row < p.numel) p.out_s[static_cast<size_t>(row) * (p.N / 256) + tile_n] = scale;
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < BM * 8; e += 512) {
+      const uint32_t r = e / 8, c = e % 8, row = ids[r];
+      if (row < p.numel)
+        *reinterpret_cast<u32x4*>(static_cast<uint8_t*>(p.out) + static_cast<size_t>(row) * (p.N / 2) + tile_n * 128 + c * 16) =
+            *reinterpret_cast<const u32x4*>(codes + r * PITCH + c * 16);
+    }
+    return;
+  }
 
   // ---- store: lane holds token m = l%16 of the tile and weight rows (output columns) 4*(l/16) .. +3
   // Grouped form: the slot ids and routing weights of this lane's rows, fetched before the first store.  Read next to

@@ -546,6 +546,13 @@ def _fp8_experts(oracle, seed, E, n, k):
     return q, s
 
 
+def _streams(numel, E, bm, k=1024):
+    """Whether a grouped call in blocks of 128 or 256 slots runs the streaming tile kernel (a paired first GEMM of these sizes is
+    served by that kernel alone) or the MFMA tile kernel."""
+    from ksanallm_amd import lib as L
+    return L.load().ksq_moe_fp8_fused_quant(numel, E, 256, k, bm) == 1
+
+
 @pytest.mark.parametrize("T,E,topk,n,k,bm,colmajor,with_w", [
     (1, 8, 2, 256, 256, 16, False, False), (70, 8, 2, 208, 384, 16, True, True), (300, 6, 3, 512, 1024, 32, False, True),
     (33, 16, 4, 4096, 7168, 32, False, False),
@@ -656,7 +663,10 @@ def test_grouped_fp8_streaming_tile_over_its_ring(ops, oracle, bm, rows, kb):
 
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
 @pytest.mark.parametrize("bm,rows,k,inter", [(128, [1, 16, 17, 127, 128, 65], 128, 128), (128, [5, 33, 100, 2], 640, 384),
-                                             (256, [129, 256, 208, 209, 16, 0], 512, 256), (256, [250, 7], 1152, 640)])
+                                             (256, [129, 256, 208, 209, 16, 0], 512, 256), (256, [250, 7], 1152, 640),
+                                             # full 256-slot blocks (241 rows and more), several of an expert's among them
+                                             (256, [240, 241, 256, 257, 512, 0, 3, 0], 128, 128), (256, [700, 241, 0, 0, 30], 384, 384),
+                                             (256, [256, 1], 2944, 1408)])
 def test_fp8_gate_up_gemm_with_the_second_quantization(ops, oracle, dtype, bm, rows, k, inter):
     """The activation and the second quantization in the first GEMM's epilogue: the codes and scales of the two launches, bit
     for bit, over row tile counts of every ring depth, with rows of zeros, of infinite and of NaN sums among them."""
@@ -689,6 +699,56 @@ def test_fp8_gate_up_gemm_with_the_second_quantization(ops, oracle, dtype, bm, r
     with pytest.raises(L.KsqError):
         L.check(lib.ksq_moe_fp8_gate_up_quant(q1.data_ptr(), s1.data_ptr(), q.data_ptr(), s.data_ptr(), 0, T, w.data_ptr(), ws.data_ptr(),
                                               *(a.data_ptr() for a in aligned), T, topk, E, n, k, 32, dtype, st))
+
+
+@pytest.mark.parametrize("n,k", [(256, 128), (272, 256), (512, 384), (784, 1152)])
+def test_grouped_fp8_full_row_blocks(ops, oracle, n, k):
+    """A full 256-slot block (241 rows and more) leaves the streaming tile kernel for the tile kernel's code, next to blocks that
+    stay: the bits of 128-slot blocks on the tile kernel, and the oracle's sums."""
+    rows = [240, 241, 255, 256, 257, 512, 700, 16, 1, 0, 0, 0]
+    E, T = len(rows), sum(rows)
+    g = H.gen(8300 + n + k)
+    bq, bs = _fp8_experts(oracle, 8310 + n, E, n, k)
+    x = torch.randn((T, k), generator=g).to(torch.bfloat16)
+    ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
+    ids = ids[torch.randperm(T, generator=g)].reshape(T, 1).contiguous()
+    tw = torch.rand((T, 1), generator=g) + 0.1
+    q, s = ops.per_token_group_quant_fp8(x.cuda(), k, 128, False)
+    wp, wsc = ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda()
+    assert _streams(T, E, 256) and not _streams(T, E, 128)
+    outs = []
+    for bm in (128, 256):
+        out = torch.full((T, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, tw.reshape(-1).cuda(), *ops.moe_align_block_size(ids.cuda(), E, bm), T, 1, bm,
+                                   torch.bfloat16, out=out)
+        outs.append(out)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    qh, sh = q.cpu().numpy(), s.cpu().numpy()
+    ref = np.zeros((T, n), np.float32)
+    flat = ids.reshape(-1).numpy()
+    for e in range(E):
+        slots = np.nonzero(flat == e)[0]
+        if slots.size:
+            ref[slots] = oracle.fp8_blockwise_gemm(qh[slots], np.ascontiguousarray(sh[slots]), bq[e], bs[e], False)
+    H.check_gemm(outs[1], ref * tw.numpy(), H.BF16, "fp8 full row blocks n=%d k=%d" % (n, k))
+
+
+def test_grouped_fp8_full_row_blocks_where_the_stages_do_not_fit(ops):
+    """K > 491520: the tile kernel's two stages and K's weight scales do not fit the LDS, and full 256-slot blocks stay with the
+    streaming loop - the bits of 128-slot blocks."""
+    n, k, T, E = 256, 491648, 250, 2
+    assert _streams(T, E, 256, k)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(8400)
+    q = torch.randint(0, 120, (T, k), generator=g, device="cuda", dtype=torch.uint8)
+    s = torch.rand((T, k // 128), generator=g, device="cuda") * 1e-4
+    w = torch.randint(0, 120, (E, n, k), generator=g, device="cuda", dtype=torch.uint8)
+    ws = torch.rand((E, n // 128, k // 128), generator=g, device="cuda") * 1e-4
+    ids = torch.full((T, 1), 1, dtype=torch.int32, device="cuda")
+    outs = [ops.moe_fp8_blockwise_gemm(q, s, False, w, ws, None, *ops.moe_align_block_size(ids, E, bm), T, 1, bm, torch.bfloat16)
+            for bm in (128, 256)]
+    assert torch.isfinite(outs[0].float()).all() and outs[0].float().abs().min() > 0
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
 
 
 def test_grouped_fp8_tile_kernel_where_three_stages_do_not_fit(ops, oracle):
