@@ -322,7 +322,7 @@ int ksq_moe_w4a16_down_sum(void* out, const void* x, const void* w_packed, const
  * a_s_column_major, [k/128, a_rows] - the two layouts ksq_fp8_group_quant writes; b [E, n, k] e4m3 packed by
  * ksq_fp8_repack_weight(E = experts), b_s fp32 [E, ceil(n/128), k/128] as in the checkpoint, out [numel, n] in out_dtype.  top_k = 1 reads a_q rows by slot (second MoE GEMM).
  * block_m is the block size the permutation was aligned with: 16 or 32 run the streaming (decode) kernel, 128 or 256
- * the streaming tile kernel while numel <= block_m * E and the MFMA tile kernel above; ksq_moe_fp8_row_block() gives the
+ * the streaming tile kernel while numel <= block_m * E * 15 / 16 and the MFMA tile kernel above; ksq_moe_fp8_row_block() gives the
  * choice for a block of experts whose gate / up projection is [2 * inter, hidden] and whose down projection is [hidden, inter].
  * ksq_moe_fp8_block_m_sized() and ksq_moe_fp8_block_m() (unknown sizes) are the choice between the decode kernel and the MFMA
  * tile kernel alone.

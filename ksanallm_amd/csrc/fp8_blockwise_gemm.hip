@@ -559,13 +559,19 @@ KSQ_EXPORT int ksq_fp8_blockwise_gemm_f32(const void* a_q, const void* a_s, cons
 }
 
 namespace {
-// The streaming tile kernel takes row blocks of 128 and 256 slots while an expert has one of them on average: its weights are
-// read once, and the kernel that streams them is the faster one (256 experts, hidden 7168, inter 2048, whole block,
-// fp8_tile.h / fp8_stream.h: 2.74 / 2.33 ms at 112 slots per expert, 4.05 / 3.78 at 224; 64, 2048, 1408: 0.258 / 0.243 at 200,
-// but 0.410 / 0.433 at 375, where weights are shared).
+// The streaming tile kernel takes row blocks of 128 and 256 slots up to a mean of 15/16 of a block per expert.  Under even
+// routing the experts then have one block but for a few (a seventh at 240 of 256 slots), whose weights are read twice; at a whole
+// block half of them do.  Whole block, fp8_tile.h over this launch's time, mean (least) of ten sizes of 8 to 256 experts: 1.05
+// (1.00) at 224 slots, 1.04 (0.99) at 232, 1.02 (0.98) at 240, 1.00 (0.99) at 248, 0.98 (0.95) at 256; in 128-slot blocks 1.10
+// (1.01) at 104, 1.05 (1.00) at 112, 1.01 (0.96) at 120, 1.00 (0.95) at 124, 0.99 (0.95) at 127.  The mean is all that the host
+// knows; where the routing prefers some experts, full blocks take care of themselves (fp8_stream.h): logits with a spread of 1.5
+// per expert, 1.04 at 104 to 127 slots, 0.99 at 224 to 240 (least 0.90: 16, 4096, 2048 at 224).
+// A K whose weight scales do not fit beside the tile kernel's stages is the streaming kernel's in any case.
 bool use_fp8_stream(size_t numel, size_t E, size_t k, size_t block_m) {
-  return (block_m == 128 || block_m == 256) && numel <= block_m * E &&
-         fp8_stream_lds_bytes(block_m == 128 ? 8 : 16, k / 128) <= static_cast<size_t>(kFp8StreamLdsMax);
+  if (block_m != 128 && block_m != 256) return false;
+  const size_t lds = kFp8StreamLdsMax, kb = k / 128;
+  const bool tile_fits = fp8_tile_lds_bytes(block_m == 128 ? 4 : 8, kb) <= lds;
+  return (numel <= block_m / 16 * 15 * E || !tile_fits) && fp8_stream_lds_bytes(block_m == 128 ? 8 : 16, kb) <= lds;
 }
 
 // out_s given: the gate / up GEMM with the activation and the second quantization in its epilogue

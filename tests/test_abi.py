@@ -135,6 +135,19 @@ def test_block_fp8_expert_row_blocks():
             assert per * E * max(hidden, inter) <= 0xffffffff
 
 
+def test_block_fp8_streaming_launch_serves_means_of_up_to_15_sixteenths_of_a_block():
+    from ksanallm_amd import lib as L
+    served = L.load().ksq_moe_fp8_fused_quant
+    for bm in (128, 256):
+        for E in (1, 3, 8, 256):
+            most = bm // 16 * 15 * E
+            assert (served(most, E, 512, 1024, bm), served(most + 1, E, 512, 1024, bm)) == (1, 0), (bm, E)
+    # (more of them where the tile kernel's stages and the weight scales of K do not fit the LDS)
+    for bm, k in ((128, 212992), (256, 491520)):
+        assert [served(bm * 8, 8, 512, kk, bm) for kk in (k, k + 128, 1000064, 2000000)] == [0, 1, 1, 0], bm
+    assert [served(100, 8, n, k, bm) for n, k, bm in ((512, 1024, 32), (384, 1024, 128), (512, 1000, 128))] == [0, 0, 0]
+
+
 def test_descriptor_of_the_grouped_streaming_launch():
     """KSQ_KIND_MOE_W4A16 describes the grouped streaming launch, which never cuts K over workgroups: its K slices are its
     wavefronts, four of them while fewer than 32 slots are routed, and then, through LDS, as many as that form has."""
