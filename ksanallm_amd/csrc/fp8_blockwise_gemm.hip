@@ -407,13 +407,13 @@ int launch_fp8_stream_grouped(const Fp8Params& q, unsigned blocks, hipStream_t s
 }
 
 // dense form of the streaming tile kernel: one block of 129..240 rows
-template <typename TO>
+template <typename TO, bool SHORT_K>
 int launch_fp8_stream_dense(const Fp8Params& q, const TilePlan& plan, float* partial, hipStream_t s) {
   const size_t kb_max = (plan.main_items || plan.splits == 1) ? q.K / 128 : plan.kt_per_split;  // whole tiles span all of K
   constexpr int RT_MAX = 16;
   // more dynamic LDS than a kernel may use without asking: once per device
   static std::atomic<uint64_t> configured{0};
-  if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&fp8_stream_tile_kernel<TO, RT_MAX, false, true>), kFp8StreamLdsMax)) return rc;
+  if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&fp8_stream_tile_kernel<TO, RT_MAX, false, true, SHORT_K>), kFp8StreamLdsMax)) return rc;
   Fp8StreamParams p{};
   p.a = q.a;
   p.a_s = q.a_s;
@@ -434,7 +434,7 @@ int launch_fp8_stream_dense(const Fp8Params& q, const TilePlan& plan, float* par
   p.as_kb_bytes = 4 * q.M;
   p.numel = q.M;
   p.top_k = 1;
-  fp8_stream_tile_kernel<TO, RT_MAX, false, true><<<plan.grid, 512, fp8_stream_lds_bytes(RT_MAX, kb_max), s>>>(p);
+  fp8_stream_tile_kernel<TO, RT_MAX, false, true, SHORT_K><<<plan.grid, 512, fp8_stream_lds_bytes(RT_MAX, kb_max), s>>>(p);
   if (plan.splits > 1) {
     const unsigned cut = plan.tiles_m * plan.tiles_n - plan.main_items;
     splitk_reduce_kernel<TO, 16 * RT_MAX><<<cut * (2 * RT_MAX), 256, 0, s>>>(partial, static_cast<uint16_t*>(p.out), q.M, p.N, p.tiles_m,
@@ -474,6 +474,18 @@ KSQ_EXPORT size_t ksq_fp8_blockwise_workspace_size(size_t max_m, size_t n, size_
 }
 
 namespace {
+// k-blocks of a workgroup that computes the least
+size_t fp8_plan_kb(const TilePlan& plan, size_t k) { return plan.splits == 1 ? k / 128 : plan.kt_per_split; }
+
+// Weights non-temporally from 16 k-blocks per workgroup on, cached below: a short part of K is over before its ring runs full,
+// and cached loads come back sooner.  us with weights out of HBM, 129 / 150 / 200 / 240 rows, non-temporally and cached (and with
+// fp8_tile.h): parts of six, n = 8832, k = 2816 27.0 28.1 31.4 32.2 and 23.0 24.6 28.5 30.6 (24.0 26.4 28.8 30.9), n = 24576, k = 1536
+// 21.7 23.1 27.1 29.0 and 22.0 23.2 27.2 29.0 (28.6 29.4 31.2 33.2); of eight, n = 8512, k = 4992 29.5 30.5 33.2 34.8 and 25.3
+// 27.7 32.3 34.6 (27.5 30.5 33.0 35.4); of 16, n = 28672, k = 4096 40.0 42.2 48.3 52.1 and 38.9 41.9 48.8 52.3; of 19, n = 18432,
+// k = 7168 45.7 45.4 51.0 55.9 and 45.9 45.5 52.3 55.9; of 28, n = k = 14336 55.2 58.5 67.4 74.5 and 58.2 58.9 70.8 75.6.  (Without the
+// cached form the worst of 19 shapes was 12 % behind fp8_tile.h, and 20 % where the weights came out of the last-level cache.)
+constexpr size_t kFp8StreamShortK = 16;
+
 // One 256-row block of 129..240 rows: every weight is read once, by one workgroup, and the streaming tile kernel takes the tile
 // kernel's plan with three (to 13 row tiles) or two k-blocks of weights in flight, activation slots for the row tiles that hold
 // rows alone and eight wavefronts that share no weights.  fp8_tile.h / fp8_stream.h in us, GEMM alone, same bits: n = 18432,
@@ -487,8 +499,7 @@ namespace {
 // 100 rows 19.2 / 26.0; ahead by 4 to 6 % at n = k = 14336 only.
 bool use_fp8_stream_dense(const TilePlan& plan, size_t m, size_t k) {
   const size_t kb_max = (plan.main_items || plan.splits == 1) ? k / 128 : plan.kt_per_split;
-  const size_t kb_min = plan.splits == 1 ? k / 128 : plan.kt_per_split;
-  return plan.tiles_m == 1 && plan.block_m == 256 && m <= 16 * kFp8StreamDenseTiles && plan.tiles_n >= 20 && kb_min >= 6 &&
+  return plan.tiles_m == 1 && plan.block_m == 256 && m <= 16 * kFp8StreamDenseTiles && plan.tiles_n >= 20 && fp8_plan_kb(plan, k) >= 6 &&
          fp8_stream_lds_bytes(16, kb_max) <= static_cast<size_t>(kFp8StreamLdsMax);
 }
 
@@ -524,9 +535,13 @@ int fp8_blockwise_gemm_impl(const char* fn, const void* a_q, const void* a_s, co
                   n, k, plan.workspace_bytes, workspace ? workspace_bytes : size_t(0));
     if (256 * k > 0xffffffffull) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: k too large", fn);
     float* partial = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
-    if (use_fp8_stream_dense(plan, m, k))
-      rc = out_dtype == KSQ_F16 ? launch_fp8_stream_dense<F16>(p, plan, partial, as_stream(stream))
-                                : launch_fp8_stream_dense<BF16>(p, plan, partial, as_stream(stream));
+    const bool streamed = use_fp8_stream_dense(plan, m, k);
+    if (streamed && fp8_plan_kb(plan, k) < kFp8StreamShortK)
+      rc = out_dtype == KSQ_F16 ? launch_fp8_stream_dense<F16, true>(p, plan, partial, as_stream(stream))
+                                : launch_fp8_stream_dense<BF16, true>(p, plan, partial, as_stream(stream));
+    else if (streamed)
+      rc = out_dtype == KSQ_F16 ? launch_fp8_stream_dense<F16, false>(p, plan, partial, as_stream(stream))
+                                : launch_fp8_stream_dense<BF16, false>(p, plan, partial, as_stream(stream));
     else if (plan.block_m == 128)
       rc = out_dtype == KSQ_F16 ? launch_fp8_tile<F16, 4>(p, plan, partial, as_stream(stream))
                                 : launch_fp8_tile<BF16, 4>(p, plan, partial, as_stream(stream));

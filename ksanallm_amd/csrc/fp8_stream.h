@@ -4,8 +4,8 @@
 // What bounds it is the stream of the weights out of HBM and what stands in its way in each CU's one vector memory path:
 //   - weights never touch LDS: every fragment belongs to one wavefront (two strips of 16 columns each), which loads it from
 //     its packed 2 KiB form (ksq_fp8_repack_weight) straight into a register ring of D k-blocks, non-temporally unless the
-//     block is full: they are read once, and cached they turn the L2 over (256 experts, hidden 7168, inter 2048, 512 tokens,
-//     whole block: 2.05 -> 1.88 ms, 6.0 TB/s of weights).
+//     block is full or, dense, K is short: they are read once, and cached they turn the L2 over (256 experts, hidden 7168,
+//     inter 2048, 512 tokens, whole block: 2.05 -> 1.88 ms, 6.0 TB/s of weights).
 //   - activations go global -> LDS (global_load_lds_dwordx4, whole 128-byte lines) into D slots that hold only the row tiles
 //     with tokens; all eight wavefronts read them from there.  Four wavefronts and 128 columns, two workgroups to a CU,
 //     overlap a workgroup's ends with the other's stream but fetch the activations twice as often: 4000 tokens 2.79 against
@@ -86,7 +86,8 @@ __device__ __forceinline__ P* scalar_ptr(P* ptr) {
 // DENSE: tile m holds rows m * block .., results go to their rows or, from a workgroup that computes a part of K, to fp32
 // partial tiles (splitk_reduce.h).  200 rows, n = 18432, k = 7168: 59.8 us with fp8_tile.h, 55.2 with this form (2.4 TB/s of
 // weights; 150 rows 55.7 -> 47.3): the MFMAs of 13 row tiles in whole waves of 32 columns and the partial sums are the rest.
-template <typename TO, int RT_MAX, bool PAIRED, bool DENSE = false>
+// SHORT_K: a workgroup multiplies fewer than 16 k-blocks; the weights are loaded cached (fp8_blockwise_gemm.hip).
+template <typename TO, int RT_MAX, bool PAIRED, bool DENSE = false, bool SHORT_K = false>
 __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];  // fp8_stream_lds_bytes
   constexpr int WAVES = 8;
@@ -218,7 +219,7 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
     // inter 2048 at 80 slots 2190 / 1928 (2107); 64, 7168, 2048 at 104 663 / 597 (626); 128, 2944, 768 at 80 291 / 257 (274).
     // Even routing, where a full block is its expert's only one: level (2182 / 2198, 610 / 625, 261 / 261).  (Full 256-slot blocks
     // come here where tile_full is 0.)
-    constexpr bool SHARED = !DENSE && RT == RT_MAX;
+    constexpr bool CACHED = DENSE ? SHORT_K : RT == RT_MAX;
     const uint32_t sv = s_voff, wv = w_voff;  // (an assembly operand in a lambda inside a generic lambda is no capture)
     static_assert(D * (GROUP_LOADS + 1) < 64, "vmcnt is a 6-bit counter");
 
@@ -264,7 +265,7 @@ __global__ void __launch_bounds__(512, 1) fp8_stream_tile_kernel(Fp8StreamParams
     auto load_w = [&](uint32_t kb, i32x4 (&dst)[2][2]) {
       const uint8_t* w0 = w_base[0] + static_cast<size_t>(kb) * FRAG;
       const uint8_t* w1 = w_base[1] + static_cast<size_t>(kb) * FRAG;
-      if constexpr (SHARED)
+      if constexpr (CACHED)
         asm volatile(
             "s_nop 4\n\t"
             "global_load_dwordx4 %0, %4, %5\n\t"

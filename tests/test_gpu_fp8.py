@@ -265,6 +265,31 @@ def test_blockwise_gemm_one_block_of_129_to_256_rows(ops, oracle, n, k, cut):
             assert torch.equal(ops.fp8_blockwise_gemm(q, s, w, ws, dt).view(torch.int16), y32.to(dt).view(torch.int16)), m
 
 
+# the same kernel with 16 and more k-blocks per workgroup (whole tiles, parts of K), whose weights are loaded non-temporally, and with
+# 256 whole tiles beside 60 that are cut in three parts of eight; n = 16 columns past a tile each
+@pytest.mark.parametrize("n,k,cut,grid", [(32784, 2048, 1, 129), (16400, 6144, 3, 195), (80656, 3072, 3, 436)])
+def test_blockwise_gemm_one_block_with_long_parts_and_whole_tiles_beside_parts(ops, oracle, n, k, cut, grid):
+    from ksanallm_amd import lib as L
+    g = torch.Generator(device="cuda")
+    g.manual_seed(4480 + n)
+    codes = torch.randint(0, 256, (n, k), generator=g, device="cuda", dtype=torch.uint8)
+    codes &= torch.where(codes & 0x7f == 0x7f, 0xfe, 0xff).to(torch.uint8)   # no NaN
+    w, ws = ops.fp8_repack_weight(codes), torch.rand((-(-n // 128), k // 128), generator=g, device="cuda") * 2e-3 + 1e-4
+    x = make_act(4490 + n, 240, k, H.BF16) * 0.02
+    first, last = (codes[c].cpu().numpy() for c in (slice(0, 256), slice(n - 16, n)))
+    wsc = ws.cpu().numpy()
+    for m in (240, 129, 161, 208, 209):
+        d = L.select_tile(L.KIND_FP8_BLOCKWISE, m, n, k, H.BF16)
+        assert (d["block_m"], d["split_k"], d["grid"]) == (256, cut, grid)
+        q, s = ops.per_token_group_quant_fp8(x[:m].contiguous().cuda(), k, 128, True)
+        qc, sc = q.cpu().numpy(), s.cpu().numpy()
+        y32 = ops.fp8_blockwise_gemm_f32(q, s, w, ws)
+        H.check_gemm_f32(y32[:, :256], oracle.fp8_blockwise_gemm(qc, sc, first, wsc[:2], True), "m=%d n=%d k=%d, first columns" % (m, n, k))
+        H.check_gemm_f32(y32[:, n - 16:], oracle.fp8_blockwise_gemm(qc, sc, last, wsc[-1:], True), "m=%d n=%d k=%d, last columns" % (m, n, k))
+        for dt in (torch.float16, torch.bfloat16):
+            assert torch.equal(ops.fp8_blockwise_gemm(q, s, w, ws, dt).view(torch.int16), y32.to(dt).view(torch.int16)), m
+
+
 # small problems of more than 32 tokens (ceil(m / 32) * n * k <= 5 * 2^24, m <= 512): the streaming kernel over blocks of
 # 32 tokens, ragged last block included
 @pytest.mark.parametrize("m,n,k", [(65, 256, 128), (100, 272, 384), (128, 4096, 4096), (300, 2320, 1152), (500, 768, 640),
