@@ -517,7 +517,8 @@ def test_few_tokens_form_drops_ids_outside_the_experts_and_rejects_what_it_canno
 def test_grouped_tile_kernel_ends_over_k_tiles(ops, dtype, kt):
     """The loads that are on their way when the main loop ends (its turns are three k-tiles long, and it prefetches past the
     end of K) leave the epilogue's registers alone: experts with every row tile count, in 256- and 128-row blocks, which sum in
-    the same order - the same bits."""
+    the same order - the same bits -, and every row that of the decode form, which has no such loop: the two differ by the
+    rounding of the weights and of the result to T, 2.8e-3 of a row's norm in bf16."""
     from ksanallm_amd import lib as L
     rows = [16 * c - 3 for c in range(1, 17)] * 4
     E, T, n, k = len(rows), sum(rows), 512, 128 * kt
@@ -529,9 +530,14 @@ def test_grouped_tile_kernel_ends_over_k_tiles(ops, dtype, kt):
     x = torch.randn((T, k), generator=g, device="cuda").to(H.TORCH_DT[dtype])
     ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)]).cuda()
     ids = ids[torch.randperm(T, generator=g, device="cuda")].reshape(T, 1).contiguous()
-    outs = [ops.moe_w4a16_gemm(x, w, sp, None, *ops.moe_align_block_size(ids, E, bm), T, 1, E, n, k, 128, bm) for bm in (256, 128)]
+    outs = []
+    for bm in (256, 128, 32):
+        out = torch.full((T, n), float("nan"), dtype=x.dtype, device="cuda")
+        outs.append(ops.moe_w4a16_gemm(x, w, sp, None, *ops.moe_align_block_size(ids, E, bm), T, 1, E, n, k, 128, bm, out=out))
     assert torch.isfinite(outs[0].float()).all()
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    tile, decode = outs[0].double(), outs[2].double()
+    assert ((tile - decode).norm(dim=1) / decode.norm(dim=1)).max() <= 1e-2
 
 
 # ---- block-quantized fp8 experts -------------------------------------------------------------------------------------
@@ -553,15 +559,17 @@ def _streams(numel, E, bm, k=1024):
     return L.load().ksq_moe_fp8_fused_quant(numel, E, 256, k, bm) == 1
 
 
-@pytest.mark.parametrize("T,E,topk,n,k,bm,colmajor,with_w", [
-    (1, 8, 2, 256, 256, 16, False, False), (70, 8, 2, 208, 384, 16, True, True), (300, 6, 3, 512, 1024, 32, False, True),
-    (33, 16, 4, 4096, 7168, 32, False, False),
-    # 256-slot blocks: the MFMA tile kernel in its grouped form (ragged n, both scale layouts, routing weight)
-    (300, 6, 3, 512, 1024, 256, False, True), (700, 4, 2, 784, 512, 256, True, False), (130, 2, 1, 256, 128, 256, False, True),
-    # 128-slot blocks of the same kernel
-    (300, 6, 3, 512, 1024, 128, False, True), (700, 4, 2, 784, 512, 128, True, False), (130, 2, 1, 256, 128, 128, False, True),
-    (90, 3, 2, 2064, 640, 128, True, True)])
-def test_grouped_fp8_gemm_stage(ops, oracle, T, E, topk, n, k, bm, colmajor, with_w):
+@pytest.mark.parametrize("T,E,topk,n,k,bm,colmajor,with_w,streamed", [
+    (1, 8, 2, 256, 256, 16, False, False, None), (70, 8, 2, 208, 384, 16, True, True, None), (300, 6, 3, 512, 1024, 32, False, True, None),
+    (33, 16, 4, 4096, 7168, 32, False, False, None),
+    # 256- and 128-slot blocks of the streaming tile kernel (ragged n, both scale layouts, routing weight)
+    (300, 6, 3, 512, 1024, 256, False, True, True), (130, 2, 1, 256, 128, 256, False, True, True), (130, 2, 1, 256, 128, 128, False, True, True),
+    (90, 3, 2, 2064, 640, 128, True, True, True),
+    # ... and of the MFMA tile kernel in its grouped form
+    (700, 4, 2, 784, 512, 256, True, False, False), (600, 3, 2, 512, 1024, 256, False, True, False), (257, 1, 1, 256, 128, 256, False, True, False),
+    (300, 6, 3, 512, 1024, 128, False, True, False), (700, 4, 2, 784, 512, 128, True, False, False), (260, 2, 1, 256, 128, 128, False, True, False),
+    (200, 3, 2, 2064, 640, 128, True, True, False)])
+def test_grouped_fp8_gemm_stage(ops, oracle, T, E, topk, n, k, bm, colmajor, with_w, streamed):
     """One grouped blockwise-fp8 GEMM launch against the per-expert oracle GEMM on the codes the GPU quantizer wrote."""
     g = H.gen(7000 + T + n)
     bq, bs = _fp8_experts(oracle, 7100 + n, E, n, k)
@@ -569,6 +577,8 @@ def test_grouped_fp8_gemm_stage(ops, oracle, T, E, topk, n, k, bm, colmajor, wit
     ids = torch.stack([torch.randperm(E, generator=g)[:topk] for _ in range(T)]).to(torch.int32)
     tw = torch.rand((T, topk), generator=g)
     numel = T * topk
+    if bm >= 128:
+        assert _streams(numel, E, bm) == streamed
     q, s = ops.per_token_group_quant_fp8(x.cuda(), k, 128, colmajor)
     sorted_ids, expert_ids, npp = ops.moe_align_block_size(ids.cuda(), E, bm)
     out = ops.moe_fp8_blockwise_gemm(q, s, colmajor, ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda(),
@@ -588,13 +598,16 @@ def test_grouped_fp8_gemm_stage(ops, oracle, T, E, topk, n, k, bm, colmajor, wit
     H.check_gemm(out, ref, H.BF16, "grouped fp8 T=%d n=%d k=%d" % (T, n, k))
 
 
-@pytest.mark.parametrize("bm", [128, 256])
-def test_grouped_fp8_tile_kernel_every_count_of_live_row_tiles(ops, oracle, bm):
-    """Every wavefront of the fp8 tile kernel has an instance of its main loop per number of its row tiles that hold
-    tokens: experts with 16c - 5 slots for c = 1..16 meet every count of the lower and of the upper wavefronts of a
-    256-slot block (cut into 128-slot blocks: of that form)."""
+@pytest.mark.parametrize("bm,streamed", [(128, False), (128, True), (256, False), (256, True)])
+def test_grouped_fp8_tile_kernel_every_count_of_live_row_tiles(ops, oracle, bm, streamed):
+    """Both tile kernels have an instance of their main loop per number of row tiles that hold tokens, the MFMA tile kernel of a
+    wavefront's row tiles: experts with 16c - 5 slots for c = 1..16 meet every count of the lower and of the upper wavefronts of a
+    256-slot block (cut into 128-slot blocks: of that form).  An expert of many slots, or experts without any, bring the mean to
+    where one kernel or the other runs."""
     rows = [16 * c - 5 for c in range(1, 17)]
+    rows += [0] * 4 if streamed else [17 * 256 - 5]
     E, T, n, k = len(rows), sum(rows), 256, 384
+    assert _streams(T, E, bm) == streamed
     g = H.gen(7700 + bm)
     bq, bs = _fp8_experts(oracle, 7710, E, n, k)
     x = torch.randn((T, k), generator=g).to(torch.bfloat16)
@@ -610,17 +623,20 @@ def test_grouped_fp8_tile_kernel_every_count_of_live_row_tiles(ops, oracle, bm):
     for e in range(E):
         slots = np.nonzero(flat == e)[0]
         ref[slots] = oracle.fp8_blockwise_gemm(qh[slots], np.ascontiguousarray(sh[slots]), bq[e], bs[e], False)
-    H.check_gemm(out, ref, H.BF16, "grouped fp8 tile kernel, %d-slot blocks" % bm)
+    H.check_gemm(out, ref, H.BF16, "grouped fp8 tile kernels, %d-slot blocks, streamed: %s" % (bm, streamed))
 
 
 @pytest.mark.parametrize("n,k", [(256, 128), (272, 384), (528, 1024)])
 def test_grouped_fp8_tile_kernel_at_the_edges_of_the_three_stage_tile(ops, oracle, n, k):
-    """A 256-slot block of at most 160 slots runs on three LDS stages, a larger one on two, a 128-slot block on its own
-    tile: every output is the same sum in the same order of k, so the bits are the same."""
-    rows = [1, 16, 17, 32, 33, 127, 128, 129, 144, 145, 159, 160, 161, 176, 255, 256, 257, 417]
+    """A 256-slot block of at most 160 slots runs on three LDS stages of the MFMA tile kernel, a larger one on two, a 128-slot
+    block on its own tile, and where experts without slots bring the mean down the streaming tile kernel runs: every output is the
+    same sum in the same order of k, so the bits are the same."""
+    rows = [1, 16, 17, 32, 33, 127, 128, 129, 144, 145, 159, 160, 161, 176, 255, 256, 257, 417, 12 * 256]
     E, T = len(rows), sum(rows)
+    few = [E, E + 40]   # (as many experts to the alignment and the launch)
+    assert [_streams(T, e, bm) for bm in (128, 256) for e in few] == [False, True] * 2
     g = H.gen(7800 + n + k)
-    bq, bs = _fp8_experts(oracle, 7810 + n, E, n, k)
+    bq, bs = _fp8_experts(oracle, 7810 + n, few[1], n, k)
     x = torch.randn((T, k), generator=g).to(torch.bfloat16)
     ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
     ids = ids[torch.randperm(T, generator=g)].reshape(T, 1).contiguous().cuda()
@@ -628,9 +644,13 @@ def test_grouped_fp8_tile_kernel_at_the_edges_of_the_three_stage_tile(ops, oracl
     wp, wsc = ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda()
     outs = []
     for bm in (128, 256):
-        sorted_ids, expert_ids, npp = ops.moe_align_block_size(ids, E, bm)
-        outs.append(ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, None, sorted_ids, expert_ids, npp, T, 1, bm, torch.bfloat16))
-    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+        for e in few:
+            out = torch.full((T, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+            outs.append(ops.moe_fp8_blockwise_gemm(q, s, False, wp[:e], wsc[:e], None, *ops.moe_align_block_size(ids, e, bm), T, 1, bm,
+                                                   torch.bfloat16, out=out))
+    assert torch.isfinite(outs[0].float()).all()
+    for out in outs[1:]:
+        assert torch.equal(outs[0].view(torch.int16), out.view(torch.int16))
 
 
 @pytest.mark.parametrize("kb", [1, 2, 3, 4, 5, 6, 7, 8, 9, 13])
@@ -752,27 +772,34 @@ def test_grouped_fp8_full_row_blocks_where_the_stages_do_not_fit(ops):
 
 
 def test_grouped_fp8_tile_kernel_where_three_stages_do_not_fit(ops, oracle):
-    """K > 28672 leaves no room in the LDS for three stages: every 256-slot block then runs on two, one without any token
-    (which the alignment never makes, but a caller's own permutation may) among them."""
-    n, k, rows = 272, 28800, [100, 0, 200, 160]
+    """K > 28672 leaves no room in the LDS for three stages: every 256-slot block of the MFMA tile kernel (an expert of many slots
+    brings the mean to it) then runs on two, one without any token (which the alignment never makes, but a caller's own
+    permutation may) among them."""
+    n, k, rows = 272, 28800, [100, 0, 200, 160, 1200]
     E, T = len(rows), sum(rows)
+    assert not _streams(T, E, 256) and not _streams(T, E, 128)
     g = H.gen(7900)
     bq, bs = _fp8_experts(oracle, 7910, E, n, k)
     x = torch.randn((T, k), generator=g).to(torch.bfloat16)
     q, s = ops.per_token_group_quant_fp8(x.cuda(), k, 128, False)
     wp, wsc = ops.fp8_repack_weight(torch.from_numpy(bq).cuda()), torch.from_numpy(bs).cuda()
     flat = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
-    sorted_ids = torch.full((E, 256), T, dtype=torch.int32)   # one block per expert, pad slots at the end
+    sorted_ids, expert_ids = [], []   # at least one block per expert, pad slots at the end
     for e in range(E):
         mine = torch.nonzero(flat == e).flatten().to(torch.int32)
-        sorted_ids[e, :mine.numel()] = mine
-    out = ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, None, sorted_ids.flatten().cuda(), torch.arange(E, dtype=torch.int32).cuda(),
-                                     torch.tensor([E * 256], dtype=torch.int32).cuda(), T, 1, 256, torch.bfloat16)
+        for c in range(0, max(mine.numel(), 1), 256):
+            block = torch.full((256,), T, dtype=torch.int32)
+            block[:mine[c:c + 256].numel()] = mine[c:c + 256]
+            sorted_ids.append(block)
+            expert_ids.append(e)
+    out = torch.full((T, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, None, torch.cat(sorted_ids).cuda(), torch.tensor(expert_ids, dtype=torch.int32).cuda(),
+                               torch.tensor([len(sorted_ids) * 256], dtype=torch.int32).cuda(), T, 1, 256, torch.bfloat16, out=out)
     aligned = ops.moe_align_block_size(flat.reshape(T, 1).cuda(), E, 128)
     short = ops.moe_fp8_blockwise_gemm(q, s, False, wp, wsc, None, *aligned, T, 1, 128, torch.bfloat16)
     assert torch.equal(out.view(torch.int16), short.view(torch.int16))
     qh, sh = q.cpu().numpy(), s.cpu().numpy()
-    pick = [0, 15, 99, 100, 260, 299, 300, 459]   # the oracle on some rows of every expert
+    pick = [0, 15, 99, 100, 260, 299, 300, 459, 460, 715, 716, 1659]   # the oracle on some rows of every expert
     ref = np.stack([oracle.fp8_blockwise_gemm(qh[t:t + 1], np.ascontiguousarray(sh[t:t + 1]), bq[flat[t]], bs[flat[t]], False)[0]
                     for t in pick])
     H.check_gemm(out[pick], ref, H.BF16, "grouped fp8 tile kernel, K = %d" % k)
