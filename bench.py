@@ -82,7 +82,7 @@ def copies_needed(weight_bytes):
 
 def kernel_label(L, kind, prefix, M, N, K, dt):
     d = L.select_tile(kind, M, N, K, dt)
-    return "%s<%dx%d,w%d>" % (prefix + ("_splitk_kernel" if d["kernel"] == 0 else "_tile_kernel"),
+    return "%s<%dx%d,w%d>" % (prefix + ("_splitk_kernel", "_tile_kernel", "_stream_tile_kernel")[d["kernel"]],
                               d["block_m"], d["block_n"], d["waves"])
 
 

@@ -401,7 +401,11 @@ int ksq_moe_sum(const void* in, void* out, size_t tokens, size_t topk, size_t d,
  * and the threshold sweep of BlockwiseMatMulLayer::Preprocess (S/layers/nvidia/blockwise_matmul_layer.cpp:71-181).
  * ------------------------------------------------------------------------------------------------------------------ */
 enum { KSQ_KIND_W4A16 = 0, KSQ_KIND_FP8_BLOCKWISE = 1, KSQ_KIND_MOE_W4A16 = 2, KSQ_KIND_W4A8 = 3 };
-enum { KSQ_KERNEL_SPLITK_WAVE = 0, KSQ_KERNEL_MFMA_TILE = 1 };
+enum {
+  KSQ_KERNEL_SPLITK_WAVE = 0,
+  KSQ_KERNEL_MFMA_TILE = 1,
+  KSQ_KERNEL_STREAM_TILE = 2 /* block fp8: the MFMA tile kernel's grid, weights through registers */
+};
 
 typedef struct ksq_tile_desc {
   int32_t kernel;   /* KSQ_KERNEL_* */

@@ -43,6 +43,10 @@ TilePlan plan_mfma_tile(size_t m, size_t n, size_t k);
 // and its grid (kt_per_split counts 128-deep k-blocks).
 bool use_fp8_tile(size_t m, size_t n, size_t k);
 TilePlan plan_fp8_tile(size_t m, size_t n, size_t k);
+// k-blocks of a workgroup that computes the least
+size_t fp8_plan_kb(const TilePlan& plan, size_t k);
+// whether the streaming tile kernel (fp8_stream.h) takes the place of the MFMA tile kernel under that plan
+bool use_fp8_stream_dense(const TilePlan& plan, size_t m, size_t k);
 // W4A8 (w4a8_tile.h): the same regime rule with its own size limit, the same tile shapes with its own costs of a cut along K
 bool use_w4a8_tile(size_t m, size_t n, size_t k);
 TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k);

@@ -3,6 +3,7 @@
 #include <atomic>
 #include <cmath>
 
+#include "fp8_stream.h"
 #include "ksq_common.h"
 #include "tile_select.h"
 
@@ -278,6 +279,25 @@ TilePlan plan_fp8_tile(size_t m, size_t n, size_t k) {
   return t;
 }
 
+size_t fp8_plan_kb(const TilePlan& plan, size_t k) { return plan.splits == 1 ? k / 128 : plan.kt_per_split; }
+
+// One 256-row block of 129..240 rows: every weight is read once, by one workgroup, and the streaming tile kernel takes the tile
+// kernel's plan with three (to 13 row tiles) or two k-blocks of weights in flight, activation slots for the row tiles that hold
+// rows alone and eight wavefronts that share no weights.  fp8_tile.h / fp8_stream.h in us, GEMM alone, same bits: n = 18432,
+// k = 7168 at 129, 150, 200, 224 rows 50.7 / 44.3, 55.7 / 47.3, 59.8 / 55.2, 61.6 / 59.8; n = 7168, k = 18432 49.5 / 41.7, 51.8 /
+// 44.2, 55.3 / 52.3, 58.5 / 54.7; n = 24576, k = 1536, six k-blocks a workgroup, 27.9 / 22.2, 28.9 / 23.7, 30.7 / 27.7, 31.5 / 28.2;
+// n = k = 14336 68.8 / 58.0, 73.6 / 61.3, 78.8 / 75.7, 81.1 / 77.2.  With all sixteen row tiles the two cross (n = 28672, k = 4096
+// at 256 rows 60.5 / 62.8, n = k = 14336 84.9 / 84.9, n = 24576, k = 1536 33.4 / 30.7), and a few column tiles cut very often spend
+// their time on partial sums (n = 1040, k = 28672: 129 rows 31.6 / 32.6, 150 36.4 / 33.7, 200 37.5 / 38.2); n = 5120, k = 25600, 20
+// column tiles, at 129 and 200 rows 48.8 / 41.0, 55.1 / 50.6.  Workgroups of fewer than six k-blocks are not measured.
+// Blocks of 128 rows stay on fp8_tile.h: n = 28672, k = 4096 at 33 and 100 rows 29.1 / 30.9, 35.8 / 39.0, n = 4096, k = 7168 at
+// 100 rows 19.2 / 26.0; ahead by 4 to 6 % at n = k = 14336 only.
+bool use_fp8_stream_dense(const TilePlan& plan, size_t m, size_t k) {
+  const size_t kb_max = (plan.main_items || plan.splits == 1) ? k / 128 : plan.kt_per_split;
+  return plan.tiles_m == 1 && plan.block_m == 256 && m <= 16 * kFp8StreamDenseTiles && plan.tiles_n >= 20 && fp8_plan_kb(plan, k) >= 6 &&
+         fp8_stream_lds_bytes(16, kb_max) <= static_cast<size_t>(kFp8StreamLdsMax);
+}
+
 // W4A8: the blockwise-FP8 tile shapes; a k-step moves three quarters of the bytes and its prologue is shorter, so a
 // cut along K pays earlier (measured at n = 25600, k = 5120: with the FP8 costs 64 / 128 / 256 tokens ran whole tiles
 // on 100 of the 256 CUs in 38 / 51 / 83 us, with these they are cut in two or three: 28 / 38 / 60 us)
@@ -442,7 +462,7 @@ KSQ_EXPORT int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype
     case KSQ_KIND_FP8_BLOCKWISE: {
       if (use_fp8_tile(m, n, k)) {
         const TilePlan t = plan_fp8_tile(m, n, k);
-        d->kernel = KSQ_KERNEL_MFMA_TILE;
+        d->kernel = use_fp8_stream_dense(t, m, k) ? KSQ_KERNEL_STREAM_TILE : KSQ_KERNEL_MFMA_TILE;
         d->block_m = t.block_m;
         d->block_n = 256;
         d->block_k = 128;

@@ -148,6 +148,20 @@ def test_block_fp8_streaming_launch_serves_means_of_up_to_15_sixteenths_of_a_blo
     assert [served(100, 8, n, k, bm) for n, k, bm in ((512, 1024, 32), (384, 1024, 128), (512, 1000, 128))] == [0, 0, 0]
 
 
+def test_block_fp8_streaming_tile_kernel_serves_one_block_of_129_to_240_rows():
+    """From 20 column tiles and six k-blocks per workgroup on."""
+    from ksanallm_amd import lib as L
+
+    def kernel(m, n, k):
+        return L.select_tile(L.KIND_FP8_BLOCKWISE, m, n, k, L.BF16)["kernel"]
+    stream, tile, decode = L.KERNEL_STREAM_TILE, L.KERNEL_MFMA_TILE, L.KERNEL_SPLITK_WAVE
+    assert [kernel(m, 18432, 7168) for m in (32, 33, 128, 129, 240, 241, 256, 400)] == [decode, tile, tile, stream, stream, tile, tile, tile]
+    assert [kernel(200, n, 20480) for n in (4864, 4880, 5120)] == [tile, stream, stream]        # 19 and 20 column tiles
+    assert [kernel(200, 8704, k) for k in (640, 768)] == [tile, stream]                          # whole tiles of five and six k-blocks
+    assert [kernel(200, n, k) for n, k in ((66064, 2048), (80656, 3072))] == [tile, stream]      # whole tiles beside parts of four, of eight
+    assert [kernel(200, n, 4096) for n in (4096, 8192, 8208)] == [tile, tile, stream]            # 128-row tiles up to 32 column tiles
+
+
 def test_descriptor_of_the_grouped_streaming_launch():
     """KSQ_KIND_MOE_W4A16 describes the grouped streaming launch, which never cuts K over workgroups: its K slices are its
     wavefronts, four of them while fewer than 32 slots are routed, and then, through LDS, as many as that form has."""

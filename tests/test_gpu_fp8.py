@@ -253,6 +253,7 @@ def test_blockwise_gemm_one_block_of_129_to_256_rows(ops, oracle, n, k, cut):
     for m in (256, 129, 144, 145, 160, 176, 177, 193, 208, 224, 225, 240, 241):
         d = L.select_tile(L.KIND_FP8_BLOCKWISE, m, n, k, H.BF16)
         assert d["block_m"] == 256 and (d["split_k"] > 1) == cut
+        assert d["kernel"] == (L.KERNEL_STREAM_TILE if k > 256 and m <= 240 else L.KERNEL_MFMA_TILE)
         q, s = ops.per_token_group_quant_fp8(x[:m].contiguous().cuda(), k, 128, True)
         if ref is None:
             qc, sc = q.cpu().numpy(), s.cpu().numpy()
@@ -280,7 +281,7 @@ def test_blockwise_gemm_one_block_with_long_parts_and_whole_tiles_beside_parts(o
     wsc = ws.cpu().numpy()
     for m in (240, 129, 161, 208, 209):
         d = L.select_tile(L.KIND_FP8_BLOCKWISE, m, n, k, H.BF16)
-        assert (d["block_m"], d["split_k"], d["grid"]) == (256, cut, grid)
+        assert (d["kernel"], d["block_m"], d["split_k"], d["grid"]) == (L.KERNEL_STREAM_TILE, 256, cut, grid)
         q, s = ops.per_token_group_quant_fp8(x[:m].contiguous().cuda(), k, 128, True)
         qc, sc = q.cpu().numpy(), s.cpu().numpy()
         y32 = ops.fp8_blockwise_gemm_f32(q, s, w, ws)
