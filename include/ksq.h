@@ -324,8 +324,7 @@ int ksq_moe_w4a16_down_sum(void* out, const void* x, const void* w_packed, const
  * block_m is the block size the permutation was aligned with: 16 or 32 run the streaming (decode) kernel, 128 or 256
  * the streaming tile kernel while numel <= block_m * E * 15 / 16 and the MFMA tile kernel above; ksq_moe_fp8_row_block() gives the
  * choice for a block of experts whose gate / up projection is [2 * inter, hidden] and whose down projection is [hidden, inter].
- * ksq_moe_fp8_block_m_sized() and ksq_moe_fp8_block_m() (unknown sizes) are the choice between the decode kernel and the MFMA
- * tile kernel alone.
+ * It is ksq_moe_fp8_block_m_sized() but for 4 to 15 slots per expert; ksq_moe_fp8_block_m() is the choice for unknown sizes.
  * Replaces the fp8_w8a8 block-quantized branch of InvokeFusedMoe's fused_moe_kernel launches
  * (S/kernels/nvidia/moe_kernel_wrapper.cpp:435-456, 498-522, 560-600). */
 size_t ksq_moe_fp8_block_m(size_t numel, size_t E);

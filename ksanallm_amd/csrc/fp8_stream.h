@@ -14,7 +14,8 @@
 //     256 bytes, and one per k-block was 7 % of the call.
 //   - results leave through LDS as whole rows of the tile, non-temporally (8-byte stores of 32 bytes a row: 2.71 against 2.60 ms).
 //   - a loop instance per number of row tiles, chosen once per workgroup; full 256-slot blocks run fp8_tile.h's code.
-// Whole block at 4000 tokens, bf16: 2.87 ms with fp8_tile.h's grouped form, 2.60 with this one.
+// Whole block at 4000 tokens, bf16: 2.87 ms with fp8_tile.h's grouped form, 2.60 with this one.  The sums run over k in one order,
+// as fp8_tile.h's do: the same bits.  (The decode form of 16- and 32-row blocks adds four partial sums, one of each wavefront.)
 #pragma once
 
 #include "fp8_encode.h"

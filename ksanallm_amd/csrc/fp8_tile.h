@@ -542,9 +542,10 @@ __device__ __forceinline__ void fp8_tile_body(const Fp8TileParams& p, char* lds)
 
 // A 256-slot block of the grouped form with at most 160 tokens (deep_limit - 1) runs the 160-token tile's code: three stages
 // of 52 KiB instead of two of 64, because what bounds such a block is the stream of its weights, and only the activation
-// fragments that hold tokens are fetched.  160 is what the LDS has room for; that it lies above 128 matters: with 125
-// tokens per expert on average four experts in ten hold more than 128, and in 128-slot blocks each of those reads its
-// weights a second time (256 experts, hidden 7168, inter 2048, 4000 tokens, whole block: 3.18 -> 2.87 ms).
+// fragments that hold tokens are fetched.  160 is what the LDS has room for.  Such blocks come here as the ends of experts whose
+// mean lies above 240 slots - below it fp8_stream.h runs - and where a caller's few experts hold most of the slots.  (Measured
+// when all 256-slot blocks ran here: 256 experts, hidden 7168, inter 2048, 4000 tokens, whole block 3.18 ms in 128-slot blocks,
+// 2.87 with this form.)
 template <typename TO, bool GROUPED = false, int WM = 8>
 __global__ void __launch_bounds__(512, 1) fp8_tile_kernel(Fp8TileParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];  // fp8_tile_lds_bytes (the larger of both forms)

@@ -343,15 +343,16 @@ SplitKChoice select_w4a8_splitk(size_t m, size_t n) {
 
 using namespace ksq;
 
-// The same for block-fp8 experts (ksq_moe_fp8_blockwise_gemm): 16- and 32-row blocks stream through the split-K
-// kernel; from 16 rows per expert the MFMA tile kernel is faster even with most of a 128-row block padding (each of its
-// wavefronts multiplies the row tiles that hold rows), and 256-row blocks take over from 104 rows per expert, where
-// experts begin to need a second block of 128 and their weights a second pass (a 256-row block of at most 160 rows runs
-// on three stages like a 128-row block, so that the larger block costs nothing where it is not needed).  E = 256,
-// hidden 7168, inter 2048, top-8, whole call with 16- / 32- / 128- / 256-row blocks: 1.50 / 1.49 / 1.61 / - ms at 2 rows
-// per expert, 1.85 / 1.84 / 1.95 / - at 8, - / 1.95 / 1.98 / 2.02 at 12, - / 2.06 / 2.00 / 2.04 at 16, - / 3.18 / 2.12 /
-// 2.12 at 32, - / - / 2.31 / 2.33 at 64, - / - / 2.56 / 2.60 at 96, - / - / 2.85 / 2.75 at 112, - / - / 3.22 / 2.87 at 125,
-// - / - / 3.29 / 2.91 at 128, - / - / 3.85 / 3.40 at 160, - / - / 5.45 / 4.92 at 256.  (Other sizes: ksq_moe_fp8_block_m_sized.)
+// Row blocks of block-fp8 experts (ksq_moe_fp8_blockwise_gemm) where their sizes are not known: 16- and 32-row blocks stream
+// through the split-K kernel, 128- and 256-row blocks run a tile kernel.  The lines were measured with the MFMA tile kernel
+// (fp8_tile.h) for all of the latter; up to a mean of 15/16 of a block the streaming one (fp8_stream.h) runs there now, a sixth
+// faster in the mean at 16 slots per expert, a tenth at 64, and the lines hold for it (ksq_moe_fp8_row_block).  With fp8_tile.h: from
+// 16 rows per expert it is faster even with most of a 128-row block padding (each of its wavefronts multiplies the row tiles that
+// hold rows), and 256-row blocks take over from 104 rows per expert, where experts begin to need a second block of 128 and their
+// weights a second pass.  E = 256, hidden 7168, inter 2048, top-8, whole call with 16- / 32- / 128- / 256-row blocks: 1.50 / 1.49 /
+// 1.61 / - ms at 2 rows per expert, 1.85 / 1.84 / 1.95 / - at 8, - / 1.95 / 1.98 / 2.02 at 12, - / 2.06 / 2.00 / 2.04 at 16, - /
+// 3.18 / 2.12 / 2.12 at 32, - / - / 2.31 / 2.33 at 64, - / - / 2.56 / 2.60 at 96, - / - / 2.85 / 2.75 at 112, - / - / 3.22 / 2.87
+// at 125, - / - / 3.29 / 2.91 at 128, - / - / 3.85 / 3.40 at 160, - / - / 5.45 / 4.92 at 256.
 KSQ_EXPORT size_t ksq_moe_fp8_block_m(size_t numel, size_t E) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E;
@@ -370,6 +371,9 @@ KSQ_EXPORT size_t ksq_moe_fp8_block_m(size_t numel, size_t E) {
 // 120 61.4 / 65.0; 16, 1152, 512 at 120 78.9 / 82.2; 8, 7168, 2048 at 112 134.9 / 138.6, at 127 156.1 / 143.1.  Over 92
 // sizes of 4 to 160 experts the choice was at most 4.5 % behind the other one, the constant line at 104 slots 7 %.
 // (From 128 slots on every second expert has a second row block, and the line is the one above.)
+// These are times of the MFMA tile kernel; with the streaming one the choice was ahead or level at 104 and 116 slots in ten
+// sizes, 128- / 256-slot blocks at 116: 16 experts, hidden 4096, inter 2048 198 / 142 us, 32, 4096, 2048 274 / 225, 64, 2048, 1408
+// 221 / 191, where it takes 256; 8, 4096, 1536 86 / 92, 16, 2048, 1408 100 / 104, 32, 1024, 512 62 / 64.5, where it takes 128.
 KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidden, size_t inter) {
   const size_t block_m = ksq_moe_fp8_block_m(numel, E);
   if (block_m != 256 || numel / E >= 128) return block_m;
@@ -397,7 +401,7 @@ KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidde
 // 79, 16, 5120, 2048, top-1, at 6 40 / 75), of 48 or more experts rarely (128, 1024, 512, top-8, at 4 32 / 39; 160, 5120,
 // 1536, top-6, 144 / 84).
 //
-// From 16 slots on the lines are those of the tile kernel, for both kernels: 256-slot blocks gain nothing at 64 slots where
+// From 16 slots on the lines are those of ksq_moe_fp8_block_m_sized, for both tile kernels: 256-slot blocks gain nothing at 64 slots where
 // the routing is even (16, 4096, 2048 97.8 / 97.8) and leave half as many workgroups where it is not (logits with a spread
 // of 0.7 per expert, 128- / 256-slot blocks at 64 slots: 16, 2048, 1408 69 / 94; 8, 4096, 1536 81 / 105).
 KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {

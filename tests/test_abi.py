@@ -96,7 +96,7 @@ def test_w4a8_64_token_tiles_serve_whole_tiles_and_long_parts():
 
 
 def test_block_fp8_expert_blocks_follow_the_rounds_of_workgroups():
-    """Slots per expert below 104 or from 128 on: the rule of unknown sizes.  Between: 256-slot blocks where the experts that
+    """The block size from 16 slots per expert on, for both tile kernels.  Below 104 and from 128 on: the rule of unknown sizes.  Between: 256-slot blocks where the experts that
     need a second 128-slot block start another round of 256 workgroups in either GEMM."""
     from ksanallm_amd import lib as L
     lib = L.load()
