@@ -392,18 +392,19 @@ KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidde
 // 16 experts or more give at least every other CU a 256-column tile in both GEMMs, us in 32-slot / 128-slot blocks at 4 and
 // 8 slots, even routing: 256 experts, hidden 7168, inter 2048 1786 / 1653 and 1831 / 1695; 256, 1024, 512 132 / 100 and 148
 // 106; 64, 1024, 512 51 / 43 and 54 / 39; 16, 7168, 2048 132 / 125 and 136 / 126; 24, 2048, 768 (144 tiles) 48.7 / 38.3 and
-// 50.5 / 38.8; 32, 1024, 512 (128 tiles) 32.5 / 31.4 and 34.2 / 32.5; 16, 2048, 1408 (128) 47.5 / 45.3 and 49.5 / 46.2; 64,
-// 4096, 1024 160 / 172 and 174 / 169; but 8, 7168, 2048 (128) 78 / 82 and 80 / 83, with uneven routing 71 / 76 and 76 / 82;
-// 8, 4096, 1536 (96) 48.2 / 51.2 and 49.9 / 52.2, 16, 1024, 512 (64) 25.2 / 28.9 and 25.6 / 29.2.  (Below four: 32, 4096,
-// 2048 at 1 and 2 slots 106 / 118 and 138 / 139, 128, 2944, 768 at 1 118 / 122.)  Routing that prefers some experts keeps
-// the order (logits with a spread of 0.7 per expert, 4 to 15 slots, 25 sizes: 0.85 to 1.4 times as fast, 1.12 in the mean);
+// 50.5 / 38.8; 32, 1024, 512 (128 tiles) 32.5 / 31.4 and 34.2 / 32.5; 16, 2048, 1408 (128) 47.5 / 45.3 and 49.5 / 46.2; but
+// 8, 7168, 2048 (128) 78 / 82 and 80 / 83, with uneven routing 71 / 76 and 76 / 82; 8, 4096, 1536 (96) 48.2 / 51.2 and 49.9
+// / 52.2, 16, 1024, 512 (64) 25.2 / 28.9 and 25.6 / 29.2.  (Below four: 32, 4096, 2048 at 1 and 2 slots 106 / 118 and 138 /
+// 139, 128, 2944, 768 at 1 118 / 122.)  Over 44 sizes drawn between 16 and 160 experts, hidden 1024 to 7168, inter 512 to
+// 2048, at 4 to 12 slots, the row blocks are 0.98 to 1.44 times as fast as the decode form under even routing, 1.20 in the
+// mean, and 0.87 to 1.54, 1.21 in the mean, where routing prefers some experts (logits with a spread of 0.7 per expert);
 // where every token takes the same top-k of 16 or 32 experts too few tiles are left (16, 7168, 2048, top-2, at 8 slots 54 /
 // 79, 16, 5120, 2048, top-1, at 6 40 / 75), of 48 or more experts rarely (128, 1024, 512, top-8, at 4 32 / 39; 160, 5120,
 // 1536, top-6, 144 / 84).
 //
-// From 16 slots on the lines are those of ksq_moe_fp8_block_m_sized, for both tile kernels: 256-slot blocks gain nothing at 64 slots where
-// the routing is even (16, 4096, 2048 97.8 / 97.8) and leave half as many workgroups where it is not (logits with a spread
-// of 0.7 per expert, 128- / 256-slot blocks at 64 slots: 16, 2048, 1408 69 / 94; 8, 4096, 1536 81 / 105).
+// From 16 slots on the lines are those of ksq_moe_fp8_block_m_sized, for both tile kernels: 256-slot blocks gain nothing at
+// 64 slots where the routing is even (16, 4096, 2048 97.8 / 97.8) and leave half as many workgroups where it is not (logits
+// with a spread of 0.7 per expert, 128- / 256-slot blocks at 64 slots: 16, 2048, 1408 69 / 94; 8, 4096, 1536 81 / 105).
 KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E, tiles = E * div_up(2 * inter < hidden ? 2 * inter : hidden, 256);
