@@ -391,7 +391,7 @@ KSQ_EXPORT size_t ksq_moe_fp8_block_m_sized(size_t numel, size_t E, size_t hidde
 // (fp8_stream.h) counted in.  From four slots per expert on its row blocks beat the 32-row blocks of the decode form where
 // 16 experts or more give at least every other CU a 256-column tile in both GEMMs, us in 32-slot / 128-slot blocks at 4 and
 // 8 slots, even routing: 256 experts, hidden 7168, inter 2048 1786 / 1653 and 1831 / 1695; 256, 1024, 512 132 / 100 and 148
-// 106; 64, 1024, 512 51 / 43 and 54 / 39; 16, 7168, 2048 132 / 125 and 136 / 126; 24, 2048, 768 (144 tiles) 48.7 / 38.3 and
+// / 106; 64, 1024, 512 51 / 43 and 54 / 39; 16, 7168, 2048 132 / 125 and 136 / 126; 24, 2048, 768 (144 tiles) 48.7 / 38.3 and
 // 50.5 / 38.8; 32, 1024, 512 (128 tiles) 32.5 / 31.4 and 34.2 / 32.5; 16, 2048, 1408 (128) 47.5 / 45.3 and 49.5 / 46.2; but
 // 8, 7168, 2048 (128) 78 / 82 and 80 / 83, with uneven routing 71 / 76 and 76 / 82; 8, 4096, 1536 (96) 48.2 / 51.2 and 49.9
 // / 52.2, 16, 1024, 512 (64) 25.2 / 28.9 and 25.6 / 29.2.  (Below four: 32, 4096, 2048 at 1 and 2 slots 106 / 118 and 138 /
