@@ -69,14 +69,6 @@ constexpr int fp8_stream_area_max(int rt_max) {
 // ... then the block's slot ids, then the weight scales of the tile's two 128-column blocks
 constexpr size_t fp8_stream_lds_bytes(int rt_max, size_t kb_max) { return fp8_stream_area_max(rt_max) + 1024 + 2 * kb_max * 4; }
 
-// a wave-uniform pointer in scalar registers (64-bit products are formed on the vector unit)
-template <typename P>
-__device__ __forceinline__ P* scalar_ptr(P* ptr) {
-  const uint64_t v = reinterpret_cast<uint64_t>(ptr);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-  return reinterpret_cast<P*>(static_cast<uint64_t>(hi) << 32 | lo);
-}
-
 // PAIRED: gate / up weights [2 * inter, K], and the result is the second GEMM's quantized input: a wavefront's strips are a
 // gate strip and the matching up strip, a workgroup covers 128 channels of the activation, one quantization group, and stores
 // e4m3(T(silu(T(gate)) * T(up)) / scale) with the group's scale - the bits of the plain GEMM followed by the quantizer with

@@ -120,6 +120,14 @@ __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) {
   return static_cast<uint32_t>(lo) | (static_cast<uint32_t>(hi) << 16);
 }
 
+// a wave-uniform pointer in scalar registers (64-bit products are formed on the vector unit)
+template <typename P>
+__device__ __forceinline__ P* scalar_ptr(P* ptr) {
+  const uint64_t v = reinterpret_cast<uint64_t>(ptr);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+  return reinterpret_cast<P*>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
 inline size_t div_up(size_t a, size_t b) { return (a + b - 1) / b; }
 inline size_t round_up(size_t a, size_t b) { return div_up(a, b) * b; }
 

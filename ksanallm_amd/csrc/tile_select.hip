@@ -139,6 +139,17 @@ SplitKChoice select_splitk_grouped(size_t block_m, size_t blocks, size_t numel, 
   return c;
 }
 
+// 32-slot blocks: the streaming kernel, where its workgroups of 256 columns come to three quarters of the CUs.  Whole int4 block,
+// decode kernel / streaming kernel in us (experts, top-k, hidden, inter, tokens): 256, 8, 7168, 2048 at 512 tokens 1140 / 1066, at
+// 1024 tokens 1690 / 1542; 128, 8, 4480, 640 at 352 210 / 177; 64, 8, 6656, 512 at 128 110 / 101; 32, 8, 3328, 512 at 124 (192
+// workgroups in the first GEMM) 65.6 / 59.4; 16, 2, 4096, 1792 at 128 (224) 59.5 / 59.0.  Fewer leave the chip to a few long
+// workgroups: 8, 2, 4096, 1536 at 96 (120) 44.6 / 50.8; 16, 2, 1024, 512 at 300 (108) 30.4 / 33.2; 16, 2, 2432, 512 at 144 (68)
+// 33.1 / 39.4.  (Workgroups of 128 columns instead: 44.5, 30.0 and 35.8, and slower than the decode kernel above.)
+bool use_w4a16_stream(size_t block_m, size_t blocks, size_t n, size_t k) {
+  return block_m == 32 && blocks * div_up(n, 256) >= static_cast<size_t>(kNumCU) * 3 / 4 &&
+         n * k <= (size_t(1) << 36);  // 32-bit offsets into an expert's scales
+}
+
 // Regime switch.  Up to 32 rows the split-K (decode) kernel; above, the MFMA tile kernel - except while the problem is
 // small: the tile kernel has a floor of 17-22 us (a workgroup's prologue, the fp32 partial tiles of the cut along K and
 // the pass that sums them), and the decode kernel run over blocks of 32 rows, each streaming the weights again (out of
@@ -416,16 +427,17 @@ KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, s
 }
 
 // Rows per expert block for numel routed (token, slot) pairs over E experts.  Replaces the M thresholds of
-// InvokeFusedMoe (16 / 32 / 64 rows by token count): below about 40 rows per expert the weights are streamed once per
+// InvokeFusedMoe (16 / 32 / 64 rows by token count): below 48 rows per expert the weights are streamed once per
 // 16- or 32-row block (HBM-bound); above, the MFMA tile kernel takes 256-row blocks, of which it multiplies the row
 // tiles that hold rows (an instance of its main loop per count), so that an expert's weights are dequantized once
-// however many of the 256 rows it fills.  E = 256, hidden 7168, inter 2048, top-8, whole call with 32- / 128- /
-// 256-row blocks: 1.97 / 2.34 / 2.37 ms at 32 rows per expert, 2.41 / 2.40 / 2.39 at 40, 2.58 / 2.46 / 2.45 at 48,
-// 3.21 / 2.60 / 2.55 at 64, 4.39 / 3.06 / 3.02 at 96, 4.96 / 3.44 / 3.30 at 112, 5.60 / 4.40 / 3.57 at 128.
+// however many of the 256 rows it fills.  E = 256, hidden 7168, inter 2048, top-8, whole call with 32- / 256-row
+// blocks: 1.54 / 2.37 ms at 32 rows per expert, 1.88 / 2.15 at 40, 2.53 / 2.31 at 64, 3.45 / 2.69 at 94; 128 experts, hidden
+// 4096, inter 768 297 / 288 us at 48; 64, 2048, 1408 161 / 180 at 48, 249 / 215 at 96; 16, 5504, 768 72 / 100 at 47; 8, 4096, 1536
+// 56 / 80 at 48, 81 / 99 at 100.  128-row blocks are not ahead of 256-row ones anywhere (4.40 / 3.57 ms at 128 rows).
 KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E;
-  if (per_expert >= 40) return 256;
+  if (per_expert >= 48) return 256;
   return per_expert < 16 ? 16 : 32;
 }
 

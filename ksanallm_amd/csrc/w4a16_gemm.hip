@@ -7,6 +7,7 @@
 
 #include "tile_select.h"
 #include "w4a16_splitk.h"
+#include "w4a16_stream.h"
 #include "w4a16_tile.h"
 
 namespace ksq {
@@ -482,7 +483,14 @@ int moe_w4a16_gemm_impl(const char* fn, bool fuse_silu, void* out, const void* x
   p.num_experts = static_cast<uint32_t>(E);
   p.x_bytes = static_cast<uint32_t>(x_rows * k * 2);
   // about numel/block_m + E/2 of the aligned blocks hold rows; K is never split across workgroups here
-  SplitKChoice c = select_splitk_grouped(block_m, few ? numel : std::min(cap_blocks, numel / block_m + E / 2 + 1), numel, n, k);
+  const size_t blocks = few ? numel : std::min(cap_blocks, numel / block_m + E / 2 + 1);
+  if (use_w4a16_stream(block_m, blocks, n, k)) {
+    p.nibble_mask = 0x000f000fu;
+    p.magic2 = dtype == KSQ_F16 ? F16::kMagic2 : BF16::kMagic2;
+    if (int rc = launch_w4a16_stream(p, fuse_silu, static_cast<uint32_t>(cap_blocks), dtype, as_stream(stream))) return rc;
+    return check_launch(fn);
+  }
+  SplitKChoice c = select_splitk_grouped(block_m, blocks, numel, n, k);
   if (fuse_silu) {
     if (c.nt < 2) c.nt = 2;  // a workgroup holds gate and up tiles in pairs
     p.pair_tiles = static_cast<uint32_t>(n / 32);

@@ -294,6 +294,37 @@ def test_grouped_tile_kernel_every_count_of_live_row_tiles(ops, oracle, dtype, b
     H.check_gemm(c1, ref1, dtype, "grouped tile kernel, %d-row blocks" % bm, weights_rounded=True)
 
 
+@pytest.mark.parametrize("dtype", [H.F16, H.BF16])
+@pytest.mark.parametrize("kt", [1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 12])
+def test_grouped_streaming_kernel_over_its_ring(ops, oracle, dtype, kt):
+    """32-slot blocks in 192 and more workgroups of 256 columns run the kernel that streams the weights through a ring of four
+    k-tiles and x by halves of two: every way its loop can end, one and two row tiles, experts with one and with several blocks,
+    a last workgroup with a few columns; the bound is the decode form's, whose weights are exact too.  With silu*mul in the
+    epilogue: the bits of the two launches."""
+    from ksanallm_amd import lib as L
+    rows = [1, 16, 17, 32, 33, 48, 49, 64, 65, 15, 31, 100]
+    E, T, k = len(rows), sum(rows), 128 * kt
+    inter = 1312
+    assert (T // 32 + E // 2 + 1) * -(-2 * inter // 256) >= 192
+    d = make_moe(oracle, 6100 + kt, E, k, inter, T, 1, 128, dtype)
+    ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
+    ids = ids[torch.randperm(T, generator=H.gen(78))].reshape(T, 1).contiguous()
+    w13p = ops.repack_weight(d["w13"].cuda(), L.SRC_MOE_NK, E, k, 2 * inter)
+    s13p = ops.repack_scales(d["s13"].cuda(), L.SCALE_NG, E, k, 2 * inter, 128)
+    al = ops.moe_align_block_size(ids.cuda(), E, 32)
+    for tw in (None, d["tw"]):
+        out = torch.full((T, 2 * inter), float("nan"), dtype=d["x"].dtype, device="cuda")
+        ops.moe_w4a16_gemm(d["x"].cuda(), w13p, s13p, None if tw is None else tw.cuda().reshape(-1), *al, T, 1, E, 2 * inter, k, 128,
+                           32, out=out)
+        ref = oracle.moe_w4a16_gemm(H.bits_of(d["x"]), d["w13"].numpy(), H.bits_of(d["s13"]), ids.numpy(), d["tw"].numpy(), 1, 128,
+                                    tw is not None, dtype)
+        H.check_gemm(out, ref, dtype, "streaming kernel, %d k-tiles" % kt)
+        if tw is None:
+            one = torch.full((T, inter), float("nan"), dtype=d["x"].dtype, device="cuda")
+            ops.moe_w4a16_gate_up_silu(d["x"].cuda(), w13p, s13p, *al, T, 1, E, 2 * inter, k, 128, 32, out=one)
+            assert torch.equal(one.view(torch.int16), ops.silu_and_mul(out).view(torch.int16))
+
+
 @pytest.mark.parametrize("T", [1, 64, 2048])
 def test_moe_block_deepseek_shape(ops, oracle, T):
     """256 experts, hidden 7168, inter 2048, top-8; weights for all experts are generated but only touched ones
