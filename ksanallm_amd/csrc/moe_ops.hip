@@ -4,83 +4,11 @@
 namespace ksq {
 namespace {
 
-constexpr int kAlignThreads = 1024;
+// Stable counting sort by expert: positions inside an expert ascend with the flat index, every expert's slots start at a
+// multiple of block_m, slots without an id hold numel.
 
-// Stable counting sort by expert in one workgroup.
-//   chunk c (one thread) owns ids [c*per, (c+1)*per); cnt[c+1][e] = #ids == e in chunk c  (global scratch)
-//   column scan over chunks turns cnt[c][e] into "ids == e before chunk c";  padded totals are scanned over experts
-//   in LDS; every chunk then places its ids in order, so positions inside an expert ascend with the flat index.
-__global__ void __launch_bounds__(kAlignThreads) moe_align_kernel(const int32_t* __restrict__ ids, uint32_t numel,
-                                                                  uint32_t E, uint32_t block_m, uint32_t capacity,
-                                                                  int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids,
-                                                                  int32_t* __restrict__ num_post_pad,
-                                                                  int32_t* __restrict__ cnt, uint32_t chunks,
-                                                                  uint32_t per) {
-  extern __shared__ int32_t lds[];  // [2][E_pad + 1] ping-pong scan buffers
-  const uint32_t tid = threadIdx.x;
-  const uint32_t EP = E + 1;
-  int32_t* scan_a = lds;
-  int32_t* scan_b = lds + EP;
-
-  // fill: every slot starts as padding
-  for (uint32_t i = tid; i < capacity; i += kAlignThreads) sorted[i] = static_cast<int32_t>(numel);
-  // clear counters
-  for (uint32_t i = tid; i < (chunks + 1) * E; i += kAlignThreads) cnt[i] = 0;
-  __syncthreads();
-
-  const uint32_t begin = tid * per;
-  const uint32_t end = (begin + per < numel) ? begin + per : numel;
-  if (tid < chunks) {
-    for (uint32_t i = begin; i < end; ++i) {
-      uint32_t e = static_cast<uint32_t>(ids[i]);
-      if (e < E) cnt[(tid + 1) * E + e] += 1;
-    }
-  }
-  __syncthreads();
-
-  // per expert: running sum over chunks
-  for (uint32_t e = tid; e < E; e += kAlignThreads) {
-    int32_t run = 0;
-    for (uint32_t c = 1; c <= chunks; ++c) {
-      run += cnt[c * E + e];
-      cnt[c * E + e] = run;
-    }
-    // cnt[chunks][e] == total of expert e ; padded size goes into the scan buffer (shifted by one: exclusive scan)
-    scan_a[e + 1] = (run + static_cast<int32_t>(block_m) - 1) / static_cast<int32_t>(block_m) * static_cast<int32_t>(block_m);
-  }
-  if (tid == 0) scan_a[0] = 0;
-  __syncthreads();
-
-  // inclusive Hillis-Steele scan over EP entries -> scan[e] = first slot of expert e, scan[E] = padded total
-  int32_t* src = scan_a;
-  int32_t* dst = scan_b;
-  for (uint32_t off = 1; off < EP; off <<= 1) {
-    for (uint32_t i = tid; i < EP; i += kAlignThreads) dst[i] = src[i] + (i >= off ? src[i - off] : 0);
-    __syncthreads();
-    int32_t* t = src;
-    src = dst;
-    dst = t;
-  }
-  const int32_t* first = src;
-
-  if (tid == 0) num_post_pad[0] = first[E];
-  for (uint32_t e = tid; e < E; e += kAlignThreads)
-    for (int32_t s = first[e]; s < first[e + 1]; s += static_cast<int32_t>(block_m)) expert_ids[s / static_cast<int32_t>(block_m)] = static_cast<int32_t>(e);
-
-  if (tid < chunks) {
-    for (uint32_t i = begin; i < end; ++i) {
-      uint32_t e = static_cast<uint32_t>(ids[i]);
-      if (e < E) {
-        int32_t r = cnt[tid * E + e];
-        cnt[tid * E + e] = r + 1;
-        sorted[first[e] + r] = static_cast<int32_t>(i);
-      }
-    }
-  }
-}
-
-// ---- the same sort for up to 1024 ids (decode batches), one id per thread, everything in LDS: no counter ever makes
-// a round trip through global memory, which is what the launch above spends most of its microseconds on.
+// ---- up to 1024 ids (decode batches), one workgroup, one id per thread, everything in LDS: no counter ever makes a round
+// trip through global memory.
 //   r        = lower lanes of the wavefront with the same id (64 readlanes)
 //   wcnt[w][e] = ids == e in wavefront w, then, scanned over w, ids == e in the wavefronts before w
 //   position = first[e] + wcnt[w][e] + r : ascending with the flat index inside an expert, as above
@@ -248,6 +176,104 @@ __global__ void __launch_bounds__(kChunkThreads) moe_align_place_kernel(const in
   }
 }
 
+// ---- the same sort in one launch: every workgroup counts all ids itself, those before its chunk and the others apart, instead of
+// waiting for a launch that counts them (32768 ids are 128 KiB out of the L2 and 32 LDS atomics a thread); it scans the padded
+// totals and places its own 256 ids.  Inside a wavefront an id's rank is the number of lower lanes that hold the same id, found
+// by one ballot per bit of the id; the four wavefronts take turns.  The slots of the padding are filled by whoever is at the
+// expert, no launch ahead of the others.
+// us, graph-replayed, before / this one: 1120 ids over 64 experts 24.4 / 4.4 and 1536 over 256 34.9 / 5.5 (one workgroup with its
+// counters in global memory), 4096 over 256 14.7 / 5.1, 32000 over 256 20.2 / 9.6, 64000 over 256 28.3 / 15.2 (the two launches below).
+constexpr int kOnePassThreads = 1024;
+constexpr uint32_t kOnePassChunk = 256;
+
+__global__ void __launch_bounds__(kOnePassThreads) moe_align_one_pass_kernel(const int32_t* __restrict__ ids, uint32_t numel, uint32_t E,
+                                                                             uint32_t block_m, uint32_t capacity,
+                                                                             int32_t* __restrict__ sorted, int32_t* __restrict__ expert_ids,
+                                                                             int32_t* __restrict__ num_post_pad) {
+  extern __shared__ int32_t lds[];  // next[E] total[E] first[E + 1]
+  __shared__ int32_t wave_sum[kOnePassThreads / 64];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int32_t* next = lds;
+  int32_t* total = lds + E;
+  int32_t* first = lds + 2 * E;
+  const int32_t bm = static_cast<int32_t>(block_m);
+  const uint32_t begin = blockIdx.x * kOnePassChunk;
+
+  for (uint32_t e = tid; e < 2 * E; e += kOnePassThreads) lds[e] = 0;
+  // the chunk's own id of this thread, on its way while the others are counted
+  const uint32_t own = begin + tid;
+  uint32_t id = (tid < kOnePassChunk && own < numel) ? static_cast<uint32_t>(ids[own]) : 0xffffffffu;
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t i = tid; i < numel; i += kOnePassThreads) {
+    const uint32_t e = static_cast<uint32_t>(ids[i]);
+    int32_t* const counts = i < begin ? next : total;  // (the same for the whole wavefront)
+    // sixty-four ids of one expert are one addition instead of sixty-four, one after the other, to one place
+    const uint64_t active = __builtin_amdgcn_ballot_w64(true);
+    if (__builtin_amdgcn_ballot_w64(e == static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(e))) == active) {
+      if (lane == 0 && e < E) atomicAdd(&counts[e], __builtin_popcountll(active));
+    } else if (e < E) {
+      atomicAdd(&counts[e], 1);
+    }
+  }
+  __syncthreads();
+
+  // exclusive scan of the padded totals: every thread a run of experts, then over lanes, then over wavefronts
+  const uint32_t run = (E + kOnePassThreads - 1) / kOnePassThreads, e0 = tid * run;
+  int32_t sum = 0;
+  for (uint32_t e = e0; e < e0 + run && e < E; ++e) {
+    const int32_t t = total[e] + next[e];
+    total[e] = t;
+    sum += (t + bm - 1) / bm * bm;
+  }
+  int32_t scan = sum;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int32_t v = __shfl_up(scan, off);
+    if (lane >= static_cast<uint32_t>(off)) scan += v;
+  }
+  if (lane == 63) wave_sum[wave] = scan;
+  __syncthreads();
+  int32_t at = scan - sum;
+  for (uint32_t w = 0; w < wave; ++w) at += wave_sum[w];
+  for (uint32_t e = e0; e < e0 + run && e < E; ++e) {
+    first[e] = at;
+    next[e] += at;
+    at += (total[e] + bm - 1) / bm * bm;
+    if (e == E - 1) first[E] = at;
+  }
+  __syncthreads();
+
+  // this workgroup's ids
+  if (id >= E) id = 0xffffffffu;
+  uint64_t same = ~0ull;  // lanes of the wavefront with this id
+  for (uint32_t b = 1; b < E; b <<= 1) {
+    const uint64_t m = __builtin_amdgcn_ballot_w64((id & b) != 0);
+    same &= (id & b) ? m : ~m;
+  }
+  same &= __builtin_amdgcn_ballot_w64(id != 0xffffffffu);
+  const int32_t rank = __builtin_popcountll(same & ((1ull << lane) - 1));
+  for (uint32_t w = 0; w < kOnePassChunk / 64; ++w) {
+    if (wave == w && id != 0xffffffffu) {
+      const int32_t pos = next[id] + rank;
+      sorted[pos] = static_cast<int32_t>(own);
+      if (same >> lane == 1) next[id] = pos + 1;  // (the last lane with this id; every lane has read the counter by then)
+    }
+    __syncthreads();
+  }
+
+  // the padding behind every expert's slots and behind the last expert, and the blocks' experts
+  const uint32_t waves = gridDim.x * (kOnePassThreads / 64);
+  for (uint32_t e = blockIdx.x * (kOnePassThreads / 64) + wave; e < E; e += waves) {
+    const int32_t from = first[e], to = first[e + 1];
+    for (int32_t p = from + total[e] + static_cast<int32_t>(lane); p < to; p += 64) sorted[p] = static_cast<int32_t>(numel);
+    for (int32_t b = from / bm + static_cast<int32_t>(lane); b < to / bm; b += 64) expert_ids[b] = static_cast<int32_t>(e);
+  }
+  for (uint32_t p = static_cast<uint32_t>(first[E]) + blockIdx.x * kOnePassThreads + tid; p < capacity; p += gridDim.x * kOnePassThreads)
+    sorted[p] = static_cast<int32_t>(numel);
+  if (blockIdx.x == 0 && tid == 0) num_post_pad[0] = first[E];
+}
+
 void chunk_geometry(size_t numel, uint32_t* chunks, uint32_t* per) {
   size_t c = div_up(numel, kChunkThreads);
   if (c > kMaxChunks) c = kMaxChunks;
@@ -256,8 +282,8 @@ void chunk_geometry(size_t numel, uint32_t* chunks, uint32_t* per) {
   *chunks = static_cast<uint32_t>(div_up(numel, p));
 }
 
-// ids from which the two-launch sort is used
-constexpr size_t kParallelAlignFrom = 2048;
+// ids up to which the one-launch sort is used (256 workgroups), the two-launch sort above
+constexpr size_t kOnePassUpTo = 256 * kOnePassChunk;
 
 // 8 elements per thread.  A workgroup covers 2^log2p column pieces of 256 >> log2p rows; the row comes from
 // blockIdx.y/z, the column piece from blockIdx.x, so that no index is divided (a 64-bit division is some fifty
@@ -586,14 +612,6 @@ __global__ void __launch_bounds__(256) grouped_topk_kernel(const void* __restric
   }
 }
 
-void align_geometry(size_t numel, uint32_t* chunks, uint32_t* per) {
-  size_t c = div_up(numel, 8);
-  if (c < 1) c = 1;
-  if (c > kAlignThreads) c = kAlignThreads;
-  *chunks = static_cast<uint32_t>(c);
-  *per = static_cast<uint32_t>(div_up(numel, c));
-}
-
 }  // namespace
 }  // namespace ksq
 
@@ -606,11 +624,8 @@ KSQ_EXPORT size_t ksq_moe_align_capacity(size_t numel, size_t E, size_t block_m)
 
 KSQ_EXPORT size_t ksq_moe_align_scratch_bytes(size_t numel, size_t E) {
   uint32_t chunks, per;
-  align_geometry(numel, &chunks, &per);
-  size_t bytes = (static_cast<size_t>(chunks) + 1) * E * sizeof(int32_t);
-  chunk_geometry(numel, &chunks, &per);
-  const size_t parallel = static_cast<size_t>(chunks) * E * sizeof(int32_t);
-  return bytes > parallel ? bytes : parallel;
+  chunk_geometry(numel ? numel : 1, &chunks, &per);
+  return static_cast<size_t>(chunks) * E * sizeof(int32_t);
 }
 
 KSQ_EXPORT int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_t block_m, void* sorted_ids,
@@ -622,18 +637,6 @@ KSQ_EXPORT int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_
   if (block_m == 0 || block_m > 1024) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: block_m %zu outside 1..1024", fn, block_m);
   const size_t cap = ksq_moe_align_capacity(numel, E, block_m);
   if (cap > 0x7fffffffull) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: too many ids", fn);
-  uint32_t chunks, per;
-  if (numel >= kParallelAlignFrom) {
-    chunk_geometry(numel, &chunks, &per);
-    moe_align_count_kernel<<<chunks, kChunkThreads, E * sizeof(int32_t), as_stream(stream)>>>(
-        static_cast<const int32_t*>(topk_ids), static_cast<uint32_t>(numel), static_cast<uint32_t>(E),
-        static_cast<uint32_t>(cap), static_cast<int32_t*>(sorted_ids), static_cast<int32_t*>(scratch), per);
-    moe_align_place_kernel<<<chunks, kChunkThreads, (3 * E + 2 + kChunkThreads) * sizeof(int32_t), as_stream(stream)>>>(
-        static_cast<const int32_t*>(topk_ids), static_cast<uint32_t>(numel), static_cast<uint32_t>(E),
-        static_cast<uint32_t>(block_m), static_cast<int32_t*>(sorted_ids), static_cast<int32_t*>(expert_ids),
-        static_cast<int32_t*>(num_post_pad), static_cast<const int32_t*>(scratch), chunks, per);
-    return check_launch(fn);
-  }
   if (numel <= 1024 && div_up(numel, 64) * E <= 12288) {  // one id per thread, counters in LDS (at most 48 KiB of them)
     const size_t small_lds = (div_up(numel, 64) * E + 2 * (E + 1)) * sizeof(int32_t);
     const unsigned threads = numel <= 256 ? 256u : 1024u;
@@ -643,13 +646,23 @@ KSQ_EXPORT int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_
         static_cast<int32_t*>(expert_ids), static_cast<int32_t*>(num_post_pad));
     return check_launch(fn);
   }
-  align_geometry(numel, &chunks, &per);
-  const size_t lds = 2 * (E + 1) * sizeof(int32_t);
-  moe_align_kernel<<<1, kAlignThreads, lds, as_stream(stream)>>>(
+  if (numel <= kOnePassUpTo) {
+    const unsigned wgs = static_cast<unsigned>(div_up(numel, kOnePassChunk));
+    moe_align_one_pass_kernel<<<wgs, kOnePassThreads, (3 * E + 1) * sizeof(int32_t), as_stream(stream)>>>(
+        static_cast<const int32_t*>(topk_ids), static_cast<uint32_t>(numel), static_cast<uint32_t>(E),
+        static_cast<uint32_t>(block_m), static_cast<uint32_t>(cap), static_cast<int32_t*>(sorted_ids),
+        static_cast<int32_t*>(expert_ids), static_cast<int32_t*>(num_post_pad));
+    return check_launch(fn);
+  }
+  uint32_t chunks, per;
+  chunk_geometry(numel, &chunks, &per);
+  moe_align_count_kernel<<<chunks, kChunkThreads, E * sizeof(int32_t), as_stream(stream)>>>(
       static_cast<const int32_t*>(topk_ids), static_cast<uint32_t>(numel), static_cast<uint32_t>(E),
-      static_cast<uint32_t>(block_m), static_cast<uint32_t>(cap), static_cast<int32_t*>(sorted_ids),
-      static_cast<int32_t*>(expert_ids), static_cast<int32_t*>(num_post_pad), static_cast<int32_t*>(scratch), chunks,
-      per);
+      static_cast<uint32_t>(cap), static_cast<int32_t*>(sorted_ids), static_cast<int32_t*>(scratch), per);
+  moe_align_place_kernel<<<chunks, kChunkThreads, (3 * E + 2 + kChunkThreads) * sizeof(int32_t), as_stream(stream)>>>(
+      static_cast<const int32_t*>(topk_ids), static_cast<uint32_t>(numel), static_cast<uint32_t>(E),
+      static_cast<uint32_t>(block_m), static_cast<int32_t*>(sorted_ids), static_cast<int32_t*>(expert_ids),
+      static_cast<int32_t*>(num_post_pad), static_cast<const int32_t*>(scratch), chunks, per);
   return check_launch(fn);
 }
 

@@ -72,6 +72,22 @@ def test_align_many_ids_ragged(ops, oracle, numel, E, bm):
     np.testing.assert_array_equal(e.cpu().numpy()[:nb], eo[:nb])
 
 
+@pytest.mark.parametrize("numel,E,bm", [(1025, 1, 16), (1280, 65, 32), (1281, 64, 128), (700, 2000, 16), (4000, 1024, 256),
+                                        (5000, 1025, 16), (65536, 256, 32), (65537, 256, 32)])
+def test_align_in_one_launch_at_the_edges(ops, oracle, numel, E, bm):
+    """Chunks that just end, a last chunk of one id, expert counts around what a wavefront and a workgroup scan at once, many ids of
+    one expert, experts without any, and the first count of ids that takes two launches."""
+    g = H.gen(numel + E)
+    ids = torch.randint(-1, E + 1, (numel,), generator=g, dtype=torch.int32)
+    ids[torch.rand((numel,), generator=g) < 0.3] = E // 2
+    ids[ids == E // 3] = E
+    s, e, npp = ops.moe_align_block_size(ids.cuda(), E, bm)
+    so, eo, nppo = oracle.moe_align(ids.numpy(), E, bm)
+    assert npp.item() == nppo
+    np.testing.assert_array_equal(s.cpu().numpy(), so)
+    np.testing.assert_array_equal(e.cpu().numpy()[:nppo // bm], eo[:nppo // bm])
+
+
 @pytest.mark.parametrize("T,E,topk", [(1, 256, 8), (77, 256, 8), (5, 60, 4), (9, 1000, 6)])
 def test_topk_softmax(ops, oracle, T, E, topk):
     g = H.gen(T + E)
