@@ -182,7 +182,7 @@ __global__ void __launch_bounds__(kChunkThreads) moe_align_place_kernel(const in
 // by one ballot per bit of the id; the four wavefronts take turns.  The slots of the padding are filled by whoever is at the
 // expert, no launch ahead of the others.
 // us, graph-replayed, before / this one: 1120 ids over 64 experts 24.4 / 4.4 and 1536 over 256 34.9 / 5.5 (one workgroup with its
-// counters in global memory), 4096 over 256 14.7 / 5.1, 32000 over 256 20.2 / 9.6, 64000 over 256 28.3 / 15.2 (the two launches below).
+// counters in global memory), 4096 over 256 14.7 / 5.1, 32000 over 256 20.2 / 11.3, 64000 over 256 28.3 / 18.9 (the two launches below).
 constexpr int kOnePassThreads = 1024;
 constexpr uint32_t kOnePassChunk = 256;
 

@@ -46,6 +46,8 @@ TilePlan plan_mfma_tile(size_t m, size_t n, size_t k);
 // and its grid (kt_per_split counts 128-deep k-blocks).
 bool use_fp8_tile(size_t m, size_t n, size_t k);
 TilePlan plan_fp8_tile(size_t m, size_t n, size_t k);
+// ... and the decode form's strips of 16 columns per workgroup: 1, 2 or 4
+int fp8_decode_strips(size_t m, size_t n, size_t k);
 // k-blocks of a workgroup that computes the least
 size_t fp8_plan_kb(const TilePlan& plan, size_t k);
 // whether the streaming tile kernel (fp8_stream.h) takes the place of the MFMA tile kernel under that plan

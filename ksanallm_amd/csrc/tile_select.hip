@@ -272,6 +272,32 @@ bool use_w4a8_tile(size_t m, size_t n, size_t k) {
   return true;
 }
 
+// Blockwise FP8, decode form: strips of 16 columns per workgroup.
+// One strip up to 32 tokens while every workgroup has a CU to itself: halving their number leaves CUs idle.  GEMM alone in us, two
+// strips / one: n = 4096, k = 14336 at 2, 16, 32 rows 13.4 / 12.2, 16.8 / 13.4, 22.0 / 19.1; n = k = 4096 at 16 6.4 / 5.8; n = 2048,
+// k = 7168 at 16 9.0 / 7.6; n = 4224 (264 strips), k = 4096 at 16 6.4 / 8.4.
+// Above, the activation fragments are as large as the weight fragments: two strips share them once there are several
+// tokens, or when K is the long dimension (few strips, long streams).  With up to 8 tokens and no long K it is the last round
+// of the CUs that tells: n = 13312, k = 4096 (416 workgroups of two strips) at 1 and 8 rows 10.9 / 11.3, 11.5 / 12.6, n = 24576,
+// k = 1536 (768) at 8 9.8 / 10.9, but n = 18432, k = 7168 (576) 24.4 / 22.7, 25.4 / 25.0 and n = 28672, k = 4096 (896) 21.1 / 19.7;
+// n = 8192, k = 4096, one round, 7.3 / 6.9 at one row, 7.3 / 7.6 at 8; n = 5120, k = 5120 6.6 / 6.8, 7.0 / 8.2.
+int fp8_decode_strips(size_t m, size_t n, size_t k) {
+  const size_t pairs = n / 32, rounds = div_up(pairs, kNumCU);
+  int nt;
+  if (m <= 32 && n <= 16 * static_cast<size_t>(kNumCU))
+    nt = 1;
+  else if (m > 8 || k > n)
+    nt = 2;
+  else if (rounds == 1)
+    nt = m >= 5 ? 2 : 1;
+  else
+    nt = pairs * 10 >= rounds * kNumCU * (rounds == 2 ? 8 : 9) ? 2 : 1;
+  // several blocks of 32 tokens (small problems above 32 tokens): four strips share a block's activation fragments while
+  // the blocks together still give every other CU a workgroup
+  if (m > 32 && n % 64 == 0 && n / 64 * div_up(m, 32) >= 128) nt = 4;
+  return n % (16 * nt) == 0 ? nt : 1;
+}
+
 TilePlan plan_fp8_tile(size_t m, size_t n, size_t k) {
   TilePlan t{};
   // 128-token tiles where 256-token ones would be half padding (the weights are then fetched once per 128 tokens);
@@ -492,8 +518,7 @@ KSQ_EXPORT int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype
       const int mt = m <= 16 ? 1 : 2;
       const int waves = 4;
       d->kernel = KSQ_KERNEL_SPLITK_WAVE;
-      int nt = ((m > 8 || k > n) && n % 32 == 0) ? 2 : 1;
-      if (m > 32 && n % 64 == 0 && n / 64 * div_up(m, 32) >= 128) nt = 4;  // as fp8_blockwise_gemm.hip's dispatch
+      const int nt = fp8_decode_strips(m, n, k);
       d->block_m = 16 * mt;
       d->block_n = 16 * nt;
       d->block_k = 128;
