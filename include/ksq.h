@@ -403,7 +403,8 @@ enum { KSQ_KIND_W4A16 = 0, KSQ_KIND_FP8_BLOCKWISE = 1, KSQ_KIND_MOE_W4A16 = 2, K
 enum {
   KSQ_KERNEL_SPLITK_WAVE = 0,
   KSQ_KERNEL_MFMA_TILE = 1,
-  KSQ_KERNEL_STREAM_TILE = 2 /* block fp8: the MFMA tile kernel's grid, weights through registers */
+  KSQ_KERNEL_STREAM_TILE = 2 /* block fp8: the MFMA tile kernel's grid, weights through registers (W4A8's form of it reports
+                                MFMA_TILE, whose grid and bits it has) */
 };
 
 typedef struct ksq_tile_desc {

@@ -55,6 +55,9 @@ bool use_fp8_stream_dense(const TilePlan& plan, size_t m, size_t k);
 // W4A8 (w4a8_tile.h): the same regime rule with its own size limit, the same tile shapes with its own costs of a cut along K
 bool use_w4a8_tile(size_t m, size_t n, size_t k);
 TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k);
+// group 128: strips of 16 columns per wavefront of the streaming kernel (w4a8_stream.h) where it takes the place of the tile kernel
+// under that plan (2), or over half as many columns per workgroup with K whole (1); 0: the tile kernel
+int w4a8_stream_strips(const TilePlan& plan, size_t m, size_t k);
 // W4A8 streaming kernel (up to 32 tokens): column tiles per workgroup and wavefronts that split K (parts is always 1)
 SplitKChoice select_w4a8_splitk(size_t m, size_t n);
 

@@ -361,6 +361,22 @@ TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k) {
   return t;
 }
 
+// One row block, 33..128 tokens.  Tile kernel / streaming kernel in us, GEMM with its reduction, same bits:
+// - 65..112 tokens: n = 25600, k = 5120 at 80 33.4 / 27.9, n = 12384, k = 14592 at 70 38.6 / 31.6, n = 23872, k = 2816, whole K, at 69
+//   28.4 / 20.7, n = 8896, k = 17920 at 82 35.9 / 31.8; the least n = 5120, k = 25600 at 100 36.0 / 33.1 and, parts of 6 to 8
+//   k-blocks, n = 3424, k = 12288 at 108 23.7 / 23.4.  113..128, all eight row tiles: 25600, 5120 at 128 35.9 / 34.9, parts of 12 at
+//   121 30.3 / 29.3, of 8 level to 2 % behind (n = 4128, k = 15360 at 115 25.6 / 26.1).
+// - 33..64 tokens, parts of 20 k-blocks and more: 25600, 5120 at 33 and 64 26.0 / 22.5, 26.0 / 25.6, n = 14336, k = 8192 21.5 / 20.1,
+//   23.7 / 23.2; shorter ones are over before the ring runs: parts of 8, 16224, 3968 at 64 18.5 / 19.6, of 11, 4352, 20480 23.9 / 25.0.
+// - ... and whole K: workgroups of 128 columns while that is one round of them, tile kernel / 256 / 128 columns: n = 28672, k = 1024 at
+//   33 and 64 10.8 / 9.5 / 8.5, 11.7 / 11.2 / 9.7, n = 8192, k = 1024 at 64 10.4 / 10.6 / 8.2.
+int w4a8_stream_strips(const TilePlan& plan, size_t m, size_t k) {
+  if (plan.tiles_m != 1 || m <= 32 || m > 128) return 0;
+  if (m <= 64 && plan.splits == 1 && 2 * plan.tiles_n <= static_cast<unsigned>(kNumCU)) return 1;
+  const size_t kb = plan.splits == 1 ? k / 128 : plan.kt_per_split;
+  return kb >= (m <= 64 ? 20u : m > 112 ? 10u : 1u) ? 2 : 0;
+}
+
 // W4A8 decode: a workgroup takes as many 16-column strips (up to 4) as still leave 128 workgroups - counting the row
 // blocks of a problem of more than 32 tokens: n = k = 5120 at 64 tokens 16.8 -> 11.4 us with four strips instead of
 // two -, and splits K over 8 wavefronts instead of 4 when fewer than 256 workgroups are left.
@@ -532,11 +548,12 @@ KSQ_EXPORT int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype
         const TilePlan t = plan_w4a8_tile(m, n, k);
         d->kernel = KSQ_KERNEL_MFMA_TILE;
         d->block_m = t.block_m;
-        d->block_n = 256;
+        const bool narrow = w4a8_stream_strips(t, m, k) == 1;
+        d->block_n = narrow ? 128 : 256;
         d->block_k = 128;
         d->waves = 8;
         d->split_k = static_cast<int32_t>(t.splits);
-        d->grid = static_cast<int32_t>(t.grid);
+        d->grid = static_cast<int32_t>(narrow ? 2 * t.grid : t.grid);
         return KSQ_OK;
       }
       const SplitKChoice c = select_w4a8_splitk(m, n);

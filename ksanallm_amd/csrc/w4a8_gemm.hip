@@ -19,6 +19,7 @@
 #include "ksq_common.h"
 #include "splitk_reduce.h"
 #include "tile_select.h"
+#include "w4a8_stream.h"
 #include "w4a8_tile.h"
 
 namespace ksq {
@@ -333,13 +334,22 @@ int dispatch_splitk(const W4A8Params& p, hipStream_t s) {
   return fail(KSQ_ERR_UNSUPPORTED, "no w4a8 kernel for mt=%d nt=%d waves=%d", mt, nt, waves);
 }
 
+// One row block of 33..128 tokens through the streaming kernel, strips of 16 columns per wavefront
+template <typename TO, int NS>
+int launch_stream(W4A8TileParams p, unsigned grid, int block_m, hipStream_t s) {
+  constexpr int kLds = w4a8_stream_lds_bytes(NS);
+  static std::atomic<uint64_t> configured{0};
+  if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&w4a8_stream_tile_kernel<TO, NS>), kLds)) return rc;
+  if (NS == 1) p.tiles_n *= 2;
+  w4a8_stream_tile_kernel<TO, NS><<<grid, 512, kLds, s>>>(p, static_cast<uint32_t>(block_m));
+  return KSQ_OK;
+}
+
 // Prefill regime: the MFMA tile kernel of w4a8_tile.h on the grid plan_w4a8_tile lays out (the blockwise-FP8 tile
 // shapes; a k-step is one 128-deep group).
 template <typename TO, int WM, int GROUP = 128>
 int launch_tile(const W4A8Params& q, const TilePlan& plan, float* partial, hipStream_t s) {
   constexpr int kLds = static_cast<int>(w4a8_tile_lds_bytes(WM));
-  static std::atomic<uint64_t> configured{0};
-  if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&w4a8_tile_kernel<TO, WM, GROUP>), kLds)) return rc;
   W4A8TileParams p{};
   p.a = q.a;
   p.xsum = q.xsum;
@@ -356,7 +366,15 @@ int launch_tile(const W4A8Params& q, const TilePlan& plan, float* partial, hipSt
   p.splits = plan.splits;
   p.kb_per_split = plan.kt_per_split;
   p.alpha512 = q.alpha512;
-  w4a8_tile_kernel<TO, WM, GROUP><<<plan.grid, 512, kLds, s>>>(p);
+  const int strips = GROUP == 128 && WM <= 4 ? w4a8_stream_strips(plan, q.M, q.K) : 0;
+  if (strips == 1) return launch_stream<TO, 1>(p, 2 * plan.tiles_n, plan.block_m, s);  // (the plan leaves K whole)
+  if (strips == 2) {
+    if (int rc = launch_stream<TO, 2>(p, plan.grid, plan.block_m, s)) return rc;
+  } else {
+    static std::atomic<uint64_t> configured{0};
+    if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&w4a8_tile_kernel<TO, WM, GROUP>), kLds)) return rc;
+    w4a8_tile_kernel<TO, WM, GROUP><<<plan.grid, 512, kLds, s>>>(p);
+  }
   if (plan.splits > 1) {
     const unsigned cut = plan.tiles_m * plan.tiles_n - plan.main_items;
     splitk_reduce_kernel<TO, 32 * WM><<<cut * (4 * WM), 256, 0, s>>>(partial, static_cast<uint16_t*>(p.out), p.M, p.N,

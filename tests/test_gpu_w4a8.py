@@ -163,6 +163,24 @@ def test_gemm_tile_kernel_few_tokens(ops, oracle, tile_kernels, m, n, k, parts):
     H.check_gemm(out, ref, H.BF16, "w4a8 tile m=%d n=%d k=%d" % (m, n, k))
 
 
+@pytest.mark.parametrize("m,n,k,narrow", [
+    (33, 272, 128, True), (64, 400, 1408, True), (49, 272, 256, True), (40, 23056, 1536, True), (64, 23056, 1664, True), (37, 23056, 3200, True),
+    (65, 272, 512, False), (80, 272, 640, False), (81, 288, 768, False), (112, 272, 896, False), (113, 23056, 1408, False),
+    (128, 23056, 1280, False), (97, 23056, 2816, False), (70, 4112, 3840, False)])
+def test_gemm_streaming_tile_over_its_rings(ops, oracle, tile_kernels, m, n, k, narrow):
+    """The weight rings of 12 k-blocks (128 columns, up to 64 tokens, K whole) and of 5 (256 columns, 65 to 128 tokens): fewer
+    k-blocks, as many, one more and several turns; three to eight row tiles; a last workgroup with one strip and one with none."""
+    from ksanallm_amd import lib as L
+    desc = L.select_tile(L.KIND_W4A8, m, n, k, H.BF16)
+    assert desc["block_n"] == (128 if narrow else 256)
+    w, scales = make_weight(n + k + m, k, n)
+    x = make_act(m * 7 + n, m, k, H.F16)
+    xq, xsum = ops.w4a8_static_quant(x.cuda(), torch.tensor([0.05], dtype=torch.float32).cuda(), False)
+    out = ops.w4a8_gemm(xq, xsum, ops.w4a8_repack_weight(w.cuda()), scales.cuda(), 0.03, n, torch.float16)
+    ref = oracle.w4a8_gemm(xq.cpu().numpy(), w.numpy().view(np.int8), H.bits_of(scales), 0.03)
+    H.check_gemm(out, ref, H.F16, "w4a8 streaming tile m=%d n=%d k=%d" % (m, n, k))
+
+
 @pytest.mark.parametrize("m,n,k", [(3, 8192, 512), (20, 8192, 512), (16, 16384, 256), (32, 16384, 256), (1, 4096, 1024)])
 def test_gemm_streaming_kernel_variants(ops, oracle, m, n, k):
     """The streaming kernel's other instantiations: four strips per workgroup with eight wavefronts (n = 8192) and with
