@@ -469,17 +469,21 @@ KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, s
 }
 
 // Rows per expert block for numel routed (token, slot) pairs over E experts.  Replaces the M thresholds of
-// InvokeFusedMoe (16 / 32 / 64 rows by token count): below 48 rows per expert the weights are streamed once per
+// InvokeFusedMoe (16 / 32 / 64 rows by token count): with few rows per expert the weights are streamed once per
 // 16- or 32-row block (HBM-bound); above, the MFMA tile kernel takes 256-row blocks, of which it multiplies the row
 // tiles that hold rows (an instance of its main loop per count), so that an expert's weights are dequantized once
-// however many of the 256 rows it fills.  E = 256, hidden 7168, inter 2048, top-8, whole call with 32- / 256-row
-// blocks: 1.54 / 2.37 ms at 32 rows per expert, 1.88 / 2.15 at 40, 2.53 / 2.31 at 64, 3.45 / 2.69 at 94; 128 experts, hidden
-// 4096, inter 768 297 / 288 us at 48; 64, 2048, 1408 161 / 180 at 48, 249 / 215 at 96; 16, 5504, 768 72 / 100 at 47; 8, 4096, 1536
-// 56 / 80 at 48, 81 / 99 at 100.  128-row blocks are not ahead of 256-row ones anywhere (4.40 / 3.57 ms at 128 rows).
+// however many of the 256 rows it fills.  Few experts make few 256-row workgroups: the line lies the higher, the fewer there
+// are.  Whole block, time in 32-row blocks over time in 256-row blocks at 48 / 64 / 80 / 100 / 128 rows per expert (hidden, inter):
+//   8 experts   7168, 2048 0.79 0.99 0.79 0.82 0.90   2048, 1408 0.72 0.73 0.77 0.79 0.80   6144, 640 0.61 0.59 0.60 0.69 0.68
+//   16          7168, 2048 0.69 0.75 0.80 0.86 0.90   2048, 1408 0.92 0.99 1.06 1.03 1.13   6144, 640 0.72 0.73 0.73 0.94 0.92
+//   32          7168, 2048 0.80 0.84 0.92 1.06 1.11   2048, 1408 0.92 1.04 1.13 1.14 1.16   6144, 640 0.92 0.95 0.97 1.22 1.20
+//   64          4096, 1536 0.84 0.94 1.06 1.25 1.31   2048, 1408 0.86 0.92 1.02 1.09 1.31   1024, 512 1.09 1.19 1.17 1.18 1.19
+//   256         7168, 2048 0.65 at 32, 0.87 at 40, 1.10 at 64, 1.28 at 94
+// 128-row blocks are not ahead of 256-row ones anywhere (256 experts, 128 rows 4.40 against 3.57 ms).
 KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E;
-  if (per_expert >= 48) return 256;
+  if (per_expert >= (E <= 8 ? 129u : E <= 16 ? 72u : E <= 32 ? 56u : 44u)) return 256;
   return per_expert < 16 ? 16 : 32;
 }
 
