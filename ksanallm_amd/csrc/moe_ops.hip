@@ -623,9 +623,10 @@ KSQ_EXPORT size_t ksq_moe_align_capacity(size_t numel, size_t E, size_t block_m)
 }
 
 KSQ_EXPORT size_t ksq_moe_align_scratch_bytes(size_t numel, size_t E) {
-  uint32_t chunks, per;
-  chunk_geometry(numel ? numel : 1, &chunks, &per);
-  return static_cast<size_t>(chunks) * E * sizeof(int32_t);
+  // the count table of the two-launch sort; as many rows for any smaller numel, whose chunks may be more (a caller sizes the
+  // scratch for its largest call)
+  const size_t chunks = div_up(numel, kChunkThreads);
+  return (chunks < 1 ? 1 : chunks < kMaxChunks ? chunks : kMaxChunks) * E * sizeof(int32_t);
 }
 
 KSQ_EXPORT int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_t block_m, void* sorted_ids,

@@ -186,3 +186,14 @@ def test_decode_with_k_cut_over_workgroups_takes_x_through_lds_where_that_pays()
         d = L.select_tile(L.KIND_W4A16, m, n, k, L.BF16)
         assert d["kernel"] == 0 and d["split_k"] > d["waves"]
         assert (d["waves"], d["x_chunk"]) == (waves, chunk), (m, n, k)
+
+
+def test_align_scratch_covers_every_smaller_call():
+    """A caller sizes the alignment's scratch for its largest call: never less than what a smaller one needs, whose chunks of whole
+    256 ids may be more (98304 ids are 128 chunks, 98305 are 97), a row of E counts each."""
+    from ksanallm_amd import lib as L
+    lib = L.load()
+    for E in (1, 256):
+        sizes = [lib.ksq_moe_align_scratch_bytes(n, E) for n in (0, 1, 256, 257, 32768, 32769, 65536, 65537, 98304, 98305, 131072, 131073)]
+        assert sizes == sorted(sizes) and sizes[0] > 0
+        assert lib.ksq_moe_align_scratch_bytes(98305, E) >= 128 * E * 4
