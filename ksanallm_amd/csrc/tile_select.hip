@@ -479,12 +479,20 @@ KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, s
 //   32          7168, 2048 0.80 0.84 0.92 1.06 1.11   2048, 1408 0.92 1.04 1.13 1.14 1.16   6144, 640 0.92 0.95 0.97 1.22 1.20
 //   64          4096, 1536 0.84 0.94 1.06 1.25 1.31   2048, 1408 0.86 0.92 1.02 1.09 1.31   1024, 512 1.09 1.19 1.17 1.18 1.19
 //   256         7168, 2048 0.65 at 32, 0.87 at 40, 1.10 at 64, 1.28 at 94
+// 16- and 32-row blocks: half-empty blocks of 32 run one row tile of the streaming kernel, which keeps more in flight than the
+// decode kernel over 16-row blocks, and an expert with more than 16 rows reads its weights once.  Time in 32-row blocks over time in
+// 16-row blocks at 3 / 5 / 7 / 9 / 11 / 13 / 15 rows per expert:
+//   16 experts  4096, 1536 1.01 1.02 0.99 1.00 1.01 0.99 0.99   4096, 768 1.12 1.14 1.12 1.15 1.13 1.08 1.02
+//   32          7168, 2048 1.06 1.05 1.06 1.01 0.98 0.95 0.89   1024, 512 1.30 1.23 1.07 0.99 1.01 0.98 0.96
+//   64          4096, 1536 0.98 0.99 0.99 1.01 0.94 0.92 0.89   7168, 2048 1.05 1.05 1.03 1.03 0.99 0.96 0.88
+//   128         4096, 768  0.93 0.92 0.95 0.91 0.91 0.85 0.81   7168, 2048 1.03 1.02 1.01 1.01 0.98 0.92 0.85
+//   256         7168, 2048 1.02 1.01 0.99 0.98 0.96 0.90 0.83   1024, 512 0.82 0.83 0.81 0.81 0.81 0.80 0.77
 // 128-row blocks are not ahead of 256-row ones anywhere (256 experts, 128 rows 4.40 against 3.57 ms).
 KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
   if (E == 0) return 16;
   const size_t per_expert = numel / E;
   if (per_expert >= (E <= 8 ? 129u : E <= 16 ? 72u : E <= 32 ? 56u : 44u)) return 256;
-  return per_expert < 16 ? 16 : 32;
+  return per_expert < (E >= 128 ? 7u : E >= 32 ? 10u : 16u) ? 16 : 32;
 }
 
 KSQ_EXPORT int ksq_set_small_problem_rule(int enabled) { return g_small_problem_rule.exchange(enabled ? 1 : 0); }
