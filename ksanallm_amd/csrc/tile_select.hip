@@ -370,9 +370,14 @@ TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k) {
 //   23.7 / 23.2; shorter ones are over before the ring runs: parts of 8, 16224, 3968 at 64 18.5 / 19.6, of 11, 4352, 20480 23.9 / 25.0.
 // - ... and whole K: workgroups of 128 columns while that is one round of them, tile kernel / 256 / 128 columns: n = 28672, k = 1024 at
 //   33 and 64 10.8 / 9.5 / 8.5, 11.7 / 11.2 / 9.7, n = 8192, k = 1024 at 64 10.4 / 10.6 / 8.2.
+// - ... and K that the plan cuts, where those workgroups come to three quarters of the CUs and K is not long, for no partial sums: 25600,
+//   5120 (200 workgroups) at 33 and 64 26.0 / 22.5 / 21.4, 26.0 / 25.6 / 25.0, n = 28672, k = 4096 (224) 21.5 / 20.7 / 18.2, 23.4 / 23.9 /
+//   20.9; but n = 20480, k = 8192 (160) at 64 29.0 / 29.1 / 36.0.
 int w4a8_stream_strips(const TilePlan& plan, size_t m, size_t k) {
   if (plan.tiles_m != 1 || m <= 32 || m > 128) return 0;
-  if (m <= 64 && plan.splits == 1 && 2 * plan.tiles_n <= static_cast<unsigned>(kNumCU)) return 1;
+  const unsigned narrow = 2 * plan.tiles_n;  // workgroups of 128 columns
+  if (m <= 64 && narrow <= static_cast<unsigned>(kNumCU) && (plan.splits == 1 || (narrow >= static_cast<unsigned>(kNumCU) * 3 / 4 && k <= 6144)))
+    return 1;
   const size_t kb = plan.splits == 1 ? k / 128 : plan.kt_per_split;
   return kb >= (m <= 64 ? 20u : m > 112 ? 10u : 1u) ? 2 : 0;
 }
@@ -559,13 +564,13 @@ KSQ_EXPORT int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype
       if (use_w4a8_tile(m, n, k)) {
         const TilePlan t = plan_w4a8_tile(m, n, k);
         d->kernel = KSQ_KERNEL_MFMA_TILE;
-        d->block_m = t.block_m;
-        const bool narrow = w4a8_stream_strips(t, m, k) == 1;
+        const bool narrow = w4a8_stream_strips(t, m, k) == 1;  // 128 columns per workgroup, K whole
+        d->block_m = narrow ? 64 : t.block_m;
         d->block_n = narrow ? 128 : 256;
         d->block_k = 128;
         d->waves = 8;
-        d->split_k = static_cast<int32_t>(t.splits);
-        d->grid = static_cast<int32_t>(narrow ? 2 * t.grid : t.grid);
+        d->split_k = narrow ? 1 : static_cast<int32_t>(t.splits);
+        d->grid = static_cast<int32_t>(narrow ? 2 * t.tiles_n : t.grid);
         return KSQ_OK;
       }
       const SplitKChoice c = select_w4a8_splitk(m, n);

@@ -340,7 +340,11 @@ int launch_stream(W4A8TileParams p, unsigned grid, int block_m, hipStream_t s) {
   constexpr int kLds = w4a8_stream_lds_bytes(NS);
   static std::atomic<uint64_t> configured{0};
   if (int rc = allow_dynamic_lds(configured, reinterpret_cast<const void*>(&w4a8_stream_tile_kernel<TO, NS>), kLds)) return rc;
-  if (NS == 1) p.tiles_n *= 2;
+  if (NS == 1) {  // 128 columns per workgroup over all of K, whatever the plan cuts
+    p.tiles_n *= 2;
+    p.main_items = 0;
+    p.splits = 1;
+  }
   w4a8_stream_tile_kernel<TO, NS><<<grid, 512, kLds, s>>>(p, static_cast<uint32_t>(block_m));
   return KSQ_OK;
 }
@@ -367,7 +371,7 @@ int launch_tile(const W4A8Params& q, const TilePlan& plan, float* partial, hipSt
   p.kb_per_split = plan.kt_per_split;
   p.alpha512 = q.alpha512;
   const int strips = GROUP == 128 && WM <= 4 ? w4a8_stream_strips(plan, q.M, q.K) : 0;
-  if (strips == 1) return launch_stream<TO, 1>(p, 2 * plan.tiles_n, plan.block_m, s);  // (the plan leaves K whole)
+  if (strips == 1) return launch_stream<TO, 1>(p, 2 * plan.tiles_n, 64, s);
   if (strips == 2) {
     if (int rc = launch_stream<TO, 2>(p, plan.grid, plan.block_m, s)) return rc;
   } else {

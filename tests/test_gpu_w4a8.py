@@ -165,6 +165,7 @@ def test_gemm_tile_kernel_few_tokens(ops, oracle, tile_kernels, m, n, k, parts):
 
 @pytest.mark.parametrize("m,n,k,narrow", [
     (33, 272, 128, True), (64, 400, 1408, True), (49, 272, 256, True), (40, 23056, 1536, True), (64, 23056, 1664, True), (37, 23056, 3200, True),
+    (33, 24336, 4736, True), (61, 32768, 3968, True),
     (65, 272, 512, False), (80, 272, 640, False), (81, 288, 768, False), (112, 272, 896, False), (113, 23056, 1408, False),
     (128, 23056, 1280, False), (97, 23056, 2816, False), (70, 4112, 3840, False)])
 def test_gemm_streaming_tile_over_its_rings(ops, oracle, tile_kernels, m, n, k, narrow):
@@ -172,7 +173,7 @@ def test_gemm_streaming_tile_over_its_rings(ops, oracle, tile_kernels, m, n, k, 
     k-blocks, as many, one more and several turns; three to eight row tiles; a last workgroup with one strip and one with none."""
     from ksanallm_amd import lib as L
     desc = L.select_tile(L.KIND_W4A8, m, n, k, H.BF16)
-    assert desc["block_n"] == (128 if narrow else 256)
+    assert desc["block_n"] == (128 if narrow else 256) and (desc["split_k"] == 1 or not narrow)
     w, scales = make_weight(n + k + m, k, n)
     x = make_act(m * 7 + n, m, k, H.F16)
     xq, xsum = ops.w4a8_static_quant(x.cuda(), torch.tensor([0.05], dtype=torch.float32).cuda(), False)
