@@ -82,6 +82,21 @@ __global__ void __launch_bounds__(512, 4) w4a16_stream_tile_kernel(SplitKParams 
   const uint32_t w_voff = lane * 16;
   const char* const x_base = static_cast<const char*>(p.x);
 
+  // An expert with several blocks: they run side by side and share the caches' copy of the weights.
+  const bool several = (pos0 + kW4StreamRows < slots && static_cast<uint32_t>(p.expert_ids[blockIdx.y + 1]) == e) ||
+                       (blockIdx.y > 0 && static_cast<uint32_t>(p.expert_ids[blockIdx.y - 1]) == e);
+  // A strip is K / 128 KiB, so where K is a multiple of 4096 the strips of all workgroups start on the same HBM channels, where it is
+  // one of 2048 on one of two sets of them, and the workgroups walk over the channels in step.  There an expert starts at a place
+  // of its own and goes round (the same one for all its columns, which share x in the L2, and for all its blocks).  us, from k-tile 0
+  // by all / with this: 64 experts of n = k = 4096 at 8, 16, 20, 32 rows 118 / 98, 121 / 108, 131 / 118, 146 / 142 (decode kernel 107,
+  // 114, 122, 168); n = 4096, k = 2048 at 8 and 20 61 / 53, 70 / 66; gate / up with n = k = 4096, 256 experts at 8 393 / 371, 16 at 16
+  // 34 / 31; whole int4 block, 16 experts of hidden 4096, inter 2048 at 16 66 / 59 (decode kernel 58).  With k = 2048 and several blocks to
+  // an expert it is 3-5 % behind (256 experts, n = 7168 at 32 rows 529 / 547); per workgroup instead of per expert it
+  // loses 3-9 % from 20 rows on, as every column then reads x at another place.
+  const bool spread = KT % 32 == 0 || (KT % 16 == 0 && !several);
+  const uint32_t first_kt = __builtin_amdgcn_readfirstlane(spread ? 2 * (5 * e % (KT / 2)) : 0);
+  auto k_tile = [&](uint32_t i) { return i + first_kt < KT ? i + first_kt : i + first_kt - KT; };  // k-tile of place i
+
   uint32_t magic2 = p.magic2;
   asm volatile("" : "+v"(magic2));  // no instruction: keeps the value in a VGPR so that and / or fold into one instruction
   const uint32_t nmask = p.nibble_mask;
@@ -113,9 +128,9 @@ __global__ void __launch_bounds__(512, 4) w4a16_stream_tile_kernel(SplitKParams 
     // half h -> LDS slot h % 4 (assembly statements open with s_nop 4: scalar operands that a v_readfirstlane produced need
     // five wait states before a vector memory instruction reads them, and the compiler inserts none inside a statement)
     auto stage = [&](uint32_t to) __attribute__((always_inline)) {
-      const uint32_t h = 2 * to < KT ? to : 0;  // (a half past the end, of a short K, repeats the first; nothing uses it)
-      const uint32_t left = (KT - 2 * h) * 16;  // pieces of a row from this half on; lanes past them re-read the first
-      const uint32_t xv = (x_piece < left ? x_piece : 0) * 16 + h * 512;
+      const uint32_t kt = k_tile(2 * to < KT ? 2 * to : 0);  // (a half past the end, of a short K, repeats the first; nothing uses it)
+      const uint32_t left = (KT - kt) * 16;  // pieces of a row from this half on; lanes past them re-read the first
+      const uint32_t xv = (x_piece < left ? x_piece : 0) * 16 + kt * 256;
       const char* const xs = x_base;
       const char* const sb = s_base;
 #pragma unroll
@@ -123,14 +138,14 @@ __global__ void __launch_bounds__(512, 4) w4a16_stream_tile_kernel(SplitKParams 
         asm volatile("s_nop 4\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2" ::"v"(x_off[i] + xv), "s"(x_dst[i] + (to & 3) * SLOT),
                      "s"(xs)
                      : "memory", "m0");
-      const uint32_t o = h * 64 + s_byte;
+      const uint32_t o = kt * 32 + s_byte;
       asm volatile("s_nop 4\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2" ::"v"(s_off + (o < s_last ? o : s_last)),
                    "s"(s_dst + (to & 3) * SC_SLOT), "s"(sb)
                    : "memory", "m0");
     };
     u32x4 ring[4][NS];
     auto load_w = [&](uint32_t kt, u32x4 (&dst)[NS]) __attribute__((always_inline)) {  // (k-tiles past the end: 16 bytes of the last one)
-      const uint32_t o = (kt < KT ? kt : KT - 1) * 1024, wv = kt < KT ? w_voff : 0;
+      const uint32_t o = k_tile(kt < KT ? kt : KT - 1) * 1024, wv = kt < KT ? w_voff : 0;
 #pragma unroll
       for (int t = 0; t < NS; t += 2) {
         const char *const w0 = w_base[t] + o, *const w1 = w_base[t + 1] + o;
@@ -314,9 +329,6 @@ __global__ void __launch_bounds__(512, 4) w4a16_stream_tile_kernel(SplitKParams 
         }
       }
   };
-  // An expert with several blocks: they run side by side on one XCD and share its L2's copy of the weights.
-  const bool several = (pos0 + kW4StreamRows < slots && static_cast<uint32_t>(p.expert_ids[blockIdx.y + 1]) == e) ||
-                       (blockIdx.y > 0 && static_cast<uint32_t>(p.expert_ids[blockIdx.y - 1]) == e);
   if (several)
     for_tile_count<1, 2>((nrows + 15) / 16, [&](auto rt_c) __attribute__((always_inline)) { run(rt_c, std::true_type{}); });
   else

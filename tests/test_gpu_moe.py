@@ -341,6 +341,31 @@ def test_grouped_streaming_kernel_over_its_ring(ops, oracle, dtype, kt):
             assert torch.equal(one.view(torch.int16), ops.silu_and_mul(out).view(torch.int16))
 
 
+@pytest.mark.parametrize("dtype", [H.F16, H.BF16])
+@pytest.mark.parametrize("kt", [16, 32, 48])
+def test_grouped_streaming_kernel_that_goes_round_k(ops, oracle, dtype, kt):
+    """K of a multiple of 2048: experts start at different k-tiles and go round - those with one block (all three sizes) and, with a
+    multiple of 4096, those with several.  Sixteen slots and fewer, 17 to 32, several blocks, and one expert without any; with
+    silu*mul in the epilogue the bits of the two launches."""
+    from ksanallm_amd import lib as L
+    rows = [1, 16, 17, 32, 33, 48, 0, 64, 65, 15, 31, 100, 5, 20, 2, 40]
+    E, T, k, inter = len(rows), sum(rows), 128 * kt, 1152
+    assert (T // 32 + E // 2 + 1) * -(-2 * inter // 256) >= 192
+    d = make_moe(oracle, 6200 + kt, E, k, inter, T, 1, 128, dtype)
+    ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
+    ids = ids[torch.randperm(T, generator=H.gen(79))].reshape(T, 1).contiguous()
+    w13p = ops.repack_weight(d["w13"].cuda(), L.SRC_MOE_NK, E, k, 2 * inter)
+    s13p = ops.repack_scales(d["s13"].cuda(), L.SCALE_NG, E, k, 2 * inter, 128)
+    al = ops.moe_align_block_size(ids.cuda(), E, 32)
+    out = torch.full((T, 2 * inter), float("nan"), dtype=d["x"].dtype, device="cuda")
+    ops.moe_w4a16_gemm(d["x"].cuda(), w13p, s13p, None, *al, T, 1, E, 2 * inter, k, 128, 32, out=out)
+    ref = oracle.moe_w4a16_gemm(H.bits_of(d["x"]), d["w13"].numpy(), H.bits_of(d["s13"]), ids.numpy(), d["tw"].numpy(), 1, 128, False, dtype)
+    H.check_gemm(out, ref, dtype, "streaming kernel, round %d k-tiles" % kt)
+    one = torch.full((T, inter), float("nan"), dtype=d["x"].dtype, device="cuda")
+    ops.moe_w4a16_gate_up_silu(d["x"].cuda(), w13p, s13p, *al, T, 1, E, 2 * inter, k, 128, 32, out=one)
+    assert torch.equal(one.view(torch.int16), ops.silu_and_mul(out).view(torch.int16))
+
+
 @pytest.mark.parametrize("T", [1, 64, 2048])
 def test_moe_block_deepseek_shape(ops, oracle, T):
     """256 experts, hidden 7168, inter 2048, top-8; weights for all experts are generated but only touched ones
