@@ -276,8 +276,8 @@ int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_t block_m, 
  *   out[s, :] = x[s / top_k, :] . dequant(W[expert of s's block]) * (topk_w ? topk_w[s] : 1)
  * x [rows, k] T, out [numel, n] T, W/scales packed per expert as by ksq_w4a16_repack(E = experts),
  * zeros_packed NULL for symmetric (code-8).  top_k = 1 reads x rows by slot (second MoE GEMM).
- * block_m is the block size the permutation was aligned with: 16 or 32 run the decode kernel or, in blocks of 32 and from 192
- * workgroups on, the streaming kernel (the sums over k in one order instead of four), 128 or 256
+ * block_m is the block size the permutation was aligned with: 16 or 32 run the decode kernel or, in blocks of 32 and by the
+ * number of its workgroups (ksq_moe_w4a16_kernel()), the streaming kernel (the sums over k in one order instead of four), 128 or 256
  * the MFMA tile kernel (which multiplies only the 16-row tiles of a block that hold rows); ksq_moe_block_m() gives the
  * choice for a problem size.
  * A handful of slots (numel <= 64, block_m 16) need no aligned permutation: with sorted_ids NULL, expert_ids is the
@@ -287,6 +287,8 @@ int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_t block_m, 
  * Replaces InvokeMoeWna16Gemm (K/moe/moe_wna16/moe_wna16.cu:263-288) and the Triton
  * InvokeFusedMoeGptqAwqKernel (S/kernels/nvidia/triton_wrapper.h:68-75). */
 size_t ksq_moe_block_m(size_t numel, size_t E);
+/* The kernel (KSQ_KERNEL_*, below) that such a launch over an aligned permutation runs: a pure host function. */
+int ksq_moe_w4a16_kernel(size_t numel, size_t E, size_t n, size_t k, size_t block_m);
 int ksq_moe_w4a16_gemm(void* out, const void* x, const void* w_packed, const void* scales_packed,
                        const void* zeros_packed, const void* topk_w, const void* sorted_ids, const void* expert_ids,
                        const void* num_post_pad, size_t numel, size_t top_k, size_t E, size_t n, size_t k,
@@ -422,8 +424,8 @@ typedef struct ksq_tile_desc {
 /* The descriptor describes group size 128.  Other group sizes of W4A16 keep the kernel and block shape but carry more
  * scales per k-tile; W4A8 with group 64 runs 128-token tiles whose K range is not cut (split_k and grid then differ
  * from what is reported here).  KSQ_KIND_MOE_W4A16 describes the grouped streaming launch of m slots of one expert, in
- * blocks of 16 slots (m <= 16) or 32, of few workgroups: from 192 workgroups of 256 columns over all experts on, blocks of 32
- * slots run a streaming kernel that no descriptor shows; the blocks of 128 and 256 slots run the tile kernel. */
+ * blocks of 16 slots (m <= 16) or 32; ksq_moe_w4a16_kernel() says where blocks of 32 slots run the streaming kernel instead and
+ * blocks of 128 and 256 the tile kernel. */
 int ksq_select_tile(int kind, size_t m, size_t n, size_t k, int dtype, ksq_tile_desc* out_desc);
 
 /* Above 32 rows ksq_w4a16_gemm, ksq_fp8_blockwise_gemm and ksq_w4a8_gemm run the MFMA tile kernels, but for small

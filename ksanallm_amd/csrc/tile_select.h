@@ -19,8 +19,12 @@ SplitKChoice select_splitk_blocks(int mt, size_t m_blocks, size_t n, size_t k);
 // grouped W4A16 launch over about `blocks` blocks of block_m (16 or 32) slots, numel of them routed; K is never cut over workgroups
 SplitKChoice select_splitk_grouped(size_t block_m, size_t blocks, size_t numel, size_t n, size_t k);
 
+// row blocks of an aligned permutation that hold rows, about: numel / block_m + E / 2
+size_t grouped_row_blocks(size_t numel, size_t E, size_t block_m);
+
 // grouped W4A16 launch: whether the streaming kernel (w4a16_stream.h) takes the place of the decode kernel over about `blocks` blocks
-bool use_w4a16_stream(size_t block_m, size_t blocks, size_t n, size_t k);
+// of block_m slots, numel of them routed to E experts
+bool use_w4a16_stream(size_t block_m, size_t blocks, size_t numel, size_t E, size_t n, size_t k);
 
 // The decode-form kernels also serve small problems of more than 32 rows, in blocks of 32 rows; never more than this
 // many rows (the workspace queries walk every m up to it).

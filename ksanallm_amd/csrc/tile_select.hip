@@ -1,5 +1,6 @@
 // Per-shape tile selection: closed-form rules of (kind, m, n, k, dtype) for a 256-CU, 8-XCD MI355X.
 // Host code only; no timing and no device queries, so the answer is the same at load time and at run time.
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 
@@ -139,15 +140,43 @@ SplitKChoice select_splitk_grouped(size_t block_m, size_t blocks, size_t numel, 
   return c;
 }
 
+// Row blocks of block_m slots that numel slots fill where the router prefers none of the E experts, on average: c slots of an expert
+// fill ceil(c / block_m), and c is about normal.
+static double expected_row_blocks(size_t numel, size_t E, size_t block_m) {
+  const double mean = static_cast<double>(numel) / E, deviation = std::sqrt(mean * (1.0 - 1.0 / E));
+  if (mean > 8.0 * block_m) return E * (mean / block_m + 0.5);
+  double blocks = 0;
+  for (double least = 0.5; least < mean + 6.0 * deviation + 1.0; least += block_m)
+    blocks += deviation > 0 ? 0.5 * std::erfc((least - mean) / (deviation * std::sqrt(2.0))) : least < mean;
+  return E * blocks;
+}
+
+size_t grouped_row_blocks(size_t numel, size_t E, size_t block_m) {
+  return std::min((numel + E * (block_m - 1)) / block_m, numel / block_m + E / 2 + 1);
+}
+
 // 32-slot blocks: the streaming kernel, where its workgroups of 256 columns come to three quarters of the CUs.  Whole int4 block,
 // decode kernel / streaming kernel in us (experts, top-k, hidden, inter, tokens): 256, 8, 7168, 2048 at 512 tokens 1140 / 1066, at
 // 1024 tokens 1690 / 1542; 128, 8, 4480, 640 at 352 210 / 177; 64, 8, 6656, 512 at 128 110 / 101; 32, 8, 3328, 512 at 124 (192
 // workgroups in the first GEMM) 65.6 / 59.4; 16, 2, 4096, 1792 at 128 (224) 59.5 / 59.0.  Fewer leave the chip to a few long
 // workgroups: 8, 2, 4096, 1536 at 96 (120) 44.6 / 50.8; 16, 2, 1024, 512 at 300 (108) 30.4 / 33.2; 16, 2, 2432, 512 at 144 (68)
 // 33.1 / 39.4.  (Workgroups of 128 columns instead: 44.5, 30.0 and 35.8, and slower than the decode kernel above.)
-bool use_w4a16_stream(size_t block_m, size_t blocks, size_t n, size_t k) {
-  return block_m == 32 && blocks * div_up(n, 256) >= static_cast<size_t>(kNumCU) * 3 / 4 &&
-         n * k <= (size_t(1) << 36);  // 32-bit offsets into an expert's scales
+//
+// A little more than one round of its workgroups over the CUs leaves it behind too, where the decode kernel has eight strips to a
+// workgroup (n a multiple of 128, its fastest form) and k is long.  Decode kernel / streaming kernel over 217 GEMMs of 2 to 64 experts, by
+// the workgroups that even routing is expected to give: 140-192 1.05 in the mean (0.96-1.19), 192-256 1.04 (0.93-1.22), 256-320 0.96
+// (0.76-1.10), 320-372 0.99 (0.88-1.15), 372-400 1.03.  Whole int4 block, streaming / decode kernel in such launches: 8, 2, 4480,
+// 4736 at 17 rows per expert 90.3 / 83.6, 16, 4, 2432, 5888 at 35 151 / 130, 16, 1, 3584, 2176 at 19 73.0 / 68.7; and, k below
+// 4096, where it does not hold: 16, 4, 2816, 1280 at 41 67.0 / 71.5, 8, 8, 2688, 4096 at 24 52.4 / 55.5.
+bool use_w4a16_stream(size_t block_m, size_t blocks, size_t numel, size_t E, size_t n, size_t k) {
+  const size_t tiles = div_up(n, 256);
+  if (block_m != 32 || blocks * tiles < static_cast<size_t>(kNumCU) * 3 / 4) return false;
+  if (n * k > (size_t(1) << 36)) return false;  // 32-bit offsets into an expert's scales
+  if (n % 128 == 0 && k >= 4096 && blocks * tiles < 2 * static_cast<size_t>(kNumCU)) {
+    const double wgs = expected_row_blocks(numel, E, block_m) * static_cast<double>(tiles);
+    if (wgs > kNumCU * 1.03 && wgs <= kNumCU * 1.25) return false;  // (a few more than expected are no round)
+  }
+  return true;
 }
 
 // Regime switch.  Up to 32 rows the split-K (decode) kernel; above, the MFMA tile kernel - except while the problem is
@@ -498,6 +527,12 @@ KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
   const size_t per_expert = numel / E;
   if (per_expert >= (E <= 8 ? 129u : E <= 16 ? 72u : E <= 32 ? 56u : 44u)) return 256;
   return per_expert < (E >= 128 ? 7u : E >= 32 ? 10u : 16u) ? 16 : 32;
+}
+
+KSQ_EXPORT int ksq_moe_w4a16_kernel(size_t numel, size_t E, size_t n, size_t k, size_t block_m) {
+  if (block_m >= 128) return KSQ_KERNEL_MFMA_TILE;
+  if (block_m == 0 || E == 0) return KSQ_KERNEL_SPLITK_WAVE;
+  return use_w4a16_stream(block_m, grouped_row_blocks(numel, E, block_m), numel, E, n, k) ? KSQ_KERNEL_STREAM_TILE : KSQ_KERNEL_SPLITK_WAVE;
 }
 
 KSQ_EXPORT int ksq_set_small_problem_rule(int enabled) { return g_small_problem_rule.exchange(enabled ? 1 : 0); }

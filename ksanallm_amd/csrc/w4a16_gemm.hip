@@ -482,9 +482,9 @@ int moe_w4a16_gemm_impl(const char* fn, bool fuse_silu, void* out, const void* x
   p.top_k = static_cast<uint32_t>(top_k);
   p.num_experts = static_cast<uint32_t>(E);
   p.x_bytes = static_cast<uint32_t>(x_rows * k * 2);
-  // about numel/block_m + E/2 of the aligned blocks hold rows; K is never split across workgroups here
-  const size_t blocks = few ? numel : std::min(cap_blocks, numel / block_m + E / 2 + 1);
-  if (use_w4a16_stream(block_m, blocks, n, k)) {
+  // (K is never split across workgroups here)
+  const size_t blocks = few ? numel : grouped_row_blocks(numel, E, block_m);
+  if (use_w4a16_stream(block_m, blocks, numel, E, n, k)) {
     p.nibble_mask = 0x000f000fu;
     p.magic2 = dtype == KSQ_F16 ? F16::kMagic2 : BF16::kMagic2;
     if (int rc = launch_w4a16_stream(p, fuse_silu, static_cast<uint32_t>(cap_blocks), dtype, as_stream(stream))) return rc;

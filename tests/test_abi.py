@@ -197,3 +197,19 @@ def test_align_scratch_covers_every_smaller_call():
         sizes = [lib.ksq_moe_align_scratch_bytes(n, E) for n in (0, 1, 256, 257, 32768, 32769, 65536, 65537, 98304, 98305, 131072, 131073)]
         assert sizes == sorted(sizes) and sizes[0] > 0
         assert lib.ksq_moe_align_scratch_bytes(98305, E) >= 128 * E * 4
+
+
+def test_grouped_int4_launches_of_the_streaming_kernel():
+    """32-slot blocks from 192 workgroups of 256 columns on, but for more than one and up to five quarters of a round of the 256 CUs
+    (as even routing is expected to fill the blocks) where the decode kernel has eight strips to a workgroup and k is 4096 or more."""
+    from ksanallm_amd import lib as L
+    kernel = L.load().ksq_moe_w4a16_kernel
+    stream, tile, decode = L.KERNEL_STREAM_TILE, L.KERNEL_MFMA_TILE, L.KERNEL_SPLITK_WAVE
+    assert [kernel(4096, 256, 4096, 7168, bm) for bm in (16, 32, 128, 256)] == [decode, stream, tile, tile]
+    assert [kernel(numel, 32, 1024, 3328, 32) for numel in (991, 992)] == [decode, stream]
+    assert [kernel(128, 8, n, 4096, 32) for n in (8192, 8320, 8448, 10240, 10368)] == [stream, decode, decode, decode, stream]   # 32 .. 41 tiles
+    assert [kernel(128, 8, n, 4096, 32) for n in (8256, 8512)] == [stream, stream]                   # n not a multiple of 128
+    assert [kernel(128, 8, 9216, k, 32) for k in (3968, 4096, 7168)] == [stream, decode, decode]
+    assert [kernel(per * 16, 16, 4096, 4096, 32) for per in (16, 20, 28, 32)] == [stream, stream, decode, stream]   # 16, 16, 19 and 23 expected blocks
+    assert kernel(256, 1, 8192, 4096, 32) == stream and kernel(256, 1, 9216, 4096, 32) == decode     # one expert: exactly 8 blocks
+    assert kernel(4096, 256, 1 << 20, 1 << 16, 32) == stream and kernel(4096, 256, 1 << 20, (1 << 16) + 128, 32) == decode

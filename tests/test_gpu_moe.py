@@ -313,7 +313,7 @@ def test_grouped_tile_kernel_every_count_of_live_row_tiles(ops, oracle, dtype, b
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
 @pytest.mark.parametrize("kt", [1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 12])
 def test_grouped_streaming_kernel_over_its_ring(ops, oracle, dtype, kt):
-    """32-slot blocks in 192 and more workgroups of 256 columns run the kernel that streams the weights through a ring of four
+    """32-slot blocks in enough workgroups of 256 columns run the kernel that streams the weights through a ring of four
     k-tiles and x by halves of two: every way its loop can end, one and two row tiles, experts with one and with several blocks,
     a last workgroup with a few columns; the bound is the decode form's, whose weights are exact too.  With silu*mul in the
     epilogue: the bits of the two launches."""
@@ -321,7 +321,7 @@ def test_grouped_streaming_kernel_over_its_ring(ops, oracle, dtype, kt):
     rows = [1, 16, 17, 32, 33, 48, 49, 64, 65, 15, 31, 100]
     E, T, k = len(rows), sum(rows), 128 * kt
     inter = 1312
-    assert (T // 32 + E // 2 + 1) * -(-2 * inter // 256) >= 192
+    assert L.load().ksq_moe_w4a16_kernel(T, E, 2 * inter, k, 32) == L.KERNEL_STREAM_TILE
     d = make_moe(oracle, 6100 + kt, E, k, inter, T, 1, 128, dtype)
     ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
     ids = ids[torch.randperm(T, generator=H.gen(78))].reshape(T, 1).contiguous()
@@ -350,7 +350,7 @@ def test_grouped_streaming_kernel_that_goes_round_k(ops, oracle, dtype, kt):
     from ksanallm_amd import lib as L
     rows = [1, 16, 17, 32, 33, 48, 0, 64, 65, 15, 31, 100, 5, 20, 2, 40]
     E, T, k, inter = len(rows), sum(rows), 128 * kt, 1152
-    assert (T // 32 + E // 2 + 1) * -(-2 * inter // 256) >= 192
+    assert L.load().ksq_moe_w4a16_kernel(T, E, 2 * inter, k, 32) == L.KERNEL_STREAM_TILE
     d = make_moe(oracle, 6200 + kt, E, k, inter, T, 1, 128, dtype)
     ids = torch.cat([torch.full((r,), e, dtype=torch.int32) for e, r in enumerate(rows)])
     ids = ids[torch.randperm(T, generator=H.gen(79))].reshape(T, 1).contiguous()
