@@ -554,7 +554,7 @@ def cpu_baseline(keeps, L, ops):
                         ref_f = ref if few else orc.from_bits(np.asarray(ref).reshape(rows, -1), orc.BF16)
                         # two GEMMs in a row: where both run on the tile kernel, which rounds every dequantized weight
                         # to T, two independent rounding errors compound
-                        tiled = L.load().ksq_moe_block_m(T * k["topk"], k["E"]) >= 128
+                        tiled = L.load().ksq_moe_w4a16_row_block(T * k["topk"], k["E"], k["hidden"], k["inter"]) >= 128
                         accuracy.append(dict(case="c%d/moe:T=%d" % (cfg, T), rows=rows,
                                              **_err(k["out"][T][:rows], ref_f, REL_L2_MAX * (2 ** 0.5 if tiled else 1))))
         if t > 0:

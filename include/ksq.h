@@ -278,8 +278,9 @@ int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_t block_m, 
  * zeros_packed NULL for symmetric (code-8).  top_k = 1 reads x rows by slot (second MoE GEMM).
  * block_m is the block size the permutation was aligned with: 16 or 32 run the decode kernel or, in blocks of 32 and by the
  * number of its workgroups (ksq_moe_w4a16_kernel()), the streaming kernel (the sums over k in one order instead of four), 128 or 256
- * the MFMA tile kernel (which multiplies only the 16-row tiles of a block that hold rows); ksq_moe_block_m() gives the
- * choice for a problem size.
+ * the MFMA tile kernel (which multiplies only the 16-row tiles of a block that hold rows); ksq_moe_w4a16_row_block()
+ * gives the choice for a block of experts whose gate / up projection is [2 * inter, hidden] and whose down projection is [hidden,
+ * inter], ksq_moe_block_m() the one for unknown sizes.
  * A handful of slots (numel <= 64, block_m 16) need no aligned permutation: with sorted_ids NULL, expert_ids is the
  * router's topk_ids [numel] itself, num_post_pad is not read, and every slot is a block of its own (a slot whose id is
  * outside [0, E) leaves its output row unwritten, as the alignment would have dropped it).  One launch fewer in front
@@ -287,6 +288,7 @@ int ksq_moe_align(const void* topk_ids, size_t numel, size_t E, size_t block_m, 
  * Replaces InvokeMoeWna16Gemm (K/moe/moe_wna16/moe_wna16.cu:263-288) and the Triton
  * InvokeFusedMoeGptqAwqKernel (S/kernels/nvidia/triton_wrapper.h:68-75). */
 size_t ksq_moe_block_m(size_t numel, size_t E);
+size_t ksq_moe_w4a16_row_block(size_t numel, size_t E, size_t hidden, size_t inter);
 /* The kernel (KSQ_KERNEL_*, below) that such a launch over an aligned permutation runs: a pure host function. */
 int ksq_moe_w4a16_kernel(size_t numel, size_t E, size_t n, size_t k, size_t block_m);
 int ksq_moe_w4a16_gemm(void* out, const void* x, const void* w_packed, const void* scales_packed,

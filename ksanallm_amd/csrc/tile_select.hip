@@ -529,6 +529,20 @@ KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
   return per_expert < (E >= 128 ? 7u : E >= 32 ? 10u : 16u) ? 16 : 32;
 }
 
+// The block size of a whole int4 expert block (both GEMMs and their alignment).  Up to 8 experts whose first GEMM has four rounds of
+// 256-row workgroups (1024 of them) give the tile kernel its workgroups: its line is that of 16 experts.  Whole block, even routing,
+// 32- / 256-row blocks in us at 68 / 72 / 80 / 90 / 100 / 128 rows per expert: 8 experts, hidden 6144, inter 16384 534 / 555, 595 / 561, 631 /
+// 573, 693 / 600, 762 / 752, 950 / 849; 8, 8192, 28672 1346 / 1443, 1421 / 1470, 1478 / 1501, 1646 / 1574, 1828 / 1640, 2231 / 1875; 8,
+// 4096, 28672 712 / 766, 739 / 801, 767 / 813, 845 / 846, 927 / 875, 1165 / 982.  With fewer 32-row blocks are ahead, or level at the
+// end: 8, 4096, 14336 (896 workgroups) at 80, 100, 128 372 / 423, 435 / 511, 566 / 569, 8, 8192, 14336 702 / 794, 894 / 941, 1085 / 1065.
+// Where routing prefers some experts (logits with a spread of 0.7 per expert) 32-row blocks are ahead longer, up to a quarter.
+KSQ_EXPORT size_t ksq_moe_w4a16_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {
+  (void)hidden;
+  const size_t block_m = ksq_moe_block_m(numel, E);
+  if (E != 0 && E <= 8 && numel / E >= 72 && E * div_up(2 * inter, 256) >= 4 * static_cast<size_t>(kNumCU)) return 256;
+  return block_m;
+}
+
 KSQ_EXPORT int ksq_moe_w4a16_kernel(size_t numel, size_t E, size_t n, size_t k, size_t block_m) {
   if (block_m >= 128) return KSQ_KERNEL_MFMA_TILE;
   if (block_m == 0 || E == 0) return KSQ_KERNEL_SPLITK_WAVE;

@@ -30,7 +30,7 @@ namespace {
 #define KSQ_FOR_EACH_FN(F) \
   F(w4a16_workspace_size) F(w4a16_gemm) F(fp8_group_quant) F(fp8_blockwise_workspace_size) F(fp8_blockwise_gemm) \
   F(w4a8_static_quant) F(w4a8_workspace_size) F(w4a8_gemm) F(moe_topk_softmax) F(moe_grouped_topk) \
-  F(moe_align_capacity) F(moe_align_scratch_bytes) F(moe_align) F(moe_block_m) F(moe_fp8_row_block) F(moe_w4a16_gemm) \
+  F(moe_align_capacity) F(moe_align_scratch_bytes) F(moe_align) F(moe_w4a16_row_block) F(moe_fp8_row_block) F(moe_w4a16_gemm) \
   F(moe_w4a16_gate_up_silu) F(moe_w4a16_down_sum) F(moe_fp8_blockwise_gemm) F(moe_fp8_fused_quant) F(moe_fp8_gate_up_quant) \
   F(moe_fp8_down_sum) F(moe_silu_mul) F(moe_sum)
 
@@ -405,13 +405,13 @@ at::Tensor fused_moe_w4a16(const Args& a) {
     });
     return out;
   }
-  if (!block_given) block_m = lib.moe_block_m(r.numel, E);
+  if (!block_given) block_m = lib.moe_w4a16_row_block(r.numel, E, hidden, inter);
   if (block_m == 0) raise(PyExc_ZeroDivisionError, "block size 0");
   const Aligned al = moe_align(r.ids, E, block_m, st);
   void *ps = ptr(al.sorted_ids), *pe = ptr(al.expert_ids), *pn = ptr(al.num_post_pad);
   at::Tensor c2 = empty({r.numel, inter}, t, x);
   void* p2 = ptr(c2);
-  // the activation runs in the first GEMM's epilogue, except with 128-row blocks (a size moe_block_m does not pick but
+  // the activation runs in the first GEMM's epilogue, except with 128-row blocks (a size moe_w4a16_row_block does not pick but
   // a caller may ask for), where the two launches measured faster (64 rows per expert: 1.75 against 1.87 ms)
   if (block_m != 128 && (2 * inter) % 32 == 0) {
     call([&] {

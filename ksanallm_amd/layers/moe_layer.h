@@ -37,7 +37,7 @@ class MoeLayer : public BaseLayer {
   size_t BlockM(size_t tokens) const {
     if (IsFp8())
       return ksq_moe_fp8_row_block(tokens * expert_topk_, expert_num_per_node_, expert_hidden_size_, expert_inter_size_);
-    return ksq_moe_block_m(tokens * expert_topk_, expert_num_per_node_);
+    return ksq_moe_w4a16_row_block(tokens * expert_topk_, expert_num_per_node_, expert_hidden_size_, expert_inter_size_);
   }
   bool IsFp8() const { return compute_dtype_ == TYPE_BLOCK_FP8_E4M3; }
 

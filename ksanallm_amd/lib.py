@@ -65,6 +65,7 @@ SIGNATURES = {
     "ksq_fp8_tensor_gemm_workspace_size": (c_sz, [c_sz, c_sz, c_sz]),
     "ksq_fp8_tensor_gemm": (c_i, [c_p, c_p, c_p, c_p, c_p, c_sz, c_sz, c_sz, c_i, c_p, c_sz, c_p]),
     "ksq_moe_block_m": (c_sz, [c_sz, c_sz]),
+    "ksq_moe_w4a16_row_block": (c_sz, [c_sz, c_sz, c_sz, c_sz]),
     "ksq_moe_w4a16_kernel": (c_i, [c_sz, c_sz, c_sz, c_sz, c_sz]),
     "ksq_moe_fp8_block_m": (c_sz, [c_sz, c_sz]),
     "ksq_moe_fp8_block_m_sized": (c_sz, [c_sz, c_sz, c_sz, c_sz]),

@@ -213,3 +213,20 @@ def test_grouped_int4_launches_of_the_streaming_kernel():
     assert [kernel(per * 16, 16, 4096, 4096, 32) for per in (16, 20, 28, 32)] == [stream, stream, decode, stream]   # 16, 16, 19 and 23 expected blocks
     assert kernel(256, 1, 8192, 4096, 32) == stream and kernel(256, 1, 9216, 4096, 32) == decode     # one expert: exactly 8 blocks
     assert kernel(4096, 256, 1 << 20, 1 << 16, 32) == stream and kernel(4096, 256, 1 << 20, (1 << 16) + 128, 32) == decode
+
+
+def test_int4_expert_row_blocks():
+    """One value on each side of every line of the sizes-unknown rule, and where the sizes move them: up to 8 experts with 1024
+    workgroups of 256 columns in the first GEMM have the line of 16 experts."""
+    from ksanallm_amd import lib as L
+    lib = L.load()
+    for E, small, large in ((1, 16, 129), (8, 16, 129), (9, 16, 72), (16, 16, 72), (17, 16, 56), (31, 16, 56), (32, 10, 56), (33, 10, 44),
+                            (127, 10, 44), (128, 7, 44), (256, 7, 44)):
+        blocks = [lib.ksq_moe_block_m(per * E + E // 2, E) for per in (small - 1, small, large - 1, large)]
+        assert blocks == [16, 32, 32, 256], (E, blocks)
+        for per in (small - 1, small, large - 1, large):
+            assert lib.ksq_moe_w4a16_row_block(per * E, E, 2048, 1408) == lib.ksq_moe_block_m(per * E, E)
+    assert lib.ksq_moe_block_m(100, 0) == 16 and lib.ksq_moe_w4a16_row_block(100, 0, 2048, 1408) == 16
+    for E, hidden, inter, line in ((8, 6144, 16384, 72), (8, 4096, 28672, 72), (8, 6144, 16256, 129), (4, 8192, 32768, 72), (4, 8192, 28672, 129)):
+        rule = [lib.ksq_moe_w4a16_row_block(per * E, E, hidden, inter) for per in (15, 16, line - 1, line)]
+        assert rule == [16, 32, 32, 256], (E, hidden, inter, rule)
