@@ -536,9 +536,13 @@ KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
 // 4096, 28672 712 / 766, 739 / 801, 767 / 813, 845 / 846, 927 / 875, 1165 / 982.  With fewer 32-row blocks are ahead, or level at the
 // end: 8, 4096, 14336 (896 workgroups) at 80, 100, 128 372 / 423, 435 / 511, 566 / 569, 8, 8192, 14336 702 / 794, 894 / 941, 1085 / 1065.
 // Where routing prefers some experts (logits with a spread of 0.7 per expert) 32-row blocks are ahead longer, up to a quarter.
+//
+// From 40 rows each on, activations of 1 GiB, which the launches of 16- and 32-row blocks refuse (32-bit offsets), run the tile kernel,
+// which takes 4 GiB.  (As many rows as slots: the second GEMM's, and the first one's behind a gather.)
 KSQ_EXPORT size_t ksq_moe_w4a16_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {
-  (void)hidden;
   const size_t block_m = ksq_moe_block_m(numel, E);
+  const size_t longest = hidden > inter ? hidden : inter;
+  if (E != 0 && numel / E >= 40 && numel > 0x3fffffffull / 2 / (longest ? longest : 1)) return 256;
   if (E != 0 && E <= 8 && numel / E >= 72 && E * div_up(2 * inter, 256) >= 4 * static_cast<size_t>(kNumCU)) return 256;
   return block_m;
 }

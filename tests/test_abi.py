@@ -230,3 +230,17 @@ def test_int4_expert_row_blocks():
     for E, hidden, inter, line in ((8, 6144, 16384, 72), (8, 4096, 28672, 72), (8, 6144, 16256, 129), (4, 8192, 32768, 72), (4, 8192, 28672, 129)):
         rule = [lib.ksq_moe_w4a16_row_block(per * E, E, hidden, inter) for per in (15, 16, line - 1, line)]
         assert rule == [16, 32, 32, 256], (E, hidden, inter, rule)
+
+
+def test_int4_expert_row_blocks_of_more_activations_than_32_row_blocks_take():
+    """The launches of 16- and 32-row blocks refuse activations of 1 GiB.  From 40 rows per expert on the rule gives such a call the tile
+    kernel's blocks, whatever its other lines say; below it never did."""
+    from ksanallm_amd import lib as L
+    rule = L.load().ksq_moe_w4a16_row_block
+    numel = 43 * 1024
+    most = 0x3fffffff // 2 // numel
+    assert L.load().ksq_moe_block_m(numel, 1024) == 32
+    for hidden, inter in ((1024, most), (most, 1024), (1024, most + 1), (most + 1, 1024)):
+        fits = max(hidden, inter) * numel * 2 < 1 << 30
+        assert rule(numel, 1024, hidden, inter) == (32 if fits else 256), (hidden, inter)
+    assert rule(39 * 1024, 1024, 1024, 2 * most) == 32 and rule(40 * 1024, 1024, 1024, 2 * most) == 256
