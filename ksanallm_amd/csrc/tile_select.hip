@@ -537,12 +537,19 @@ KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
 // end: 8, 4096, 14336 (896 workgroups) at 80, 100, 128 372 / 423, 435 / 511, 566 / 569, 8, 8192, 14336 702 / 794, 894 / 941, 1085 / 1065.
 // Where routing prefers some experts (logits with a spread of 0.7 per expert) 32-row blocks are ahead longer, up to a quarter.
 //
+// With hidden a multiple of 4096 and inter of 4096 and more the gate / up projection's strips share their HBM channels (w4a16_stream.h)
+// and the streaming kernel does not make up for half-empty blocks before 11 rows per expert.  Even routing, 16- / 32-row blocks at 7, 10,
+// 11, 13 rows: 128 experts, hidden 4096, inter 4096 525 / 577, 549 / 586, 566 / 591, 603 / 590 us; 64, 8192, 4096 529 / 592, 536 / 594,
+// 551 / 604, 602 / 618; 64, 4096, 14336 882 / 938, 913 / 951, 966 / 958, 1055 / 972; inter 2048, 128, 4096 291 / 296, 296 / 298.  (Uneven
+// as above: 471 / 460, 535 / 457, 599 / 511 for the first.)
+//
 // From 40 rows each on, activations of 1 GiB, which the launches of 16- and 32-row blocks refuse (32-bit offsets), run the tile kernel,
 // which takes 4 GiB.  (As many rows as slots: the second GEMM's, and the first one's behind a gather.)
 KSQ_EXPORT size_t ksq_moe_w4a16_row_block(size_t numel, size_t E, size_t hidden, size_t inter) {
   const size_t block_m = ksq_moe_block_m(numel, E);
   const size_t longest = hidden > inter ? hidden : inter;
   if (E != 0 && numel / E >= 40 && numel > 0x3fffffffull / 2 / (longest ? longest : 1)) return 256;
+  if (block_m == 32 && numel / E < 11 && hidden % 4096 == 0 && inter >= 4096) return 16;
   if (E != 0 && E <= 8 && numel / E >= 72 && E * div_up(2 * inter, 256) >= 4 * static_cast<size_t>(kNumCU)) return 256;
   return block_m;
 }

@@ -230,6 +230,11 @@ def test_int4_expert_row_blocks():
     for E, hidden, inter, line in ((8, 6144, 16384, 72), (8, 4096, 28672, 72), (8, 6144, 16256, 129), (4, 8192, 32768, 72), (4, 8192, 28672, 129)):
         rule = [lib.ksq_moe_w4a16_row_block(per * E, E, hidden, inter) for per in (15, 16, line - 1, line)]
         assert rule == [16, 32, 32, 256], (E, hidden, inter, rule)
+    # hidden a multiple of 4096 and inter from 4096 on: 32-row blocks from 11 rows on
+    for E, hidden, inter, line in ((128, 4096, 4096, 11), (32, 8192, 14336, 11), (128, 4096, 3968, 7), (128, 4224, 4096, 7), (32, 4096, 2048, 10),
+                                   (8, 4096, 14336, 16)):
+        rule = [lib.ksq_moe_w4a16_row_block(per * E + E // 2, E, hidden, inter) for per in (line - 1, line)]
+        assert rule == [16, 32], (E, hidden, inter, rule)
 
 
 def test_int4_expert_row_blocks_of_more_activations_than_32_row_blocks_take():
