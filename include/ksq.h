@@ -252,6 +252,8 @@ int ksq_w4a8_unpack_weight(const void* packed, void* dst, size_t n, size_t k, vo
 int ksq_w4a8_static_quant(const void* x, const void* scale, void* q, void* xsum, size_t m, size_t k, int mode,
                           int dtype, void* stream);
 size_t ksq_w4a8_workspace_size(size_t max_m, size_t n, size_t k);
+/* The kernel (KSQ_KERNEL_*, below) that such a GEMM runs with group 128: a pure host function. */
+int ksq_w4a8_kernel(size_t m, size_t n, size_t k);
 int ksq_w4a8_gemm(const void* a_q, const void* xsum, const void* w_packed, const void* scales, float alpha, void* out,
                   size_t m, size_t n, size_t k, size_t group, int out_dtype, void* workspace, size_t workspace_bytes,
                   void* stream);
@@ -408,8 +410,9 @@ enum { KSQ_KIND_W4A16 = 0, KSQ_KIND_FP8_BLOCKWISE = 1, KSQ_KIND_MOE_W4A16 = 2, K
 enum {
   KSQ_KERNEL_SPLITK_WAVE = 0,
   KSQ_KERNEL_MFMA_TILE = 1,
-  KSQ_KERNEL_STREAM_TILE = 2 /* block fp8: the MFMA tile kernel's grid, weights through registers (W4A8's form of it reports
-                                MFMA_TILE, whose grid and bits it has) */
+  KSQ_KERNEL_STREAM_TILE = 2 /* weights through registers: block fp8 on the MFMA tile kernel's grid; W4A8 and int4 experts where
+                                ksq_w4a8_kernel() and ksq_moe_w4a16_kernel() say so.  ksq_select_tile reports W4A8's as MFMA_TILE: with
+                                block_n 256 it has that kernel's grid and bits, with 128 a grid of its own over all of K */
 };
 
 typedef struct ksq_tile_desc {

@@ -402,12 +402,16 @@ TilePlan plan_w4a8_tile(size_t m, size_t n, size_t k) {
 // - ... and K that the plan cuts, where those workgroups come to three quarters of the CUs and K is not long, for no partial sums: 25600,
 //   5120 (200 workgroups) at 33 and 64 26.0 / 22.5 / 21.4, 26.0 / 25.6 / 25.0, n = 28672, k = 4096 (224) 21.5 / 20.7 / 18.2, 23.4 / 23.9 /
 //   20.9; but n = 20480, k = 8192 (160) at 64 29.0 / 29.1 / 36.0.
+// - From 97 tokens on not with parts of up to 16 k-blocks of a K whose strips, and its parts, lie whole numbers of 16 KiB apart and
+//   start on the same HBM channels: n = 4096, k = 16384 (parts of 8) at 80, 97, 112 level, 27.3 / 28.6, 27.9 / 29.3, n = 8192 (of 16) at
+//   116 and 128 35.5 / 37.5, 36.2 / 37.9, n = 4096, k = 32768 at 128 37.0 / 38.5; k = 12288, 16256, 20480 ahead or level.
 int w4a8_stream_strips(const TilePlan& plan, size_t m, size_t k) {
   if (plan.tiles_m != 1 || m <= 32 || m > 128) return 0;
   const unsigned narrow = 2 * plan.tiles_n;  // workgroups of 128 columns
   if (m <= 64 && narrow <= static_cast<unsigned>(kNumCU) && (plan.splits == 1 || (narrow >= static_cast<unsigned>(kNumCU) * 3 / 4 && k <= 6144)))
     return 1;
   const size_t kb = plan.splits == 1 ? k / 128 : plan.kt_per_split;
+  if (m > 96 && plan.splits > 1 && kb <= 16 && k % 16384 == 0) return 0;
   return kb >= (m <= 64 ? 20u : m > 112 ? 10u : 1u) ? 2 : 0;
 }
 
@@ -558,6 +562,11 @@ KSQ_EXPORT int ksq_moe_w4a16_kernel(size_t numel, size_t E, size_t n, size_t k, 
   if (block_m >= 128) return KSQ_KERNEL_MFMA_TILE;
   if (block_m == 0 || E == 0) return KSQ_KERNEL_SPLITK_WAVE;
   return use_w4a16_stream(block_m, grouped_row_blocks(numel, E, block_m), numel, E, n, k) ? KSQ_KERNEL_STREAM_TILE : KSQ_KERNEL_SPLITK_WAVE;
+}
+
+KSQ_EXPORT int ksq_w4a8_kernel(size_t m, size_t n, size_t k) {
+  if (n == 0 || k == 0 || !use_w4a8_tile(m, n, k)) return KSQ_KERNEL_SPLITK_WAVE;
+  return w4a8_stream_strips(plan_w4a8_tile(m, n, k), m, k) ? KSQ_KERNEL_STREAM_TILE : KSQ_KERNEL_MFMA_TILE;
 }
 
 KSQ_EXPORT int ksq_set_small_problem_rule(int enabled) { return g_small_problem_rule.exchange(enabled ? 1 : 0); }

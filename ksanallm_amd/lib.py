@@ -85,6 +85,7 @@ SIGNATURES = {
     "ksq_w4a8_unpack_weight": (c_i, [c_p, c_p, c_sz, c_sz, c_p]),
     "ksq_w4a8_static_quant": (c_i, [c_p, c_p, c_p, c_p, c_sz, c_sz, c_i, c_i, c_p]),
     "ksq_w4a8_workspace_size": (c_sz, [c_sz, c_sz, c_sz]),
+    "ksq_w4a8_kernel": (c_i, [c_sz, c_sz, c_sz]),
     "ksq_w4a8_gemm": (c_i, [c_p, c_p, c_p, c_p, ctypes.c_float, c_p, c_sz, c_sz, c_sz, c_sz, c_i, c_p, c_sz, c_p]),
     "ksq_select_tile": (c_i, [c_i, c_sz, c_sz, c_sz, c_i, ctypes.POINTER(TileDesc)]),
     "ksq_set_small_problem_rule": (c_i, [c_i]),

@@ -249,3 +249,24 @@ def test_int4_expert_row_blocks_of_more_activations_than_32_row_blocks_take():
         fits = max(hidden, inter) * numel * 2 < 1 << 30
         assert rule(numel, 1024, hidden, inter) == (32 if fits else 256), (hidden, inter)
     assert rule(39 * 1024, 1024, 1024, 2 * most) == 32 and rule(40 * 1024, 1024, 1024, 2 * most) == 256
+
+
+def test_w4a8_streaming_tile_kernel_serves_one_row_block():
+    """33 to 128 tokens: up to 64 in workgroups of 128 columns that are one round of the 256 CUs, or in 256 columns with parts of 20
+    k-blocks and more; above, parts of any length up to 112 tokens and of 10 up to 128, but for short parts of a K of 16384 and its
+    multiples from 97 tokens on."""
+    from ksanallm_amd import lib as L
+    lib = L.load()
+    stream, tile, decode = L.KERNEL_STREAM_TILE, L.KERNEL_MFMA_TILE, L.KERNEL_SPLITK_WAVE
+
+    def form(m, n, k):
+        d = L.select_tile(L.KIND_W4A8, m, n, k, L.BF16)
+        return lib.ksq_w4a8_kernel(m, n, k), d["block_n"], d["split_k"]
+    assert [form(m, 25600, 5120)[0] for m in (32, 33, 64, 65, 128, 129)] == [decode, stream, stream, stream, stream, tile]
+    assert [form(m, 25600, 5120)[1:] for m in (64, 65)] == [(128, 1), (256, 2)]
+    assert form(64, 32768, 1024) == (stream, 128, 1) and form(64, 32784, 1024) == (tile, 256, 1)      # 256 and 258 workgroups
+    assert form(64, 40960, 2432) == (tile, 256, 1) and form(64, 40960, 2560) == (stream, 256, 1)      # 19 and 20 k-blocks
+    assert form(64, 14336, 8192) == (tile, 256, 4) and form(64, 20480, 8192) == (stream, 256, 3)      # parts of 16 and of 22
+    assert [lib.ksq_w4a8_kernel(m, 4096, 16384) for m in (96, 97, 112)] == [stream, tile, tile]       # parts of 8
+    assert [lib.ksq_w4a8_kernel(m, 8192, 16384) for m in (96, 97, 128)] == [stream, tile, tile]       # of 16
+    assert [lib.ksq_w4a8_kernel(128, n, k) for n, k in ((12288, 16384), (8192, 16256))] == [stream, stream]
