@@ -470,6 +470,11 @@ KSQ_EXPORT int ksq_w4a8_static_quant(const void* x, const void* scale, void* q, 
   return check_launch(fn);
 }
 
+// what a call under that plan writes its fp32 partial tiles to (128 columns per workgroup over all of K: none)
+static size_t w4a8_workspace_bytes(const TilePlan& plan, size_t m, size_t k) {
+  return plan.splits > 1 && w4a8_stream_strips(plan, m, k) != 1 ? plan.workspace_bytes : 0;
+}
+
 KSQ_EXPORT size_t ksq_w4a8_workspace_size(size_t max_m, size_t n, size_t k) {
   if (n == 0 || k == 0 || k % 128 != 0) return 0;
   // only the split-K form of the tile kernel needs scratch (fp32 partial tiles); the plan is the same for
@@ -478,7 +483,8 @@ KSQ_EXPORT size_t ksq_w4a8_workspace_size(size_t max_m, size_t n, size_t k) {
   for (size_t band_end = 64; max_m > 32; band_end += band_end == 64 ? 64 : 128) {
     const size_t m = band_end < max_m ? band_end : max_m;
     const TilePlan t = plan_w4a8_tile(m, n, k);
-    need = t.workspace_bytes > need ? t.workspace_bytes : need;
+    const size_t bytes = w4a8_workspace_bytes(t, m, k);
+    need = bytes > need ? bytes : need;
     if (m == max_m) break;
   }
   return need;
@@ -528,11 +534,12 @@ KSQ_EXPORT int ksq_w4a8_gemm(const void* a_q, const void* xsum, const void* w_pa
     }
   } else if (use_w4a8_tile(m, n, k)) {
     const TilePlan plan = plan_w4a8_tile(m, n, k);
-    if (plan.splits > 1 && (!workspace || workspace_bytes < plan.workspace_bytes || !aligned16(workspace)))
+    const size_t need = w4a8_workspace_bytes(plan, m, k);
+    if (need > 0 && (!workspace || workspace_bytes < need || !aligned16(workspace)))
       return fail(KSQ_ERR_WORKSPACE, "%s: m=%zu n=%zu k=%zu needs %zu bytes of 16-byte aligned workspace, got %zu", fn, m,
-                  n, k, plan.workspace_bytes, workspace ? workspace_bytes : size_t(0));
+                  n, k, need, workspace ? workspace_bytes : size_t(0));
     if (256 * k > 0xffffffffull || 16 * (k / 128) * 1024 > 0xffffffffull) return fail(KSQ_ERR_INVALID_ARGUMENT, "%s: k too large", fn);
-    float* partial = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
+    float* partial = need > 0 ? static_cast<float*>(workspace) : nullptr;
     if (plan.block_m == 64)
       rc = out_dtype == KSQ_F16 ? launch_tile<F16, 2>(p, plan, partial, st) : launch_tile<BF16, 2>(p, plan, partial, st);
     else if (plan.block_m == 128)

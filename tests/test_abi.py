@@ -270,3 +270,16 @@ def test_w4a8_streaming_tile_kernel_serves_one_row_block():
     assert [lib.ksq_w4a8_kernel(m, 4096, 16384) for m in (96, 97, 112)] == [stream, tile, tile]       # parts of 8
     assert [lib.ksq_w4a8_kernel(m, 8192, 16384) for m in (96, 97, 128)] == [stream, tile, tile]       # of 16
     assert [lib.ksq_w4a8_kernel(128, n, k) for n, k in ((12288, 16384), (8192, 16256))] == [stream, stream]
+
+
+def test_w4a8_workspace_of_a_form_that_writes_none():
+    """Up to 64 tokens in workgroups of 128 columns over all of K, also where the plan cuts it: no partial tiles and no workspace; a
+    buffer sized for more tokens still covers every smaller call."""
+    from ksanallm_amd import lib as L
+    size = L.load().ksq_w4a8_workspace_size
+    for n, k in ((25600, 5120), (24336, 4736)):
+        assert L.select_tile(L.KIND_W4A8, 64, n, k, L.BF16)["block_n"] == 128 and L.select_tile(L.KIND_W4A8, 65, n, k, L.BF16)["split_k"] == 2
+        assert [size(m, n, k) for m in (1, 32, 33, 64)] == [0, 0, 0, 0], (n, k)
+        assert size(128, n, k) >= size(65, n, k) >= -(-n // 256) * 2 * 128 * 256 * 4
+    for m, n, k in ((33, 20480, 8192), (64, 14336, 8192)):          # K cut at 64 tokens and below
+        assert size(m, n, k) >= L.select_tile(L.KIND_W4A8, m, n, k, L.BF16)["grid"] * 128 * 256 * 4
