@@ -138,10 +138,11 @@ def test_gemm_tile_kernel(ops, oracle, tile_kernels, out_dtype, m, n, k):
     H.check_gemm(out, ref, out_dtype, "w4a8 tile m=%d n=%d k=%d" % (m, n, k))
 
 
-# 64- and 128-token tiles keep four and three k-blocks of loads in flight: fewer k-blocks than that, as many, one more; parts of
-# K (`parts`: k-blocks of a part, and of the last one) of one to five k-blocks on the 128-token tile and of 18 to 33, even and
-# odd, on the 64-token tile, which takes parts of 32 and more; and every count of row tiles that hold tokens, with M % 4 == 0 and
-# without
+# Row blocks of 33 to 128 tokens at K whole and cut, with every count of row tiles that hold tokens, with M % 4 == 0 and without.
+# `parts`: k-blocks of a part of K, and of the last one.  What runs them: the first six the streaming kernel in workgroups of 128
+# columns, parts of 18 to 33 k-blocks and 65 to 112 tokens the streaming kernel in 256 columns, the other short parts and 113 to 128
+# tokens the 128-token tile kernel, which keeps three k-blocks of loads in flight: as many k-blocks, fewer and more.  (The 64-token tile
+# kernel: test_gemm_tile_kernel_of_64_tokens.)
 @pytest.mark.parametrize("m,n,k,parts", [
     (33, 272, 128, None), (48, 4112, 512, None), (49, 256, 640, None), (63, 528, 768, None), (64, 256, 896, None), (64, 272, 1152, None),
     (65, 272, 256, None), (96, 256, 384, None), (127, 528, 512, None), (128, 256, 640, None),
@@ -153,6 +154,8 @@ def test_gemm_tile_kernel_few_tokens(ops, oracle, tile_kernels, m, n, k, parts):
     desc = L.select_tile(L.KIND_W4A8, m, n, k, H.BF16)
     kb, cut = k // 128, desc["split_k"]
     per = -(-kb // cut)
+    streams = m <= 64 and (cut == 1 or per >= 20) or 64 < m <= 112
+    assert L.load().ksq_w4a8_kernel(m, n, k) == (L.KERNEL_STREAM_TILE if streams else L.KERNEL_MFMA_TILE)
     assert desc["block_m"] == (64 if m <= 64 and (cut == 1 or per >= 32) else 128)
     assert (cut == 1) if parts is None else (cut > 1 and (per, kb - (cut - 1) * per) == parts)
     w, scales = make_weight(n + k + m, k, n)
@@ -180,6 +183,42 @@ def test_gemm_streaming_tile_over_its_rings(ops, oracle, tile_kernels, m, n, k, 
     out = ops.w4a8_gemm(xq, xsum, ops.w4a8_repack_weight(w.cuda()), scales.cuda(), 0.03, n, torch.float16)
     ref = oracle.w4a8_gemm(xq.cpu().numpy(), w.numpy().view(np.int8), H.bits_of(scales), 0.03)
     H.check_gemm(out, ref, H.F16, "w4a8 streaming tile m=%d n=%d k=%d" % (m, n, k))
+
+
+@pytest.mark.parametrize("m,k", [(33, 128), (64, 256), (48, 384), (49, 512), (64, 640), (61, 768), (33, 1152), (64, 2432)])
+def test_gemm_tile_kernel_of_64_tokens(ops, oracle, tile_kernels, m, k):
+    """More than 256 workgroups of 128 columns and fewer than 20 k-blocks: the MFMA tile kernel of 64 tokens, which keeps four k-blocks of
+    loads in flight and takes two to a barrier - fewer k-blocks, as many, odd and even numbers, three and four row tiles, and a last
+    column tile of one strip."""
+    from ksanallm_amd import lib as L
+    n = 32784
+    desc = L.select_tile(L.KIND_W4A8, m, n, k, H.F16)
+    assert L.load().ksq_w4a8_kernel(m, n, k) == L.KERNEL_MFMA_TILE and (desc["block_m"], desc["block_n"], desc["split_k"]) == (64, 256, 1)
+    _check_w4a8(ops, oracle, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k,parts", [
+    (33, 272, 39424, (20, 8)), (64, 272, 41472, (21, 9)), (49, 272, 42496, (21, 17)),   # partial tiles of 128 rows, a short last part
+    (50, 32784, 2560, None), (64, 32784, 2688, None)])                                  # K whole, 20 and 21 k-blocks
+def test_gemm_streaming_tile_of_256_columns_up_to_64_tokens(ops, oracle, tile_kernels, m, n, k, parts):
+    """The weight ring of eight k-blocks: parts of 20 k-blocks and a few more, and a last part of as many as the ring, one more and two
+    turns and one."""
+    from ksanallm_amd import lib as L
+    desc = L.select_tile(L.KIND_W4A8, m, n, k, H.F16)
+    assert L.load().ksq_w4a8_kernel(m, n, k) == L.KERNEL_STREAM_TILE and desc["block_n"] == 256
+    kb, cut = k // 128, desc["split_k"]
+    per = -(-kb // cut)
+    assert (cut == 1 and desc["block_m"] == 64) if parts is None else (cut > 1 and desc["block_m"] == 128 and (per, kb - (cut - 1) * per) == parts)
+    _check_w4a8(ops, oracle, m, n, k)
+
+
+def _check_w4a8(ops, oracle, m, n, k):
+    w, scales = make_weight(n + k + m, k, n)
+    x = make_act(m * 7 + n, m, k, H.F16)
+    xq, xsum = ops.w4a8_static_quant(x.cuda(), torch.tensor([0.05], dtype=torch.float32).cuda(), False)
+    out = ops.w4a8_gemm(xq, xsum, ops.w4a8_repack_weight(w.cuda()), scales.cuda(), 0.03, n, torch.float16)
+    ref = oracle.w4a8_gemm(xq.cpu().numpy(), w.numpy().view(np.int8), H.bits_of(scales), 0.03)
+    H.check_gemm(out, ref, H.F16, "w4a8 m=%d n=%d k=%d" % (m, n, k))
 
 
 @pytest.mark.parametrize("m,n,k", [(3, 8192, 512), (20, 8192, 512), (16, 16384, 256), (32, 16384, 256), (1, 4096, 1024)])
