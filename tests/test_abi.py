@@ -283,3 +283,21 @@ def test_w4a8_workspace_of_a_form_that_writes_none():
         assert size(128, n, k) >= size(65, n, k) >= -(-n // 256) * 2 * 128 * 256 * 4
     for m, n, k in ((33, 20480, 8192), (64, 14336, 8192)):          # K cut at 64 tokens and below
         assert size(m, n, k) >= L.select_tile(L.KIND_W4A8, m, n, k, L.BF16)["grid"] * 128 * 256 * 4
+
+
+def test_block_fp8_decode_strips():
+    """Up to 32 rows: one strip of 16 columns per workgroup up to 256 strips; above, two with more than 8 rows or a K longer than n, else by
+    rows in one round of the CUs and by how full the last round is in several.  Above 32 rows in row blocks: four where every other CU
+    still gets a workgroup.  Always as many as divide n."""
+    from ksanallm_amd import lib as L
+
+    def strips(m, n, k):
+        d = L.select_tile(L.KIND_FP8_BLOCKWISE, m, n, k, L.BF16)
+        assert d["kernel"] == L.KERNEL_SPLITK_WAVE and d["grid"] == n // d["block_n"] * -(-m // 32)
+        return d["block_n"] // 16
+    assert [strips(m, 4096, 14336) for m in (1, 8, 16, 32)] == [1, 1, 1, 1]
+    assert [strips(m, 4128, 14336) for m in (1, 8, 16, 32)] == [2, 2, 2, 2] and strips(16, 4112, 4096) == 1      # (257 strips)
+    assert [strips(m, 8192, 4096) for m in (1, 4, 5, 8, 9, 32)] == [1, 1, 2, 2, 2, 2]                            # one round of pairs
+    assert [strips(8, n, 4096) for n in (12800, 13088, 13120, 16384)] == [1, 1, 2, 2]                            # 409 and 410 of 512
+    assert [strips(8, n, 1536) for n in (18432, 22112, 22144, 24576)] == [1, 1, 2, 2]                            # 691 and 692 of 768
+    assert [strips(33, n, 4096) for n in (2048, 4096)] == [2, 4]

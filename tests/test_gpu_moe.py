@@ -366,6 +366,32 @@ def test_grouped_streaming_kernel_that_goes_round_k(ops, oracle, dtype, kt):
     assert torch.equal(one.view(torch.int16), ops.silu_and_mul(out).view(torch.int16))
 
 
+@pytest.mark.parametrize("kt", [3, 32])
+def test_grouped_streaming_kernel_with_ids_outside_the_experts(ops, oracle, kt):
+    """Slots whose id is no expert are in no block: their output rows stay as they were, the others are the oracle's - rows shared by
+    the two slots of a token, and an expert that no slot takes."""
+    from ksanallm_amd import lib as L
+    E, T, topk, k, inter, dtype = 12, 300, 2, 128 * kt, 1312, H.BF16
+    assert L.load().ksq_moe_w4a16_kernel(T * topk, E, 2 * inter, k, 32) == L.KERNEL_STREAM_TILE
+    d = make_moe(oracle, 6300 + kt, E, k, inter, T, topk, 128, dtype)
+    g = H.gen(80 + kt)
+    ids = torch.randint(0, E - 1, (T, topk), generator=g, dtype=torch.int32)
+    outside = torch.rand((T, topk), generator=g) < 0.2
+    ids[outside] = torch.tensor([-1, E, E + 5, 1 << 30], dtype=torch.int32)[torch.randint(0, 4, (int(outside.sum()),), generator=g)]
+    w13p = ops.repack_weight(d["w13"].cuda(), L.SRC_MOE_NK, E, k, 2 * inter)
+    s13p = ops.repack_scales(d["s13"].cuda(), L.SCALE_NG, E, k, 2 * inter, 128)
+    al = ops.moe_align_block_size(ids.cuda(), E, 32)
+    out = torch.full((T * topk, 2 * inter), float("nan"), dtype=d["x"].dtype, device="cuda")
+    ops.moe_w4a16_gemm(d["x"].cuda(), w13p, s13p, d["tw"].cuda().reshape(-1), *al, T * topk, topk, E, 2 * inter, k, 128, 32, out=out)
+    one = torch.full((T * topk, inter), float("nan"), dtype=d["x"].dtype, device="cuda")
+    ops.moe_w4a16_gate_up_silu(d["x"].cuda(), w13p, s13p, *al, T * topk, topk, E, 2 * inter, k, 128, 32, out=one)
+    valid = ~outside.reshape(-1)
+    assert torch.isnan(out.cpu()[~valid]).all() and torch.isnan(one.cpu()[~valid]).all() and torch.isfinite(one.cpu()[valid]).all()
+    ref = oracle.moe_w4a16_gemm(H.bits_of(d["x"]), d["w13"].numpy(), H.bits_of(d["s13"]), ids.masked_fill(outside, 0).numpy(),
+                                d["tw"].numpy(), topk, 128, True, dtype)
+    H.check_gemm(out.cpu()[valid], ref[valid.numpy()], dtype, "streaming kernel, ids outside the experts")
+
+
 @pytest.mark.parametrize("T", [1, 64, 2048])
 def test_moe_block_deepseek_shape(ops, oracle, T):
     """256 experts, hidden 7168, inter 2048, top-8; weights for all experts are generated but only touched ones
@@ -422,6 +448,33 @@ def test_moe_block_benchmark_token_counts(ops, oracle, T):
                                  128, H.BF16)
         H.check_gemm(out[sel], oracle.from_bits(ref, H.BF16), H.BF16, "moe block T=%d tokens %s" % (T, sel),
                      weights_rounded=rounded, rel_l2_max=5e-3 * (2 ** 0.5 if rounded else 1.0))
+
+
+def test_moe_block_deepseek_shape_through_the_streaming_kernel(ops, oracle):
+    """The block above at 512 tokens, 16 slots per expert: both GEMMs in 32-slot blocks of the streaming kernel, as the rule has it, and the
+    same block in 16-slot blocks of the decode kernel.  Shares of experts and their sum are rounded to T, and one that falls the other way
+    moves an output by a unit of its last place whatever the kernel (0.03 from 4 on), so the bounds are the relative ones."""
+    from ksanallm_amd import lib as L
+    E, hidden, inter, topk, T = 256, 7168, 2048, 8, 512
+    lib = L.load()
+    assert lib.ksq_moe_w4a16_row_block(T * topk, E, hidden, inter) == 32
+    for n, k in ((2 * inter, hidden), (hidden, inter)):
+        assert [lib.ksq_moe_w4a16_kernel(T * topk, E, n, k, bm) for bm in (16, 32)] == [L.KERNEL_SPLITK_WAVE, L.KERNEL_STREAM_TILE]
+    base = make_moe(oracle, 5200 + T, 8, hidden, inter, T, topk, 128, H.BF16)
+    d = dict(base)
+    d["E"] = E
+    for k in ("w13", "w2", "s13", "s2"):
+        d[k] = base[k].repeat((E // 8, 1, 1))
+    tw, ids = torch.topk(torch.softmax(torch.randn((T, E), generator=H.gen(78 + T)), -1), topk, dim=-1)
+    d["ids"], d["tw"] = ids.to(torch.int32), tw.float().contiguous()
+    packed = pack_moe(ops, d)
+    outs = [ops.fused_moe_w4a16(d["x"].cuda(), *packed, d["ids"].cuda(), d["tw"].cuda(), E, hidden, inter, 128, bm) for bm in (None, 16)]
+    for sel in (slice(0, 8), slice(T - 4, T)):
+        ref = oracle.moe_forward(H.bits_of(d["x"][sel]), d["w13"].numpy(), H.bits_of(d["s13"]), d["w2"].numpy(),
+                                 H.bits_of(d["s2"]), d["ids"][sel].contiguous().numpy(), d["tw"][sel].contiguous().numpy(),
+                                 128, H.BF16)
+        for out in outs:
+            H.check_gemm(out[sel], oracle.from_bits(ref, H.BF16), H.BF16, "moe block T=%d tokens %s" % (T, sel), weights_rounded=True)
 
 
 @pytest.mark.parametrize("dtype", [H.F16, H.BF16])
