@@ -511,15 +511,22 @@ KSQ_EXPORT size_t ksq_moe_fp8_row_block(size_t numel, size_t E, size_t hidden, s
 // 16- or 32-row block (HBM-bound); above, the MFMA tile kernel takes 256-row blocks, of which it multiplies the row
 // tiles that hold rows (an instance of its main loop per count), so that an expert's weights are dequantized once
 // however many of the 256 rows it fills.  Few experts make few 256-row workgroups: the line lies the higher, the fewer there
-// are.  Whole block, time in 32-row blocks over time in 256-row blocks at 48 / 64 / 80 / 100 / 128 rows per expert (hidden, inter):
-//   8 experts   7168, 2048 0.79 0.99 0.79 0.82 0.90   2048, 1408 0.72 0.73 0.77 0.79 0.80   6144, 640 0.61 0.59 0.60 0.69 0.68
-//   16          7168, 2048 0.69 0.75 0.80 0.86 0.90   2048, 1408 0.92 0.99 1.06 1.03 1.13   6144, 640 0.72 0.73 0.73 0.94 0.92
-//   32          7168, 2048 0.80 0.84 0.92 1.06 1.11   2048, 1408 0.92 1.04 1.13 1.14 1.16   6144, 640 0.92 0.95 0.97 1.22 1.20
-//   64          4096, 1536 0.84 0.94 1.06 1.25 1.31   2048, 1408 0.86 0.92 1.02 1.09 1.31   1024, 512 1.09 1.19 1.17 1.18 1.19
-//   256         7168, 2048 0.65 at 32, 0.87 at 40, 1.10 at 64, 1.28 at 94
+// are.  Whole block, time in 32-row blocks over time in 256-row blocks at 48 / 64 / 80 / 100 / 128 rows per expert (hidden, inter), where
+// routing prefers no expert and, in brackets, where it prefers some (logits with a spread of 0.7 per expert):
+//   8 experts   7168, 2048 0.74 0.96 0.78 0.81 0.89 (0.81 0.67 0.71 0.63 0.68)   4096, 4096 0.75 at 60, 0.77 at 84, 0.78 at 105, 0.90
+//   16          7168, 2048 0.66 0.71 0.71 0.80 0.77 (0.63 0.71 0.70 0.64 0.76)   2048, 1408 0.86 0.94 0.92 1.02 1.16 (0.78 0.67 0.73 0.71 0.87)
+//   32          7168, 2048 0.68 0.74 0.80 0.99 1.00 (0.67 0.72 0.75 0.81 0.86)   2048, 1408 0.85 0.99 1.08 1.14 1.15 (0.62 0.73 0.85 0.84 0.80)
+//   64          4096, 1536 0.80 0.86 0.95 1.21 1.27 (0.63 0.68 0.75 0.82 0.84)   1024, 512  1.16 1.14 1.16 1.19 1.22 (0.69 0.78 0.63 0.67 0.76)
+//   128         4096, 1536 0.92 1.02 1.08 1.23 1.29 (0.70 0.83 0.87 0.96 0.99)   2048, 768  0.94 1.04 1.15 1.27 1.29 (0.67 0.81 0.81 0.77 0.91)
+//   256         4096, 2048 0.89 at 50, 0.99 1.11 (0.75 at 50, 0.82 0.97)
+// With 9 experts and more a line lies where the first of the sizes that were timed with so many nears its crossing without
+// preferences, so that none is behind; larger ones would bear a higher line (7168, 2048 with 16 experts 0.77 at 128 rows, with 32 0.80 at
+// 80; 4096, 1536 with 64 0.86 at 64), and uneven routing nearly all.  Up to 8 it lies at the end of what was timed: 0.6 to 1.0 before it,
+// but for hidden 4480 with inter 6144 to 12032 from 105 rows on, 1.01-1.12 (0.82-0.91), and the sizes that
+// ksq_moe_w4a16_row_block takes out.
 // 16- and 32-row blocks: half-empty blocks of 32 run one row tile of the streaming kernel, which keeps more in flight than the
-// decode kernel over 16-row blocks, and an expert with more than 16 rows reads its weights once.  Time in 32-row blocks over time in
-// 16-row blocks at 3 / 5 / 7 / 9 / 11 / 13 / 15 rows per expert:
+// decode kernel over 16-row blocks, and an expert with more than 16 rows reads its weights once (under uneven routing 32-row blocks are
+// ahead sooner, by 5 to 15 %).  Time in 32-row blocks over time in 16-row blocks, no preferences, at 3 / 5 / 7 / 9 / 11 / 13 / 15 rows per expert:
 //   16 experts  4096, 1536 1.01 1.02 0.99 1.00 1.01 0.99 0.99   4096, 768 1.12 1.14 1.12 1.15 1.13 1.08 1.02
 //   32          7168, 2048 1.06 1.05 1.06 1.01 0.98 0.95 0.89   1024, 512 1.30 1.23 1.07 0.99 1.01 0.98 0.96
 //   64          4096, 1536 0.98 0.99 0.99 1.01 0.94 0.92 0.89   7168, 2048 1.05 1.05 1.03 1.03 0.99 0.96 0.88

@@ -3,8 +3,10 @@
 //
 //   - every weight tile belongs to one wavefront (two strips of 16 columns each), which loads it straight into a register ring
 //     of four k-tiles: 64 KiB in flight per workgroup, two workgroups to a CU.  Non-temporally, for a weight is read once,
-//     unless its expert has several blocks, which run at the same time and share the L2's copy (256 experts, hidden 7168, inter
-//     2048, 32 slots each 1.62 -> 1.54 ms).
+//     unless its expert has several blocks, which run at the same time and share a cached copy: the L2's where the columns are a
+//     multiple of eight workgroups (the same columns of the next block are then on the same XCD), the Infinity Cache's otherwise.
+//     32 / 48 slots each, non-temporal / cached, us: 256 experts, n = 4096, k = 7168 (16 column workgroups) 1002 / 942, 1410 / 1273, n =
+//     7168, k = 2048 (28) 569 / 526, 777 / 707; 64, n = k = 5120 (20) 250 / 226, 352 / 305; n = 3072, k = 4096 (12) 125 / 125, 173 / 168.
 //   - x goes global -> LDS (global_load_lds_dwordx4) by halves of two k-tiles, three halves ahead; all wavefronts read it from
 //     there.  A strip's scales of a half are 64 contiguous bytes and come the same way, one load for a wavefront's strips.
 //   - the sums of x that make up for the codes' offset are taken once per workgroup, a half ahead, and handed round through
@@ -13,7 +15,8 @@
 //     the ring in flight, also across the one barrier per half.
 // The decode kernel (w4a16_splitk.h), four wavefronts that divide K among them, keeps 64 KiB per CU in flight at best, waits for
 // more of it than it needs (the compiler's counts do not know the staging loads) and fetches x twice as often.  512 tokens,
-// 256 experts, hidden 7168, inter 2048, bf16: first GEMM 663 -> 618 us (6.3 TB/s), second 415 -> 362 us, whole block 1140 -> 1066;
+// 256 experts, hidden 7168, inter 2048, bf16, GEMMs alone: the first 663 -> 618 us (6.3 TB/s), the second 415 -> 362 us, whole block 1140 ->
+// 1066 (single launches behind a write of 600 MiB, in one session: 841 -> 816 and 475 -> 420);
 // with weights out of the L2 484 -> 400 and 326 -> 222 (one row tile), 634 -> 562 and 417 -> 326 (two): what the SIMDs take to
 // issue it, about 1.4 times the unpacking (28 instructions a tile), scaling and MFMAs added up.  Measured against it and not
 // kept: four strips to a wavefront and four wavefronts, 594 / 369 us; eight of those, one workgroup to a CU, 603 / 388; two
@@ -82,7 +85,7 @@ __global__ void __launch_bounds__(512, 4) w4a16_stream_tile_kernel(SplitKParams 
   const uint32_t w_voff = lane * 16;
   const char* const x_base = static_cast<const char*>(p.x);
 
-  // An expert with several blocks: they run side by side and share the caches' copy of the weights.
+  // an expert with several blocks (they run side by side and share a cached copy of the weights)
   const bool several = (pos0 + kW4StreamRows < slots && static_cast<uint32_t>(p.expert_ids[blockIdx.y + 1]) == e) ||
                        (blockIdx.y > 0 && static_cast<uint32_t>(p.expert_ids[blockIdx.y - 1]) == e);
   // A strip is K / 128 KiB, so where K is a multiple of 4096 the strips of all workgroups start on the same HBM channels, where it is

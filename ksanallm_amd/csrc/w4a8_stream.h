@@ -1,5 +1,6 @@
-// W4A8 kernel for one row block of 33 to 128 tokens, under the tile kernel's plan (w4a8_tile.h) and with its bits: a workgroup of
-// eight wavefronts side by side along N computes up to 128 tokens x 128 * NS columns over a range of 128-deep k-blocks.
+// W4A8 kernel for one row block of 33 to 128 tokens: a workgroup of eight wavefronts side by side along N computes up to 128 tokens x
+// 128 * NS columns over a range of 128-deep k-blocks.  NS = 2 runs under the tile kernel's plan (w4a8_tile.h) and with its bits; NS = 1, up
+// to 64 tokens, has workgroups of 128 columns over all of K, whatever that plan cuts, and so its own grid and one order of the sums.
 //
 //   - weights and their scales go straight into a register ring of D k-blocks, each fragment to the one wavefront that
 //     multiplies it (NS strips of 16 columns each); activations (whole 128-byte lines) and group sums go global -> LDS into D
@@ -7,11 +8,13 @@
 //     few ring lengths, and non-temporal loads come back later (n = 25600, k = 5120 at 40 and 64 tokens 27.1 / 30.1 us, cached
 //     22.5 / 25.6).
 //   - all loads are issued from inline assembly in a fixed order, so every wait has a constant count.
-//   - NS = 1: 128 columns per workgroup over all of K, for a single round of workgroups: no partial sums, no second launch.
-// What bounds it: a launch and a reduction (about 7 us of the 25 at n = 25600, k = 5120, 64 tokens), the ramp, and per k-block the
-// chain of LDS reads, code expansion, MFMAs and scale FMAs, 2.5 us per row tile over 20 k-blocks, in two wavefronts per SIMD.  The
-// tile kernel pays for all eight row tiles of its 128-token form in two of four wavefronts' time.  80 tokens 33.4 -> 27.9 us, 33
-// tokens 26.0 -> 22.5.  Fragments read four ahead instead of two: 26.9 us at 64 tokens (25.6); the group sums read behind the
+//   - NS = 1 is for a single round of workgroups: no partial sums, no workspace, no second launch.
+// What bounds it: a launch, the ramp, and per k-block the chain of LDS reads, code expansion, MFMAs and scale FMAs in two wavefronts per
+// SIMD; with NS = 2 also the pass over the partial sums where the plan cuts K, 4.4 us behind the kernel.  n = 25600, k = 5120 at 64 tokens,
+// which takes NS = 1 (40 k-blocks on 200 CUs): 25.6 us as NS = 2 (20 k-blocks, reduction included), 25.0 as NS = 1; single launches behind a
+// write of 600 MiB 34.5 + 4.4 (tile kernel and reduction) -> 33.4.  As NS = 2 a row tile more costs 2.5 us over 20 k-blocks; the tile kernel
+// pays for all eight row tiles of its 128-token form in two of four wavefronts' time.  80 tokens (NS = 2) 33.4 -> 27.9 us, 33 tokens 26.0 ->
+// 22.5, as NS = 1 21.4.  Of NS = 2 at 64 tokens: fragments read four ahead instead of two 26.9 us (25.6); the group sums read behind the
 // first fragments instead of in front of them 25.6 -> 26.
 #pragma once
 
