@@ -174,7 +174,7 @@ bool use_w4a16_stream(size_t block_m, size_t blocks, size_t numel, size_t E, siz
   if (n * k > (size_t(1) << 36)) return false;  // 32-bit offsets into an expert's scales
   if (n % 128 == 0 && k >= 4096 && blocks * tiles < 2 * static_cast<size_t>(kNumCU)) {
     const double wgs = expected_row_blocks(numel, E, block_m) * static_cast<double>(tiles);
-    if (wgs > kNumCU * 1.03 && wgs <= kNumCU * 1.25) return false;  // (a few more than expected are no round)
+    if (wgs > kNumCU * 1.03 && wgs <= kNumCU * 1.25) return false;  // (a handful more than 256 make no second round)
   }
   return true;
 }
@@ -546,7 +546,8 @@ KSQ_EXPORT size_t ksq_moe_block_m(size_t numel, size_t E) {
 // 573, 693 / 600, 762 / 752, 950 / 849; 8, 8192, 28672 1346 / 1443, 1421 / 1470, 1478 / 1501, 1646 / 1574, 1828 / 1640, 2231 / 1875; 8,
 // 4096, 28672 712 / 766, 739 / 801, 767 / 813, 845 / 846, 927 / 875, 1165 / 982.  With fewer 32-row blocks are ahead, or level at the
 // end: 8, 4096, 14336 (896 workgroups) at 80, 100, 128 372 / 423, 435 / 511, 566 / 569, 8, 8192, 14336 702 / 794, 894 / 941, 1085 / 1065.
-// Where routing prefers some experts (logits with a spread of 0.7 per expert) 32-row blocks are ahead longer, up to a quarter.
+// Where routing prefers some experts (logits with a spread of 0.7 per expert) 32-row blocks are ahead longer, up to a quarter.  (The tile
+// kernel rounds dequantized weights to T, where 16- and 32-row blocks keep them exact: 2.2e-3 and 1.7e-3 off in bf16.)
 //
 // With hidden a multiple of 4096 and inter of 4096 and more the gate / up projection's strips share their HBM channels (w4a16_stream.h)
 // and the streaming kernel does not make up for half-empty blocks before 11 rows per expert.  Even routing, 16- / 32-row blocks at 7, 10,
